@@ -26,6 +26,7 @@
 #include <mutex>
 
 #include "rk_device.h"
+#include "rk_face_bounds.h"
 
 namespace {
 
@@ -134,19 +135,47 @@ __device__ __forceinline__ void tri_setup(const uint4* __restrict__ faces, const
 // A face's tri_setup terms, v0, e1 = v1 - v0 and e2 = v2 - v0 (w 0),
 // precomputed per call in face order (nine floats, 36 B per face): one
 // contiguous load per face test instead of the face's indices, then its
-// vertices.
+// vertices. And the bound of each kFaceGroup faces (rk_face_bounds.h), 2 B per
+// face: 16 lanes share a group, reduced by shuffles.
 constexpr size_t kRecFloats = 9;
+constexpr uint32_t kGroup = rk::kFaceGroup;
+static_assert(kGroup == 16, "a group is a quarter of a wave");
 __global__ __launch_bounds__(256) void k_tri_records(const uint4* __restrict__ faces,
                                                      const float4* __restrict__ verts, uint32_t face_count,
-                                                     float* __restrict__ tris) {
+                                                     float* __restrict__ tris, rk::FaceBound* __restrict__ bounds) {
   const uint32_t f = blockIdx.x * 256 + threadIdx.x;
-  if (f >= face_count) return;
-  float4 v0, e1, e2;
-  tri_setup(faces, verts, f, v0, e1, e2);
-  float3* r = reinterpret_cast<float3*>(tris + kRecFloats * (size_t)f);
-  r[0] = make_float3(v0.x, v0.y, v0.z);
-  r[1] = make_float3(e1.x, e1.y, e1.z);
-  r[2] = make_float3(e2.x, e2.y, e2.z);
+  const bool in = f < face_count;
+  float lo[3], hi[3], e2m = 0.0f, nan = 0.0f;
+  for (int q = 0; q < 3; ++q) { lo[q] = RK_HUGE; hi[q] = -RK_HUGE; }
+  if (in) {
+    const uint4 face = faces[f];
+    const float4 a = verts[face.x], b = verts[face.y], c = verts[face.z];
+    const float4 e1 = rk::sub4(b, a), e2 = rk::sub4(c, a);
+    float3* r = reinterpret_cast<float3*>(tris + kRecFloats * (size_t)f);
+    r[0] = make_float3(a.x, a.y, a.z);
+    r[1] = make_float3(e1.x, e1.y, e1.z);
+    r[2] = make_float3(e2.x, e2.y, e2.z);
+    lo[0] = fminf(fminf(a.x, b.x), c.x); hi[0] = fmaxf(fmaxf(a.x, b.x), c.x);
+    lo[1] = fminf(fminf(a.y, b.y), c.y); hi[1] = fmaxf(fmaxf(a.y, b.y), c.y);
+    lo[2] = fminf(fminf(a.z, b.z), c.z); hi[2] = fmaxf(fmaxf(a.z, b.z), c.z);
+    const float l1 = e1.x * e1.x + e1.y * e1.y + e1.z * e1.z, l2 = e2.x * e2.x + e2.y * e2.y + e2.z * e2.z;
+    e2m = fmaxf(l1, l2);
+    nan = l1 + l2;  // NaN or infinite when a vertex is (fminf and fmaxf drop NaN)
+  }
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1) {
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      lo[q] = fminf(lo[q], __shfl_xor(lo[q], off, 16));
+      hi[q] = fmaxf(hi[q], __shfl_xor(hi[q], off, 16));
+    }
+    e2m = fmaxf(e2m, __shfl_xor(e2m, off, 16));
+    nan += __shfl_xor(nan, off, 16);
+  }
+  if (in && f % kGroup == 0) {
+    const float e = (nan == nan) ? 1.00001f * e2m : nan;
+    bounds[f / kGroup] = rk::face_bound(lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], e);
+  }
 }
 
 // One of a record's three vectors, w 0 as tri_setup leaves it.
@@ -155,17 +184,80 @@ __device__ __forceinline__ float4 rec_vec(const float* __restrict__ r) {
   return make_float4(v.x, v.y, v.z, 0.0f);
 }
 
+// The call's faces: the mesh, and the records and bounds k_tri_records wrote
+// (both NULL when there was no memory for them).
+struct RefMesh {
+  const uint4* faces;
+  const float4* verts;
+  const float* tris;
+  const rk::FaceBound* bounds;
+};
+
 // tri_setup from the records when the call has them, else from the mesh.
-__device__ __forceinline__ void tri_get(const uint4* __restrict__ faces, const float4* __restrict__ verts,
-                                        const float* __restrict__ tris, uint32_t f, float4& v0, float4& e1,
-                                        float4& e2) {
-  if (tris) {
-    const float* r = tris + kRecFloats * (size_t)f;
+__device__ __forceinline__ void tri_get(const RefMesh& m, uint32_t f, float4& v0, float4& e1, float4& e2) {
+  if (m.tris) {
+    const float* r = m.tris + kRecFloats * (size_t)f;
     v0 = rec_vec(r);
     e1 = rec_vec(r + 3);
     e2 = rec_vec(r + 6);
   } else {
-    tri_setup(faces, verts, f, v0, e1, e2);
+    tri_setup(m.faces, m.verts, f, v0, e1, e2);
+  }
+}
+
+__device__ __forceinline__ rk::CullRay cull_ray4(float4 o, float4 d) {
+  return rk::cull_ray(o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w);
+}
+
+// Which of the groups g0 .. g0 + ng - 1 (ng <= 32) may hold a face the ray's
+// part [0, depth] hits: bit j for group g0 + j. Every group without bounds.
+__device__ __forceinline__ uint32_t groups_near(const rk::FaceBound* __restrict__ bounds, uint32_t g0, uint32_t ng,
+                                                float4 o, float4 d, const rk::CullRay& cr, float depth) {
+  if (!bounds) return ng >= 32u ? 0xFFFFFFFFu : (1u << ng) - 1u;
+  uint32_t mask = 0u;
+  for (uint32_t j = 0; j < ng; j += 2) {  // two bounds in flight
+    const rk::FaceBound b0 = bounds[g0 + j], b1 = bounds[g0 + min(j + 1u, ng - 1u)];
+    if (!rk::bound_missed(b0, o.x, o.y, o.z, d.x, d.y, d.z, cr, depth)) mask |= 1u << j;
+    if (j + 1u < ng && !rk::bound_missed(b1, o.x, o.y, o.z, d.x, d.y, d.z, cr, depth)) mask |= 2u << j;
+  }
+  return mask;
+}
+
+// One lane's pass over faces [first, first + cnt) in face order, keeping a hit
+// when t < depth: (depth, fid, uv) as a sequential pass over all of them ends.
+// Faces of groups the ray misses are skipped; the lanes of a wave step through
+// the faces left to each, so the pass lasts as long as the most any lane has.
+#ifndef RK_REF_LEAF_BATCH
+#define RK_REF_LEAF_BATCH 2
+#endif
+constexpr uint32_t kLeafBatch = RK_REF_LEAF_BATCH;
+__device__ __forceinline__ void lane_leaf(const RefMesh& mesh, uint32_t first, uint32_t cnt, float4 o, float4 d,
+                                          const rk::CullRay& cr, float& depth, uint32_t& fid, float2& coord) {
+  if (cnt == 0u) return;
+  const uint32_t end = first + cnt, g_end = (end - 1u) / kGroup + 1u;
+  for (uint32_t g0 = first / kGroup; g0 < g_end; g0 += 32u) {
+    uint32_t mask = groups_near(mesh.bounds, g0, min(32u, g_end - g0), o, d, cr, depth);
+    uint32_t f = 0u, stop = 0u;
+    for (;;) {
+      if (f >= stop) {
+        if (mask == 0u) break;
+        const uint32_t g = (g0 + (uint32_t)__builtin_ctz(mask)) * kGroup;
+        mask &= mask - 1u;
+        f = max(first, g);
+        stop = g + min(end - g, kGroup);
+      }
+      float4 v0[kLeafBatch], e1[kLeafBatch], e2[kLeafBatch];
+#pragma unroll
+      for (uint32_t b = 0; b < kLeafBatch; ++b) tri_get(mesh, min(f + b, stop - 1u), v0[b], e1[b], e2[b]);
+#pragma unroll
+      for (uint32_t b = 0; b < kLeafBatch; ++b) {
+        float t, u, v;
+        if (f + b < stop && tri_ray(o, d, v0[b], e1[b], e2[b], t, u, v)) {
+          if (t < depth) { fid = f + b; coord = make_float2(u, v); depth = t; }
+        }
+      }
+      f += kLeafBatch;
+    }
   }
 }
 
@@ -211,10 +303,6 @@ constexpr uint32_t kHandoffHead = 64;
 constexpr uint32_t kHandoffCap = 1u << 16;  // rays per call (256 KB)
 constexpr uint32_t kWaveGrid = 2048;     // one-wave workgroups merging the split rays
 constexpr uint32_t kRayWaveGrid = 8192;  // one-wave workgroups walking the other rays handed off
-#ifndef RK_REF_WAVE_PER
-#define RK_REF_WAVE_PER 4
-#endif
-constexpr int kWavePer = RK_REF_WAVE_PER;  // faces per lane per round of the second pass's leaf tests
 
 struct LeafBest { float t, u, v; uint32_t k; bool found; };
 
@@ -222,16 +310,13 @@ struct LeafBest { float t, u, v; uint32_t k; bool found; };
 // the same in every lane) and returns the first face of smallest t < dep, the
 // face a sequential pass keeping hits with t < depth would end on: its depth
 // after such a pass is the smallest t below dep, and a later face with the
-// same t fails t < depth. A round takes up to 64 * kPer faces, lane x the
-// consecutive faces [x * per, x * per + per), so that lane order is face
-// order: each lane keeps its first face of smallest t below dep, and the
-// lowest lane holding the wave's smallest t has the first such face. The
-// next round compares with that t.
-template <int kPer>
-__device__ __forceinline__ LeafBest wave_leaf(const uint4* __restrict__ faces, const float4* __restrict__ verts,
-                                              const float* __restrict__ tris, float4 o, float4 d, uint32_t first,
-                                              uint32_t cnt, float dep) {
-  const uint32_t lane = threadIdx.x & 63u;
+// same t fails t < depth. Each lane tests one group's bound, then the faces of
+// four groups the ray may hit at a time, one face per lane, so that lane
+// order is face order: the lowest lane holding the wave's smallest t has the
+// first such face. The next four compare with that t.
+__device__ __forceinline__ LeafBest wave_leaf(const RefMesh& mesh, float4 o, float4 d, const rk::CullRay& cr,
+                                              uint32_t first, uint32_t cnt, float dep) {
+  const uint32_t lane = threadIdx.x & 63u, quarter = lane / kGroup;
   LeafBest r;
   r.t = dep;
   r.u = 0.0f;
@@ -239,68 +324,50 @@ __device__ __forceinline__ LeafBest wave_leaf(const uint4* __restrict__ faces, c
   r.k = 0;
   r.found = false;
   const float inf = __int_as_float(0x7f800000);
-  for (uint32_t c0 = 0; c0 < cnt; c0 += 64u * kPer) {
-    const uint32_t m = min(cnt - c0, 64u * kPer);
-    const uint32_t per = (m + 63u) >> 6;
-    const uint32_t k0 = lane * per;
-    float4 p0[kPer], p1[kPer], p2[kPer];
-    if (tris) {  // v0, e1, e2
+  const uint32_t end = first + cnt, g_end = cnt ? (end - 1u) / kGroup + 1u : 0u;
+  for (uint32_t g0 = first / kGroup; g0 < g_end; g0 += 64u) {
+    bool near = lane < g_end - g0;
+    if (near && mesh.bounds)
+      near = !rk::bound_missed(mesh.bounds[g0 + lane], o.x, o.y, o.z, d.x, d.y, d.z, cr, r.t);
+    uint64_t mask = __ballot(near);
+    while (mask != 0ull) {
+      uint32_t g = 0u;  // this quarter's group
+      bool has = false;
 #pragma unroll
-      for (int j = 0; j < kPer; ++j) {
-        if ((uint32_t)j < per && k0 + j < m) {
-          const float* q = tris + kRecFloats * (size_t)(first + c0 + k0 + j);
-          p0[j] = rec_vec(q);
-          p1[j] = rec_vec(q + 3);
-          p2[j] = rec_vec(q + 6);
+      for (uint32_t q = 0; q < 4; ++q) {
+        if (mask != 0ull) {
+          if (quarter == q) {
+            g = (uint32_t)__builtin_ctzll(mask);
+            has = true;
+          }
+          mask &= mask - 1ull;
         }
       }
-    } else {  // the vertices
-      uint4 f[kPer];
-#pragma unroll
-      for (int j = 0; j < kPer; ++j)
-        f[j] = ((uint32_t)j < per && k0 + j < m) ? faces[first + c0 + k0 + j] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-      for (int j = 0; j < kPer; ++j) {
-        if ((uint32_t)j < per && k0 + j < m) {
-          p0[j] = verts[f[j].x];
-          p1[j] = verts[f[j].y];
-          p2[j] = verts[f[j].z];
-        }
-      }
-    }
-    float bt = inf, bu = 0.0f, bv = 0.0f;
-    uint32_t bk = 0;
-    bool any = false;
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-      if ((uint32_t)j < per && k0 + j < m) {
-        float4 v0 = p0[j], e1 = p1[j], e2 = p2[j];
-        if (!tris) {  // tri_setup's arithmetic: v0, v1 - v0, v2 - v0, w cleared
-          e1 = rk::sub4(p1[j], v0);
-          e2 = rk::sub4(p2[j], v0);
-          v0.w = 0.0f;
-          e1.w = 0.0f;
-          e2.w = 0.0f;
-        }
+      const uint32_t f = (g0 + g) * kGroup + lane % kGroup;
+      has = has && f >= first && f < end;
+      float bt = inf, bu = 0.0f, bv = 0.0f;
+      bool any = false;
+      if (has) {
+        float4 v0, e1, e2;
+        tri_get(mesh, f, v0, e1, e2);
         float t, u, v;
-        if (tri_ray(o, d, v0, e1, e2, t, u, v) && t < r.t && t < bt) {
+        if (tri_ray(o, d, v0, e1, e2, t, u, v) && t < r.t) {
           bt = t;  // t < dep <= FLT_MAX or +inf: t is finite, below the sentinel
           bu = u;
           bv = v;
-          bk = c0 + k0 + (uint32_t)j;
           any = true;
         }
       }
+      if (__ballot(any) == 0ull) continue;
+      float mn = bt;
+      for (int off = 32; off > 0; off >>= 1) mn = fminf(mn, __shfl_xor(mn, off, 64));
+      const int w = __builtin_ctzll(__ballot(any && bt == mn));
+      r.t = __shfl(bt, w, 64);  // the winner's own bits (bt == mn holds for -0 against +0 too)
+      r.u = __shfl(bu, w, 64);
+      r.v = __shfl(bv, w, 64);
+      r.k = (uint32_t)__shfl((int)(f - first), w, 64);
+      r.found = true;
     }
-    if (__ballot(any) == 0ull) continue;
-    float mn = any ? bt : inf;
-    for (int off = 32; off > 0; off >>= 1) mn = fminf(mn, __shfl_xor(mn, off, 64));
-    const int w = __builtin_ctzll(__ballot(any && bt == mn));
-    r.t = __shfl(bt, w, 64);  // the winner's own bits (bt == mn holds for -0 against +0 too)
-    r.u = __shfl(bu, w, 64);
-    r.v = __shfl(bv, w, 64);
-    r.k = (uint32_t)__shfl((int)bk, w, 64);
-    r.found = true;
   }
   return r;
 }
@@ -384,22 +451,15 @@ constexpr uint32_t kBucketHead = 8;  // handoff[8 + o]: rays of octant o
 // kLdsStack entries of each lane live in LDS (entry e of lane x at
 // e * 64 + x), deeper ones in scratch (trees of depth <= 31 need at most 33),
 // so a CU holds 20 waves of this kernel instead of 6.
-#ifndef RK_REF_LEAF_BATCH
-#define RK_REF_LEAF_BATCH 2
-#endif
-constexpr int kLeafBatch = RK_REF_LEAF_BATCH;
-
 template <int kCoopMax>
 __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ nodes,
-                                                  const uint4* __restrict__ faces,
-                                                  const float4* __restrict__ verts,
+                                                  RefMesh mesh,
                                                   const float4* __restrict__ origins,
                                                   const float4* __restrict__ dirs, uint32_t n_rays,
                                                   uint32_t node_count, uint32_t face_count,
                                                   uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
                                                   float* __restrict__ depths, uint32_t* __restrict__ handoff,
-                                                  uint32_t handoff_cap, uint32_t handoff_faces, UnitArgs ua,
-                                                  const float* __restrict__ tris) {
+                                                  uint32_t handoff_cap, uint32_t handoff_faces, UnitArgs ua) {
   __shared__ uint32_t s_stack[kLdsStack * 64];
   const int lane = (int)threadIdx.x;
   const uint32_t l = blockIdx.x * 64 + (uint32_t)lane;
@@ -407,6 +467,7 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
   const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   const float4 orig = has_ray ? origins[l] : zero4, dir = has_ray ? dirs[l] : zero4;
   const float4 invdir = has_ray ? invdir_of(dir) : zero4;
+  const rk::CullRay cr = cull_ray4(orig, dir);
   float depth = has_ray ? depths[l] : 0.0f;
   uint32_t fid = has_ray ? faces_id[l] : 0u;
   float2 coord = has_ray ? coords[l] : make_float2(0.0f, 0.0f);
@@ -493,60 +554,16 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
     if (pending == 0ull) break;  // every lane is done
     if (__popcll(pending) > kCoopMax) {
       // each lane its own leaf, in face order
-      if (at_leaf) {
-        for (uint32_t k0 = 0; k0 < leaf_cnt; k0 += kLeafBatch) {
-          float4 p0[kLeafBatch], p1[kLeafBatch], p2[kLeafBatch];
-          if (tris) {  // v0, e1, e2
-#pragma unroll
-            for (int b = 0; b < kLeafBatch; ++b) {
-              if (k0 + b < leaf_cnt) {
-                const float* q = tris + kRecFloats * (size_t)(leaf_first + k0 + b);
-                p0[b] = rec_vec(q);
-                p1[b] = rec_vec(q + 3);
-                p2[b] = rec_vec(q + 6);
-              }
-            }
-          } else {  // the vertices
-            uint4 f[kLeafBatch];
-#pragma unroll
-            for (int b = 0; b < kLeafBatch; ++b)
-              f[b] = k0 + b < leaf_cnt ? faces[leaf_first + k0 + b] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-            for (int b = 0; b < kLeafBatch; ++b) {
-              if (k0 + b < leaf_cnt) {
-                p0[b] = verts[f[b].x];
-                p1[b] = verts[f[b].y];
-                p2[b] = verts[f[b].z];
-              }
-            }
-          }
-#pragma unroll
-          for (int b = 0; b < kLeafBatch; ++b) {
-            if (k0 + b < leaf_cnt) {
-              float4 v0 = p0[b], e1 = p1[b], e2 = p2[b];
-              if (!tris) {  // tri_setup's arithmetic: v0, v1 - v0, v2 - v0, w cleared
-                e1 = rk::sub4(p1[b], v0);
-                e2 = rk::sub4(p2[b], v0);
-                v0.w = 0.0f;
-                e1.w = 0.0f;
-                e2.w = 0.0f;
-              }
-              float t, u, v;
-              if (tri_ray(orig, dir, v0, e1, e2, t, u, v)) {
-                if (t < depth) { fid = leaf_first + k0 + b; coord = make_float2(u, v); depth = t; }
-              }
-            }
-          }
-        }
-      }
+      if (at_leaf) lane_leaf(mesh, leaf_first, leaf_cnt, orig, dir, cr, depth, fid, coord);
     } else {
       // the whole wave on each pending leaf in turn
       while (pending != 0ull) {
         const int L = __builtin_ctzll(pending);
         pending &= pending - 1;
         const uint32_t first = readlane_u32(leaf_first, L);
-        const LeafBest b = wave_leaf<1>(faces, verts, tris, readlane_f4(orig, L), readlane_f4(dir, L), first,
-                                     readlane_u32(leaf_cnt, L), readlane_f32(depth, L));
+        const float4 oL = readlane_f4(orig, L), dL = readlane_f4(dir, L);
+        const LeafBest b = wave_leaf(mesh, oL, dL, rk::CullRay{readlane_f32(cr.dl, L), readlane_f32(cr.d2, L)},
+                                     first, readlane_u32(leaf_cnt, L), readlane_f32(depth, L));
         if (lane == L && b.found) {
           depth = b.t;
           fid = first + b.k;
@@ -637,14 +654,15 @@ struct WalkResult { float depth; uint32_t fid; float2 coord; uint32_t pops; bool
 
 __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint32_t sp_base, float depth,
                                                 uint32_t fid, float2 coord, const rk::Node* __restrict__ nodes,
-                                                const uint4* __restrict__ faces, const float4* __restrict__ verts,
+                                                RefMesh mesh,
                                                 const float4* __restrict__ origins,
                                                 const float4* __restrict__ dirs, uint32_t node_count,
-                                                uint32_t face_count, const float* __restrict__ tris) {
+                                                uint32_t face_count) {
   const int lane = (int)(threadIdx.x & 63u);
   const uint32_t max_visits = 2 * node_count + 2;
   const float4 orig = origins[l], dir = dirs[l];
   const float4 invdir = invdir_of(dir);
+  const rk::CullRay cr = cull_ray4(orig, dir);
   uint32_t st0 = lane == 0 ? root : 0u, st1 = 0u;
   int sp = 1;
   uint32_t visits = 0;
@@ -660,7 +678,7 @@ __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint3
     if (rk::node_is_leaf(nd.w0)) {
       const uint32_t first = nd.w1;
       const uint32_t cnt = first < face_count ? min(rk::leaf_count(nd.w0), face_count - first) : 0u;
-      const LeafBest b = wave_leaf<kWavePer>(faces, verts, tris, orig, dir, first, cnt, depth);
+      const LeafBest b = wave_leaf(mesh, orig, dir, cr, first, cnt, depth);
       if (b.found) {
         depth = b.t;
         fid = first + b.k;
@@ -700,19 +718,17 @@ __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint3
 // The second pass of the per-ray traversal: one wave per ray handed off, its
 // walk again from the root.
 __global__ __launch_bounds__(64) void k_trace_ray_wave(const rk::Node* __restrict__ nodes,
-                                                       const uint4* __restrict__ faces,
-                                                       const float4* __restrict__ verts,
+                                                       RefMesh mesh,
                                                        const float4* __restrict__ origins,
                                                        const float4* __restrict__ dirs, uint32_t node_count,
                                                        uint32_t face_count, const uint32_t* __restrict__ handoff,
                                                        uint32_t handoff_cap, uint32_t* __restrict__ faces_id,
-                                                       float2* __restrict__ coords, float* __restrict__ depths,
-                                                       const float* __restrict__ tris) {
+                                                       float2* __restrict__ coords, float* __restrict__ depths) {
   const uint32_t count = min(handoff[0], handoff_cap);
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
     const uint32_t l = handoff[kHandoffHead + i];
-    const WalkResult r = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, faces, verts, origins,
-                                   dirs, node_count, face_count, tris);
+    const WalkResult r = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, mesh, origins, dirs,
+                                   node_count, face_count);
     if (threadIdx.x == 0) {
       faces_id[l] = r.fid;
       coords[l] = r.coord;
@@ -734,13 +750,11 @@ __global__ __launch_bounds__(64) void k_trace_ray_wave(const rk::Node* __restric
 // the leader's is marked diverged too. Each ray gets its UnitResult.
 template <int kUW>
 __global__ __launch_bounds__(64 * kUW) void k_units_walk(const rk::Node* __restrict__ nodes,
-                                                   const uint4* __restrict__ faces,
-                                                   const float4* __restrict__ verts,
+                                                   RefMesh mesh,
                                                    const float4* __restrict__ origins,
                                                    const float4* __restrict__ dirs, const float* __restrict__ depths,
                                                    uint32_t node_count, uint32_t face_count,
-                                                   const uint32_t* __restrict__ handoff, UnitArgs ua,
-                                                   const float* __restrict__ tris) {
+                                                   const uint32_t* __restrict__ handoff, UnitArgs ua) {
   __shared__ float4 s_v0[64 * kUW], s_e1[64 * kUW], s_e2[64 * kUW];
   __shared__ float4 s_part[kUW > 1 ? 64 * kUW : 1];  // a wave's first smallest (t, u, v, face) per ray
   const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
@@ -807,7 +821,7 @@ __global__ __launch_bounds__(64 * kUW) void k_units_walk(const rk::Node* __restr
           const uint32_t cc = min(64u * kUW, cnt - c0);
           if (threadIdx.x < cc) {
             float4 v0, e1, e2;
-            tri_get(faces, verts, tris, first + c0 + threadIdx.x, v0, e1, e2);
+            tri_get(mesh, first + c0 + threadIdx.x, v0, e1, e2);
             s_v0[threadIdx.x] = shared ? rk::sub4(orig0, v0) : v0;  // tvec, or v0
             s_e1[threadIdx.x] = e1;
             s_e2[threadIdx.x] = e2;
@@ -898,14 +912,12 @@ __global__ __launch_bounds__(64 * kUW) void k_units_walk(const rk::Node* __restr
 // the walk), when the pops add up to no more than the visit limit; else the
 // ray's walk by the whole wave.
 __global__ __launch_bounds__(64) void k_units_merge(const rk::Node* __restrict__ nodes,
-                                                    const uint4* __restrict__ faces,
-                                                    const float4* __restrict__ verts,
+                                                    RefMesh mesh,
                                                     const float4* __restrict__ origins,
                                                     const float4* __restrict__ dirs, uint32_t node_count,
                                                     uint32_t face_count, const uint32_t* __restrict__ handoff,
                                                     UnitArgs ua, uint32_t* __restrict__ faces_id,
-                                                    float2* __restrict__ coords, float* __restrict__ depths,
-                                                    const float* __restrict__ tris) {
+                                                    float2* __restrict__ coords, float* __restrict__ depths) {
   const uint32_t count = min(handoff[1], ua.cap);
   const uint64_t max_visits = 2 * node_count + 2;
   for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
@@ -926,8 +938,8 @@ __global__ __launch_bounds__(64) void k_units_merge(const rk::Node* __restrict__
       if (r.flags & kUnitStop) break;
     }
     if (pops > max_visits || ua.diverged[i] != 0u) {
-      const WalkResult w = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, faces, verts, origins,
-                                     dirs, node_count, face_count, tris);
+      const WalkResult w = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, mesh, origins, dirs,
+                                   node_count, face_count);
       depth = w.depth;
       fid = w.fid;
       coord = w.coord;
@@ -977,13 +989,12 @@ constexpr uint32_t kNone = 0xffffffffu, kDone = 0xfffffffeu;
 
 template <int kS>
 __device__ __forceinline__ bool trace_packet_job(
-    const rk::Node* __restrict__ nodes, const uint4* __restrict__ faces, const float4* __restrict__ verts,
+    const rk::Node* __restrict__ nodes, RefMesh mesh,
     const float4* __restrict__ origins, const float4* __restrict__ dirs, int width, int height, uint32_t node_count,
     uint32_t face_count, uint32_t* __restrict__ faces_id, float2* __restrict__ coords, float* __restrict__ depths,
     int bx, int by, uint32_t* __restrict__ handoff, uint32_t handoff_cap, uint32_t handoff_faces,
     uint32_t* __restrict__ state, uint32_t* __restrict__ forced_list, uint32_t forced_cap,
-    const uint32_t* __restrict__ resume, const float* __restrict__ tris, uint32_t* s_stack, float4* s_v0,
-    float4* s_e1, float4* s_e2, float4* s_dir0, uint32_t* s_slot, float* s_pt, float* s_pu, float* s_pv,
+    const uint32_t* __restrict__ resume, uint32_t* s_stack, float4* s_dir0, uint32_t* s_slot, float* s_pt, float* s_pu, float* s_pv,
     uint32_t* s_pk) {
   const int ray = (int)threadIdx.x % kPT, part = (int)threadIdx.x / kPT;
   const int tx = ray % kPW, ty = ray / kPW;
@@ -1002,6 +1013,7 @@ __device__ __forceinline__ bool trace_packet_job(
     fid = faces_id[l];
     coord = coords[l];
   }
+  const rk::CullRay cr = cull_ray4(orig, dir);
   int sp = 1;
   uint32_t visits = 0;
   if (resume) {
@@ -1072,57 +1084,40 @@ __device__ __forceinline__ bool trace_packet_job(
           tested += cnt;
         }
       }
-      for (uint32_t c0 = 0; c0 < cnt; c0 += kPCache) {
-        const uint32_t cc = (cnt - c0) < (uint32_t)kPCache ? (cnt - c0) : (uint32_t)kPCache;
-        __syncthreads();
-        for (uint32_t k = threadIdx.x; k < cc; k += kPT * kS) {
-          float4 v0, e1, e2;
-          tri_get(faces, verts, tris, tri_id + c0 + k, v0, e1, e2);
-          s_v0[k] = v0; s_e1[k] = e1; s_e2[k] = e2;
+      if (kS == 1) {
+        if (in_image) lane_leaf(mesh, tri_id, cnt, orig, dir, cr, depth, fid, coord);
+      } else {
+        // part p: an equal run of the leaf's groups of faces
+        const uint32_t end = tri_id + cnt, g_first = tri_id / kGroup;
+        const uint32_t ng = cnt ? (end - 1u) / kGroup + 1u - g_first : 0u, q = (ng + kS - 1) / kS;
+        const uint32_t ga = min((uint32_t)part * q, ng), gb = min(ga + q, ng);
+        float pt = depth;
+        float2 puv = make_float2(0.0f, 0.0f);
+        uint32_t pk = 0xffffffffu;  // none
+        if (in_image && ga < gb) {
+          const uint32_t a = max(tri_id, (g_first + ga) * kGroup);
+          const uint32_t m = gb == ng ? end - a : (g_first + gb) * kGroup - a;
+          lane_leaf(mesh, a, m, orig, dir, cr, pt, pk, puv);
         }
+        s_pt[threadIdx.x] = pt;
+        s_pu[threadIdx.x] = puv.x;
+        s_pv[threadIdx.x] = puv.y;
+        s_pk[threadIdx.x] = pk;
         __syncthreads();
-        if (kS == 1) {
-          if (in_image) {
-            for (uint32_t k = 0; k < cc; ++k) {
-              float t, u, v;
-              if (tri_ray(orig, dir, s_v0[k], s_e1[k], s_e2[k], t, u, v)) {
-                if (t < depth) { fid = tri_id + c0 + k; coord = make_float2(u, v); depth = t; }
-              }
-            }
-          }
-        } else {
-          const uint32_t q = (cc + kS - 1) / kS;
-          const uint32_t k0 = (uint32_t)part * q, k1 = min(cc, k0 + q);
-          float pt = depth, pu = 0.0f, pv = 0.0f;
-          uint32_t pk = 0xffffffffu;  // none
-          if (in_image) {
-            for (uint32_t k = k0; k < k1; ++k) {
-              float t, u, v;
-              if (tri_ray(orig, dir, s_v0[k], s_e1[k], s_e2[k], t, u, v)) {
-                if (t < pt) { pk = k; pu = u; pv = v; pt = t; }
-              }
-            }
-          }
-          s_pt[threadIdx.x] = pt;
-          s_pu[threadIdx.x] = pu;
-          s_pv[threadIdx.x] = pv;
-          s_pk[threadIdx.x] = pk;
-          __syncthreads();
-          if (in_image) {
+        if (in_image) {
 #pragma unroll
-            for (int p = 0; p < kS; ++p) {
-              const int o = p * kPT + ray;
-              const uint32_t k = s_pk[o];
-              if (k != 0xffffffffu && s_pt[o] < depth) {
-                depth = s_pt[o];
-                fid = tri_id + c0 + k;
-                coord = make_float2(s_pu[o], s_pv[o]);
-              }
+          for (int p = 0; p < kS; ++p) {
+            const int o = p * kPT + ray;
+            const uint32_t k = s_pk[o];
+            if (k != 0xffffffffu && s_pt[o] < depth) {
+              depth = s_pt[o];
+              fid = k;
+              coord = make_float2(s_pu[o], s_pv[o]);
             }
           }
         }
+        __syncthreads();
       }
-      __syncthreads();
     } else {
       int hit = 0;
       if (in_image) {
@@ -1150,24 +1145,21 @@ __device__ __forceinline__ bool trace_packet_job(
 
 // The packet traversal's first pass: one 192-thread block per packet.
 __global__ __launch_bounds__(kPT) void k_trace_packet(const rk::Node* __restrict__ nodes,
-                                                      const uint4* __restrict__ faces,
-                                                      const float4* __restrict__ verts,
+                                                      RefMesh mesh,
                                                       const float4* __restrict__ origins,
                                                       const float4* __restrict__ dirs, int width, int height,
                                                       uint32_t node_count, uint32_t face_count,
                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
                                                       float* __restrict__ depths, uint32_t* __restrict__ handoff,
                                                       uint32_t handoff_cap, uint32_t handoff_faces,
-                                                      uint32_t* __restrict__ forced_list, uint32_t forced_cap,
-                                                      const float* __restrict__ tris) {
+                                                      uint32_t* __restrict__ forced_list, uint32_t forced_cap) {
   __shared__ uint32_t s_stack[kPStack];
-  __shared__ float4 s_v0[kPCache], s_e1[kPCache], s_e2[kPCache];
   __shared__ float4 s_dir0;
   __shared__ uint32_t s_slot;
-  trace_packet_job<1>(nodes, faces, verts, origins, dirs, width, height, node_count, face_count, faces_id, coords,
+  trace_packet_job<1>(nodes, mesh, origins, dirs, width, height, node_count, face_count, faces_id, coords,
                       depths, (int)blockIdx.x, (int)blockIdx.y, handoff, handoff_cap, handoff_faces,
-                      handoff + kHandoffHead + handoff_cap, forced_list, forced_cap, nullptr, tris, s_stack, s_v0,
-                      s_e1, s_e2, &s_dir0, &s_slot, nullptr, nullptr, nullptr, nullptr);
+                      handoff + kHandoffHead + handoff_cap, forced_list, forced_cap, nullptr, s_stack, &s_dir0,
+                      &s_slot, nullptr, nullptr, nullptr, nullptr);
 }
 
 // The second pass: the packets handed off, each resumed from its record,
@@ -1178,13 +1170,11 @@ __global__ __launch_bounds__(kPT) void k_trace_packet(const rk::Node* __restrict
 constexpr int kPacketSplit = RK_REF_PACKET_SPLIT;
 
 __global__ __launch_bounds__(kPT * kPacketSplit) void k_trace_packet_split(
-    const rk::Node* __restrict__ nodes, const uint4* __restrict__ faces, const float4* __restrict__ verts,
+    const rk::Node* __restrict__ nodes, RefMesh mesh,
     const float4* __restrict__ origins, const float4* __restrict__ dirs, int width, int height, int packets_x,
     uint32_t node_count, uint32_t face_count, const uint32_t* __restrict__ handoff, uint32_t handoff_cap,
-    uint32_t* __restrict__ faces_id, float2* __restrict__ coords, float* __restrict__ depths,
-    const float* __restrict__ tris) {
+    uint32_t* __restrict__ faces_id, float2* __restrict__ coords, float* __restrict__ depths) {
   __shared__ uint32_t s_stack[kPStack];
-  __shared__ float4 s_v0[kPCache], s_e1[kPCache], s_e2[kPCache];
   __shared__ float4 s_dir0;
   __shared__ uint32_t s_slot;
   __shared__ float s_pt[kPT * kPacketSplit], s_pu[kPT * kPacketSplit], s_pv[kPT * kPacketSplit];
@@ -1194,10 +1184,10 @@ __global__ __launch_bounds__(kPT * kPacketSplit) void k_trace_packet_split(
     const uint32_t pk = handoff[kHandoffHead + i];
     const uint32_t* rec = handoff + kHandoffHead + handoff_cap + (size_t)i * kPStateWords;
     if (rec[3] == kDone) continue;  // traced by the forced walk
-    trace_packet_job<kPacketSplit>(nodes, faces, verts, origins, dirs, width, height, node_count, face_count,
+    trace_packet_job<kPacketSplit>(nodes, mesh, origins, dirs, width, height, node_count, face_count,
                                    faces_id, coords, depths, (int)(pk % (uint32_t)packets_x),
                                    (int)(pk / (uint32_t)packets_x), nullptr, 0u, 0u, nullptr, nullptr, 0u, rec,
-                                   tris, s_stack, s_v0, s_e1, s_e2, &s_dir0, &s_slot, s_pt, s_pu, s_pv, s_pk);
+                                   s_stack, &s_dir0, &s_slot, s_pt, s_pu, s_pv, s_pk);
     __syncthreads();  // the next packet rewrites the stack and s_dir0
   }
 }
@@ -1225,12 +1215,12 @@ constexpr uint32_t kForcedCap = 1024;    // forced packets per call
 constexpr uint32_t kForcedGrid = 2048;
 
 __global__ __launch_bounds__(kFThreads) void k_packet_forced(
-    const rk::Node* __restrict__ nodes, const uint4* __restrict__ faces, const float4* __restrict__ verts,
+    const rk::Node* __restrict__ nodes, RefMesh mesh,
     const float4* __restrict__ origins, const float4* __restrict__ dirs, int width, int height, int packets_x,
     uint32_t node_count, uint32_t face_count, const uint32_t* __restrict__ handoff, uint32_t handoff_cap,
     const uint32_t* __restrict__ forced_list, uint32_t forced_cap, float4* __restrict__ temp,
     uint32_t* __restrict__ fflags, const uint32_t* __restrict__ faces_id, const float2* __restrict__ coords,
-    const float* __restrict__ depths, const float* __restrict__ tris) {
+    const float* __restrict__ depths) {
   __shared__ uint32_t s_stack[kPStack];
   __shared__ float4 s_v0[kPCache], s_e1[kPCache], s_e2[kPCache];
   __shared__ float s_pt[kFThreads], s_pu[kFThreads], s_pv[kFThreads];
@@ -1282,7 +1272,7 @@ __global__ __launch_bounds__(kFThreads) void k_packet_forced(
           __syncthreads();
           for (uint32_t k = threadIdx.x; k < cc; k += kFThreads) {
             float4 v0, e1, e2;
-            tri_get(faces, verts, tris, tri_id + c0 + k, v0, e1, e2);
+            tri_get(mesh, tri_id + c0 + k, v0, e1, e2);
             s_v0[k] = v0;
             s_e1[k] = e1;
             s_e2[k] = e2;
@@ -1451,21 +1441,28 @@ static uint32_t* handoff_alloc(hipStream_t st, size_t words, uint32_t faces) {
 #define RK_REF_TRI_RECORDS 1
 #endif
 
-// The call's triangle records (k_tri_records), from the same pool, or nullptr:
-// the kernels then read the faces and vertices.
-static float* tri_records_alloc(hipStream_t st, const uint4* faces, const float4* verts, uint32_t face_count) {
-  if (!RK_REF_TRI_RECORDS) return nullptr;
-  float* tris = nullptr;
+// The call's triangle records and group bounds (k_tri_records), one block from
+// the same pool; without it the kernels read the faces and vertices.
+static RefMesh ref_mesh_alloc(hipStream_t st, const uint4* faces, const float4* verts, uint32_t face_count) {
+  RefMesh m{faces, verts, nullptr, nullptr};
+  if (!RK_REF_TRI_RECORDS) return m;
+  char* block = nullptr;
   hipMemPool_t pool = handoff_pool();
-  const size_t bytes = (size_t)face_count * kRecFloats * sizeof(float);
-  const hipError_t e = pool ? hipMallocFromPoolAsync(reinterpret_cast<void**>(&tris), bytes, pool, st)
-                            : hipMallocAsync(reinterpret_cast<void**>(&tris), bytes, st);
+  const size_t rec_bytes = rk_align_up((size_t)face_count * kRecFloats * sizeof(float));
+  const size_t bytes = rec_bytes + ((size_t)face_count + kGroup - 1) / kGroup * sizeof(rk::FaceBound);
+  const hipError_t e = pool ? hipMallocFromPoolAsync(reinterpret_cast<void**>(&block), bytes, pool, st)
+                            : hipMallocAsync(reinterpret_cast<void**>(&block), bytes, st);
   if (e != hipSuccess) {
     (void)hipGetLastError();
-    return nullptr;
+    return m;
   }
-  hipLaunchKernelGGL(k_tri_records, dim3((face_count + 255) / 256), dim3(256), 0, st, faces, verts, face_count, tris);
-  return tris;
+  float* tris = reinterpret_cast<float*>(block);
+  rk::FaceBound* bounds = reinterpret_cast<rk::FaceBound*>(block + rec_bytes);
+  hipLaunchKernelGGL(k_tri_records, dim3((face_count + 255) / 256), dim3(256), 0, st, faces, verts, face_count, tris,
+                     bounds);
+  m.tris = tris;
+  m.bounds = bounds;
+  return m;
 }
 
 extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* nodes, uint32_t node_count,
@@ -1495,30 +1492,30 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
     uint32_t* flist = ho ? ho + flist_off : nullptr;
     uint32_t* fflags = ho ? ho + flist_off + fcap : nullptr;
     float4* temp = ho ? reinterpret_cast<float4*>(ho + temp_off) : nullptr;
-    float* tris = tri_records_alloc(st, reinterpret_cast<const uint4*>(faces),
-                                     reinterpret_cast<const float4*>(vertices), face_count);
+    const RefMesh mesh = ref_mesh_alloc(st, reinterpret_cast<const uint4*>(faces),
+                                        reinterpret_cast<const float4*>(vertices), face_count);
     hipLaunchKernelGGL(k_trace_packet, dim3(gx, gy), dim3(kPT), 0, st, reinterpret_cast<const rk::Node*>(nodes),
-                       reinterpret_cast<const uint4*>(faces), reinterpret_cast<const float4*>(vertices),
+                       mesh,
                        reinterpret_cast<const float4*>(origins), reinterpret_cast<const float4*>(directions), width,
                        height, node_count, face_count, faces_id, reinterpret_cast<float2*>(coords), depths, ho,
-                       ho ? cap : 0u, faces_limit, flist, fcap, tris);
+                       ho ? cap : 0u, faces_limit, flist, fcap);
     if (ho) {
       hipLaunchKernelGGL(k_packet_forced, dim3(std::min<uint32_t>(fcap * kFPackets, kForcedGrid)), dim3(kFThreads), 0,
-                         st, reinterpret_cast<const rk::Node*>(nodes), reinterpret_cast<const uint4*>(faces),
-                         reinterpret_cast<const float4*>(vertices), reinterpret_cast<const float4*>(origins),
+                         st, reinterpret_cast<const rk::Node*>(nodes), mesh,
+                       reinterpret_cast<const float4*>(origins),
                          reinterpret_cast<const float4*>(directions), width, height, (int)gx, node_count, face_count,
                          ho, cap, flist, fcap, temp, fflags, faces_id, reinterpret_cast<const float2*>(coords),
-                         depths, tris);
+                         depths);
       hipLaunchKernelGGL(k_packet_commit, dim3(fcap), dim3(kPT), 0, st, width, height, (int)gx, ho, cap, flist, fcap,
                          temp, fflags, faces_id, reinterpret_cast<float2*>(coords), depths);
       hipLaunchKernelGGL(k_trace_packet_split, dim3(std::min<uint32_t>(cap, kPacketGrid)), dim3(kPT * kPacketSplit),
-                         0, st, reinterpret_cast<const rk::Node*>(nodes), reinterpret_cast<const uint4*>(faces),
-                         reinterpret_cast<const float4*>(vertices), reinterpret_cast<const float4*>(origins),
+                         0, st, reinterpret_cast<const rk::Node*>(nodes), mesh,
+                       reinterpret_cast<const float4*>(origins),
                          reinterpret_cast<const float4*>(directions), width, height, (int)gx, node_count, face_count,
-                         ho, cap, faces_id, reinterpret_cast<float2*>(coords), depths, tris);
+                         ho, cap, faces_id, reinterpret_cast<float2*>(coords), depths);
       if (hipFreeAsync(ho, st) != hipSuccess) return RK_ERROR_DEVICE;
     }
-    if (tris && hipFreeAsync(tris, st) != hipSuccess) return RK_ERROR_DEVICE;
+    if (mesh.tris && hipFreeAsync(const_cast<float*>(mesh.tris), st) != hipSuccess) return RK_ERROR_DEVICE;
   } else {
     // A ray whose leaves pass g_ray_faces faces, or a ray that passes every
     // box test (at its first leaf), is traced again by the second pass, one
@@ -1545,34 +1542,32 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
       ua.cap = ucap;
     }
     const rk::Node* nd = reinterpret_cast<const rk::Node*>(nodes);
-    const uint4* fc = reinterpret_cast<const uint4*>(faces);
-    const float4* vt = reinterpret_cast<const float4*>(vertices);
     const float4* org = reinterpret_cast<const float4*>(origins);
     const float4* drs = reinterpret_cast<const float4*>(directions);
     float2* uv = reinterpret_cast<float2*>(coords);
-    float* tris = tri_records_alloc(st, fc, vt, face_count);
-    hipLaunchKernelGGL(k_trace_ray<RK_REF_COOP_MAX>, dim3((n + 63) / 64), dim3(64), 0, st, nd, fc, vt, org,
-                       drs, n, node_count, face_count, faces_id, uv, depths, ho, ho ? cap : 0u, faces_limit, ua,
-                       tris);
+    const RefMesh mesh = ref_mesh_alloc(st, reinterpret_cast<const uint4*>(faces),
+                                        reinterpret_cast<const float4*>(vertices), face_count);
+    hipLaunchKernelGGL(k_trace_ray<RK_REF_COOP_MAX>, dim3((n + 63) / 64), dim3(64), 0, st, nd, mesh, org,
+                       drs, n, node_count, face_count, faces_id, uv, depths, ho, ho ? cap : 0u, faces_limit, ua);
     if (ho && ucap != 0u) {
       hipLaunchKernelGGL(k_units_split, dim3((ucap + 63) / 64), dim3(64), 0, st, nd, org, drs, depths, node_count,
                          ho, ua);
       const dim3 ugrid(std::min<uint32_t>(ucap * kUnits, kUnitGrid));
       if ((uint64_t)face_count >= (uint64_t)kUnitWaveFaces * ((node_count + 1) / 2))
-        hipLaunchKernelGGL(k_units_walk<RK_REF_UNIT_WAVES>, ugrid, dim3(64 * RK_REF_UNIT_WAVES), 0, st, nd, fc, vt, org,
-                           drs, depths, node_count, face_count, ho, ua, tris);
+        hipLaunchKernelGGL(k_units_walk<RK_REF_UNIT_WAVES>, ugrid, dim3(64 * RK_REF_UNIT_WAVES), 0, st, nd, mesh, org,
+                           drs, depths, node_count, face_count, ho, ua);
       else
-        hipLaunchKernelGGL(k_units_walk<1>, ugrid, dim3(64), 0, st, nd, fc, vt, org, drs, depths, node_count,
-                           face_count, ho, ua, tris);
-      hipLaunchKernelGGL(k_units_merge, dim3(std::min<uint32_t>(ucap, kWaveGrid)), dim3(64), 0, st, nd, fc, vt, org,
-                         drs, node_count, face_count, ho, ua, faces_id, uv, depths, tris);
+        hipLaunchKernelGGL(k_units_walk<1>, ugrid, dim3(64), 0, st, nd, mesh, org, drs, depths, node_count,
+                           face_count, ho, ua);
+      hipLaunchKernelGGL(k_units_merge, dim3(std::min<uint32_t>(ucap, kWaveGrid)), dim3(64), 0, st, nd, mesh, org,
+                         drs, node_count, face_count, ho, ua, faces_id, uv, depths);
     }
     if (ho) {
-      hipLaunchKernelGGL(k_trace_ray_wave, dim3(std::min<uint32_t>(cap, kRayWaveGrid)), dim3(64), 0, st, nd, fc, vt,
-                         org, drs, node_count, face_count, ho, cap, faces_id, uv, depths, tris);
+      hipLaunchKernelGGL(k_trace_ray_wave, dim3(std::min<uint32_t>(cap, kRayWaveGrid)), dim3(64), 0, st, nd, mesh,
+                         org, drs, node_count, face_count, ho, cap, faces_id, uv, depths);
       if (hipFreeAsync(ho, st) != hipSuccess) return RK_ERROR_DEVICE;
     }
-    if (tris && hipFreeAsync(tris, st) != hipSuccess) return RK_ERROR_DEVICE;
+    if (mesh.tris && hipFreeAsync(const_cast<float*>(mesh.tris), st) != hipSuccess) return RK_ERROR_DEVICE;
   }
   RK_CHECK_LAUNCH();
   return RK_SUCCESS;
