@@ -1,24 +1,24 @@
 // Closest-hit traversal of the reference tree layout (bvnode, 32 B) with the
 // reference arithmetic (CUDA_raytraceMeshTree.cu), for gfx950:
+//   k_tri_records   the call's triangle records, and bounds of each 16 and 64
+//                   faces (rk_face_bounds.h): every leaf test below skips the
+//                   groups of faces its ray misses
 //   k_trace_ray     per-ray DFS (kernel_raytraceMeshTree, :111-219), one lane
 //                   per ray for the nodes; a leaf's faces tested by its lane,
 //                   or by the whole wave when few lanes hold a leaf; stack in
-//                   LDS and scratch; a ray that passes every box test is
-//                   handed off to
-//   k_units_split, k_units_walk, k_units_merge  its walk cut into subtrees,
-//                   walked for groups of rays of one direction octant, and
-//                   merged in walk order; another ray past a face budget to
-//   k_trace_ray_wave  the same walk, one wave per ray, leaves tested by the
-//                   whole wave;
+//                   LDS and scratch
 //   k_trace_packet  the 16x12 packet traversal (kernel_raytraceMeshTreePacket,
 //                   :222-377), one 192-thread workgroup (3 waves) per tile,
-//                   block-uniform stack in LDS, one barrier vote per node; a
-//                   packet past a face budget is handed off to
-//   k_trace_packet_split  the same walk with five threads per ray, each
-//                   testing a fifth of every chunk of faces, or, for a packet
-//                   holding a ray that passes every box test, to
-//   k_packet_forced  the packet's walk by parts of 16 rays on different CUs.
-// The results of both passes are bit-identical to the reference's.
+//                   block-uniform stack in LDS, one barrier vote per node
+//   k_units_cut, k_unit_walk, k_units_merge, k_packet_commit
+//                   rays that pass every box test, and the packets that hold
+//                   one: their walks cut into subtrees, walked for groups of
+//                   64 rays and merged in walk order
+//   k_trace_ray_wave  other rays past a face budget: the same walk, one wave
+//                   per ray, leaves tested by the whole wave
+//   k_trace_packet_split  other packets past a face budget: the same walk with
+//                   five threads per ray, each testing a fifth of every leaf
+// The results are bit-identical to the reference's.
 // Built with -ffp-contract=off, so the triangle and box tests are the same
 // float operations in the same order as the reference source.
 #include <algorithm>
@@ -34,9 +34,6 @@ constexpr float kEps = 0.000001f;  // CUDA_raytraceMeshTree.cu:36
 constexpr float kUMargin = 0.001f;
 #ifndef RK_REF_U_PRETEST
 #define RK_REF_U_PRETEST 1
-#endif
-#ifndef RK_REF_SHARED_TVEC
-#define RK_REF_SHARED_TVEC 1
 #endif
 
 // intersectTriRay, CUDA_raytraceMeshTree.cu:57-89.
@@ -64,34 +61,6 @@ __device__ __forceinline__ bool tri_ray(float4 orig, float4 dir, float4 v0, floa
   if (v < 0.0f || u + v > 1.0f) return false;
   t = rk::dot4(e2, qvec) * inv_det;
   return t >= 0.0f;
-}
-
-// tri_ray with tvec = orig - v0 given: for rays that share an origin (bit for
-// bit, w included) it is computed once per face, with tri_ray's operation.
-// The same results as tri_ray.
-__device__ __forceinline__ bool tri_ray_tv(float4 dir, float4 tvec, float4 e1, float4 e2, float& t, float& u,
-                                           float& v) {
-  float4 pvec = rk::cross4(dir, e2);
-  float det = rk::dot4(e1, pvec);
-  if (det > -kEps && det < kEps) return false;
-  const float un = rk::dot4(tvec, pvec);
-#if RK_REF_U_PRETEST
-  const float ua = un * __builtin_amdgcn_rcpf(det);
-  if (ua < -kUMargin || ua > 1.0f + kUMargin) return false;
-#endif
-  float inv_det = 1.0f / det;
-  u = un * inv_det;
-  if (u < 0.0f || u > 1.0f) return false;
-  float4 qvec = rk::cross4(tvec, e1);
-  v = rk::dot4(dir, qvec) * inv_det;
-  if (v < 0.0f || u + v > 1.0f) return false;
-  t = rk::dot4(e2, qvec) * inv_det;
-  return t >= 0.0f;
-}
-
-__device__ __forceinline__ bool same_bits(float4 a, float4 b) {
-  return __float_as_uint(a.x) == __float_as_uint(b.x) && __float_as_uint(a.y) == __float_as_uint(b.y) &&
-         __float_as_uint(a.z) == __float_as_uint(b.z) && __float_as_uint(a.w) == __float_as_uint(b.w);
 }
 
 // intersectBoxRay, CUDA_raytraceMeshTree.cu:91-105.
@@ -136,13 +105,15 @@ __device__ __forceinline__ void tri_setup(const uint4* __restrict__ faces, const
 // precomputed per call in face order (nine floats, 36 B per face): one
 // contiguous load per face test instead of the face's indices, then its
 // vertices. And the bound of each kFaceGroup faces (rk_face_bounds.h), 2 B per
-// face: 16 lanes share a group, reduced by shuffles.
+// face, and of each wave's 64: reduced by shuffles.
 constexpr size_t kRecFloats = 9;
 constexpr uint32_t kGroup = rk::kFaceGroup;
+constexpr uint32_t kSuper = 64 / kGroup;
 static_assert(kGroup == 16, "a group is a quarter of a wave");
 __global__ __launch_bounds__(256) void k_tri_records(const uint4* __restrict__ faces,
                                                      const float4* __restrict__ verts, uint32_t face_count,
-                                                     float* __restrict__ tris, rk::FaceBound* __restrict__ bounds) {
+                                                     float* __restrict__ tris, rk::FaceBound* __restrict__ bounds,
+                                                     rk::FaceBound* __restrict__ supers) {
   const uint32_t f = blockIdx.x * 256 + threadIdx.x;
   const bool in = f < face_count;
   float lo[3], hi[3], e2m = 0.0f, nan = 0.0f;
@@ -162,20 +133,21 @@ __global__ __launch_bounds__(256) void k_tri_records(const uint4* __restrict__ f
     e2m = fmaxf(l1, l2);
     nan = l1 + l2;  // NaN or infinite when a vertex is (fminf and fmaxf drop NaN)
   }
+  // (lane 0 of a group or wave with any face holds one: faces fill them from the front)
 #pragma unroll
-  for (int off = 8; off > 0; off >>= 1) {
+  for (int off = 1; off < 64; off <<= 1) {
+    if (off == (int)kGroup && in && f % kGroup == 0)
+      bounds[f / kGroup] = rk::face_bound(lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], nan == nan ? 1.00001f * e2m : nan);
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
-      lo[q] = fminf(lo[q], __shfl_xor(lo[q], off, 16));
-      hi[q] = fmaxf(hi[q], __shfl_xor(hi[q], off, 16));
+      lo[q] = fminf(lo[q], __shfl_xor(lo[q], off, 64));
+      hi[q] = fmaxf(hi[q], __shfl_xor(hi[q], off, 64));
     }
-    e2m = fmaxf(e2m, __shfl_xor(e2m, off, 16));
-    nan += __shfl_xor(nan, off, 16);
+    e2m = fmaxf(e2m, __shfl_xor(e2m, off, 64));
+    nan += __shfl_xor(nan, off, 64);
   }
-  if (in && f % kGroup == 0) {
-    const float e = (nan == nan) ? 1.00001f * e2m : nan;
-    bounds[f / kGroup] = rk::face_bound(lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], e);
-  }
+  if (in && f % 64 == 0)
+    supers[f / 64] = rk::face_bound(lo[0], lo[1], lo[2], hi[0], hi[1], hi[2], nan == nan ? 1.00001f * e2m : nan);
 }
 
 // One of a record's three vectors, w 0 as tri_setup leaves it.
@@ -190,7 +162,8 @@ struct RefMesh {
   const uint4* faces;
   const float4* verts;
   const float* tris;
-  const rk::FaceBound* bounds;
+  const rk::FaceBound* bounds;  // per kGroup faces
+  const rk::FaceBound* supers;  // per kSuper groups (a wave's 64 faces)
 };
 
 // tri_setup from the records when the call has them, else from the mesh.
@@ -209,16 +182,23 @@ __device__ __forceinline__ rk::CullRay cull_ray4(float4 o, float4 d) {
   return rk::cull_ray(o.x, o.y, o.z, o.w, d.x, d.y, d.z, d.w);
 }
 
+#ifndef RK_REF_BOUND_BATCH
+#define RK_REF_BOUND_BATCH 4
+#endif
+constexpr uint32_t kBoundBatch = RK_REF_BOUND_BATCH;
 // Which of the groups g0 .. g0 + ng - 1 (ng <= 32) may hold a face the ray's
 // part [0, depth] hits: bit j for group g0 + j. Every group without bounds.
 __device__ __forceinline__ uint32_t groups_near(const rk::FaceBound* __restrict__ bounds, uint32_t g0, uint32_t ng,
                                                 float4 o, float4 d, const rk::CullRay& cr, float depth) {
   if (!bounds) return ng >= 32u ? 0xFFFFFFFFu : (1u << ng) - 1u;
   uint32_t mask = 0u;
-  for (uint32_t j = 0; j < ng; j += 2) {  // two bounds in flight
-    const rk::FaceBound b0 = bounds[g0 + j], b1 = bounds[g0 + min(j + 1u, ng - 1u)];
-    if (!rk::bound_missed(b0, o.x, o.y, o.z, d.x, d.y, d.z, cr, depth)) mask |= 1u << j;
-    if (j + 1u < ng && !rk::bound_missed(b1, o.x, o.y, o.z, d.x, d.y, d.z, cr, depth)) mask |= 2u << j;
+  for (uint32_t j0 = 0; j0 < ng; j0 += kBoundBatch) {  // their loads in flight together
+    rk::FaceBound b[kBoundBatch];
+#pragma unroll
+    for (uint32_t j = 0; j < kBoundBatch; ++j) b[j] = bounds[g0 + min(j0 + j, ng - 1u)];
+#pragma unroll
+    for (uint32_t j = 0; j < kBoundBatch; ++j)
+      if (j0 + j < ng && !rk::bound_missed(b[j], o.x, o.y, o.z, d.x, d.y, d.z, cr, depth)) mask |= 1u << (j0 + j);
   }
   return mask;
 }
@@ -227,8 +207,13 @@ __device__ __forceinline__ uint32_t groups_near(const rk::FaceBound* __restrict_
 // when t < depth: (depth, fid, uv) as a sequential pass over all of them ends.
 // Faces of groups the ray misses are skipped; the lanes of a wave step through
 // the faces left to each, so the pass lasts as long as the most any lane has.
+// On the 1920x1080 frame of the 1M-face terrain (leaves of 155 faces, 10
+// groups, of which a ray meets one or two) the per-ray first pass takes 1.48 ms
+// with the groups skipped and 2.97 without, the packets' 0.66 and 1.58 ms. It
+// is bound by the latency of its loads: 4 faces and 4 bounds in flight per
+// lane against 2 and 2, 2.02 against 2.13 ms per frame (1 face: 2.31; 8: 2.11).
 #ifndef RK_REF_LEAF_BATCH
-#define RK_REF_LEAF_BATCH 2
+#define RK_REF_LEAF_BATCH 4
 #endif
 constexpr uint32_t kLeafBatch = RK_REF_LEAF_BATCH;
 __device__ __forceinline__ void lane_leaf(const RefMesh& mesh, uint32_t first, uint32_t cnt, float4 o, float4 d,
@@ -301,7 +286,6 @@ __device__ __forceinline__ float4 readlane_f4(float4 v, int l) {
 // off, the ray indices start at word kHandoffHead.
 constexpr uint32_t kHandoffHead = 64;
 constexpr uint32_t kHandoffCap = 1u << 16;  // rays per call (256 KB)
-constexpr uint32_t kWaveGrid = 2048;     // one-wave workgroups merging the split rays
 constexpr uint32_t kRayWaveGrid = 8192;  // one-wave workgroups walking the other rays handed off
 
 struct LeafBest { float t, u, v; uint32_t k; bool found; };
@@ -372,60 +356,76 @@ __device__ __forceinline__ LeafBest wave_leaf(const RefMesh& mesh, float4 o, flo
   return r;
 }
 
-// Rays that pass every box test (crosses_every_box) are split by subtree. The
-// walk of such a ray visits every node below one that passes its box test,
-// in an order fixed by the direction, as long as its depth stays above 0
-// (its box tests give t = +-0); at depth 0 no later face can be kept (t < 0
-// never holds). So the subtrees at tree level kUnitLevel (and the leaves
-// above it), each walked on its own from the ray's starting depth, give the
-// walk's result when merged in walk order, first smallest t winning. A
-// subtree's walk differs from the reference's only after the reference's
-// depth has reached 0, when its result can no longer change. The stack the
-// reference holds when it pops a subtree's root is known from the walk above
-// the cut, so a stack overflow stops both at the same node; the visit limit
-// is checked on the sum (past it, the ray is walked again by one wave). The
-// subtrees are walked for groups of up to 64 rays of one direction octant at
-// once (k_units_walk). On the 1920x1080 heightfield (1,949 such rays), cuts
-// at levels 6, 8, 9 and 10 gave 15.7, 8.5, 9.9 and 9.4 ms per frame on the
-// depth-12 LBVH and 8.8, 5.9, 6.2 and 6.8 ms on the SAH tree.
+// Walks split by subtree: rays that pass every box test (crosses_every_box).
+// The walk of such a ray visits every node below one that passes its box
+// test, in an order fixed by its direction's octant, as long as its depth
+// stays above 0 (its box tests give t = +-0); at depth 0 no later face can be
+// kept (t < 0 never holds). So the subtrees at tree level kUnitLevel (and the
+// leaves above it), each walked on its own from the ray's starting depth,
+// give the walk's result when merged in walk order, first smallest t winning.
+// A packet holding such a ray (the forcing ray) visits the same nodes in the
+// order its first ray gives, whatever its other rays hold, as long as the
+// forcing ray's depth stays above 0: its rays' walks are split the same way.
+//
+// k_units_cut finds the subtrees' roots once per octant, on the assumption
+// that every box above the cut is passed; k_unit_walk walks one subtree for a
+// group of 64 rays (rays of one octant, or a third of a packet), checking the
+// boxes, and lists each ray's best hit in it; k_units_merge and
+// k_packet_commit take each ray's first smallest t. What does not fit the
+// assumption (a box failed, a stack overflow, a child out of range, more pops
+// than the visit limit, the hit list full) is walked again as the reference
+// does: a ray by one wave, a packet by k_trace_packet_split.
+//
+// Nearly every face of the tree is far from any one ray, so a walk is a scan
+// of bounds, 64 faces at a time. On the 1920x1080 frame of the 1M-face terrain
+// (1,949 such rays; 149 packets holding one; depth-12 LBVH, 155 faces per
+// leaf) the subtree walks take 0.24 ms for the rays and 1.36 ms for the
+// packets. With every face tested by every ray they took 2.76 ms, and the
+// packets 37.9 ms in parts of 16 rays that each walked the whole tree. Cut
+// level 7: 2.20 ms per per-ray frame against 2.02, packets the same.
 #ifndef RK_REF_UNIT_LEVEL
 #define RK_REF_UNIT_LEVEL 8
 #endif
 constexpr int kUnitLevel = RK_REF_UNIT_LEVEL;
-constexpr uint32_t kUnits = 1u << kUnitLevel;  // subtrees per ray at most: the cut has <= 2^kUnitLevel nodes
+constexpr uint32_t kUnits = 1u << kUnitLevel;  // subtrees at most: the cut has <= 2^kUnitLevel nodes
 #ifndef RK_REF_CROSS_CAP
 #define RK_REF_CROSS_CAP 4096
 #endif
-constexpr uint32_t kCrossCap = RK_REF_CROSS_CAP;          // rays split per call
-constexpr uint32_t kUnitGrid = 8192;          // workgroups walking the subtrees
-// A subtree walk takes two waves, each testing half of every batch of faces,
-// when the tree's leaves hold 64 faces or more on average (node_count / 2
-// leaves): the heightfield's depth-12 LBVH (155 faces per leaf) 7.7 -> 6.8 ms
-// per frame; with small leaves the second wave only repeats the walk
-// (depth-31 LBVH, 42 faces per leaf: 9.5 against 9.2 ms; SAH tree, 21 faces
-// per leaf: 5.6 against 6.7 ms), and four waves were slower on all three.
-#ifndef RK_REF_UNIT_WAVES
-#define RK_REF_UNIT_WAVES 2
-#endif
-constexpr uint32_t kUnitWaveFaces = 64;  // faces per leaf from which a walk takes RK_REF_UNIT_WAVES waves
-constexpr uint32_t kNoFace = 0xffffffffu;
-constexpr uint32_t kUnitStop = 1u;            // the walk stopped here (stack overflow, child out of range)
+constexpr uint32_t kCrossCap = RK_REF_CROSS_CAP;  // rays split per call
+constexpr uint32_t kUnitGrid = 8192;              // one-wave workgroups walking the subtrees
+constexpr uint32_t kNone = 0xffffffffu;
 
-struct UnitResult { float t, u, v; uint32_t face, pops, flags, pad0, pad1; };
-
-// The split rays' state in the hand-off buffer.
-struct UnitArgs {
-  uint32_t* list;        // [cap] the rays, in hand-off order
-  uint32_t* nunits;      // [cap] subtrees of each
-  uint32_t* top_pops;    // [cap] pops of the walk above the cut
-  uint32_t* diverged;    // [cap] 1: the ray's walk left its group's; walked again by one wave
-  uint32_t* bucket;      // [8 * cap] the slots of the rays of each direction octant
-  uint32_t* unit_node;   // [cap * kUnits] each subtree's root, in walk order
-  uint32_t* unit_sp;     // [cap * kUnits] the reference's stack size after popping that root
-  UnitResult* res;       // [cap * kUnits]
-  uint32_t cap;
+// The subtrees of each direction octant (bit 0: x < 0, 1: y, 2: z), in walk order.
+struct UnitCut {
+  uint32_t units[8];            // subtrees
+  uint32_t tops[8];             // internal nodes above them
+  uint32_t node[8][kUnits];     // each subtree's root
+  uint32_t sp[8][kUnits];       // the reference's stack size after popping that root
+  uint32_t top[8][kUnits];      // the internal nodes above
 };
-constexpr uint32_t kBucketHead = 8;  // handoff[8 + o]: rays of octant o
+
+// A ray's best hit in one subtree; next: the ray's previous entry, or kNone.
+struct UnitHit { float t, u, v; uint32_t face, unit, next; };
+
+// The split walks' state in the hand-off buffer. A slot is a crossing ray's
+// place in list, or a forced packet's ray (packet's place * kPT + ray).
+struct UnitArgs {
+  uint32_t* list;            // crossing rays: [cap] the rays, in hand-off order
+  uint32_t* bucket;          // crossing rays: [8 * cap] the slots of each octant
+  uint32_t* redo;            // crossing rays: [cap] the rays to walk again
+  uint32_t* diverged;        // [cap] per crossing ray or forced packet: walk it again
+  unsigned long long* pops;  // per group: pops of its subtree walks
+  uint32_t* head;            // per slot: its last hit entry, or kNone
+  UnitHit* hits;             // [hit_cap]
+  UnitCut* cut;
+  uint32_t cap, hit_cap;
+};
+// Words of the hand-off buffer's head: [0] handed off, [1] crossing rays, [2]
+// forced packets, [3] hit entries, [4] crossing rays to walk again.
+constexpr uint32_t kBucketHead = 8;  // [8 + o]: crossing rays of octant o
+__device__ __forceinline__ uint32_t octant_of(float4 dir) {
+  return (dir.x < 0.0f ? 1u : 0u) | (dir.y < 0.0f ? 2u : 0u) | (dir.z < 0.0f ? 4u : 0u);
+}
 
 // The per-ray traversal (kernel_raytraceMeshTree, :111-219), one lane per ray:
 // pop a node, test its box against the depth so far, push the far child, then
@@ -438,14 +438,9 @@ constexpr uint32_t kBucketHead = 8;  // handoff[8 + o]: rays of octant o
 // hundred faces each: on the 1920x1080 heightfield the waves that hold them
 // ran alone for most of the frame (0.5 waves per CU on average). So when at
 // most kCoopMax lanes hold a leaf, the whole wave tests each of those leaves
-// in turn, 64 faces at a time, one face per lane: the reference keeps the
-// first face of smallest t below the depth the leaf was entered with, so a
-// round keeps the smallest t below the current depth, ties to the smallest
-// face index, and the next round compares with the depth that leaves (the
-// same depth after every leaf as the reference's, and so the same later
-// pops). When more lanes hold a leaf, each lane tests its own, its faces
-// fetched kLeafBatch at a time with all their loads issued before the first
-// test (a face costs two dependent loads: the face, then its vertices).
+// in turn (wave_leaf): the same depth after every leaf as the reference's, and
+// so the same later pops. When more lanes hold a leaf, each lane tests its own
+// (lane_leaf). Both skip the groups of faces the ray misses.
 //
 // The stack keeps the reference's 96 entries and its overflow rule; the first
 // kLdsStack entries of each lane live in LDS (entry e of lane x at
@@ -484,9 +479,21 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
   uint32_t tested = 0;  // faces of the leaves reached, while may_hand_off
   // A direction with a component of 0 leaves a NaN in invdir: every box test
   // then passes (at t = 0, while depth > 0) and the ray walks the whole tree,
-  // so it goes to the split at its first leaf (else to the second pass).
-  const bool crossing = crosses_every_box(invdir);
+  // so it goes to the split at once (else to the second pass at its first leaf).
+  const bool crossing = has_ray && crosses_every_box(invdir);
   const uint32_t limit = crossing ? 0u : handoff_faces;
+  if (crossing && may_hand_off && ua.cap != 0u) {
+    const uint32_t slot = atomicAdd(handoff + 1, 1u);
+    if (slot < ua.cap) {
+      const uint32_t o = octant_of(dir);
+      ua.list[slot] = l;
+      ua.diverged[slot] = 0u;
+      ua.head[slot] = kNone;
+      ua.bucket[o * ua.cap + atomicAdd(handoff + kBucketHead + o, 1u)] = slot;  // at most cap rays in all
+      handed_off = true;
+      active = false;
+    }
+  }
   uint32_t visits = 0;
   const uint32_t max_visits = 2 * node_count + 2;
   for (;;) {
@@ -511,15 +518,6 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
         if (may_hand_off) {
           if (leaf_cnt > limit - tested) {
             may_hand_off = false;
-            if (crossing && ua.cap != 0u) {
-              const uint32_t slot = atomicAdd(handoff + 1, 1u);
-              if (slot < ua.cap) {
-                ua.list[slot] = l;
-                handed_off = true;
-                active = false;
-                break;
-              }
-            }
             const uint32_t slot = atomicAdd(handoff, 1u);
             if (slot < handoff_cap) {
               handoff[kHandoffHead + slot] = l;
@@ -579,70 +577,80 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
   }
 }
 
-__global__ __launch_bounds__(64) void k_handoff_clear(uint32_t* __restrict__ handoff) {
-  if (threadIdx.x < kHandoffHead) handoff[threadIdx.x] = 0u;
+// Clears the head's counters and the groups' pops.
+__global__ __launch_bounds__(256) void k_handoff_clear(uint32_t* __restrict__ handoff, unsigned long long* __restrict__ pops,
+                                                       uint32_t groups) {
+  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+  if (t < kHandoffHead) handoff[t] = 0u;
+  if (t < groups) pops[t] = 0ull;
 }
 
-// The walk of a split ray above the cut, one lane per ray: the reference's
-// pops of the nodes above kUnitLevel (box tests at the starting depth), each
-// node at the cut, leaf above it or child out of range recorded as a subtree
-// root with the stack size after its pop. The stack holds at most
-// kUnitLevel + 1 entries here.
-__global__ __launch_bounds__(64) void k_units_split(const rk::Node* __restrict__ nodes,
-                                                    const float4* __restrict__ origins,
-                                                    const float4* __restrict__ dirs,
-                                                    const float* __restrict__ depths, uint32_t node_count,
-                                                    uint32_t* __restrict__ handoff, UnitArgs ua) {
-  const uint32_t i = blockIdx.x * 64 + threadIdx.x;
-  if (i >= min(handoff[1], ua.cap)) return;
-  const uint32_t l = ua.list[i];
-  const float4 orig = origins[l], dir = dirs[l];
-  const float4 invdir = invdir_of(dir);
-  const float depth = depths[l];
-  uint32_t st[2 * kUnitLevel + 2], lv[2 * kUnitLevel + 2];
-  int sp = 1;
-  st[0] = 0u;
-  lv[0] = 0u;
-  uint32_t nu = 0, pops = 0;
-  uint32_t* unode = ua.unit_node + (size_t)i * kUnits;
-  uint32_t* usp = ua.unit_sp + (size_t)i * kUnits;
-  while (sp > 0 && nu < kUnits) {
-    --sp;
-    const uint32_t nid = st[sp], level = lv[sp];
-    bool unit = level >= (uint32_t)kUnitLevel || nid >= node_count;
-    NodeRegs nd;
-    if (!unit) {
-      nd = load_node(nodes, nid);
-      unit = rk::node_is_leaf(nd.w0);
-    }
-    if (unit) {  // its walk counts its pop and stops at a child out of range
-      unode[nu] = nid;
-      usp[nu] = (uint32_t)sp;
-      ++nu;
-      if (nid >= node_count) break;
-      continue;
-    }
-    ++pops;
-    float t;
-    if (box_ray(nd.bmin, nd.bmax, orig, invdir, t) && t < depth) {
-      uint32_t nearc, farc;
-      children_order(nd.w0, nd.w1, dir, nearc, farc);
-      if (sp + 2 > 2 * kUnitLevel + 2) break;  // cannot occur: one entry per level, two at the deepest
-      st[sp] = farc;
-      lv[sp] = level + 1u;
-      ++sp;
-      st[sp] = nearc;
-      lv[sp] = level + 1u;
-      ++sp;
-    }
+// The cut: one workgroup per octant expands the tree level by level, in walk
+// order, down to kUnitLevel; a leaf or a child out of range ends where it is.
+// The reference's stack holds, after it pops a node, one far child for every
+// near step on the path to it.
+__global__ __launch_bounds__(256) void k_units_cut(const rk::Node* __restrict__ nodes, uint32_t node_count,
+                                                   const uint32_t* __restrict__ handoff, UnitCut* __restrict__ cut) {
+  static_assert(kUnits <= 256, "one thread per subtree");
+  __shared__ uint32_t s_node[kUnits], s_sp[kUnits], s_wave[4];
+  constexpr uint32_t kDone = 0x80000000u;
+  if (handoff[1] == 0u && handoff[2] == 0u) return;  // nothing to walk
+  const uint32_t o = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
+  uint32_t n = 1, tops = 0;
+  if (t == 0) {
+    s_node[0] = 0u;
+    s_sp[0] = 0u;
   }
-  ua.nunits[i] = nu;
-  ua.top_pops[i] = pops;
-  ua.diverged[i] = 0u;
-  // children_order's choice at every node: rays of one octant walk alike
-  const uint32_t o = (dir.x < 0.0f ? 1u : 0u) | (dir.y < 0.0f ? 2u : 0u) | (dir.z < 0.0f ? 4u : 0u);
-  const uint32_t slot = atomicAdd(handoff + kBucketHead + o, 1u);
-  ua.bucket[o * ua.cap + slot] = i;  // slot < cap: at most cap rays in all
+  __syncthreads();
+  for (int level = 0; level < kUnitLevel; ++level) {
+    const bool in = t < n;
+    const uint32_t nid = in ? s_node[t] : 0u;
+    uint32_t sp = in ? s_sp[t] : 0u;
+    bool expand = false;
+    uint32_t w0 = 0, w1 = 0;
+    if (in && !(sp & kDone)) {
+      if (nid < node_count) {
+        w0 = nodes[nid].w0;
+        w1 = nodes[nid].w1;
+        expand = !rk::node_is_leaf(w0);
+      }
+      if (!expand) sp |= kDone;
+    }
+    const uint64_t em = __ballot(expand);
+    if (lane == 0) s_wave[wv] = (uint32_t)__popcll(em);
+    __syncthreads();  // also: every entry has been read
+    uint32_t before = (uint32_t)__popcll(em & rk::lanemask_lt()), total = 0;
+    for (uint32_t w = 0; w < 4; ++w) {
+      if (w < wv) before += s_wave[w];
+      total += s_wave[w];
+    }
+    if (in) {
+      const uint32_t at = t + before;
+      if (expand) {
+        const uint32_t ax = rk::node_axis(w0);
+        const bool neg = ax <= 1u ? ((o >> ax) & 1u) != 0u : (o & 4u) != 0u;  // children_order
+        s_node[at] = neg ? w1 + 1u : w1;
+        s_sp[at] = sp + 1u;
+        s_node[at + 1] = neg ? w1 : w1 + 1u;
+        s_sp[at + 1] = sp;
+        cut->top[o][tops + before] = nid;
+      } else {
+        s_node[at] = nid;
+        s_sp[at] = sp;
+      }
+    }
+    n += total;
+    tops += total;
+    __syncthreads();
+  }
+  if (t < n) {
+    cut->node[o][t] = s_node[t];
+    cut->sp[o][t] = s_sp[t] & ~kDone;
+  }
+  if (t == 0) {
+    cut->units[o] = n;
+    cut->tops[o] = tops;
+  }
 }
 
 // The walk of ray l by the whole wave with the reference's rules (the same
@@ -715,18 +723,19 @@ __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint3
   return r;
 }
 
-// The second pass of the per-ray traversal: one wave per ray handed off, its
-// walk again from the root.
+// The second pass of the per-ray traversal: one wave per ray handed off (and
+// per crossing ray whose split walk did not fit), its walk again from the root.
 __global__ __launch_bounds__(64) void k_trace_ray_wave(const rk::Node* __restrict__ nodes,
                                                        RefMesh mesh,
                                                        const float4* __restrict__ origins,
                                                        const float4* __restrict__ dirs, uint32_t node_count,
                                                        uint32_t face_count, const uint32_t* __restrict__ handoff,
-                                                       uint32_t handoff_cap, uint32_t* __restrict__ faces_id,
+                                                       uint32_t handoff_cap, const uint32_t* __restrict__ redo,
+                                                       uint32_t redo_cap, uint32_t* __restrict__ faces_id,
                                                        float2* __restrict__ coords, float* __restrict__ depths) {
-  const uint32_t count = min(handoff[0], handoff_cap);
-  for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    const uint32_t l = handoff[kHandoffHead + i];
+  const uint32_t count = min(handoff[0], handoff_cap), again = min(handoff[4], redo_cap);
+  for (uint32_t i = blockIdx.x; i < count + again; i += gridDim.x) {
+    const uint32_t l = i < count ? handoff[kHandoffHead + i] : redo[i - count];
     const WalkResult r = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, mesh, origins, dirs,
                                    node_count, face_count);
     if (threadIdx.x == 0) {
@@ -737,145 +746,215 @@ __global__ __launch_bounds__(64) void k_trace_ray_wave(const rk::Node* __restric
   }
 }
 
-// The subtrees of the split rays, by groups of up to 64 rays of one octant:
-// one wave per group and subtree, lane r on the group's ray r. The rays of a
-// group walk alike (children_order depends on the octant only, and their box
-// tests pass at t = +-0 while their depth is above 0), so the wave walks the
-// subtree once, from the root its first ray (the leader) recorded: a node is
-// visited when a ray still walking (not diverged, depth above 0) passes its
-// box test, and a ray still walking that fails a visited node's test has left
-// the group's walk (diverged: the ray is walked again by one wave). A leaf's
-// faces go to LDS 64 at a time, and each ray tests them in face order against
-// its own depth, as the reference does. A ray whose subtree list differs from
-// the leader's is marked diverged too. Each ray gets its UnitResult.
-template <int kUW>
-__global__ __launch_bounds__(64 * kUW) void k_units_walk(const rk::Node* __restrict__ nodes,
-                                                   RefMesh mesh,
-                                                   const float4* __restrict__ origins,
-                                                   const float4* __restrict__ dirs, const float* __restrict__ depths,
-                                                   uint32_t node_count, uint32_t face_count,
-                                                   const uint32_t* __restrict__ handoff, UnitArgs ua) {
-  __shared__ float4 s_v0[64 * kUW], s_e1[64 * kUW], s_e2[64 * kUW];
-  __shared__ float4 s_part[kUW > 1 ? 64 * kUW : 1];  // a wave's first smallest (t, u, v, face) per ray
-  const int lane = (int)threadIdx.x & 63, wv = (int)threadIdx.x >> 6;
-  uint32_t bcount[8], groups = 0;
-#pragma unroll
-  for (int o = 0; o < 8; ++o) {
-    bcount[o] = handoff[kBucketHead + o];
-    groups += (bcount[o] + 63u) / 64u;
+// Uniform data through the scalar cache: read-only for the whole kernel.
+typedef uint32_t u32x8 __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ u32x8 load_uniform32(const void* p) {
+  return *(const __attribute__((address_space(4))) u32x8*)(uintptr_t)p;
+}
+__device__ __forceinline__ NodeRegs load_node_uniform(const rk::Node* __restrict__ nodes, uint32_t id) {
+  const u32x8 a = load_uniform32(nodes + __builtin_amdgcn_readfirstlane(id));
+  NodeRegs r;
+  r.w0 = a[0];
+  r.w1 = a[1];
+  r.bmin = make_float4(__uint_as_float(a[2]), __uint_as_float(a[3]), __uint_as_float(a[4]), 0.0f);
+  r.bmax = make_float4(__uint_as_float(a[5]), __uint_as_float(a[6]), __uint_as_float(a[7]), 0.0f);
+  return r;
+}
+__device__ __forceinline__ rk::FaceBound load_bound_uniform(const rk::FaceBound* __restrict__ p, uint32_t g) {
+  const u32x8 a = load_uniform32(p + __builtin_amdgcn_readfirstlane(g));
+  return rk::FaceBound{__uint_as_float(a[0]), __uint_as_float(a[1]), __uint_as_float(a[2]), __uint_as_float(a[3]),
+                       __uint_as_float(a[4]), __uint_as_float(a[5]), __uint_as_float(a[6]), __uint_as_float(a[7])};
+}
+
+// Faces [first, first + cnt) against the wave's rays, one per lane (test: the
+// lanes that have one), in face order, each lane keeping hits with t < its
+// depth. A group's bound is tested by every lane; the faces of a group that
+// some ray may hit are fetched one per lane and handed round by readlane.
+__device__ __forceinline__ void group_leaf(const RefMesh& mesh, uint32_t first, uint32_t cnt, bool test, float4 o,
+                                           float4 d, const rk::CullRay& cr, float& depth, uint32_t& fid,
+                                           float2& coord) {
+  if (cnt == 0u) return;
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t end = first + cnt, g_end = (end - 1u) / kGroup + 1u;
+  for (uint32_t s0 = first / kGroup; s0 < g_end;) {
+    // up to four groups at a time: all of them are missed by every ray of the
+    // wave when their common bound is
+    const uint32_t s1 = min(g_end, (s0 / kSuper + 1u) * kSuper);
+    bool near = test;
+    if (mesh.supers) {
+      const rk::FaceBound sb = load_bound_uniform(mesh.supers, s0 / kSuper);
+      near = test && !rk::bound_missed(sb, o.x, o.y, o.z, d.x, d.y, d.z, cr, depth);
+    }
+    if (__ballot(near) != 0ull) {
+      for (uint32_t g = s0; g < s1; ++g) {
+        bool hit = near;
+        if (mesh.bounds) {
+          const rk::FaceBound gb = load_bound_uniform(mesh.bounds, g);
+          hit = near && !rk::bound_missed(gb, o.x, o.y, o.z, d.x, d.y, d.z, cr, depth);
+        }
+        if (__ballot(hit) == 0ull) continue;
+        const uint32_t f0 = max(first, g * kGroup), nf = g * kGroup + min(end - g * kGroup, kGroup) - f0;
+        float4 v0, e1, e2;
+        tri_get(mesh, f0 + min(lane, nf - 1u), v0, e1, e2);
+        for (uint32_t q = 0; q < nf; ++q) {
+          const float4 qv0 = make_float4(readlane_f32(v0.x, q), readlane_f32(v0.y, q), readlane_f32(v0.z, q), 0.0f);
+          const float4 qe1 = make_float4(readlane_f32(e1.x, q), readlane_f32(e1.y, q), readlane_f32(e1.z, q), 0.0f);
+          const float4 qe2 = make_float4(readlane_f32(e2.x, q), readlane_f32(e2.y, q), readlane_f32(e2.z, q), 0.0f);
+          float t, u, v;
+          if (hit && tri_ray(o, d, qv0, qe1, qe2, t, u, v)) {
+            if (t < depth) { fid = f0 + q; coord = make_float2(u, v); depth = t; }
+          }
+        }
+      }
+    }
+    s0 = s1;
   }
-  const uint32_t jobs = groups * kUnits;
+}
+
+constexpr int kPW = 16, kPH = 12, kPT = kPW * kPH;  // PACKET_BLOCK_*, :47-49
+constexpr int kPStack = 128;                       // PACKET_STACK_SIZE, :51
+constexpr uint32_t kPGroups = kPT / 64;            // groups of a packet
+// A packet's record: sp, visits, the forcing ray (the first ray of the
+// packet that passes every box test, or kNone), its forced slot (or kNone;
+// kDone once the forced walk's results are in the outputs), the stack.
+constexpr uint32_t kPStateWords = kPStack + 4;
+constexpr uint32_t kDone = 0xfffffffeu;
+
+// The image and the packets' records, for k_unit_walk on forced packets.
+struct PacketArgs {
+  int width, height, packets_x;
+  uint32_t handoff_cap;
+  const uint32_t* forced;  // [cap] each forced packet's place in the hand-off list
+};
+
+// One wave per group of 64 rays and subtree, lane r on the group's ray r; the
+// wave walks the subtree once, and every ray tests the leaves' faces in face
+// order against its own depth, as the reference does.
+//
+// Crossing rays (kPacket false), groups of one octant: a node is visited when
+// a ray still walking (not diverged, depth above 0) passes its box test; a ray
+// still walking that fails a visited node's test is marked diverged.
+// Packets: a node is visited when the forcing ray passes its box test, and
+// the packet is marked diverged when it does not.
+//
+// The subtrees' boxes above the cut are checked by the first subtree's wave.
+template <bool kPacket>
+__global__ __launch_bounds__(64) void k_unit_walk(const rk::Node* __restrict__ nodes, RefMesh mesh,
+                                                  const float4* __restrict__ origins, const float4* __restrict__ dirs,
+                                                  const float* __restrict__ depths, uint32_t node_count,
+                                                  uint32_t face_count, uint32_t* __restrict__ handoff, UnitArgs ua,
+                                                  PacketArgs pa) {
+  const int lane = (int)threadIdx.x;
+  uint32_t bcount[8], groups = 0;
+  if (kPacket) {
+    groups = min(handoff[2], ua.cap) * kPGroups;
+  } else {
+#pragma unroll
+    for (int o = 0; o < 8; ++o) {
+      bcount[o] = handoff[kBucketHead + o];
+      groups += (bcount[o] + 63u) / 64u;
+    }
+  }
+  const uint64_t jobs = (uint64_t)groups * kUnits;
   const uint32_t max_visits = 2 * node_count + 2;
-  for (uint32_t jj = blockIdx.x; jj < jobs; jj += gridDim.x) {
+  constexpr uint32_t kLimit = kPacket ? (uint32_t)kPStack : (uint32_t)kStack;
+  for (uint64_t jj = blockIdx.x; jj < jobs; jj += gridDim.x) {
     // subtree k of every group before subtree k + 1 of any: the waves running
     // together walk the same part of the tree and share it in the L2
-    const uint32_t k = jj / groups;
-    uint32_t g = jj % groups, o = 0;
-    while (g >= (bcount[o] + 63u) / 64u) {
-      g -= (bcount[o] + 63u) / 64u;
-      ++o;
+    const uint32_t k = (uint32_t)(jj / groups), g = (uint32_t)(jj % groups);
+    uint32_t o = 0, slot = 0, l = 0, div = 0;  // octant, this lane's slot and ray, its mark
+    bool has_ray = false;
+    float4 borig, bdir, border;  // the ray whose boxes are tested, and the one that gives the order
+    if (kPacket) {
+      const uint32_t f = g / kPGroups, rslot = pa.forced[f];
+      const uint32_t* rec = handoff + kHandoffHead + pa.handoff_cap + (size_t)rslot * kPStateWords;
+      const uint32_t pk = handoff[kHandoffHead + rslot], R = rec[2];
+      const int x0 = (int)(pk % (uint32_t)pa.packets_x) * kPW, y0 = (int)(pk / (uint32_t)pa.packets_x) * kPH;
+      const int q = (int)(g % kPGroups) * 64 + lane, x = x0 + q % kPW, y = y0 + q / kPW;
+      has_ray = x < pa.width && y < pa.height;
+      l = has_ray ? (uint32_t)y * (uint32_t)pa.width + (uint32_t)x : 0u;
+      slot = f * (uint32_t)kPT + (uint32_t)q;
+      div = f;
+      const uint32_t lr = (uint32_t)(y0 + (int)R / kPW) * (uint32_t)pa.width + (uint32_t)(x0 + (int)R % kPW);
+      borig = origins[lr];
+      bdir = dirs[lr];
+      border = dirs[(uint32_t)y0 * (uint32_t)pa.width + (uint32_t)x0];
+      o = octant_of(border);
+    } else {
+      uint32_t gg = g;
+      while (gg >= (bcount[o] + 63u) / 64u) {
+        gg -= (bcount[o] + 63u) / 64u;
+        ++o;
+      }
+      has_ray = gg * 64u + (uint32_t)lane < bcount[o];
+      slot = has_ray ? ua.bucket[o * ua.cap + gg * 64u + (uint32_t)lane] : 0u;
+      l = has_ray ? ua.list[slot] : 0u;
+      div = slot;
     }
-    const uint32_t n_in = min(64u, bcount[o] - g * 64u);
-    const bool has_ray = (uint32_t)lane < n_in;
-    const uint32_t i = has_ray ? ua.bucket[o * ua.cap + g * 64u + (uint32_t)lane] : 0u;
-    const uint32_t lead = readlane_u32(i, 0);
-    const uint32_t nu_lead = ua.nunits[lead];
-    if (k == 0 && has_ray && wv == 0 && ua.nunits[i] != nu_lead) ua.diverged[i] = 1u;
-    if (k >= nu_lead) continue;
-    const uint32_t root = ua.unit_node[lead * kUnits + k], sp_base = ua.unit_sp[lead * kUnits + k];
-    bool walking = has_ray && ua.nunits[i] == nu_lead && ua.unit_node[i * kUnits + k] == root &&
-                   ua.unit_sp[i * kUnits + k] == sp_base;
-    bool diverged = has_ray && !walking;
-    const uint32_t l = has_ray ? ua.list[i] : 0u;
+    o = __builtin_amdgcn_readfirstlane(o);
+    if (k >= ua.cut->units[o]) continue;
     const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     const float4 orig = has_ray ? origins[l] : zero4, dir = has_ray ? dirs[l] : zero4;
-    const float4 invdir = has_ray ? invdir_of(dir) : zero4;
+    if (!kPacket) {
+      borig = orig;
+      bdir = dir;
+      border = readlane_f4(dir, 0);  // the octant's
+    }
+    const float4 binv = invdir_of(bdir);
+    const rk::CullRay cr = cull_ray4(orig, dir);
     float depth = has_ray ? depths[l] : 0.0f;
-    const float4 dir0 = readlane_f4(dir, 0);  // the octant's: the leader's direction
-    const float4 orig0 = readlane_f4(orig, 0);
-    // rays from one camera share their origin: tvec once per face
-    const bool shared = RK_REF_SHARED_TVEC && __ballot(has_ray && !same_bits(orig, orig0)) == 0ull;
-    uint32_t fid = kNoFace;
+    uint32_t fid = kNone;
     float2 coord = make_float2(0.0f, 0.0f);
+    bool walking = has_ray, diverged = false;
+    if (k == 0) {  // every box above the cut, at the starting depth
+      const uint32_t tops = ua.cut->tops[o];
+      for (uint32_t i = 0; i < tops; ++i) {
+        const NodeRegs nd = load_node_uniform(nodes, ua.cut->top[o][i]);
+        float t;
+        if (!(box_ray(nd.bmin, nd.bmax, borig, binv, t) && (kPacket || t < depth))) diverged = true;
+      }
+      if (!kPacket && diverged) walking = false;
+    }
+    const uint32_t root = ua.cut->node[o][k], sp_base = ua.cut->sp[o][k];
     uint32_t st0 = lane == 0 ? root : 0u, st1 = 0u;
     int sp = 1;
     uint32_t visits = 0;
-    bool stopped = false;
     while (sp > 0 && ++visits <= max_visits) {
-      if (__ballot(walking && depth > 0.0f) == 0ull) break;  // every ray's result here is final
+      if (!kPacket && __ballot(walking && depth > 0.0f) == 0ull) break;  // every ray's result here is final
       --sp;
       const uint32_t nid = readlane_u32(sp < 64 ? st0 : st1, sp & 63);
       if (nid >= node_count) {  // never taken for a tree built by this library
-        stopped = true;
+        diverged = true;
         break;
       }
-      const NodeRegs nd = load_node(nodes, nid);
+      const NodeRegs nd = load_node_uniform(nodes, nid);
       if (rk::node_is_leaf(nd.w0)) {
         const uint32_t first = nd.w1;
         const uint32_t cnt = first < face_count ? min(rk::leaf_count(nd.w0), face_count - first) : 0u;
-        // Batches of 64 * kUW faces; wave w tests [w * 64, w * 64 + 64) of each,
-        // keeping its first smallest t below the depth at the batch's start,
-        // and the waves' results are merged in wave order: a sequential pass
-        // keeping t < depth ends on the same face (the first of smallest t).
-        for (uint32_t c0 = 0; c0 < cnt; c0 += 64u * kUW) {
-          const uint32_t cc = min(64u * kUW, cnt - c0);
-          if (threadIdx.x < cc) {
-            float4 v0, e1, e2;
-            tri_get(mesh, first + c0 + threadIdx.x, v0, e1, e2);
-            s_v0[threadIdx.x] = shared ? rk::sub4(orig0, v0) : v0;  // tvec, or v0
-            s_e1[threadIdx.x] = e1;
-            s_e2[threadIdx.x] = e2;
-          }
-          __syncthreads();
-          const uint32_t q0 = (uint32_t)wv * 64u, q1 = min(cc, q0 + 64u);
-          float pt = depth, pu = 0.0f, pv = 0.0f;
-          uint32_t pq = 0xFFFFFFFFu;  // none
-          if (walking) {
-            if (shared) {
-              for (uint32_t q = q0; q < q1; ++q) {
-                float t, u, v;
-                if (tri_ray_tv(dir, s_v0[q], s_e1[q], s_e2[q], t, u, v)) {
-                  if (t < pt) { pq = q; pu = u; pv = v; pt = t; }
-                }
-              }
-            } else {
-              for (uint32_t q = q0; q < q1; ++q) {
-                float t, u, v;
-                if (tri_ray(orig, dir, s_v0[q], s_e1[q], s_e2[q], t, u, v)) {
-                  if (t < pt) { pq = q; pu = u; pv = v; pt = t; }
-                }
-              }
-            }
-          }
-          if (kUW == 1) {
-            if (pq != 0xFFFFFFFFu) { fid = first + c0 + pq; coord = make_float2(pu, pv); depth = pt; }
-          } else {
-            s_part[threadIdx.x] = make_float4(pt, pu, pv, __uint_as_float(pq));
-            __syncthreads();
-            if (walking) {
-#pragma unroll
-              for (int w = 0; w < kUW; ++w) {
-                const float4 r = s_part[w * 64 + lane];
-                const uint32_t rq = __float_as_uint(r.w);
-                if (rq != 0xFFFFFFFFu && r.x < depth) { fid = first + c0 + rq; coord = make_float2(r.y, r.z); depth = r.x; }
-              }
-            }
-          }
-          __syncthreads();
-        }
+        group_leaf(mesh, first, cnt, walking, orig, dir, cr, depth, fid, coord);
       } else {
         float t;
-        const bool pass = box_ray(nd.bmin, nd.bmax, orig, invdir, t) && t < depth;
-        const bool live = walking && depth > 0.0f;  // at depth 0 a ray's result is final
-        if (__ballot(live && pass) != 0ull) {
-          if (live && !pass) {
+        bool pass = box_ray(nd.bmin, nd.bmax, borig, binv, t);
+        bool visit;
+        if (kPacket) {
+          visit = __ballot(pass) != 0ull;  // the same in every lane
+          if (!visit) diverged = true;
+        } else {
+          pass = pass && t < depth;
+          const bool live = walking && depth > 0.0f;  // at depth 0 a ray's result is final
+          visit = __ballot(live && pass) != 0ull;
+          if (visit && live && !pass) {
             walking = false;
             diverged = true;
           }
+        }
+        if (visit) {
           uint32_t nearc, farc;
-          children_order(nd.w0, nd.w1, dir0, nearc, farc);
-          if ((uint32_t)sp + sp_base + 2u > (uint32_t)kStack) {  // cannot occur for trees of depth <= 94
-            stopped = true;
+          children_order(nd.w0, nd.w1, border, nearc, farc);
+          nearc = __builtin_amdgcn_readfirstlane(nearc);
+          farc = __builtin_amdgcn_readfirstlane(farc);
+          if ((uint32_t)sp + sp_base + 2u > kLimit) {  // cannot occur for trees of depth <= 94
+            diverged = true;
             break;
           }
           if (lane == (sp & 63)) {
@@ -891,64 +970,70 @@ __global__ __launch_bounds__(64 * kUW) void k_units_walk(const rk::Node* __restr
         }
       }
     }
-    if (has_ray && wv == 0) {
-      if (diverged) ua.diverged[i] = 1u;
-      UnitResult r;
-      r.t = depth;
-      r.u = coord.x;
-      r.v = coord.y;
-      r.face = fid;
-      r.pops = visits;
-      r.flags = stopped ? kUnitStop : 0u;
-      r.pad0 = 0u;
-      r.pad1 = 0u;
-      ua.res[i * kUnits + k] = r;
+    if (lane == 0) atomicAdd(ua.pops + g, (unsigned long long)visits);
+    const bool hit = has_ray && fid != kNone;
+    const uint64_t hm = __ballot(hit);
+    if (hm != 0ull) {
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(handoff + 3, (uint32_t)__popcll(hm));
+      base = __builtin_amdgcn_readfirstlane(base);
+      if (hit) {
+        const uint32_t e = base + (uint32_t)__popcll(hm & rk::lanemask_lt());
+        if (e < ua.hit_cap) {
+          UnitHit h;
+          h.t = depth;
+          h.u = coord.x;
+          h.v = coord.y;
+          h.face = fid;
+          h.unit = k;
+          h.next = atomicExch(ua.head + slot, e);
+          ua.hits[e] = h;
+        } else {
+          diverged = true;
+        }
+      }
     }
+    if (diverged && has_ray) ua.diverged[div] = 1u;
   }
 }
 
-// The split rays' results: the subtrees' results merged in walk order (the
-// first smallest t below the depth so far wins; a subtree that stopped ends
-// the walk), when the pops add up to no more than the visit limit; else the
-// ray's walk by the whole wave.
-__global__ __launch_bounds__(64) void k_units_merge(const rk::Node* __restrict__ nodes,
-                                                    RefMesh mesh,
-                                                    const float4* __restrict__ origins,
-                                                    const float4* __restrict__ dirs, uint32_t node_count,
-                                                    uint32_t face_count, const uint32_t* __restrict__ handoff,
-                                                    UnitArgs ua, uint32_t* __restrict__ faces_id,
-                                                    float2* __restrict__ coords, float* __restrict__ depths) {
-  const uint32_t count = min(handoff[1], ua.cap);
+// A slot's result: of its entries, the smallest t, the first subtree's of
+// equal ones; false when it has none. Entries hold t below the starting depth.
+__device__ __forceinline__ bool unit_best(const UnitArgs& ua, uint32_t slot, UnitHit& best) {
+  bool any = false;
+  uint32_t e = ua.head[slot];
+  for (uint32_t n = 0; e != kNone && n < kUnits; ++n) {
+    const UnitHit h = ua.hits[e];
+    if (!any || h.t < best.t || (h.t == best.t && h.unit < best.unit)) best = h;
+    any = true;
+    e = h.next;
+  }
+  return any;
+}
+
+// The crossing rays' results, one lane per ray; a diverged ray, or one of a
+// group whose pops pass the visit limit, goes on the list to walk again.
+__global__ __launch_bounds__(64) void k_units_merge(uint32_t node_count, uint32_t* __restrict__ handoff, UnitArgs ua,
+                                                    uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
+                                                    float* __restrict__ depths) {
   const uint64_t max_visits = 2 * node_count + 2;
-  for (uint32_t i = blockIdx.x; i < count; i += gridDim.x) {
-    const uint32_t l = ua.list[i];
-    float depth = depths[l];
-    uint32_t fid = faces_id[l];
-    float2 coord = coords[l];
-    uint64_t pops = ua.top_pops[i];
-    const uint32_t nu = ua.diverged[i] != 0u ? 0u : ua.nunits[i];  // a diverged ray's results may be missing
-    for (uint32_t k = 0; k < nu; ++k) {
-      const UnitResult r = ua.res[(size_t)i * kUnits + k];
-      pops += r.pops;
-      if (r.face != kNoFace && r.t < depth) {
-        depth = r.t;
-        fid = r.face;
-        coord = make_float2(r.u, r.v);
+  uint32_t group0 = 0;
+  for (uint32_t o = 0; o < 8; ++o) {
+    const uint32_t n = handoff[kBucketHead + o];
+    for (uint32_t i = blockIdx.x * 64u + threadIdx.x; i < n; i += gridDim.x * 64u) {
+      const uint32_t slot = ua.bucket[o * ua.cap + i], l = ua.list[slot];
+      if (ua.diverged[slot] != 0u || ua.pops[group0 + i / 64u] + ua.cut->tops[o] > max_visits) {
+        ua.redo[atomicAdd(handoff + 4, 1u)] = l;  // at most cap rays
+        continue;
       }
-      if (r.flags & kUnitStop) break;
+      UnitHit h;
+      if (unit_best(ua, slot, h)) {
+        faces_id[l] = h.face;
+        coords[l] = make_float2(h.u, h.v);
+        depths[l] = h.t;
+      }
     }
-    if (pops > max_visits || ua.diverged[i] != 0u) {
-      const WalkResult w = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, mesh, origins, dirs,
-                                   node_count, face_count);
-      depth = w.depth;
-      fid = w.fid;
-      coord = w.coord;
-    }
-    if (threadIdx.x == 0) {
-      faces_id[l] = fid;
-      coords[l] = coord;
-      depths[l] = depth;
-    }
+    group0 += (n + 63u) / 64u;
   }
 }
 
@@ -959,10 +1044,6 @@ __global__ __launch_bounds__(64) void k_units_merge(const rk::Node* __restrict__
 #ifndef RK_REF_COOP_MAX
 #define RK_REF_COOP_MAX 16
 #endif
-
-constexpr int kPW = 16, kPH = 12, kPT = kPW * kPH;  // PACKET_BLOCK_*, :47-49
-constexpr int kPStack = 128;                       // PACKET_STACK_SIZE, :51
-constexpr int kPCache = 224;                       // TRIANGLES_MAX, :39
 
 // One packet of the packet traversal (kernel_raytraceMeshTreePacket,
 // :222-377): the block walks the tree once for its 16x12 rays, visiting a
@@ -981,21 +1062,15 @@ constexpr int kPCache = 224;                       // TRIANGLES_MAX, :39
 // back on top, sp and the visits before that leaf's pop (so that the second
 // pass, given the record as resume, makes the same pops from there). Returns
 // whether it was.
-// A packet's record: sp, visits, the forcing ray (the first ray of the
-// packet that passes every box test, or kNone), its forced slot (or kNone;
-// kDone once the forced walk's results are in the outputs), the stack.
-constexpr uint32_t kPStateWords = kPStack + 4;
-constexpr uint32_t kNone = 0xffffffffu, kDone = 0xfffffffeu;
-
 template <int kS>
 __device__ __forceinline__ bool trace_packet_job(
     const rk::Node* __restrict__ nodes, RefMesh mesh,
     const float4* __restrict__ origins, const float4* __restrict__ dirs, int width, int height, uint32_t node_count,
     uint32_t face_count, uint32_t* __restrict__ faces_id, float2* __restrict__ coords, float* __restrict__ depths,
     int bx, int by, uint32_t* __restrict__ handoff, uint32_t handoff_cap, uint32_t handoff_faces,
-    uint32_t* __restrict__ state, uint32_t* __restrict__ forced_list, uint32_t forced_cap,
-    const uint32_t* __restrict__ resume, uint32_t* s_stack, float4* s_dir0, uint32_t* s_slot, float* s_pt, float* s_pu, float* s_pv,
-    uint32_t* s_pk) {
+    uint32_t* __restrict__ state, uint32_t* __restrict__ forced_list, UnitArgs ua,
+    const uint32_t* __restrict__ resume, uint32_t* s_stack, float4* s_dir0, uint32_t* s_slot, float* s_pt,
+    float* s_pu, float* s_pv, uint32_t* s_pk) {
   const int ray = (int)threadIdx.x % kPT, part = (int)threadIdx.x / kPT;
   const int tx = ray % kPW, ty = ray / kPW;
   const int x = bx * kPW + tx, y = by * kPH + ty;
@@ -1026,14 +1101,50 @@ __device__ __forceinline__ bool trace_packet_job(
     if (!resume) s_stack[0] = 0;
   }
   bool may_hand_off = handoff_cap != 0u;
-  uint32_t limit = handoff_faces, forcer = kNone;
-  if (may_hand_off) {  // a packet holding a ray that passes every box test visits every node
+  // Hands the packet off where it stands (stack s_stack[0 .. sp), visits):
+  // false when the list is full. f: its place among the forced packets.
+  auto hand_off = [&](uint32_t forcer) {
+    __syncthreads();  // s_slot and s_stack are settled
+    if (threadIdx.x == 0) {
+      const uint32_t slot = atomicAdd(handoff, 1u);
+      if (slot < handoff_cap) {
+        handoff[kHandoffHead + slot] = (uint32_t)by * gridDim.x + (uint32_t)bx;
+        uint32_t f = kNone;
+        if (forcer != kNone) {
+          f = atomicAdd(handoff + 2, 1u);
+          if (f < ua.cap) {
+            forced_list[f] = slot;
+            ua.diverged[f] = 0u;
+          } else {
+            f = kNone;
+          }
+        }
+        uint32_t* rec = state + (size_t)slot * kPStateWords;
+        rec[0] = (uint32_t)sp;
+        rec[1] = visits;
+        rec[2] = f != kNone ? forcer : kNone;
+        rec[3] = f;
+      }
+      *s_slot = slot;
+    }
+    __syncthreads();
+    const uint32_t slot = *s_slot;
+    if (slot >= handoff_cap) return false;
+    uint32_t* rec = state + (size_t)slot * kPStateWords;
+    for (int k = (int)threadIdx.x; k < sp; k += kPT * kS) rec[4 + k] = s_stack[k];
+    if (forcer != kNone && rec[3] != kNone) ua.head[rec[3] * (uint32_t)kPT + (uint32_t)ray] = kNone;
+    return true;
+  };
+  if (may_hand_off) {  // a packet holding a ray that passes every box test visits every node: at once
     if (threadIdx.x == 0) *s_slot = kNone;
     __syncthreads();
     if (in_image && part == 0 && crosses_every_box(invdir)) atomicMin(s_slot, (uint32_t)ray);
     __syncthreads();
-    forcer = *s_slot;
-    if (forcer != kNone) limit = 0u;
+    const uint32_t forcer = *s_slot;
+    if (forcer != kNone) {
+      may_hand_off = false;
+      if (hand_off(forcer)) return true;
+    }
   }
   __syncthreads();
   const float4 dir0 = *s_dir0;
@@ -1047,32 +1158,11 @@ __device__ __forceinline__ bool trace_packet_job(
       const uint32_t tri_id = nd.w1;
       const uint32_t cnt = tri_id < face_count ? min(rk::leaf_count(nd.w0), face_count - tri_id) : 0u;
       if (may_hand_off) {
-        if (cnt > limit - tested) {
+        if (cnt > handoff_faces - tested) {
           may_hand_off = false;
-          if (threadIdx.x == 0) {
-            const uint32_t slot = atomicAdd(handoff, 1u);
-            if (slot < handoff_cap) handoff[kHandoffHead + slot] = (uint32_t)by * gridDim.x + (uint32_t)bx;
-            *s_slot = slot;
-          }
-          __syncthreads();
-          const uint32_t slot = *s_slot;
-          __syncthreads();
-          if (slot < handoff_cap) {
-            uint32_t* rec = state + (size_t)slot * kPStateWords;
-            for (int k = (int)threadIdx.x; k < sp; k += kPT * kS) rec[4 + k] = s_stack[k];
-            if (threadIdx.x == 0) {
-              rec[0] = (uint32_t)sp + 1u;  // sp < kPStack after the pop: the leaf fits
-              rec[1] = visits - 1u;
-              rec[4 + sp] = nid;
-              uint32_t f = kNone;
-              if (forcer != kNone) {
-                f = atomicAdd(handoff + 2, 1u);
-                if (f < forced_cap) forced_list[f] = slot;
-                else f = kNone;
-              }
-              rec[2] = f != kNone ? forcer : kNone;
-              rec[3] = f;
-            }
+          ++sp;  // the leaf goes back on top (s_stack still holds it), its pop is not counted
+          --visits;
+          if (hand_off(kNone)) {
             if (in_image && part == 0) {
               faces_id[l] = fid;
               coords[l] = coord;
@@ -1080,6 +1170,8 @@ __device__ __forceinline__ bool trace_packet_job(
             }
             return true;
           }
+          --sp;
+          ++visits;
         } else {
           tested += cnt;
         }
@@ -1152,13 +1244,13 @@ __global__ __launch_bounds__(kPT) void k_trace_packet(const rk::Node* __restrict
                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
                                                       float* __restrict__ depths, uint32_t* __restrict__ handoff,
                                                       uint32_t handoff_cap, uint32_t handoff_faces,
-                                                      uint32_t* __restrict__ forced_list, uint32_t forced_cap) {
+                                                      uint32_t* __restrict__ forced_list, UnitArgs ua) {
   __shared__ uint32_t s_stack[kPStack];
   __shared__ float4 s_dir0;
   __shared__ uint32_t s_slot;
   trace_packet_job<1>(nodes, mesh, origins, dirs, width, height, node_count, face_count, faces_id, coords,
                       depths, (int)blockIdx.x, (int)blockIdx.y, handoff, handoff_cap, handoff_faces,
-                      handoff + kHandoffHead + handoff_cap, forced_list, forced_cap, nullptr, s_stack, &s_dir0,
+                      handoff + kHandoffHead + handoff_cap, forced_list, ua, nullptr, s_stack, &s_dir0,
                       &s_slot, nullptr, nullptr, nullptr, nullptr);
 }
 
@@ -1186,179 +1278,54 @@ __global__ __launch_bounds__(kPT * kPacketSplit) void k_trace_packet_split(
     if (rec[3] == kDone) continue;  // traced by the forced walk
     trace_packet_job<kPacketSplit>(nodes, mesh, origins, dirs, width, height, node_count, face_count,
                                    faces_id, coords, depths, (int)(pk % (uint32_t)packets_x),
-                                   (int)(pk / (uint32_t)packets_x), nullptr, 0u, 0u, nullptr, nullptr, 0u, rec,
+                                   (int)(pk / (uint32_t)packets_x), nullptr, 0u, 0u, nullptr, nullptr, UnitArgs{}, rec,
                                    s_stack, &s_dir0, &s_slot, s_pt, s_pu, s_pv, s_pk);
     __syncthreads();  // the next packet rewrites the stack and s_dir0
   }
 }
 
-// The packets holding a ray that passes every box test (the forcing ray), by
-// parts of kFRays rays on different CUs. While the forcing ray's depth is
-// above 0 it passes every box that box_ray passes (at t = +-0), so the packet
-// visits every such node, in the order its first ray gives, whatever its
-// other rays hold: each part walks that order from the packet's record on its
-// own, checking the forcing ray's box test at every node (a failure ends the
-// part: diverged), and each of its rays tests every face of every leaf in face
-// order against its own depth, kFParts threads per ray (consecutive faces of
-// each chunk each, merged in part order). The results go to temp;
-// k_packet_commit puts them in the outputs when no part diverged and the
-// forcing ray's final depth is above 0 (then it was above 0 all along), and
-// otherwise leaves the packet to k_trace_packet_split, from its record. On the
-// 1920x1080 heightfield (149 such packets), parts of 48, 24, 16 and 12 rays
-// gave 68.6, 47.4, 44.9 and 59.8 ms per frame (67.1 ms with all on one CU).
-#ifndef RK_REF_FORCED_RAYS
-#define RK_REF_FORCED_RAYS 16
-#endif
-constexpr int kFRays = RK_REF_FORCED_RAYS, kFThreads = kPT, kFParts = kFThreads / kFRays;
-constexpr int kFPackets = kPT / kFRays;  // parts of a packet
-constexpr uint32_t kForcedCap = 1024;    // forced packets per call
-constexpr uint32_t kForcedGrid = 2048;
+// The forced packets' results: into the outputs (and the packet's record
+// marked kDone) when no walk diverged, the pops keep to the visit limit and
+// the forcing ray's final depth is above 0 (then it was above 0 all along);
+// otherwise k_trace_packet_split walks the packet from its record.
+constexpr uint32_t kForcedCap = 1024;  // forced packets per call
+constexpr uint32_t kHitsPerSlot = 2;   // hit entries per forced packet's ray on average
+constexpr uint32_t kHitsPerRay = 32;   // and per crossing ray
 
-__global__ __launch_bounds__(kFThreads) void k_packet_forced(
-    const rk::Node* __restrict__ nodes, RefMesh mesh,
-    const float4* __restrict__ origins, const float4* __restrict__ dirs, int width, int height, int packets_x,
-    uint32_t node_count, uint32_t face_count, const uint32_t* __restrict__ handoff, uint32_t handoff_cap,
-    const uint32_t* __restrict__ forced_list, uint32_t forced_cap, float4* __restrict__ temp,
-    uint32_t* __restrict__ fflags, const uint32_t* __restrict__ faces_id, const float2* __restrict__ coords,
-    const float* __restrict__ depths) {
-  __shared__ uint32_t s_stack[kPStack];
-  __shared__ float4 s_v0[kPCache], s_e1[kPCache], s_e2[kPCache];
-  __shared__ float s_pt[kFThreads], s_pu[kFThreads], s_pv[kFThreads];
-  __shared__ uint32_t s_pk[kFThreads];
-  const uint32_t nf = min(handoff[2], forced_cap);
-  const uint32_t jobs = nf * (uint32_t)kFPackets;
-  const uint32_t* state = handoff + kHandoffHead + handoff_cap;
-  const uint32_t max_visits = 2 * node_count + 2;
-  const int r = (int)threadIdx.x % kFRays, fp = (int)threadIdx.x / kFRays;
-  for (uint32_t job = blockIdx.x; job < jobs; job += gridDim.x) {
-    const uint32_t f = job % nf, part = job / nf;  // part k of every packet before part k + 1 of any
-    const uint32_t slot = forced_list[f];
-    const uint32_t* rec = state + (size_t)slot * kPStateWords;
-    const uint32_t pk = handoff[kHandoffHead + slot];
-    const int bx = (int)(pk % (uint32_t)packets_x), by = (int)(pk / (uint32_t)packets_x);
-    const int q = (int)part * kFRays + r;  // the ray's place in the packet
-    const int x = bx * kPW + q % kPW, y = by * kPH + q / kPW;
-    const bool in_image = x < width && y < height;
-    const uint32_t l = in_image ? (uint32_t)(y * width + x) : 0u;
-    float4 orig = make_float4(0.f, 0.f, 0.f, 0.f), dir = orig;
-    float depth = 0.0f;
-    uint32_t fid = 0;
-    float2 coord = make_float2(0.f, 0.f);
-    if (in_image) {  // the hits so far, left in the outputs at the hand-off
-      orig = origins[l];
-      dir = dirs[l];
-      depth = depths[l];
-      fid = faces_id[l];
-      coord = coords[l];
-    }
-    const uint32_t R = rec[2];
-    const uint32_t lr = (uint32_t)((by * kPH + (int)R / kPW) * width + bx * kPW + (int)R % kPW);
-    const float4 orig_r = origins[lr], invdir_r = invdir_of(dirs[lr]);
-    const float4 dir0 = dirs[(uint32_t)(by * kPH) * (uint32_t)width + (uint32_t)(bx * kPW)];
-    int sp = (int)rec[0];
-    uint32_t visits = rec[1];
-    for (int k = (int)threadIdx.x; k < sp; k += kFThreads) s_stack[k] = rec[4 + k];
-    __syncthreads();
-    bool diverged = false;
-    while (sp > 0 && ++visits <= max_visits) {
-      const uint32_t nid = s_stack[--sp];
-      if (nid >= node_count) break;  // block-uniform; never taken for a tree built by this library
-      const NodeRegs nd = load_node(nodes, nid);
-      if (rk::node_is_leaf(nd.w0)) {
-        const uint32_t tri_id = nd.w1;
-        const uint32_t cnt = tri_id < face_count ? min(rk::leaf_count(nd.w0), face_count - tri_id) : 0u;
-        for (uint32_t c0 = 0; c0 < cnt; c0 += kPCache) {
-          const uint32_t cc = (cnt - c0) < (uint32_t)kPCache ? (cnt - c0) : (uint32_t)kPCache;
-          __syncthreads();
-          for (uint32_t k = threadIdx.x; k < cc; k += kFThreads) {
-            float4 v0, e1, e2;
-            tri_get(mesh, tri_id + c0 + k, v0, e1, e2);
-            s_v0[k] = v0;
-            s_e1[k] = e1;
-            s_e2[k] = e2;
-          }
-          __syncthreads();
-          const uint32_t qn = (cc + kFParts - 1) / kFParts;
-          const uint32_t k0 = (uint32_t)fp * qn, k1 = min(cc, k0 + qn);
-          float pt = depth, pu = 0.0f, pv = 0.0f;
-          uint32_t pkf = kNone;
-          if (in_image) {
-            for (uint32_t k = k0; k < k1; ++k) {
-              float t, u, v;
-              if (tri_ray(orig, dir, s_v0[k], s_e1[k], s_e2[k], t, u, v)) {
-                if (t < pt) { pkf = k; pu = u; pv = v; pt = t; }
-              }
-            }
-          }
-          s_pt[threadIdx.x] = pt;
-          s_pu[threadIdx.x] = pu;
-          s_pv[threadIdx.x] = pv;
-          s_pk[threadIdx.x] = pkf;
-          __syncthreads();
-          if (in_image) {
-#pragma unroll
-            for (int p2 = 0; p2 < kFParts; ++p2) {
-              const int o = p2 * kFRays + r;
-              const uint32_t k = s_pk[o];
-              if (k != kNone && s_pt[o] < depth) {
-                depth = s_pt[o];
-                fid = tri_id + c0 + k;
-                coord = make_float2(s_pu[o], s_pv[o]);
-              }
-            }
-          }
-        }
-        __syncthreads();
-      } else {
-        float t;
-        if (!box_ray(nd.bmin, nd.bmax, orig_r, invdir_r, t)) {  // block-uniform
-          diverged = true;
-          break;
-        }
-        uint32_t nearc, farc;
-        children_order(nd.w0, nd.w1, dir0, nearc, farc);
-        if (sp + 2 > kPStack) break;  // block-uniform; cannot occur for trees of depth <= 126
-        __syncthreads();  // every thread has read the entry popped above
-        if (threadIdx.x == 0) { s_stack[sp] = farc; s_stack[sp + 1] = nearc; }
-        sp += 2;
-        __syncthreads();
-      }
-    }
-    if (in_image && fp == 0) temp[(size_t)f * kPT + (uint32_t)q] = make_float4(depth, coord.x, coord.y, __uint_as_float(fid));
-    if (threadIdx.x == 0) fflags[f * kFPackets + part] = diverged ? 1u : 0u;
-    __syncthreads();  // the next job rewrites the stack
-  }
-}
-
-// The forced walks' results, per packet: into the outputs (and the packet's
-// record marked kDone) when no part diverged and the forcing ray's final
-// depth is above 0.
-__global__ __launch_bounds__(kPT) void k_packet_commit(
-    int width, int height, int packets_x, uint32_t* __restrict__ handoff, uint32_t handoff_cap,
-    const uint32_t* __restrict__ forced_list, uint32_t forced_cap, const float4* __restrict__ temp,
-    const uint32_t* __restrict__ fflags, uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
-    float* __restrict__ depths) {
-  const uint32_t nf = min(handoff[2], forced_cap);
-  uint32_t* state = handoff + kHandoffHead + handoff_cap;
+__global__ __launch_bounds__(kPT) void k_packet_commit(uint32_t node_count, const float4* __restrict__ dirs,
+                                                       uint32_t* __restrict__ handoff, UnitArgs ua, PacketArgs pa,
+                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
+                                                       float* __restrict__ depths) {
+  __shared__ uint32_t s_ok;
+  const uint32_t nf = min(handoff[2], ua.cap);
+  const uint64_t max_visits = 2 * node_count + 2;
   for (uint32_t f = blockIdx.x; f < nf; f += gridDim.x) {
-    const uint32_t slot = forced_list[f];
-    uint32_t* rec = state + (size_t)slot * kPStateWords;
-    bool ok = temp[(size_t)f * kPT + rec[2]].x > 0.0f;
-    for (int p = 0; p < kFPackets; ++p) ok = ok && fflags[f * kFPackets + p] == 0u;
-    if (!ok) continue;  // block-uniform
+    const uint32_t slot = pa.forced[f];
+    uint32_t* rec = handoff + kHandoffHead + pa.handoff_cap + (size_t)slot * kPStateWords;
     const uint32_t pk = handoff[kHandoffHead + slot];
-    const int bx = (int)(pk % (uint32_t)packets_x), by = (int)(pk / (uint32_t)packets_x);
-    const int q = (int)threadIdx.x;
-    const int x = bx * kPW + q % kPW, y = by * kPH + q / kPW;
-    if (x < width && y < height) {
-      const uint32_t l = (uint32_t)(y * width + x);
-      const float4 v = temp[(size_t)f * kPT + (uint32_t)q];
-      depths[l] = v.x;
-      coords[l] = make_float2(v.y, v.z);
-      faces_id[l] = __float_as_uint(v.w);
+    const int x0 = (int)(pk % (uint32_t)pa.packets_x) * kPW, y0 = (int)(pk / (uint32_t)pa.packets_x) * kPH;
+    const uint32_t q = threadIdx.x;
+    const int x = x0 + (int)q % kPW, y = y0 + (int)q / kPW;
+    const bool in_image = x < pa.width && y < pa.height;
+    const uint32_t l = in_image ? (uint32_t)y * (uint32_t)pa.width + (uint32_t)x : 0u;
+    UnitHit h;
+    const bool hit = in_image && unit_best(ua, f * (uint32_t)kPT + q, h);
+    if (q == rec[2]) {
+      const uint32_t o = octant_of(dirs[(uint32_t)y0 * (uint32_t)pa.width + (uint32_t)x0]);
+      bool ok = ua.diverged[f] == 0u && (hit ? h.t : depths[l]) > 0.0f;
+      for (uint32_t w = 0; w < kPGroups; ++w) ok = ok && ua.pops[f * kPGroups + w] + ua.cut->tops[o] <= max_visits;
+      s_ok = ok ? 1u : 0u;
     }
-    __syncthreads();  // every thread has read the record before it is marked
-    if (threadIdx.x == 0) rec[3] = kDone;
+    __syncthreads();  // also: every thread has read the record before it is marked
+    if (s_ok != 0u) {
+      if (hit) {
+        faces_id[l] = h.face;
+        coords[l] = make_float2(h.u, h.v);
+        depths[l] = h.t;
+      }
+      if (q == 0) rec[3] = kDone;
+    }
+    __syncthreads();  // s_ok is read before the next packet's
   }
 }
 
@@ -1418,11 +1385,12 @@ static hipMemPool_t handoff_pool() {
   return g_pools[dev];
 }
 
-// The hand-off buffer of one call (words 32-bit words), its counters cleared:
+// The hand-off buffer of one call (words 32-bit words), its counters and its
+// groups' pops (at word pops_off) cleared:
 // a stream-ordered allocation, so that calls on other streams have their own.
 // Without it (nullptr) every ray or packet stays in the first pass, with the
 // same results.
-static uint32_t* handoff_alloc(hipStream_t st, size_t words, uint32_t faces) {
+static uint32_t* handoff_alloc(hipStream_t st, size_t words, size_t pops_off, uint32_t groups, uint32_t faces) {
   uint32_t* ho = nullptr;
   if (faces == kNoHandoff || words <= kHandoffHead) return nullptr;
   hipMemPool_t pool = handoff_pool();
@@ -1433,7 +1401,8 @@ static uint32_t* handoff_alloc(hipStream_t st, size_t words, uint32_t faces) {
     (void)hipGetLastError();
     return nullptr;
   }
-  hipLaunchKernelGGL(k_handoff_clear, dim3(1), dim3(64), 0, st, ho);
+  hipLaunchKernelGGL(k_handoff_clear, dim3((std::max(groups, kHandoffHead) + 255) / 256), dim3(256), 0, st, ho,
+                     reinterpret_cast<unsigned long long*>(ho + pops_off), groups);
   return ho;
 }
 
@@ -1444,12 +1413,13 @@ static uint32_t* handoff_alloc(hipStream_t st, size_t words, uint32_t faces) {
 // The call's triangle records and group bounds (k_tri_records), one block from
 // the same pool; without it the kernels read the faces and vertices.
 static RefMesh ref_mesh_alloc(hipStream_t st, const uint4* faces, const float4* verts, uint32_t face_count) {
-  RefMesh m{faces, verts, nullptr, nullptr};
+  RefMesh m{faces, verts, nullptr, nullptr, nullptr};
   if (!RK_REF_TRI_RECORDS) return m;
   char* block = nullptr;
   hipMemPool_t pool = handoff_pool();
   const size_t rec_bytes = rk_align_up((size_t)face_count * kRecFloats * sizeof(float));
-  const size_t bytes = rec_bytes + ((size_t)face_count + kGroup - 1) / kGroup * sizeof(rk::FaceBound);
+  const size_t n_groups = ((size_t)face_count + kGroup - 1) / kGroup;
+  const size_t bytes = rec_bytes + (n_groups + ((size_t)face_count + 63) / 64) * sizeof(rk::FaceBound);
   const hipError_t e = pool ? hipMallocFromPoolAsync(reinterpret_cast<void**>(&block), bytes, pool, st)
                             : hipMallocAsync(reinterpret_cast<void**>(&block), bytes, st);
   if (e != hipSuccess) {
@@ -1459,9 +1429,10 @@ static RefMesh ref_mesh_alloc(hipStream_t st, const uint4* faces, const float4* 
   float* tris = reinterpret_cast<float*>(block);
   rk::FaceBound* bounds = reinterpret_cast<rk::FaceBound*>(block + rec_bytes);
   hipLaunchKernelGGL(k_tri_records, dim3((face_count + 255) / 256), dim3(256), 0, st, faces, verts, face_count, tris,
-                     bounds);
+                     bounds, bounds + n_groups);
   m.tris = tris;
   m.bounds = bounds;
+  m.supers = bounds + n_groups;
   return m;
 }
 
@@ -1485,34 +1456,43 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
                                           RK_REF_PACKET_HANDOFF_FACES);
     const uint32_t cap = std::min<uint32_t>(gx * gy, g_list_cap.load(std::memory_order_relaxed));
     const uint32_t fcap = std::min<uint32_t>(cap, kForcedCap);
-    // [head | list | records | forced list | forced flags (4 each) | forced results (192 float4 each)]
-    const size_t flist_off = kHandoffHead + (size_t)cap * (1u + kPStateWords);
-    const size_t temp_off = (flist_off + (1ull + kFPackets) * fcap + 3) & ~size_t(3);
-    uint32_t* ho = handoff_alloc(st, temp_off + 4ull * kPT * fcap, faces_limit);
-    uint32_t* flist = ho ? ho + flist_off : nullptr;
-    uint32_t* fflags = ho ? ho + flist_off + fcap : nullptr;
-    float4* temp = ho ? reinterpret_cast<float4*>(ho + temp_off) : nullptr;
+    // [head | list | records | pops (2 words each) | forced list | diverged | slots' heads | cut | hit entries]
+    const size_t pops_off = (kHandoffHead + (size_t)cap * (1u + kPStateWords) + 1) & ~size_t(1);
+    const size_t flist_off = pops_off + 2ull * kPGroups * fcap;
+    const size_t cut_off = flist_off + (2ull + kPT) * fcap;
+    const size_t hits_off = cut_off + sizeof(UnitCut) / 4;
+    const uint32_t hit_cap = kHitsPerSlot * kPT * fcap;
+    uint32_t* ho = handoff_alloc(st, hits_off + hit_cap * (sizeof(UnitHit) / 4), pops_off, kPGroups * fcap,
+                                 faces_limit);
+    UnitArgs ua{};
+    PacketArgs pa{width, height, (int)gx, cap, ho ? ho + flist_off : nullptr};
+    if (ho) {
+      ua.pops = reinterpret_cast<unsigned long long*>(ho + pops_off);
+      ua.diverged = ho + flist_off + fcap;
+      ua.head = ho + flist_off + 2ull * fcap;
+      ua.cut = reinterpret_cast<UnitCut*>(ho + cut_off);
+      ua.hits = reinterpret_cast<UnitHit*>(ho + hits_off);
+      ua.cap = fcap;
+      ua.hit_cap = hit_cap;
+    }
+    const rk::Node* nd = reinterpret_cast<const rk::Node*>(nodes);
+    const float4* org = reinterpret_cast<const float4*>(origins);
+    const float4* drs = reinterpret_cast<const float4*>(directions);
+    float2* uv = reinterpret_cast<float2*>(coords);
     const RefMesh mesh = ref_mesh_alloc(st, reinterpret_cast<const uint4*>(faces),
                                         reinterpret_cast<const float4*>(vertices), face_count);
-    hipLaunchKernelGGL(k_trace_packet, dim3(gx, gy), dim3(kPT), 0, st, reinterpret_cast<const rk::Node*>(nodes),
-                       mesh,
-                       reinterpret_cast<const float4*>(origins), reinterpret_cast<const float4*>(directions), width,
-                       height, node_count, face_count, faces_id, reinterpret_cast<float2*>(coords), depths, ho,
-                       ho ? cap : 0u, faces_limit, flist, fcap);
+    hipLaunchKernelGGL(k_trace_packet, dim3(gx, gy), dim3(kPT), 0, st, nd, mesh, org, drs, width, height, node_count,
+                       face_count, faces_id, uv, depths, ho, ho ? cap : 0u, faces_limit, ho ? ho + flist_off : nullptr,
+                       ua);
     if (ho) {
-      hipLaunchKernelGGL(k_packet_forced, dim3(std::min<uint32_t>(fcap * kFPackets, kForcedGrid)), dim3(kFThreads), 0,
-                         st, reinterpret_cast<const rk::Node*>(nodes), mesh,
-                       reinterpret_cast<const float4*>(origins),
-                         reinterpret_cast<const float4*>(directions), width, height, (int)gx, node_count, face_count,
-                         ho, cap, flist, fcap, temp, fflags, faces_id, reinterpret_cast<const float2*>(coords),
+      hipLaunchKernelGGL(k_units_cut, dim3(8), dim3(256), 0, st, nd, node_count, ho, ua.cut);
+      hipLaunchKernelGGL(k_unit_walk<true>, dim3(kUnitGrid), dim3(64), 0, st, nd, mesh, org, drs, depths, node_count,
+                         face_count, ho, ua, pa);
+      hipLaunchKernelGGL(k_packet_commit, dim3(fcap), dim3(kPT), 0, st, node_count, drs, ho, ua, pa, faces_id, uv,
                          depths);
-      hipLaunchKernelGGL(k_packet_commit, dim3(fcap), dim3(kPT), 0, st, width, height, (int)gx, ho, cap, flist, fcap,
-                         temp, fflags, faces_id, reinterpret_cast<float2*>(coords), depths);
       hipLaunchKernelGGL(k_trace_packet_split, dim3(std::min<uint32_t>(cap, kPacketGrid)), dim3(kPT * kPacketSplit),
-                         0, st, reinterpret_cast<const rk::Node*>(nodes), mesh,
-                       reinterpret_cast<const float4*>(origins),
-                         reinterpret_cast<const float4*>(directions), width, height, (int)gx, node_count, face_count,
-                         ho, cap, faces_id, reinterpret_cast<float2*>(coords), depths);
+                         0, st, nd, mesh, org, drs, width, height, (int)gx, node_count, face_count, ho, cap, faces_id,
+                         uv, depths);
       if (hipFreeAsync(ho, st) != hipSuccess) return RK_ERROR_DEVICE;
     }
     if (mesh.tris && hipFreeAsync(const_cast<float*>(mesh.tris), st) != hipSuccess) return RK_ERROR_DEVICE;
@@ -1524,22 +1504,27 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
                                           RK_REF_HANDOFF_FACES);
     const uint32_t cap = std::min<uint32_t>(n, g_list_cap.load(std::memory_order_relaxed));
     const uint32_t ucap = std::min<uint32_t>(cap, kCrossCap);
-    // [head | list | split rays: list, nunits, top_pops, diverged, buckets (8) | unit_node, unit_sp |
-    //  results (8 words each)]
-    const size_t res_off = (kHandoffHead + cap + 12ull * ucap + 2ull * ucap * kUnits + 7) & ~size_t(7);
-    uint32_t* ho = handoff_alloc(st, res_off + 8ull * ucap * kUnits, faces_limit);
+    // [head | list | pops (2 words each) | crossing rays: list, buckets (8), redo, diverged, heads | cut | hit entries]
+    const uint32_t groups = ucap / 64 + 8;
+    const size_t pops_off = (kHandoffHead + cap + 1ull) & ~size_t(1);
+    const size_t list_off = pops_off + 2ull * groups;
+    const size_t cut_off = list_off + 12ull * ucap;
+    const size_t hits_off = cut_off + sizeof(UnitCut) / 4;
+    const uint32_t hit_cap = kHitsPerRay * ucap;
+    uint32_t* ho = handoff_alloc(st, hits_off + hit_cap * (sizeof(UnitHit) / 4), pops_off, groups, faces_limit);
     UnitArgs ua{};
     if (ho) {
-      uint32_t* p = ho + kHandoffHead + cap;
+      uint32_t* p = ho + list_off;
+      ua.pops = reinterpret_cast<unsigned long long*>(ho + pops_off);
       ua.list = p;
-      ua.nunits = p + ucap;
-      ua.top_pops = p + 2 * ucap;
-      ua.diverged = p + 3 * ucap;
-      ua.bucket = p + 4 * ucap;
-      ua.unit_node = p + 12 * ucap;
-      ua.unit_sp = p + 12 * ucap + (size_t)ucap * kUnits;
-      ua.res = reinterpret_cast<UnitResult*>(ho + res_off);
+      ua.bucket = p + ucap;
+      ua.redo = p + 9ull * ucap;
+      ua.diverged = p + 10ull * ucap;
+      ua.head = p + 11ull * ucap;
+      ua.cut = reinterpret_cast<UnitCut*>(ho + cut_off);
+      ua.hits = reinterpret_cast<UnitHit*>(ho + hits_off);
       ua.cap = ucap;
+      ua.hit_cap = hit_cap;
     }
     const rk::Node* nd = reinterpret_cast<const rk::Node*>(nodes);
     const float4* org = reinterpret_cast<const float4*>(origins);
@@ -1549,22 +1534,14 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
                                         reinterpret_cast<const float4*>(vertices), face_count);
     hipLaunchKernelGGL(k_trace_ray<RK_REF_COOP_MAX>, dim3((n + 63) / 64), dim3(64), 0, st, nd, mesh, org,
                        drs, n, node_count, face_count, faces_id, uv, depths, ho, ho ? cap : 0u, faces_limit, ua);
-    if (ho && ucap != 0u) {
-      hipLaunchKernelGGL(k_units_split, dim3((ucap + 63) / 64), dim3(64), 0, st, nd, org, drs, depths, node_count,
-                         ho, ua);
-      const dim3 ugrid(std::min<uint32_t>(ucap * kUnits, kUnitGrid));
-      if ((uint64_t)face_count >= (uint64_t)kUnitWaveFaces * ((node_count + 1) / 2))
-        hipLaunchKernelGGL(k_units_walk<RK_REF_UNIT_WAVES>, ugrid, dim3(64 * RK_REF_UNIT_WAVES), 0, st, nd, mesh, org,
-                           drs, depths, node_count, face_count, ho, ua);
-      else
-        hipLaunchKernelGGL(k_units_walk<1>, ugrid, dim3(64), 0, st, nd, mesh, org, drs, depths, node_count,
-                           face_count, ho, ua);
-      hipLaunchKernelGGL(k_units_merge, dim3(std::min<uint32_t>(ucap, kWaveGrid)), dim3(64), 0, st, nd, mesh, org,
-                         drs, node_count, face_count, ho, ua, faces_id, uv, depths);
-    }
     if (ho) {
+      hipLaunchKernelGGL(k_units_cut, dim3(8), dim3(256), 0, st, nd, node_count, ho, ua.cut);
+      hipLaunchKernelGGL(k_unit_walk<false>, dim3(kUnitGrid), dim3(64), 0, st, nd, mesh, org, drs, depths, node_count,
+                         face_count, ho, ua, PacketArgs{});
+      hipLaunchKernelGGL(k_units_merge, dim3((ucap + 63) / 64), dim3(64), 0, st, node_count, ho, ua, faces_id, uv,
+                         depths);
       hipLaunchKernelGGL(k_trace_ray_wave, dim3(std::min<uint32_t>(cap, kRayWaveGrid)), dim3(64), 0, st, nd, mesh,
-                         org, drs, node_count, face_count, ho, cap, faces_id, uv, depths);
+                         org, drs, node_count, face_count, ho, cap, ua.redo, ucap, faces_id, uv, depths);
       if (hipFreeAsync(ho, st) != hipSuccess) return RK_ERROR_DEVICE;
     }
     if (mesh.tris && hipFreeAsync(const_cast<float*>(mesh.tris), st) != hipSuccess) return RK_ERROR_DEVICE;
