@@ -11,10 +11,9 @@
 //                     (v0, v1-v0, v2-v0; 48 B) bottom-up (agglomerative
 //                     LBVH, Apetrei 2014) for the splits inside each
 //                     512-position chunk; subtrees of <= leaf_max faces
-//                     become leaves; up to 2^21 faces it also climbs the
-//                     splits that cross chunks
-//   k_fast_hierarchy_top  above that, the climbs through the splits that cross
-//                     chunks
+//                     become leaves
+//   k_hier_reduce     the same over the subtrees that 64 chunks left over,
+//                     again until one group is left
 //
 // Node record (64 B): float4 (c0.lo.x, c0.hi.x, c0.lo.y, c0.hi.y),
 //                     float4 (c1.lo.x, c1.hi.x, c1.lo.y, c1.hi.y),
@@ -62,20 +61,18 @@ __device__ __forceinline__ uint64_t spread21(uint64_t v) {
   return v;
 }
 
-// Also clears the build's info words, the hierarchy's split counters
-// (flags, n words) and the sort's error word and digit counts (sort_head,
-// head_words), which saves three fill launches per build.
+// Also clears the build's info words and the sort's error word and digit
+// counts (sort_head, head_words), which saves two fill launches per build.
 template <typename K>
 __global__ __launch_bounds__(256) void k_fast_prep(const uint4* __restrict__ faces, const float4* __restrict__ verts,
                                                    uint32_t n, float4 rmin, float4 rmax, Box* __restrict__ boxes,
                                                    K* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                   uint32_t* __restrict__ info, uint32_t* __restrict__ flags,
-                                                   uint32_t* __restrict__ sort_head, uint32_t head_words) {
+                                                   uint32_t* __restrict__ info, uint32_t* __restrict__ sort_head,
+                                                   uint32_t head_words) {
   uint32_t k = blockIdx.x * 256 + threadIdx.x;
   if (k < RK_INFO_WORDS) info[k] = 0u;
   if (k < head_words) sort_head[k] = 0u;
   if (k >= n) return;
-  flags[k] = 0u;
   uint4 f = faces[k];
   float4 v0 = verts[f.x], v1 = verts[f.y], v2 = verts[f.z];
   Box b;
@@ -127,24 +124,16 @@ __device__ __forceinline__ void pad_box(float& lo, float& hi) {
   hi = hi + p;
 }
 
-// A finished subtree as its parent sees it: box (unpadded), reference, and
-// the far end of its leaf range (the end the sibling does not know).
-struct Part {
+// A finished subtree as its sibling sees it: box (unpadded), reference, and
+// the end of its range that the sibling does not know: the item, its position
+// and the split key beyond it.
+struct alignas(16) Part {
   float lox, loy, loz, hix, hiy, hiz;
   uint32_t ref, end;
+  uint64_t key;
+  uint32_t pos, pad;
 };
-static_assert(sizeof(Part) == 32, "part is 32 B");
-// A part exchanged through global memory at a split that crosses chunks, with
-// the split key at its outer end (left end for a left child, right end for a
-// right child), which its parent's side test needs: carried with the part, so
-// the climb does not load keys after each exchange.
-struct GPart {
-  Part p;
-  uint64_t outer;
-  uint64_t pad;
-};
-static_assert(sizeof(GPart) == 48, "global part is 48 B");
-
+static_assert(sizeof(Part) == 48, "part is 48 B");
 __device__ __forceinline__ void write_node(FNode* __restrict__ nodes, uint32_t idx, const Part& c0, const Part& c1,
                                            uint32_t n0, uint32_t n1) {
   float a0 = c0.lox, a1 = c0.hix, a2 = c0.loy, a3 = c0.hiy, a4 = c0.loz, a5 = c0.hiz;
@@ -158,50 +147,10 @@ __device__ __forceinline__ void write_node(FNode* __restrict__ nodes, uint32_t i
   p->d = make_uint4(c0.ref, c1.ref, n0, n1);
 }
 
-// Max-scan over one workgroup of kLocalThreads threads (waves of 64). The
-// hierarchy pass's chunks are one position per thread: 512 measured best on
-// the 1M-face heightfield and the 10M-face soup (builds of 224 and 1718 us,
-// against 236 and 1816 with 1024 and 222 and 1810 with 256; the same trees).
 #ifndef RK_HIER_THREADS
 #define RK_HIER_THREADS 512
 #endif
-constexpr uint32_t kLocalThreads = RK_HIER_THREADS;
-constexpr uint32_t kLocalWaves = kLocalThreads / 64;
-
-__device__ __forceinline__ uint64_t shfl_up64(uint64_t v, int d) {
-  uint32_t lo = __shfl_up((uint32_t)v, d, 64), hi = __shfl_up((uint32_t)(v >> 32), d, 64);
-  return ((uint64_t)hi << 32) | lo;
-}
-__device__ __forceinline__ uint64_t shfl_down64(uint64_t v, int d) {
-  uint32_t lo = __shfl_down((uint32_t)v, d, 64), hi = __shfl_down((uint32_t)(v >> 32), d, 64);
-  return ((uint64_t)hi << 32) | lo;
-}
-// before = max of v over threads < t (0 for t = 0), after = max over threads
-// > t (0 for the last thread), t = threadIdx.x.
-__device__ __forceinline__ void block_excl_max(uint64_t v, uint64_t* s_wave, uint64_t& before, uint64_t& after) {
-  const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
-  uint64_t up = v, dn = v;
-  for (int d = 1; d < 64; d <<= 1) {
-    uint64_t u = shfl_up64(up, d), q = shfl_down64(dn, d);
-    if (lane >= (uint32_t)d) up = up > u ? up : u;
-    if (lane + d < 64) dn = dn > q ? dn : q;
-  }
-  if (lane == 63) s_wave[w] = up;  // wave max
-  __syncthreads();
-  uint64_t b = 0, a = 0;
-  for (uint32_t k = 0; k < kLocalWaves; ++k) {
-    if (k < w) b = b > s_wave[k] ? b : s_wave[k];
-    if (k > w) a = a > s_wave[k] ? a : s_wave[k];
-  }
-  uint64_t ub = shfl_up64(up, 1), da = shfl_down64(dn, 1);
-  if (lane > 0) b = b > ub ? b : ub;
-  if (lane < 63) a = a > da ? a : da;
-  before = b;
-  after = a;
-}
-
-constexpr uint32_t kChunk = kLocalThreads;  // sorted positions per workgroup, one per thread
-constexpr uint32_t kPendLeft = 0x80000000u;  // a handed-on climb whose part is its split's left child
+constexpr uint32_t kChunk = RK_HIER_THREADS;  // sorted positions per workgroup of k_fast_hierarchy, one per thread
 
 __device__ __forceinline__ Part merge_parts(const Part& lc, const Part& rc) {
   Part up;
@@ -220,198 +169,280 @@ __device__ __forceinline__ bool left_of_parent(bool has_l, bool has_r, uint64_t 
   return !has_l || (has_r && kr < kl);
 }
 
-// Completes split p from its two children: writes its record unless it
-// collapses into a leaf, and returns the merged part (end not set).
-// The tree's positions are [lo, hi]; its root record goes to lo. Any other
-// node [nl, nr] goes to nr when it is its parent's left child (next_left)
-// and to nl when it is the right child, so the two children of a split p sit
-// in records p and p + 1, next to each other (the numbering of Karras 2012).
-__device__ __forceinline__ Part finish_split(FNode* __restrict__ nodes, uint32_t lo, uint32_t hi, uint32_t leaf_max,
-                                             uint32_t p, uint32_t nl, uint32_t nr, const Part& lc, const Part& rc,
-                                             bool next_left) {
-  const uint32_t cnt = nr - nl + 1;
-  const bool root = nl == lo && nr == hi;
-  const uint32_t idx = root ? lo : (next_left ? nr : nl);
-  if (root || cnt > leaf_max) write_node(nodes, idx, lc, rc, p - nl + 1, nr - p);
-  Part up = merge_parts(lc, rc);
-  up.ref = (!root && cnt <= leaf_max) ? (kLeafBit | (nl << 4) | (cnt - 1)) : idx;
-  return up;
+// The hierarchy, bottom-up (agglomerative LBVH, Apetrei 2014): a subtree
+// covering sorted positions [l, r] is a child of the split at r or at l - 1,
+// whichever has the smaller split key; of the two subtrees that arrive at a
+// split, the second has it merged. This gives the binary radix tree of Karras
+// 2012 without per-node binary searches.
+//
+// A workgroup takes a run of up to kT consecutive items (single positions in
+// k_fast_hierarchy, subtrees left over by earlier passes in k_hier_reduce),
+// one per thread, and exchanges through LDS alone. A split whose range lies
+// inside the run sees both children arrive; at any other at most one does, and
+// that subtree is left over for the next pass. The splits that cross one end
+// of the run are nested, so at most two subtrees per level of the tree are
+// left over; 10 to 12 per 512 positions on the meshes measured.
+//
+// Merges run in rounds: a round merges the splits in a queue, one per thread,
+// and those whose parents become ready fill the next round's queue. Once at
+// most 64 are ready they fit the first wave, whose lanes go on alone, without
+// queue or barriers, each with its subtree in registers. What bounds the pass
+// is issuing the merges: a thread that climbed on by itself from its leaf left
+// its wave with a few active lanes for a dozen steps (80 wave-steps per 512
+// positions against about 20), and the splits that cross chunks took three
+// round trips to memory per level. On the 1M-face terrain the passes took 111
+// us that way.
+//
+// Slots: a subtree on items [a, b] waits for its sibling in slot b of part as
+// a left child and in slot a as a right child, so the children of split q
+// (between items q - 1 and q) are in slots q - 1 and q; end is the item at the
+// subtree's other end. Slots a..b belong to that subtree alone.
+
+// A subtree that a run left over, for the next pass: its part, its positions
+// [l, r] and the split key after r.
+struct HierItem {
+  float4 a, b, c;  // (lo.xyz, hi.x), (hi.yz, ref, l), (r, 0, key)
+};
+static_assert(sizeof(HierItem) == 48, "item is 48 B");
+
+constexpr uint32_t kFromLeft = 1u, kFromRight = 2u;  // HierLds::flag: the children that have arrived
+
+template <uint32_t kT>
+struct HierLds {
+  Part part[kT];
+  uint64_t key[kT + 1];   // key[q]: the split key before item q; key[m] after the last; ~0 past the array's ends
+  uint32_t first[kT], last[kT];  // item k's positions
+  uint32_t flag[kT + 1];  // split q's arrivals
+  uint32_t cnt[3];        // entries of the rounds' queues
+  uint32_t wcnt[kT / 64];
+  uint16_t queue[2][kT / 2];
+};
+
+// Whether a key separates two meshes of a batch (or is past an end): keys are
+// mesh << 30 | 30-bit code, so the XOR reaches bit 30.
+__device__ __forceinline__ bool between_meshes(uint64_t key) { return ((key << 1) >> 31) != 0ull; }
+
+// A subtree on items [a, b] and positions [l, r], with the split keys before
+// and after it.
+struct Sub {
+  Part p;  // box and reference
+  uint32_t a, b, l, r;
+  uint64_t kl, kr;
+};
+
+// The subtree u goes to its parent, split q (left: as the left child); the
+// children that had arrived there before.
+template <uint32_t kT>
+__device__ __forceinline__ uint32_t hier_arrive(HierLds<kT>& s, Sub& u, uint32_t n, bool& left, uint32_t& q) {
+  left = left_of_parent(u.l > 0u, u.r + 1u < n, u.kl, u.kr);
+  q = left ? u.b + 1u : u.a;
+  u.p.end = left ? u.a : u.b;
+  u.p.pos = left ? u.l : u.r;
+  u.p.key = left ? u.kl : u.kr;
+  s.part[left ? u.b : u.a] = u.p;
+  // a wave's LDS accesses keep their order, which is all the first wave's
+  // going on alone needs; between waves there is a barrier
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  const uint32_t before = __hip_atomic_fetch_add(&s.flag[q], left ? kFromLeft : kFromRight, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_WORKGROUP);
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  return before;
 }
 
-// 16-B loads and stores that are coherent across XCDs, as relaxed agent-scope
-// atomics are (the same cache policy bit), but one instruction per 16 B.
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void store_part_coherent(GPart* p, const Part& v, uint64_t outer) {
-  const u32x4 a = {__float_as_uint(v.lox), __float_as_uint(v.loy), __float_as_uint(v.loz), __float_as_uint(v.hix)};
-  const u32x4 b = {__float_as_uint(v.hiy), __float_as_uint(v.hiz), v.ref, v.end};
-  const u32x4 c = {(uint32_t)outer, (uint32_t)(outer >> 32), 0u, 0u};
-  asm volatile(
-      "global_store_dwordx4 %0, %1, off sc1\n\tglobal_store_dwordx4 %0, %2, off offset:16 sc1\n\t"
-      "global_store_dwordx4 %0, %3, off offset:32 sc1"
-      :
-      : "v"(p), "v"(a), "v"(b), "v"(c)
-      : "memory");
-}
-__device__ __forceinline__ Part load_part_coherent(const GPart* p, uint64_t& outer) {
-  u32x4 a, b, c;
-  asm volatile(
-      "global_load_dwordx4 %0, %3, off sc1\n\tglobal_load_dwordx4 %1, %3, off offset:16 sc1\n\t"
-      "global_load_dwordx4 %2, %3, off offset:32 sc1\n\ts_waitcnt vmcnt(0)"
-      : "=&v"(a), "=&v"(b), "=&v"(c)
-      : "v"(p)
-      : "memory");
-  Part v;
-  v.lox = __uint_as_float(a.x);
-  v.loy = __uint_as_float(a.y);
-  v.loz = __uint_as_float(a.z);
-  v.hix = __uint_as_float(a.w);
-  v.hiy = __uint_as_float(b.x);
-  v.hiz = __uint_as_float(b.y);
-  v.ref = b.z;
-  v.end = b.w;
-  outer = (uint64_t)c.x | ((uint64_t)c.y << 32);
-  return v;
-}
-
-// Climb of the subtree [l, r] (box and ref in me) through splits that cross
-// chunks, starting at its parent on side as_left: publish the part in its
-// slot with XCD-coherent stores, waited for before the split's counter moves
-// (published: already in its slot); the first to arrive stops, the second
-// merges both and climbs on. Every split above a crossing split crosses
-// chunks too, so the whole climb exchanges through global memory.
-// outer: the split key at the outer end of [l, r] (~0 past the array's end).
-__device__ __forceinline__ void climb_crossing(uint32_t n, uint32_t leaf_max, uint32_t* __restrict__ gflags,
-                                               GPart* __restrict__ gparts, FNode* __restrict__ nodes, uint32_t lo,
-                                               uint32_t hi, Part me, uint64_t outer, uint32_t l, uint32_t r,
-                                               bool as_left, bool published) {
-  for (uint32_t guard = 0; guard < n; ++guard) {
-    const uint32_t p = as_left ? r : l - 1;
-    const uint32_t mine = as_left ? p : p + 1, other = as_left ? p + 1 : p;
-    if (!published) {
-      me.end = as_left ? l : r;
-      store_part_coherent(gparts + mine, me, outer);
-      __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    }
-    published = false;
-    const uint32_t old = __hip_atomic_fetch_add(gflags + p, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (old == 0) return;
-    uint64_t sib_outer;
-    const Part sib = load_part_coherent(gparts + other, sib_outer);
-    const uint32_t nl = as_left ? l : sib.end, nr = as_left ? sib.end : r;
-    const bool root = nl == lo && nr == hi;  // the (mesh) root
-    bool next_left = false;
-    // the merged range's end keys: the left child's outer key and the right child's
-    const uint64_t kl = as_left ? outer : sib_outer, kr = as_left ? sib_outer : outer;
-    if (!root) next_left = left_of_parent(nl > 0, nr + 1 < n, kl, kr);
-    outer = next_left ? kl : kr;
-    me = as_left ? finish_split(nodes, lo, hi, leaf_max, p, nl, nr, me, sib, next_left)
-                 : finish_split(nodes, lo, hi, leaf_max, p, nl, nr, sib, me, next_left);
-    if (root) return;
-    l = nl;
-    r = nr;
-    as_left = next_left;
+// Merges split q's children lc and rc into u, whose range is set: the split's
+// record is written unless it collapses into a leaf (p: the left child's last
+// position), and u goes to its parent. True when that is ready too.
+template <uint32_t kT, bool kBatch>
+__device__ __forceinline__ bool hier_merge(HierLds<kT>& s, uint32_t n, uint32_t leaf_max, FNode* __restrict__ nodes,
+                                           const Part& lc, const Part& rc, uint32_t p, Sub& u, bool& left,
+                                           uint32_t& q) {
+  const bool root = kBatch ? between_meshes(u.kl) && between_meshes(u.kr) : u.l == 0u && u.r + 1u == n;
+  const uint32_t cnt = u.r - u.l + 1u;
+  uint32_t before = 0u, idx = u.l;  // a root's record goes to its first position
+  u.p = merge_parts(lc, rc);
+  if (!root) {
+    // any other to its last position as a left child and to its first as a
+    // right child: the children of the split between p and p + 1 are then
+    // records p and p + 1 (Karras 2012's numbering)
+    if (left_of_parent(u.l > 0u, u.r + 1u < n, u.kl, u.kr)) idx = u.r;
+    u.p.ref = cnt <= leaf_max ? (kLeafBit | (u.l << 4) | (cnt - 1u)) : idx;
+    before = hier_arrive(s, u, n, left, q);
   }
+  if (root || cnt > leaf_max) write_node(nodes, idx, lc, rc, p - u.l + 1u, u.r - p);
+  return before != 0u;
 }
 
-// The hierarchy in one bottom-up pass (agglomerative LBVH, Apetrei 2014): a
-// subtree covering sorted positions [l, r] is a child of the split at r or
-// at l - 1, whichever has the smaller split key; of the two subtrees that
-// reach a split, the second to arrive merges both and climbs on. This gives
-// the binary radix tree of Karras 2012 without per-node binary searches. Each
-// thread starts at its leaf, whose triangle record it also writes.
-//
-// Exchange at a split: both children publish their part before either knows
-// it is second, each in its own slot, the position next to the split (p for
-// the left child, p + 1 for the right one); then a counter decides. A slot is
-// next written by an ancestor of the split, which completes only after the
-// split's reader is done.
-//
-// A workgroup owns kChunk consecutive positions, one per thread. A split
-// whose range lies inside them is reached only by this workgroup, and its
-// exchange goes through LDS. The range of split p ends, on each side, at the
-// nearest split with a larger key, so it lies inside [c0, c1) when such a
-// split exists both in [c0 - 1, p - 1] and in [p + 1, c1 - 1] (prefix and
-// suffix maxima of the chunk's split keys). A climb that reaches a split
-// crossing chunks goes on through global memory (climb_crossing) when
-// inline_top is set; otherwise it leaves its part in the split's slot and its
-// position in the chunk's list of handed-on climbs (pend, pend_count), and
-// ends, and k_fast_hierarchy_top continues it. The chain of crossing splits
-// above a chunk takes a few memory round trips per level; on a large tree,
-// waiting for it here would hold the workgroup's LDS while other chunks queue.
-// With kBatch the positions hold many meshes, sorted by (mesh, Morton code):
-// keys are mesh << 30 | 30-bit code, so every split between two meshes ranks
-// above every split inside one, and a climb stops at its mesh's root, whose
-// record goes to the mesh's first position. Mesh m's nodes and triangle
-// records then occupy [face_offset, face_offset + face_count).
+// Completes the run's splits: every first arrival is in (ready, q: this
+// thread's second one), keys and zeroed flags since a barrier. Ends with one.
+template <uint32_t kT, bool kBatch>
+__device__ __forceinline__ void hier_rounds(HierLds<kT>& s, uint32_t n, uint32_t leaf_max, FNode* __restrict__ nodes,
+                                            bool ready, uint32_t q) {
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  auto push = [&](bool sec, uint32_t sq, uint32_t qi, uint32_t ci) {
+    const uint64_t mask = __ballot(sec);
+    if (mask == 0ull) return;
+    uint32_t base = 0;
+    if (lane == 0) base = atomicAdd(&s.cnt[ci], (uint32_t)__popcll(mask));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (sec) s.queue[qi][base + (uint32_t)__popcll(mask & rk::lanemask_lt())] = (uint16_t)sq;
+  };
+  // split sq's children and range; the left child's last position
+  auto load = [&](uint32_t sq, Part& lc, Part& rc, Sub& u) {
+    lc = s.part[sq - 1u];
+    rc = s.part[sq];
+    u.a = lc.end;
+    u.b = rc.end;
+    u.l = lc.pos;
+    u.r = rc.pos;
+    u.kl = lc.key;
+    u.kr = rc.key;
+    return s.last[sq - 1u];
+  };
+  push(ready, q, 0u, 0u);
+  for (uint32_t r = 0;; ++r) {
+    __syncthreads();
+    const uint32_t cnt = s.cnt[r % 3u];
+    if (cnt <= 64u) {
+      if (w == 0 && lane < cnt) {
+        Part lc, rc;
+        Sub u;
+        bool left;
+        uint32_t p = load(s.queue[r & 1u][lane], lc, rc, u);
+        while (hier_merge<kT, kBatch>(s, n, leaf_max, nodes, lc, rc, p, u, left, q)) {
+          const Part sib = s.part[left ? q : q - 1u];
+          p = left ? u.r : u.l - 1u;  // a split's children are next to each other
+          lc = left ? u.p : sib;
+          rc = left ? sib : u.p;
+          u.a = left ? u.a : sib.end;
+          u.l = left ? u.l : sib.pos;
+          u.kl = left ? u.kl : sib.key;
+          u.b = left ? sib.end : u.b;
+          u.r = left ? sib.pos : u.r;
+          u.kr = left ? sib.key : u.kr;
+        }
+      }
+      break;
+    }
+    if (t == 0) s.cnt[(r + 2u) % 3u] = 0u;  // last read in the round before
+    // at most kT / 2 entries: two items each
+    uint32_t nq = 0u;
+    bool sec = false;
+    if (t < cnt) {
+      Part lc, rc;
+      Sub u;
+      bool left;
+      const uint32_t p = load(s.queue[r & 1u][t], lc, rc, u);
+      sec = hier_merge<kT, kBatch>(s, n, leaf_max, nodes, lc, rc, p, u, left, nq);
+    }
+    push(sec, nq, (r & 1u) ^ 1u, (r + 1u) % 3u);
+  }
+  __syncthreads();
+}
+
+// The left-over subtree that waits at split q, if one does.
+struct Left {
+  bool has;
+  Part part;
+  uint32_t l, r;  // positions
+  uint64_t kl, kr;
+};
+template <uint32_t kT>
+__device__ __forceinline__ Left left_over(const HierLds<kT>& s, uint32_t m, uint32_t q) {
+  Left o;
+  const uint32_t f = q <= m ? s.flag[q] : 0u;
+  o.has = f == kFromLeft || f == kFromRight;
+  o.l = o.r = 0u;
+  o.kl = o.kr = 0ull;
+  if (o.has) {
+    const bool left = f == kFromLeft;
+    o.part = s.part[left ? q - 1u : q];
+    o.l = left ? o.part.pos : s.first[q];
+    o.r = left ? s.last[q - 1u] : o.part.pos;
+    o.kl = left ? o.part.key : s.key[q];
+    o.kr = left ? s.key[q] : o.part.key;
+  }
+  return o;
+}
+
+// Ranks of the left-over subtrees of splits 0 .. kT - 1 (has: this thread's),
+// and their number. Subtrees in item order wait at splits in increasing order.
+template <uint32_t kT>
+__device__ __forceinline__ uint32_t hier_rank(HierLds<kT>& s, bool has, uint32_t& total) {
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  const uint64_t mask = __ballot(has);
+  if (lane == 0) s.wcnt[w] = (uint32_t)__popcll(mask);
+  __syncthreads();
+  uint32_t before = (uint32_t)__popcll(mask & rk::lanemask_lt());
+  total = 0u;
+  for (uint32_t k = 0; k < kT / 64; ++k) {
+    if (k < w) before += s.wcnt[k];
+    total += s.wcnt[k];
+  }
+  return before;
+}
+
+__device__ __forceinline__ void store_item(HierItem* __restrict__ it, const Part& p, uint32_t l, uint32_t r,
+                                           uint64_t key) {
+  it->a = make_float4(p.lox, p.loy, p.loz, p.hix);
+  it->b = make_float4(p.hiy, p.hiz, __uint_as_float(p.ref), __uint_as_float(l));
+  it->c = make_float4(__uint_as_float(r), 0.0f, __uint_as_float((uint32_t)key), __uint_as_float((uint32_t)(key >> 32)));
+}
+
+// The chunk pass: kChunk consecutive sorted positions per workgroup, one per
+// thread, whose triangle record it also writes. With kBatch the positions hold
+// many meshes, sorted by (mesh, Morton code): keys are mesh << 30 | 30-bit
+// code, so every split between two meshes ranks above every split inside one,
+// and a subtree between two such splits is its mesh's root, whose record goes
+// to the mesh's first position. Mesh m's nodes and triangle records then
+// occupy [face_offset, face_offset + face_count).
 template <typename K, bool kBatch>
-__global__ __launch_bounds__(kLocalThreads) void k_fast_hierarchy(const K* __restrict__ keys,
-                                                                  const uint32_t* __restrict__ order,
-                                                                  const uint4* __restrict__ faces,
-                                                                  const float4* __restrict__ verts, uint32_t n,
-                                                                  uint32_t leaf_max, uint32_t* __restrict__ gflags,
-                                                                  GPart* __restrict__ gparts,
-                                                                  FNode* __restrict__ nodes,
-                                                                  float4* __restrict__ tris,
-                                                                  const rk_batch_mesh* __restrict__ meshes,
-                                                                  uint32_t* __restrict__ pend,
-                                                                  uint32_t* __restrict__ pend_count,
-                                                                  uint32_t inline_top) {
-  __shared__ Part s_part[kChunk];
-  __shared__ uint32_t s_npend;
-  __shared__ uint64_t s_key[kChunk + 1];  // s_key[k] = split_key(c0 - 1 + k), ~0 past either end
-  __shared__ uint32_t s_flag[kChunk];
-  __shared__ uint8_t s_local[kChunk];     // s_local[k]: split c0 + k lies inside the chunk
-  __shared__ uint64_t s_wave[kLocalWaves];
+__global__ __launch_bounds__(kChunk) void k_fast_hierarchy(const K* __restrict__ keys,
+                                                           const uint32_t* __restrict__ order,
+                                                           const uint4* __restrict__ faces,
+                                                           const float4* __restrict__ verts, uint32_t n,
+                                                           uint32_t leaf_max, FNode* __restrict__ nodes,
+                                                           float4* __restrict__ tris,
+                                                           const rk_batch_mesh* __restrict__ meshes,
+                                                           HierItem* __restrict__ items,
+                                                           uint32_t* __restrict__ counts) {
+  __shared__ HierLds<kChunk> s;
   const uint32_t t = threadIdx.x;
   const uint32_t c0 = blockIdx.x * kChunk;
-  const uint32_t c1 = min(c0 + kChunk, n);
+  const uint32_t m = min(kChunk, n - c0);
   const uint32_t i = c0 + t;
-  // leaf loads first: their latency overlaps the split-key scan
+  // leaf loads first: their latency overlaps the split keys'
   uint32_t fid = 0;
-  uint32_t lo = 0, hi = n - 1, voff = 0;  // this leaf's mesh: positions [lo, hi]
   float4 v0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v1 = v0, v2 = v0;
-  if (i < c1) {
+  if (t < m) {
     fid = order[i];
-    if (kBatch) {
-      const rk_batch_mesh m = meshes[(uint32_t)((uint64_t)keys[i] >> 30)];
-      lo = m.face_offset;
-      hi = m.face_offset + m.face_count - 1;
-      voff = m.vertex_offset;
-    }
+    uint32_t voff = 0;
+    if (kBatch) voff = meshes[(uint32_t)((uint64_t)keys[i] >> 30)].vertex_offset;
     const uint4 f = faces[fid];
     v0 = verts[f.x + voff];
     v1 = verts[f.y + voff];
     v2 = verts[f.z + voff];
   }
-  for (uint32_t k = t; k <= kChunk; k += kLocalThreads) {
+  for (uint32_t k = t; k <= m; k += kChunk) {
     const int64_t x = (int64_t)c0 - 1 + (int64_t)k;
-    s_key[k] = (x >= 0 && x + 1 < (int64_t)n) ? split_key(keys, (uint32_t)x) : ~0ull;
+    s.key[k] = (x >= 0 && x + 1 < (int64_t)n) ? split_key(keys, (uint32_t)x) : ~0ull;
+    s.flag[k] = 0u;
   }
-  s_flag[t] = 0u;
-  if (t == 0) s_npend = 0u;
+  s.first[t] = s.last[t] = i;
+  if (t < 3u) s.cnt[t] = 0u;
   __syncthreads();
-  {
-    // inside test of split p = c0 - 1 + k for k = t (k >= 1)
-    const uint64_t d = s_key[t];
-    uint64_t before, after;
-    block_excl_max(d, s_wave, before, after);
-    const uint64_t last = s_key[kChunk];
-    after = after > last ? after : last;
-    const bool inside = t >= 1 && c0 + t < c1 && before > d && after > d;
-    if (t >= 1) s_local[t - 1] = inside ? 1 : 0;
-    if (t == kLocalThreads - 1) s_local[kChunk - 1] = 0;  // split c0 + kChunk - 1 always crosses
-  }
-  __syncthreads();
-  // Climbs from this thread's leaf through the chunk's splits; stops as the
-  // first to arrive at a split, at the (mesh) root, or at a split that
-  // crosses chunks, whose climb k_fast_hierarchy_top continues.
-  auto climb = [&]() {
-    if (i >= c1) return;
+  bool ready = false;
+  uint32_t q = 0;
+  if (t < m) {
     const float4 e1 = rk::sub4(v1, v0), e2 = rk::sub4(v2, v0);
     tris[3 * (size_t)i + 0] = make_float4(v0.x, v0.y, v0.z, __uint_as_float(fid));
     tris[3 * (size_t)i + 1] = make_float4(e1.x, e1.y, e1.z, 0.0f);
     tris[3 * (size_t)i + 2] = make_float4(e2.x, e2.y, e2.z, 0.0f);
-    Part me;
+    Sub u;
+    u.a = u.b = t;
+    u.l = u.r = i;
+    u.kl = s.key[t];
+    u.kr = s.key[t + 1u];
+    Part& me = u.p;
     me.lox = rk::fmn(rk::fmn(v0.x, v1.x), v2.x);
     me.loy = rk::fmn(rk::fmn(v0.y, v1.y), v2.y);
     me.loz = rk::fmn(rk::fmn(v0.z, v1.z), v2.z);
@@ -419,92 +450,133 @@ __global__ __launch_bounds__(kLocalThreads) void k_fast_hierarchy(const K* __res
     me.hiy = rk::fmx(rk::fmx(v0.y, v1.y), v2.y);
     me.hiz = rk::fmx(rk::fmx(v0.z, v1.z), v2.z);
     me.ref = kLeafBit | (i << 4);  // count - 1 = 0
-    if (lo == hi) {  // a single face: root with one leaf child and one empty child
+    if (kBatch ? between_meshes(u.kl) && between_meshes(u.kr) : n == 1u) {
+      // a single face: root with one leaf child and one empty child
       Part empty;
       empty.lox = empty.loy = empty.loz = RK_HUGE;
       empty.hix = empty.hiy = empty.hiz = -RK_HUGE;
       empty.ref = kLeafBit;
-      write_node(nodes, lo, me, empty, 1, 0);
-      return;
+      write_node(nodes, i, me, empty, 1, 0);
+    } else {
+      bool left;
+      ready = hier_arrive(s, u, n, left, q) != 0u;
     }
-    // the side of [l, r] under its parent, from the split keys at its ends
-    // (and the split key at the outer end of [l, r] in outer)
-    auto side = [&](uint32_t l, uint32_t r, uint64_t& outer) {
-      const bool has_l = l > 0, has_r = r + 1 < n;
-      uint64_t kl = ~0ull, kr = ~0ull;
-      if (has_l) kl = (l >= c0 && l - c0 <= kChunk) ? s_key[l - c0] : split_key(keys, l - 1);
-      if (has_r) kr = (r + 1 >= c0 && r + 1 - c0 <= kChunk) ? s_key[r + 1 - c0] : split_key(keys, r);
-      const bool left = left_of_parent(has_l, has_r, kl, kr);
-      outer = left ? kl : kr;
-      return left;
-    };
-    uint32_t l = i, r = i;
-    uint64_t outer = ~0ull;
-    bool as_left = side(l, r, outer);
-    // Each step widens [l, r] by at least one position: n steps bound it.
-    for (uint32_t guard = 0; guard < n; ++guard) {
-      const uint32_t p = as_left ? r : l - 1;
-      const uint32_t mine = as_left ? p : p + 1, other = as_left ? p + 1 : p;
-      me.end = as_left ? l : r;
-      if (!(p >= c0 && p - c0 < kChunk && s_local[p - c0])) {
-        if (inline_top) {  // small trees: the chain above the chunks is short
-          climb_crossing(n, leaf_max, gflags, gparts, nodes, lo, hi, me, outer, l, r, as_left, false);
-          return;
-        }
-        // crossing split: publish the part in its slot and hand the climb on
-        gparts[mine].p = me;
-        gparts[mine].outer = outer;
-        const uint32_t k = atomicAdd(&s_npend, 1u);
-        pend[c0 + k] = mine | (as_left ? kPendLeft : 0u);
-        return;
-      }
-      s_part[mine - c0] = me;  // a local split has p, p + 1 in [c0, c1)
-      const uint32_t old =
-          __hip_atomic_fetch_add(s_flag + (p - c0), 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_WORKGROUP);
-      if (old == 0) return;
-      const Part sib = s_part[other - c0];
-      const uint32_t nl = as_left ? l : sib.end, nr = as_left ? sib.end : r;
-      const bool root = nl == lo && nr == hi;  // the (mesh) root
-      const bool next_left = root ? false : side(nl, nr, outer);
-      me = as_left ? finish_split(nodes, lo, hi, leaf_max, p, nl, nr, me, sib, next_left)
-                   : finish_split(nodes, lo, hi, leaf_max, p, nl, nr, sib, me, next_left);
-      if (root) return;
-      l = nl;
-      r = nr;
-      as_left = next_left;
+  }
+  hier_rounds<kChunk, kBatch>(s, n, leaf_max, nodes, ready, q);
+  const Left o = left_over(s, m, t);
+  uint32_t total;
+  const uint32_t rank = hier_rank(s, o.has, total);
+  if (o.has) store_item(items + c0 + rank, o.part, o.l, o.r, o.kr);
+  if (t == 0) {
+    if (m == kChunk) {  // the split after the last item, which no thread above has
+      const Left e = left_over(s, m, m);
+      if (e.has) store_item(items + c0 + total++, e.part, e.l, e.r, e.kr);
     }
-  };
-  climb();
-  __syncthreads();
-  if (t == 0) pend_count[blockIdx.x] = s_npend;
+    counts[blockIdx.x] = total;
+  }
 }
 
-// The splits that cross chunks, above the chunks' own: thread k of workgroup
-// c continues the k-th climb that chunk c handed on, whose part is in its
-// slot already (written by k_fast_hierarchy).
+// One group of up to kReduceFan runs, whose left-over subtrees (counts[c] of
+// them from items[c * kChunk] on, c = the run's first chunk, every stride-th)
+// become the items of one run, completed as above; what is left over goes to
+// the group's first chunk. More items than threads are taken in steps, each
+// with the subtrees the one before left over in front.
+constexpr uint32_t kReduceFan = 64, kReduceThreads = 1024;
 template <typename K, bool kBatch>
-__global__ __launch_bounds__(64) void k_fast_hierarchy_top(const K* __restrict__ keys, uint32_t n, uint32_t leaf_max,
-                                                           uint32_t* __restrict__ gflags, GPart* __restrict__ gparts,
-                                                           FNode* __restrict__ nodes,
-                                                           const rk_batch_mesh* __restrict__ meshes,
-                                                           const uint32_t* __restrict__ pend,
-                                                           const uint32_t* __restrict__ pend_count) {
-  const uint32_t c0 = blockIdx.x * kChunk;
-  const uint32_t count = pend_count[blockIdx.x];
-  for (uint32_t k = threadIdx.x; k < count; k += 64) {
-    const uint32_t e = pend[c0 + k];
-    const uint32_t mine = e & ~kPendLeft;
-    const bool as_left = (e & kPendLeft) != 0;
-    uint64_t outer;
-    const Part me = load_part_coherent(gparts + mine, outer);
-    const uint32_t l = as_left ? me.end : mine, r = as_left ? mine : me.end;
-    uint32_t lo = 0, hi = n - 1;
-    if (kBatch) {
-      const rk_batch_mesh m = meshes[(uint32_t)((uint64_t)keys[mine] >> 30)];
-      lo = m.face_offset;
-      hi = m.face_offset + m.face_count - 1;
+__global__ __launch_bounds__(kReduceThreads) void k_hier_reduce(const K* __restrict__ keys, uint32_t n,
+                                                                uint32_t leaf_max, uint32_t chunks, uint32_t stride,
+                                                                FNode* __restrict__ nodes,
+                                                                HierItem* __restrict__ items,
+                                                                uint32_t* __restrict__ counts) {
+  constexpr uint32_t kT = kReduceThreads;
+  static_assert(kReduceFan == 64, "one lane per run");
+  __shared__ HierLds<kT> s;
+  __shared__ uint32_t s_off[kReduceFan + 1];
+  const uint32_t t = threadIdx.x;
+  const uint32_t base = blockIdx.x * kReduceFan * stride;  // the group's first chunk
+  uint64_t key0 = ~0ull;  // before the group's first position
+  if (t == 0 && base > 0u) key0 = split_key(keys, base * kChunk - 1u);
+  if (t < 64u) {
+    const uint64_t c = (uint64_t)base + (uint64_t)t * stride;
+    uint32_t incl = c < chunks ? counts[c] : 0u;
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(incl, off, 64);
+      if (t >= (uint32_t)off) incl += y;
     }
-    climb_crossing(n, leaf_max, gflags, gparts, nodes, lo, hi, me, outer, l, r, as_left, true);
+    s_off[t + 1u] = incl;
+    if (t == 0) s_off[0] = 0u;
+  }
+  __syncthreads();
+  const uint32_t total = s_off[kReduceFan];
+  uint32_t done = 0, m = 0, left = 0;  // items taken; items in front from the step before; left over
+  for (;;) {
+    const uint32_t take = min(total - done, kT - m);
+    Sub u;
+    u.a = u.b = t;
+    if (t < m) {  // in place since the step before
+      u.p = s.part[t];
+      u.l = s.first[t];
+      u.r = s.last[t];
+    } else if (t < m + take) {
+      const uint32_t e = done + t - m;
+      uint32_t lo = 0, hi = kReduceFan - 1u;  // the last run with s_off <= e
+      while (lo < hi) {
+        const uint32_t mid = (lo + hi + 1u) >> 1;
+        if (s_off[mid] <= e) lo = mid;
+        else hi = mid - 1u;
+      }
+      const HierItem it = items[((size_t)base + (size_t)lo * stride) * kChunk + (e - s_off[lo])];
+      u.p.lox = it.a.x; u.p.loy = it.a.y; u.p.loz = it.a.z; u.p.hix = it.a.w;
+      u.p.hiy = it.b.x; u.p.hiz = it.b.y;
+      u.p.ref = __float_as_uint(it.b.z);
+      u.l = __float_as_uint(it.b.w);
+      u.r = __float_as_uint(it.c.x);
+      s.first[t] = u.l;
+      s.last[t] = u.r;
+      s.key[t + 1u] = (uint64_t)__float_as_uint(it.c.z) | ((uint64_t)__float_as_uint(it.c.w) << 32);
+      // (a batch's first left-over subtree may lie further on)
+      if (t == 0) s.key[0] = u.l == base * kChunk ? key0 : split_key(keys, u.l - 1u);
+    }
+    m += take;
+    done += take;
+    for (uint32_t k = t; k <= m; k += kT) s.flag[k] = 0u;
+    if (t < 3u) s.cnt[t] = 0u;
+    __syncthreads();
+    bool ready = false, as_left;
+    uint32_t q = 0;
+    if (t < m) {
+      u.kl = s.key[t];
+      u.kr = s.key[t + 1u];
+      ready = hier_arrive(s, u, n, as_left, q) != 0u;
+    }
+    hier_rounds<kT, kBatch>(s, n, leaf_max, nodes, ready, q);
+    // split kT, which no thread has when m == kT, goes last
+    const Left o = left_over(s, m, t);
+    Left e;
+    e.has = false;
+    if (t == 0 && m == kT) e = left_over(s, m, m);
+    const uint32_t rank = hier_rank(s, o.has, left);
+    const uint32_t last = left;
+    if (m == kT && (s.flag[kT] == kFromLeft || s.flag[kT] == kFromRight)) ++left;
+    if (done == total || left >= kT) {  // left < kT: the tree's depth bounds it
+      if (o.has) store_item(items + (size_t)base * kChunk + rank, o.part, o.l, o.r, o.kr);
+      if (e.has) store_item(items + (size_t)base * kChunk + last, e.part, e.l, e.r, e.kr);
+      if (t == 0) counts[base] = left;
+      return;
+    }
+    // the left-over subtrees become the next step's first items
+    __syncthreads();
+    auto keep = [&](const Left& x, uint32_t at) {
+      s.part[at] = x.part;
+      s.first[at] = x.l;
+      s.last[at] = x.r;
+      s.key[at + 1u] = x.kr;
+      if (at == 0u) s.key[0] = x.kl;
+    };
+    if (o.has) keep(o, rank);
+    if (e.has) keep(e, last);
+    m = left;
+    __syncthreads();
   }
 }
 
@@ -996,52 +1068,37 @@ __global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ 
 
 inline unsigned blocks_for(uint32_t n, uint32_t per) { return (n + per - 1) / per; }
 
-// Up to this many faces the chunk pass also climbs the splits that cross
-// chunks, in the thread that reaches them: the chain above a few thousand
-// chunks is short, and a second launch would cost more than it saves (the 1M
-// heightfield: 224 us against 229 us with k_fast_hierarchy_top). Above it, a
-// workgroup waiting on that chain would hold its LDS while thousands of
-// chunks queue, so the climbs go to k_fast_hierarchy_top.
-#ifndef RK_INLINE_TOP_FACES
-#define RK_INLINE_TOP_FACES (1u << 21)
-#endif
-constexpr uint32_t kInlineTopFaces = RK_INLINE_TOP_FACES;
-
-// Workspace of the hierarchy passes over n positions.
+// Workspace of the hierarchy passes over n positions. The spare words keep the
+// workspace sizes, and the no-allocation build's face limits, what callers know.
 struct HierWs {
-  uint32_t* flags;       // counters of splits that cross chunks (zeroed per build)
-  GPart* parts;          // parts exchanged at splits that cross chunks
-  uint32_t* pend;        // per chunk, the climbs handed on to the top pass
-  uint32_t* pend_count;  // per chunk, how many
+  HierItem* items;   // the subtrees each chunk, then each group of chunks, left over
+  uint32_t* counts;  // per chunk, how many
 };
 inline size_t hier_ws_bytes(size_t n) {
-  return rk_align_up(n * 4) + rk_align_up(n * sizeof(GPart)) + rk_align_up(n * 4) +
+  return rk_align_up(n * 4) + rk_align_up(n * sizeof(HierItem)) + rk_align_up(n * 4) +
          rk_align_up(((n + kChunk - 1) / kChunk) * 4);
 }
 inline bool take_hier_ws(RkArena& ar, uint32_t n, HierWs& w) {
-  w.flags = ar.take<uint32_t>(n);
-  w.parts = ar.take<GPart>(n);
-  w.pend = ar.take<uint32_t>(n);
-  w.pend_count = ar.take<uint32_t>(blocks_for(n, kChunk));
-  return w.flags && w.parts && w.pend && w.pend_count;
+  uint32_t* spare0 = ar.take<uint32_t>(n);
+  w.items = ar.take<HierItem>(n);
+  uint32_t* spare1 = ar.take<uint32_t>(n);
+  w.counts = ar.take<uint32_t>((n + kChunk - 1) / kChunk);
+  return spare0 && w.items && spare1 && w.counts;
 }
-// Clears the counters and runs both hierarchy passes.
+// The chunk pass, then reductions of kReduceFan groups to one until one is left.
 template <typename K, bool kBatch>
 rk_status launch_hierarchy(hipStream_t st, const K* keys, const uint32_t* order, const uint4* f, const float4* v,
                            uint32_t n, uint32_t leaf_max, const HierWs& w, FNode* nodes, float4* tris,
-                           const rk_batch_mesh* meshes, bool flags_clear = false) {
-  if (!flags_clear) {
-    rk_status s = rk_fill_u32(reinterpret_cast<rk_stream>(st), w.flags, n, 0u);
-    if (s != RK_SUCCESS) return s;
-  }
-  const unsigned chunks = blocks_for(n, kChunk);
-  const uint32_t inline_top = n <= kInlineTopFaces ? 1u : 0u;
-  hipLaunchKernelGGL((k_fast_hierarchy<K, kBatch>), dim3(chunks), dim3(kLocalThreads), 0, st, keys, order, f, v, n,
-                     leaf_max, w.flags, w.parts, nodes, tris, meshes, w.pend, w.pend_count, inline_top);
+                           const rk_batch_mesh* meshes) {
+  const uint32_t chunks = blocks_for(n, kChunk);
+  hipLaunchKernelGGL((k_fast_hierarchy<K, kBatch>), dim3(chunks), dim3(kChunk), 0, st, keys, order, f, v, n, leaf_max,
+                     nodes, tris, meshes, w.items, w.counts);
   RK_CHECK_LAUNCH();
-  if (!inline_top) {
-    hipLaunchKernelGGL((k_fast_hierarchy_top<K, kBatch>), dim3(chunks), dim3(64), 0, st, keys, n, leaf_max, w.flags,
-                       w.parts, nodes, meshes, w.pend, w.pend_count);
+  uint32_t stride = 1;
+  for (uint32_t groups = chunks; groups > 1; stride *= kReduceFan) {
+    groups = blocks_for(groups, kReduceFan);
+    hipLaunchKernelGGL((k_hier_reduce<K, kBatch>), dim3(groups), dim3(kReduceThreads), 0, st, keys, n, leaf_max,
+                       chunks, stride, nodes, w.items, w.counts);
     RK_CHECK_LAUNCH();
   }
   return RK_SUCCESS;
@@ -1068,14 +1125,13 @@ static rk_status fast_build_keys(hipStream_t st, const uint4* f, const float4* v
   const uint32_t head_words = 1u + (uint32_t)sizeof(K) * 256u;
   const uint32_t grid_n = std::max(n, std::max((uint32_t)RK_INFO_WORDS, head_words));
   hipLaunchKernelGGL(k_fast_prep<K>, dim3(blocks_for(grid_n, 256)), dim3(256), 0, st, f, v, n, rmin, rmax,
-                     reinterpret_cast<Box*>(bvh->boxes), keys, order, info, hw.flags, static_cast<uint32_t*>(sort_ws),
-                     head_words);
+                     reinterpret_cast<Box*>(bvh->boxes), keys, order, info, static_cast<uint32_t*>(sort_ws), head_words);
   RK_CHECK_LAUNCH();
   rk_status s = rk_radix_sort_impl<K>(st, keys, order, n, 0, (int)sizeof(K), sort_ws, sort_bytes,
                                       info + RK_INFO_FLAGS, true);
   if (s != RK_SUCCESS) return s;
   return launch_hierarchy<K, false>(st, keys, order, f, v, n, leaf_max, hw, static_cast<FNode*>(bvh->nodes),
-                                    static_cast<float4*>(bvh->tris), (const rk_batch_mesh*)nullptr, true);
+                                    static_cast<float4*>(bvh->tris), (const rk_batch_mesh*)nullptr);
 }
 
 static rk_status fast_build_common(rk_stream stream, const rk_uint4* faces, const rk_float4* vertices,
@@ -1167,33 +1223,9 @@ extern "C" rk_status rk_fast_build_noalloc(rk_stream stream, const rk_uint4* fac
                            kNoAllocScratchBytes);
 }
 
-static rk_status fast_refit(rk_stream stream, const rk_uint4* faces, const rk_float4* vertices, uint32_t face_count,
-                            int morton_mode, uint32_t leaf_max, const rk_fast_bvh* bvh, const void* sorted_keys,
-                            void* ws, size_t ws_bytes, bool counters_clear);
-
 extern "C" rk_status rk_fast_refit(rk_stream stream, const rk_uint4* faces, const rk_float4* vertices,
                                    uint32_t face_count, int morton_mode, uint32_t leaf_max, const rk_fast_bvh* bvh,
                                    const void* sorted_keys, void* ws, size_t ws_bytes) {
-  return fast_refit(stream, faces, vertices, face_count, morton_mode, leaf_max, bvh, sorted_keys, ws, ws_bytes,
-                    false);
-}
-
-// For the request loop: where a refit over n faces keeps its split counters
-// in ws (n words), and the refit that takes them as already zero.
-uint32_t* rk_fast_refit_counters(void* ws, size_t ws_bytes, uint32_t n) {
-  RkArena ar(ws, ws_bytes);
-  HierWs hw;
-  return take_hier_ws(ar, n, hw) ? hw.flags : nullptr;
-}
-rk_status rk_fast_refit_precleared(rk_stream stream, const rk_uint4* faces, const rk_float4* vertices,
-                                   uint32_t face_count, int morton_mode, uint32_t leaf_max, const rk_fast_bvh* bvh,
-                                   const void* sorted_keys, void* ws, size_t ws_bytes) {
-  return fast_refit(stream, faces, vertices, face_count, morton_mode, leaf_max, bvh, sorted_keys, ws, ws_bytes, true);
-}
-
-static rk_status fast_refit(rk_stream stream, const rk_uint4* faces, const rk_float4* vertices, uint32_t face_count,
-                            int morton_mode, uint32_t leaf_max, const rk_fast_bvh* bvh, const void* sorted_keys,
-                            void* ws, size_t ws_bytes, bool counters_clear) {
   const uint32_t n = face_count;
   if (n == 0 || !faces || !vertices || !bvh || !sorted_keys) return RK_ERROR_INVALID_VALUE;
   if (!bvh->nodes || !bvh->tris || !bvh->indices) return RK_ERROR_INVALID_VALUE;
@@ -1210,10 +1242,9 @@ static rk_status fast_refit(rk_stream stream, const rk_uint4* faces, const rk_fl
   float4* tris = static_cast<float4*>(bvh->tris);
   if (morton_mode == RK_MORTON_63)
     return launch_hierarchy<uint64_t, false>(st, static_cast<const uint64_t*>(sorted_keys), bvh->indices, f, v, n,
-                                             leaf_max, hw, nodes, tris, (const rk_batch_mesh*)nullptr,
-                                             counters_clear);
+                                             leaf_max, hw, nodes, tris, (const rk_batch_mesh*)nullptr);
   return launch_hierarchy<uint32_t, false>(st, static_cast<const uint32_t*>(sorted_keys), bvh->indices, f, v, n,
-                                           leaf_max, hw, nodes, tris, (const rk_batch_mesh*)nullptr, counters_clear);
+                                           leaf_max, hw, nodes, tris, (const rk_batch_mesh*)nullptr);
 }
 
 
@@ -1585,14 +1616,10 @@ __device__ __forceinline__ float u01_of(uint64_t h) { return (float)(h >> 40) * 
 
 // v = base + amplitude * sin(omega * time + phase_v) * axis_v; phase and axis
 // hashed from the vertex index (axis uniform on the sphere, or +z).
-// Threads below clear_n also zero clear[i] (the request loop clears a
-// refit's split counters here instead of in a launch of its own).
 __global__ __launch_bounds__(256) void k_deform(const float4* __restrict__ base, float4* __restrict__ out,
                                                 uint32_t count, float amplitude, float omega, float time,
-                                                uint64_t seed, int along_z, uint32_t* __restrict__ clear,
-                                                uint32_t clear_n) {
+                                                uint64_t seed, int along_z) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
-  if (i < clear_n) clear[i] = 0u;
   if (i >= count) return;
   const uint64_t h0 = mix64(seed ^ (0x9E3779B97F4A7C15ull * ((uint64_t)i + 1)));
   const uint64_t h1 = mix64(h0 + 0x632BE59BD9B4E019ull), h2 = mix64(h1 + 0x632BE59BD9B4E019ull);
@@ -1608,6 +1635,11 @@ __global__ __launch_bounds__(256) void k_deform(const float4* __restrict__ base,
   const float s = amplitude * sinf(omega * time + phase);
   const float4 b = base[i];
   out[i] = make_float4(b.x + s * ax, b.y + s * ay, b.z + s * az, b.w);
+}
+
+__device__ __forceinline__ uint64_t shfl_down64(uint64_t v, int d) {
+  uint32_t lo = __shfl_down((uint32_t)v, d, 64), hi = __shfl_down((uint32_t)(v >> 32), d, 64);
+  return ((uint64_t)hi << 32) | lo;
 }
 
 // Order-independent frame checksum: the wrapping sum over rays of a hash of
@@ -2122,25 +2154,10 @@ extern "C" rk_status rk_deform_vertices(rk_stream stream, const rk_float4* base,
   if (!base || !out) return RK_ERROR_INVALID_VALUE;
   hipLaunchKernelGGL(k_deform, dim3(blocks_for(count, 256)), dim3(256), 0, rk_hip_stream(stream),
                      reinterpret_cast<const float4*>(base), reinterpret_cast<float4*>(out), count, amplitude, omega,
-                     time, seed, along_z, (uint32_t*)nullptr, 0u);
+                     time, seed, along_z);
   RK_CHECK_LAUNCH();
   return RK_SUCCESS;
 }
-
-// For the request loop (rk_serve.hip): rk_deform_vertices that also zeroes
-// clear[0, clear_n).
-rk_status rk_deform_and_clear(hipStream_t st, const rk_float4* base, rk_float4* out, uint32_t count, float amplitude,
-                              float omega, float time, uint64_t seed, int along_z, uint32_t* clear,
-                              uint32_t clear_n) {
-  if (!base || !out || (clear_n && !clear)) return RK_ERROR_INVALID_VALUE;
-  const uint32_t n = std::max(count, clear_n);
-  if (n == 0) return RK_SUCCESS;
-  hipLaunchKernelGGL(k_deform, dim3(blocks_for(n, 256)), dim3(256), 0, st, reinterpret_cast<const float4*>(base),
-                     reinterpret_cast<float4*>(out), count, amplitude, omega, time, seed, along_z, clear, clear_n);
-  RK_CHECK_LAUNCH();
-  return RK_SUCCESS;
-}
-
 
 extern "C" rk_status rk_frame_checksum(rk_stream stream, const uint32_t* faces_id, const rk_float2* coords,
                                        const float* depths, uint32_t count, const uint32_t* indices,

@@ -7,12 +7,11 @@
 // Admitted requests run concurrently, one per slot: the GPU overlaps their
 // kernels while the host keeps admitting. Per request, on its slot's stream:
 // upload the scene if it was not resident, deform its vertices for the
-// request's time (the same launch clears a refit's split counters), rebuild
-// or refit its tree, trace the camera frame, and checksum it; the checksum
-// launch's last workgroup writes the checksum and then the request's ticket
-// to pinned host memory, which is how the host sees the request finish (four
-// launches per refit request). Requests of one scene
-// are ordered, since they share its buffers: a request whose scene's latest
+// request's time, rebuild or refit its tree, trace the camera frame, and
+// checksum it; the checksum launch's last workgroup writes the checksum and
+// then the request's ticket to pinned host memory, which is how the host sees
+// the request finish (five launches for a refit of up to 32,768 faces). Requests
+// of one scene are ordered, since they share its buffers: a request whose scene's latest
 // request still runs on another slot waits for an event recorded there.
 //
 // Nothing here allocates per request: the arena, the slot workspaces and the
@@ -35,13 +34,6 @@ rk_status rk_frame_checksum_to_host(hipStream_t st, const uint32_t* faces_id, co
                                     const float* depths, uint32_t count, const uint32_t* indices,
                                     uint32_t face_count, uint64_t* partials, uint32_t* counter, uint64_t* out_host,
                                     uint64_t done_value, const uint32_t* build_flags);
-rk_status rk_deform_and_clear(hipStream_t st, const rk_float4* base, rk_float4* out, uint32_t count, float amplitude,
-                              float omega, float time, uint64_t seed, int along_z, uint32_t* clear,
-                              uint32_t clear_n);
-uint32_t* rk_fast_refit_counters(void* ws, size_t ws_bytes, uint32_t n);
-rk_status rk_fast_refit_precleared(rk_stream stream, const rk_uint4* faces, const rk_float4* vertices,
-                                   uint32_t face_count, int morton_mode, uint32_t leaf_max, const rk_fast_bvh* bvh,
-                                   const void* sorted_keys, void* ws, size_t ws_bytes);
 
 namespace {
 
@@ -296,12 +288,8 @@ struct rk_server_st {
     const bool force_refit = (r.flags & RK_REQUEST_FORCE_REFIT) != 0;
     const bool rebuild = !s.built || force_rebuild ||
                          (!force_refit && (cfg.rebuild_every == 0 || s.refits >= cfg.rebuild_every));
-    // A refit's split counters are cleared by the deform launch; a rebuild
-    // clears its own in its key kernel.
-    uint32_t* counters = rebuild ? nullptr : rk_fast_refit_counters(sl.ws, sl.ws_bytes, s.nf);
-    if (!rebuild && !counters) return RK_ERROR_WORKSPACE;
-    if ((e = rk_deform_and_clear(sl.st, s.base, s.verts, s.nv, s.amplitude, cfg.omega, r.time,
-                                 0x5EED0000ull + r.scene, s.along_z, counters, rebuild ? 0u : s.nf)) != RK_SUCCESS)
+    if ((e = rk_deform_vertices(st, s.base, s.verts, s.nv, s.amplitude, cfg.omega, r.time, 0x5EED0000ull + r.scene,
+                                s.along_z)) != RK_SUCCESS)
       return e;
     if (rebuild) {
       s.built = false;
@@ -312,8 +300,7 @@ struct rk_server_st {
       s.refits = 0;
       ++rebuilds;
     } else {
-      e = rk_fast_refit_precleared(st, s.faces, s.verts, s.nf, RK_MORTON_30, cfg.leaf_max, &bvh, s.keys, sl.ws,
-                                   sl.ws_bytes);
+      e = rk_fast_refit(st, s.faces, s.verts, s.nf, RK_MORTON_30, cfg.leaf_max, &bvh, s.keys, sl.ws, sl.ws_bytes);
       ++s.refits;
       ++refits;
     }
