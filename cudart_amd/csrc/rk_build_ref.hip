@@ -13,11 +13,8 @@
 #include <algorithm>
 
 #include "rk_device.h"
+#include "rk_sort.h"
 
-template <typename K>
-rk_status rk_radix_sort_impl(hipStream_t st, K* keys, uint32_t* vals, uint32_t n, int first_pass, int passes,
-                             void* ws, size_t ws_bytes, uint32_t* err, bool head_cleared = false,
-                             const uint32_t** digit_counts = nullptr);
 rk_status rk_sort_general_impl(hipStream_t st, uint32_t* keys, uint32_t* indices, uint32_t length,
                                uint32_t bit_depth, int init_indices, void* ws, size_t ws_bytes, uint32_t* err);
 
@@ -98,18 +95,53 @@ __global__ __launch_bounds__(256) void k_calc_boxes(const uint4* __restrict__ fa
   indices[k] = k;
 }
 
-__global__ __launch_bounds__(256) void k_boxes_morton32(const uint4* __restrict__ faces,
-                                                        const float4* __restrict__ verts, uint32_t n, float4 rmin,
-                                                        float4 rmax, Box* __restrict__ boxes,
-                                                        uint32_t* __restrict__ indices, uint32_t* __restrict__ codes) {
-  uint32_t k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= n) return;
-  Box b = face_box(faces, verts, k);
-  float4* o = reinterpret_cast<float4*>(boxes + k);
-  o[0] = b.mn;
-  o[1] = b.mx;
-  indices[k] = k;
-  codes[k] = morton_ref32(b, rmin, rmax);
+// Boxes, indices and reference codes of the faces, per * kBoxThreads per workgroup.
+// counts (may be NULL): the sort's digit counts, zero already. copy (may be
+// NULL): receives the faces as they are, for the reorder at the end.
+constexpr uint32_t kBoxThreads = 1024;
+__global__ __launch_bounds__(kBoxThreads) void k_boxes_morton32(const uint4* __restrict__ faces,
+                                                                const float4* __restrict__ verts, uint32_t n,
+                                                                float4 rmin, float4 rmax, Box* __restrict__ boxes,
+                                                                uint32_t* __restrict__ indices,
+                                                                uint32_t* __restrict__ codes, uint32_t per,
+                                                                uint32_t* __restrict__ counts, uint32_t copies,
+                                                                uint4* __restrict__ copy) {
+  __shared__ uint32_t s_hist[4 * 256];
+  s_hist[threadIdx.x] = 0u;
+  __syncthreads();
+  for (uint32_t u = 0; u < per; ++u) {
+    const size_t kk = ((size_t)blockIdx.x * per + u) * kBoxThreads + threadIdx.x;
+    if (kk >= n) break;
+    const uint32_t k = (uint32_t)kk;
+    const uint4 f = faces[k];
+    if (copy) copy[k] = f;
+    const float4 v0 = verts[f.x], v1 = verts[f.y], v2 = verts[f.z];
+    Box b;  // CUDA_calcMeshBoxes.cu:53-55: reset(v0), merge(v1), merge(v2)
+    b.mn = rk::min4(rk::min4(v0, v1), v2);
+    b.mx = rk::max4(rk::max4(v0, v1), v2);
+    float4* o = reinterpret_cast<float4*>(boxes + k);
+    o[0] = b.mn;
+    o[1] = b.mx;
+    indices[k] = k;
+    const uint32_t code = morton_ref32(b, rmin, rmax);
+    codes[k] = code;
+    if (counts) rk_count_digits<uint32_t, 4>(s_hist, code);
+  }
+  if (counts) {
+    __syncthreads();
+    rk_flush_digits<4, (int)kBoxThreads>(s_hist, counts, copies);
+  }
+}
+
+// Zeroes the build's info words and level counts, and two runs of words.
+__global__ __launch_bounds__(256) void k_lbvh_clear(uint32_t* __restrict__ info, uint32_t* __restrict__ level_count,
+                                                    uint32_t* __restrict__ a, size_t na, uint32_t* __restrict__ b,
+                                                    size_t nb) {
+  const size_t stride = (size_t)gridDim.x * 256, t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (t < RK_INFO_WORDS) info[t] = 0u;
+  if (t < 64) level_count[t] = 0u;
+  for (size_t i = t; i < na; i += stride) a[i] = 0u;
+  for (size_t i = t; i < nb; i += stride) b[i] = 0u;
 }
 
 __global__ __launch_bounds__(256) void k_morton(const Box* __restrict__ boxes, uint32_t n, float4 rmin, float4 rmax,
@@ -126,19 +158,36 @@ __global__ __launch_bounds__(256) void k_morton(const Box* __restrict__ boxes, u
 // codes with code[s]^code[s+1] != 0, level = clz (0 = bit 31). Here every
 // position gets a key (32 = no split) so one stable 8-bit pass groups the
 // splits by level, ascending within a level.
-// The per-level counts come from the digit counts of that pass (its first
-// 33 digits), except for a single split, which no sort runs on: then this
-// kernel counts it (level_count, may be NULL otherwise).
+// Counts the levels as it goes: into level_count (33 of its words), and into
+// the sort's digit counts when it takes them (digits, may be NULL).
+constexpr uint32_t kSplitPer = 8;  // positions per thread
 __global__ __launch_bounds__(256) void k_split_levels(const uint32_t* __restrict__ codes, uint32_t n,
                                                       uint32_t* __restrict__ lev, uint32_t* __restrict__ pos,
-                                                      uint32_t* __restrict__ level_count) {
-  uint32_t s = blockIdx.x * 256 + threadIdx.x;
-  if (s + 1 < n) {
-    uint32_t diff = codes[s] ^ codes[s + 1];
-    uint32_t level = diff ? (uint32_t)__clz((int)diff) : 32u;
-    lev[s] = level;
-    pos[s] = s + 1;
-    if (level_count) atomicAdd(&level_count[level], 1u);
+                                                      uint32_t* __restrict__ level_count,
+                                                      uint32_t* __restrict__ digits, uint32_t copies) {
+  constexpr uint32_t kCopies = 16;  // most splits share a few levels: lanes count into copies
+  __shared__ uint32_t s_count[kCopies][33];
+  for (uint32_t i = threadIdx.x; i < kCopies * 33; i += 256) (&s_count[0][0])[i] = 0u;
+  __syncthreads();
+#pragma unroll 4
+  for (uint32_t u = 0; u < kSplitPer; ++u) {
+    const uint32_t s = (blockIdx.x * kSplitPer + u) * 256 + threadIdx.x;
+    if (s + 1 < n) {
+      uint32_t diff = codes[s] ^ codes[s + 1];
+      uint32_t level = diff ? (uint32_t)__clz((int)diff) : 32u;
+      lev[s] = level;
+      pos[s] = s + 1;
+      atomicAdd(&s_count[threadIdx.x % kCopies][level], 1u);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 33) {
+    uint32_t c = 0;
+    for (uint32_t i = 0; i < kCopies; ++i) c += s_count[i][threadIdx.x];
+    if (c) {
+      atomicAdd(&level_count[threadIdx.x], c);
+      if (digits) atomicAdd(&digits[(size_t)(blockIdx.x % copies) * 256 + threadIdx.x], c);
+    }
   }
 }
 
@@ -573,32 +622,44 @@ extern "C" rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_f
     return RK_ERROR_WORKSPACE;
 
   rk_status s;
-  if ((s = rk_fill_u32(stream, info, RK_INFO_WORDS, 0u)) != RK_SUCCESS) return s;
-  if ((s = rk_fill_u32(stream, level_count, 64, 0u)) != RK_SUCCESS) return s;
-  float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
-  float4 rmax = make_float4(hitbox->max.x, hitbox->max.y, hitbox->max.z, hitbox->max.w);
+  const float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
+  const float4 rmax = make_float4(hitbox->max.x, hitbox->max.y, hitbox->max.z, hitbox->max.w);
   uint4* f = reinterpret_cast<uint4*>(faces);
-  hipLaunchKernelGGL(k_boxes_morton32, dim3(blocks_for(n, 256)), dim3(256), 0, st, f,
-                     reinterpret_cast<const float4*>(vertices), n, rmin, rmax, reinterpret_cast<Box*>(boxes), indices,
-                     codes);
+  // CUDA_radixSortGeneral(codes, indices, N, 32, true), CUDA_buildMeshTreeLBVH.cu:522-528: above its bitonic
+  // class (32768) a stable sort, whose digits the box kernel counts. The sort of the splits by level has its
+  // workspace in the topology's records, which nothing uses before that.
+  const bool plain = n > 4u * 8192u;
+  RkSortPlan<uint32_t> codes_plan, levels_plan;
+  if (plain && (s = rk_sort_plan<uint32_t>(n, 32, false, codes, indices, sort_ws, sort_bytes, codes_plan)) != RK_SUCCESS)
+    return s;
+  if (n > 1 && (s = rk_sort_plan<uint32_t>(n - 1, 8, true, lev, pos, tw.ra, 7 * rk_align_up(cap * 4), levels_plan)) !=
+                   RK_SUCCESS)
+    return s;
+  const bool counted = n > 1 && !levels_plan.one;  // the levels are counted where they are found
+  const size_t clear_a = plain ? codes_plan.head_words + codes_plan.status_words : 0;
+  const size_t clear_b = counted ? levels_plan.head_words + levels_plan.status_words : 0;
+  hipLaunchKernelGGL(k_lbvh_clear, dim3(std::min<unsigned>(1024u, blocks_for((uint32_t)(clear_a + clear_b + 64), 1024))),
+                     dim3(256), 0, st, info, level_count, codes_plan.head, clear_a, levels_plan.head, clear_b);
   RK_CHECK_LAUNCH();
-  // CUDA_radixSortGeneral(codes, indices, N, 32, true), CUDA_buildMeshTreeLBVH.cu:522-528.
-  s = rk_sort_general_impl(st, codes, indices, n, 32, 0, sort_ws, sort_bytes, info + RK_INFO_FLAGS);
+  // 4 faces per thread from 2^18 on, where that still leaves a workgroup for most CUs
+  const uint32_t per = n >= (1u << 18) ? 4u : 1u;
+  hipLaunchKernelGGL(k_boxes_morton32, dim3(blocks_for(n, per * kBoxThreads)), dim3(kBoxThreads), 0, st, f,
+                     reinterpret_cast<const float4*>(vertices), n, rmin, rmax, reinterpret_cast<Box*>(boxes), indices,
+                     codes, per, plain ? codes_plan.head + 1 : (uint32_t*)nullptr, codes_plan.copies,
+                     tree_complete ? ftmp : (uint4*)nullptr);
+  RK_CHECK_LAUNCH();
+  s = plain ? rk_sort_run<uint32_t>(st, codes_plan, true, info + RK_INFO_FLAGS)
+            : rk_sort_general_impl(st, codes, indices, n, 32, 0, sort_ws, sort_bytes, info + RK_INFO_FLAGS);
   if (s != RK_SUCCESS) return s;
-  const uint32_t* counts = level_count;  // zero when there is no split
   if (n > 1) {
-    // one split is not sorted, so its level is counted here; more are counted
-    // by the sort that groups them by level
-    hipLaunchKernelGGL(k_split_levels, dim3(blocks_for(n - 1, 256)), dim3(256), 0, st, codes, n, lev, pos,
-                       n == 2 ? level_count : (uint32_t*)nullptr);
+    hipLaunchKernelGGL(k_split_levels, dim3(blocks_for(n - 1, 256 * kSplitPer)), dim3(256), 0, st, codes, n,
+                       levels_plan.src, levels_plan.vsrc, level_count,
+                       counted ? levels_plan.head + 1 : (uint32_t*)nullptr, levels_plan.copies);
     RK_CHECK_LAUNCH();
-    const uint32_t* digit_counts = nullptr;
-    s = rk_radix_sort_impl<uint32_t>(st, lev, pos, n - 1, 0, 1, sort_ws, sort_bytes, info + RK_INFO_FLAGS, false,
-                                     &digit_counts);
+    s = rk_sort_run<uint32_t>(st, levels_plan, counted, info + RK_INFO_FLAGS);
     if (s != RK_SUCCESS) return s;
-    if (digit_counts) counts = digit_counts;
   }
-  hipLaunchKernelGGL(k_topo_ref, dim3(1), dim3(kTopoThreads), 0, st, pos, counts, n, tree_depth, tree_complete,
+  hipLaunchKernelGGL(k_topo_ref, dim3(1), dim3(kTopoThreads), 0, st, pos, level_count, n, tree_depth, tree_complete,
                      tw, reinterpret_cast<Node*>(nodes), info);
   RK_CHECK_LAUNCH();
   unsigned lb = blocks_for(n, 64 * 4);
@@ -610,9 +671,7 @@ extern "C" rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_f
                      reinterpret_cast<Node*>(nodes));
   RK_CHECK_LAUNCH();
   if (tree_complete) {  // CUDA_reorderMeshFaces, CUDA_buildMeshTreeLBVH.cu:669-676
-    hipLaunchKernelGGL(k_gather_faces, dim3(blocks_for(n, 256)), dim3(256), 0, st, f, indices, ftmp, n);
-    RK_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_copy_faces, dim3(blocks_for(n, 256)), dim3(256), 0, st, ftmp, f, n);
+    hipLaunchKernelGGL(k_gather_faces, dim3(blocks_for(n, 256)), dim3(256), 0, st, ftmp, indices, f, n);
     RK_CHECK_LAUNCH();
   }
   return RK_SUCCESS;

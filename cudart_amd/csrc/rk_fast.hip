@@ -27,11 +27,7 @@
 #include <mutex>
 
 #include "rk_device.h"
-
-template <typename K>
-rk_status rk_radix_sort_impl(hipStream_t st, K* keys, uint32_t* vals, uint32_t n, int first_pass, int passes,
-                             void* ws, size_t ws_bytes, uint32_t* err, bool head_cleared = false,
-                             const uint32_t** digit_counts = nullptr);
+#include "rk_sort.h"
 
 namespace {
 
@@ -61,44 +57,61 @@ __device__ __forceinline__ uint64_t spread21(uint64_t v) {
   return v;
 }
 
-// Also clears the build's info words and the sort's error word and digit
-// counts (sort_head, head_words), which saves two fill launches per build.
-template <typename K>
-__global__ __launch_bounds__(256) void k_fast_prep(const uint4* __restrict__ faces, const float4* __restrict__ verts,
-                                                   uint32_t n, float4 rmin, float4 rmax, Box* __restrict__ boxes,
-                                                   K* __restrict__ keys, uint32_t* __restrict__ vals,
-                                                   uint32_t* __restrict__ info, uint32_t* __restrict__ sort_head,
-                                                   uint32_t head_words) {
-  uint32_t k = blockIdx.x * 256 + threadIdx.x;
-  if (k < RK_INFO_WORDS) info[k] = 0u;
-  if (k < head_words) sort_head[k] = 0u;
-  if (k >= n) return;
-  uint4 f = faces[k];
-  float4 v0 = verts[f.x], v1 = verts[f.y], v2 = verts[f.z];
-  Box b;
-  b.mn = rk::min4(rk::min4(v0, v1), v2);
-  b.mx = rk::max4(rk::max4(v0, v1), v2);
-  if (boxes) {  // the API's per-face boxes, when the caller keeps them
-    float4* o = reinterpret_cast<float4*>(boxes + k);
-    o[0] = b.mn;
-    o[1] = b.mx;
+// Per-face box (API array), Morton key and index. kPasses > 0: also counts the
+// digits of the sort's kPasses passes (counts and info are zero already);
+// otherwise it clears the build's info words. 'per' faces per thread.
+constexpr uint32_t kPrepThreads = 1024;
+constexpr uint32_t kCountInPrep = 1u << 21;
+constexpr uint32_t kCountPer4 = 1u << 18;  // 4 faces per thread from here on: below, that leaves most CUs idle
+template <typename K, int kPasses>
+__global__ __launch_bounds__(kPrepThreads) void k_fast_prep(const uint4* __restrict__ faces,
+                                                            const float4* __restrict__ verts, uint32_t n, float4 rmin,
+                                                            float4 rmax, Box* __restrict__ boxes,
+                                                            K* __restrict__ keys, uint32_t* __restrict__ vals,
+                                                            uint32_t* __restrict__ info, uint32_t per,
+                                                            uint32_t* __restrict__ counts, uint32_t copies) {
+  constexpr int kWords = kPasses * 256;
+  __shared__ uint32_t s_hist[kWords ? kWords : 1];
+  if (kPasses) {
+    for (int i = threadIdx.x; i < kWords; i += kPrepThreads) s_hist[i] = 0u;
+    __syncthreads();
+  } else if (blockIdx.x == 0 && threadIdx.x < RK_INFO_WORDS) {
+    info[threadIdx.x] = 0u;
   }
-  float4 len = rk::sub4(rmax, rmin);
-  float4 c = rk::muls4(rk::add4(b.mn, b.mx), 0.5f);
-  if (sizeof(K) == 4) {
-    float sx = 1024.0f / len.x, sy = 1024.0f / len.y, sz = 1024.0f / len.z;
-    uint32_t qx = min(rk::f2u_sat((c.x - rmin.x) * sx), 1023u);
-    uint32_t qy = min(rk::f2u_sat((c.y - rmin.y) * sy), 1023u);
-    uint32_t qz = min(rk::f2u_sat((c.z - rmin.z) * sz), 1023u);
-    keys[k] = (K)((spread10(qx) << 2) | (spread10(qy) << 1) | spread10(qz));
-  } else {
-    float sx = 2097152.0f / len.x, sy = 2097152.0f / len.y, sz = 2097152.0f / len.z;
-    uint32_t qx = min(rk::f2u_sat((c.x - rmin.x) * sx), 2097151u);
-    uint32_t qy = min(rk::f2u_sat((c.y - rmin.y) * sy), 2097151u);
-    uint32_t qz = min(rk::f2u_sat((c.z - rmin.z) * sz), 2097151u);
-    keys[k] = (K)((spread21(qx) << 2) | (spread21(qy) << 1) | spread21(qz));
+  const float4 len = rk::sub4(rmax, rmin);
+  const float cells = sizeof(K) == 4 ? 1024.0f : 2097152.0f;
+  const uint32_t top = sizeof(K) == 4 ? 1023u : 2097151u;
+  const float sx = cells / len.x, sy = cells / len.y, sz = cells / len.z;
+  const size_t base = (size_t)blockIdx.x * per * kPrepThreads + threadIdx.x;
+  for (uint32_t u = 0; u < per; ++u) {
+    const size_t kk = base + (size_t)u * kPrepThreads;
+    if (kk >= n) break;
+    const uint32_t k = (uint32_t)kk;
+    const uint4 f = faces[k];
+    const float4 v0 = verts[f.x], v1 = verts[f.y], v2 = verts[f.z];
+    Box b;
+    b.mn = rk::min4(rk::min4(v0, v1), v2);
+    b.mx = rk::max4(rk::max4(v0, v1), v2);
+    if (boxes) {  // the API's per-face boxes, when the caller keeps them
+      float4* o = reinterpret_cast<float4*>(boxes + k);
+      o[0] = b.mn;
+      o[1] = b.mx;
+    }
+    const float4 c = rk::muls4(rk::add4(b.mn, b.mx), 0.5f);
+    const uint32_t qx = min(rk::f2u_sat((c.x - rmin.x) * sx), top);
+    const uint32_t qy = min(rk::f2u_sat((c.y - rmin.y) * sy), top);
+    const uint32_t qz = min(rk::f2u_sat((c.z - rmin.z) * sz), top);
+    K key;
+    if (sizeof(K) == 4) key = (K)((spread10(qx) << 2) | (spread10(qy) << 1) | spread10(qz));
+    else key = (K)((spread21(qx) << 2) | (spread21(qy) << 1) | spread21(qz));
+    keys[k] = key;
+    vals[k] = k;
+    if (kPasses) rk_count_digits<K, kPasses>(s_hist, key);
   }
-  vals[k] = k;
+  if (kPasses) {
+    __syncthreads();
+    rk_flush_digits<kPasses, (int)kPrepThreads>(s_hist, counts, copies);
+  }
 }
 
 // Split key between sorted positions i and i+1 (Apetrei 2014, "Fast and
@@ -1068,8 +1081,9 @@ __global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ 
 
 inline unsigned blocks_for(uint32_t n, uint32_t per) { return (n + per - 1) / per; }
 
-// Workspace of the hierarchy passes over n positions. The spare words keep the
-// workspace sizes, and the no-allocation build's face limits, what callers know.
+// Workspace of the hierarchy passes over n positions. Its size has 8 B per
+// position more than the passes use, so that the workspace sizes and the
+// no-allocation build's face limits stay what callers know.
 struct HierWs {
   HierItem* items;   // the subtrees each chunk, then each group of chunks, left over
   uint32_t* counts;  // per chunk, how many
@@ -1079,11 +1093,15 @@ inline size_t hier_ws_bytes(size_t n) {
          rk_align_up(((n + kChunk - 1) / kChunk) * 4);
 }
 inline bool take_hier_ws(RkArena& ar, uint32_t n, HierWs& w) {
-  uint32_t* spare0 = ar.take<uint32_t>(n);
   w.items = ar.take<HierItem>(n);
-  uint32_t* spare1 = ar.take<uint32_t>(n);
   w.counts = ar.take<uint32_t>((n + kChunk - 1) / kChunk);
-  return spare0 && w.items && spare1 && w.counts;
+  return w.items && w.counts;
+}
+// What is left of the workspace.
+inline void* rest_of(const RkArena& ar, size_t& bytes) {
+  const size_t at = rk_align_up(ar.used);
+  bytes = at < ar.size ? ar.size - at : 0;
+  return ar.base ? ar.base + at : nullptr;
 }
 // The chunk pass, then reductions of kReduceFan groups to one until one is left.
 template <typename K, bool kBatch>
@@ -1120,15 +1138,27 @@ template <typename K>
 static rk_status fast_build_keys(hipStream_t st, const uint4* f, const float4* v, uint32_t n, float4 rmin,
                                  float4 rmax, const rk_fast_bvh* bvh, uint32_t leaf_max, K* keys, const HierWs& hw,
                                  void* sort_ws, size_t sort_bytes, uint32_t* info) {
+  constexpr int kKeyBits = sizeof(K) == 4 ? 30 : 63;
   uint32_t* order = bvh->indices;
-  // the sort's workspace starts with its error word and digit counts
-  const uint32_t head_words = 1u + (uint32_t)sizeof(K) * 256u;
-  const uint32_t grid_n = std::max(n, std::max((uint32_t)RK_INFO_WORDS, head_words));
-  hipLaunchKernelGGL(k_fast_prep<K>, dim3(blocks_for(grid_n, 256)), dim3(256), 0, st, f, v, n, rmin, rmax,
-                     reinterpret_cast<Box*>(bvh->boxes), keys, order, info, static_cast<uint32_t*>(sort_ws), head_words);
+  RkSortPlan<K> plan;
+  rk_status s = rk_sort_plan<K>(n, kKeyBits, true, keys, order, sort_ws, sort_bytes, plan);
+  if (s != RK_SUCCESS) return s;
+  // Below 2^21 faces the key kernel counts the sort's digits as well (1M
+  // faces: 14.4 us, and 4.9 to clear the counts, against 15.5 and 13.2 for a
+  // kernel of its own); above, its LDS atomics cost what that kernel does
+  // (10M faces, 63-bit keys: 274 against 203 + 65 us).
+  const bool counted = !plan.one && n < kCountInPrep;
+  if (counted && (s = rk_sort_clear<K>(st, plan, info)) != RK_SUCCESS) return s;
+  const uint32_t per = counted && n >= kCountPer4 ? 4u : 1u;
+  auto prep = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(blocks_for(n, per * kPrepThreads)), dim3(kPrepThreads), 0, st, f, v, n, rmin,
+                       rmax, reinterpret_cast<Box*>(bvh->boxes), plan.src, plan.vsrc, info, per, plan.head + 1,
+                       plan.copies);
+  };
+  if (counted) prep(k_fast_prep<K, (int)sizeof(K)>);
+  else prep(k_fast_prep<K, 0>);
   RK_CHECK_LAUNCH();
-  rk_status s = rk_radix_sort_impl<K>(st, keys, order, n, 0, (int)sizeof(K), sort_ws, sort_bytes,
-                                      info + RK_INFO_FLAGS, true);
+  s = rk_sort_run<K>(st, plan, counted, info + RK_INFO_FLAGS);
   if (s != RK_SUCCESS) return s;
   return launch_hierarchy<K, false>(st, keys, order, f, v, n, leaf_max, hw, static_cast<FNode*>(bvh->nodes),
                                     static_cast<float4*>(bvh->tris), (const rk_batch_mesh*)nullptr);
@@ -1150,9 +1180,9 @@ static rk_status fast_build_common(rk_stream stream, const rk_uint4* faces, cons
   void* keys = wide ? (void*)ar.take<uint64_t>(n) : (void*)ar.take<uint32_t>(n);
   HierWs hw;
   const bool hw_ok = take_hier_ws(ar, n, hw);
-  size_t sort_bytes = rk_sort_workspace_size(n, wide ? 8 : 4);
-  void* sort_ws = ar.take<char>(sort_bytes);
-  if (!keys || !hw_ok || !sort_ws) return RK_ERROR_WORKSPACE;
+  size_t sort_bytes = 0;
+  void* sort_ws = rest_of(ar, sort_bytes);
+  if (!keys || !hw_ok) return RK_ERROR_WORKSPACE;
   if (sorted_keys) keys = sorted_keys;
   float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
   float4 rmax = make_float4(hitbox->max.x, hitbox->max.y, hitbox->max.z, hitbox->max.w);
@@ -1406,10 +1436,10 @@ __global__ __launch_bounds__(kWG) void k_batch_trace_queue(const rk_batch_mesh* 
   }
 }
 
-uint32_t key_passes_for(uint32_t mesh_count) {
-  uint32_t bits = 30;
+int key_bits_for(uint32_t mesh_count) {
+  int bits = 30;
   while (bits < 64 && (1ull << (bits - 30)) < mesh_count) ++bits;
-  return (bits + 7) / 8;
+  return bits;
 }
 
 bool config_ok(const rk_batch_config* c) {
@@ -1455,19 +1485,20 @@ extern "C" rk_status rk_batch_build(rk_stream stream, const rk_batch_mesh* meshe
   uint64_t* keys = ar.take<uint64_t>(n);
   HierWs hw;
   const bool hw_ok = take_hier_ws(ar, n, hw);
-  const size_t sort_bytes = rk_sort_workspace_size(n, 8);
-  void* sort_ws = ar.take<char>(sort_bytes);
-  if (!keys || !hw_ok || !sort_ws) return RK_ERROR_WORKSPACE;
-  rk_status s;
-  if ((s = rk_fill_u32(stream, info, RK_INFO_WORDS, 0u)) != RK_SUCCESS) return s;
+  size_t sort_bytes = 0;
+  void* sort_ws = rest_of(ar, sort_bytes);
+  if (!keys || !hw_ok) return RK_ERROR_WORKSPACE;
   const uint4* f = reinterpret_cast<const uint4*>(faces);
   const float4* v = reinterpret_cast<const float4*>(vertices);
   uint32_t* order = bvh->indices;
+  RkSortPlan<uint64_t> plan;
+  rk_status s = rk_sort_plan<uint64_t>(n, key_bits_for(mesh_count), true, keys, order, sort_ws, sort_bytes, plan);
+  if (s != RK_SUCCESS) return s;
+  if ((s = rk_fill_u32(stream, info, RK_INFO_WORDS, 0u)) != RK_SUCCESS) return s;
   hipLaunchKernelGGL(k_batch_prep, dim3(blocks_for(n, 256)), dim3(256), 0, st, meshes, mesh_count, f, v, n, hitboxes,
-                     keys, order);
+                     plan.src, plan.vsrc);
   RK_CHECK_LAUNCH();
-  s = rk_radix_sort_impl<uint64_t>(st, keys, order, n, 0, (int)key_passes_for(mesh_count), sort_ws, sort_bytes,
-                                   info + RK_INFO_FLAGS);
+  s = rk_sort_run<uint64_t>(st, plan, false, info + RK_INFO_FLAGS);
   if (s != RK_SUCCESS) return s;
   return launch_hierarchy<uint64_t, true>(st, keys, order, f, v, n, config->leaf_max, hw,
                                           static_cast<FNode*>(bvh->nodes), static_cast<float4*>(bvh->tris), meshes);
@@ -1543,11 +1574,14 @@ extern "C" rk_status rk_batch_trace(rk_stream stream, const rk_batch_mesh* meshe
     const size_t sort_bytes = rk_sort_workspace_size(ray_count, 8);
     void* sort_ws = ar.take<char>(sort_bytes);
     if (!keys || !order || !sort_ws) return RK_ERROR_WORKSPACE;
+    RkSortPlan<uint64_t> plan;
+    rk_status s = rk_sort_plan<uint64_t>(ray_count, key_bits_for(mesh_count), true, keys, order, sort_ws, sort_bytes,
+                                         plan);
+    if (s != RK_SUCCESS) return s;
     hipLaunchKernelGGL(k_batch_ray_keys, dim3(blocks_for(ray_count, 256)), dim3(256), 0, st, meshes, mesh_count,
-                       nodes, o, ray_count, keys, order);
+                       nodes, o, ray_count, plan.src, plan.vsrc);
     RK_CHECK_LAUNCH();
-    rk_status s = rk_radix_sort_impl<uint64_t>(st, keys, order, ray_count, 0, (int)key_passes_for(mesh_count),
-                                               sort_ws, sort_bytes, flags);
+    s = rk_sort_run<uint64_t>(st, plan, false, flags);
     if (s != RK_SUCCESS) return s;
   }
 #define RK_BATCH_TRACE(WG, SD, DM)                                                                                 \
@@ -2212,11 +2246,15 @@ extern "C" rk_status rk_fast_trace_sorted(rk_stream stream, const rk_fast_bvh* b
   if (!keys || !order || !sort_ws) return RK_ERROR_WORKSPACE;
   const FNode* nodes = static_cast<const FNode*>(bvh->nodes);
   const float4* o = reinterpret_cast<const float4*>(origins);
-  hipLaunchKernelGGL(k_ray_keys, dim3(blocks_for(n_rays, 256)), dim3(256), 0, st, nodes, o, n_rays, keys, order);
-  RK_CHECK_LAUNCH();
   const TraceVariant* tv = trace_variant(options ? options->config : 0u);
   if (!tv) return RK_ERROR_INVALID_VALUE;
-  rk_status s = rk_radix_sort_impl<uint32_t>(st, keys, order, n_rays, 0, 4, sort_ws, sort_bytes, nullptr);
+  RkSortPlan<uint32_t> plan;
+  rk_status s = rk_sort_plan<uint32_t>(n_rays, 30, true, keys, order, sort_ws, sort_bytes, plan);
+  if (s != RK_SUCCESS) return s;
+  hipLaunchKernelGGL(k_ray_keys, dim3(blocks_for(n_rays, 256)), dim3(256), 0, st, nodes, o, n_rays, plan.src,
+                     plan.vsrc);
+  RK_CHECK_LAUNCH();
+  s = rk_sort_run<uint32_t>(st, plan, false, nullptr);
   if (s != RK_SUCCESS) return s;
   // the variant's workgroup, stack and exchange settings; the order replaces its ray runs
   hipLaunchKernelGGL(tv->kernel, dim3(blocks_for(n_rays, tv->wg)), dim3(tv->wg), 0, st, nodes,

@@ -1,11 +1,24 @@
 // Stable LSD radix sort for gfx950, 8-bit digits, onesweep style:
-//   1. one histogram kernel counts the digits of every pass in a single read;
-//   2. one scatter kernel per pass. Each 512-thread workgroup sorts the
-//      8192-key tile (4096 below 2^21 keys) of its block index: it ranks its keys stably with
-//      per-(wave, digit) lane masks in LDS, publishes its per-digit counts,
-//      resolves its global per-digit prefix by decoupled look-back over
-//      earlier tiles, reorders the tile by digit in LDS and writes it out in
-//      per-digit runs, keys first, then values through the same LDS.
+//   1. one kernel counts the digits of every pass in a single read (or the
+//      kernel that makes the keys does, rk_sort.h);
+//   2. one scatter kernel per pass. Each 512-thread workgroup sorts the tile
+//      of its block index (2048, 4096 or 8192 keys): it ranks its keys stably
+//      with per-(wave, digit) lane masks in LDS, publishes its per-digit
+//      counts, resolves its global per-digit prefix by decoupled look-back
+//      over earlier tiles, reorders the tile by digit in LDS and writes it
+//      out in per-digit runs, keys first, then values through the same LDS.
+// Up to 4096 keys, one workgroup does all passes in LDS in a single launch
+// instead (k_sort_one: a 3,042-face build 43 us against 52).
+// Below 2^21 keys a pass is bound by latency, at most a few tiles per CU, and
+// the look-back has two levels: a tile adds the counts of the tiles before it
+// in its group of 16, all in flight at once, and looks back over groups (1M
+// pairs: 15.1 against 16.8 us per pass; with one level the prefixes advance 8
+// tiles per round trip). Above, tiles queue on every CU and overlap each other.
+// Slower: ranks from eight ballots per key (158 against 155 us per 1M-face
+// build, 1613 against 1577 for 10M); wider digits, 10 bits (three passes for
+// 30-bit keys) at 25.9 us per pass on 1M pairs, 9 bits (seven for 63) at 85.6
+// us on 10M 64-bit pairs against 59.7, for their shorter runs and more counts to
+// look back over.
 // Tiles follow the block index rather than a counter that every workgroup
 // increments (on MI355X such a counter serialises the workgroups' start
 // across the eight XCDs). A workgroup only waits on lower tiles; workgroups
@@ -19,7 +32,10 @@
 // CUDA_bitonicSortGeneral.cu, CUDA_bitonicSort.cu, CUDA_bubbleSort512.cu)
 // differ in tie order by size class; rk_radix_sort_general reproduces that
 // order (see the size-class notes at the entry point).
-#include "rk_device.h"
+#include <algorithm>
+#include <utility>
+
+#include "rk_sort.h"
 
 namespace {
 
@@ -29,67 +45,75 @@ namespace {
 #ifndef RK_SCATTER_ITEMS
 #define RK_SCATTER_ITEMS 16
 #endif
-#ifndef RK_SCATTER_ITEMS_SMALL
-#define RK_SCATTER_ITEMS_SMALL 8
-#endif
 constexpr int kWaves = RK_SCATTER_WAVES;    // waves per scatter workgroup
 constexpr int kThreads = 64 * kWaves;
-constexpr int kItems = RK_SCATTER_ITEMS;    // keys per lane
-constexpr int kItemsSmall = RK_SCATTER_ITEMS_SMALL;  // keys per lane below kSmallTilesBelow keys
-// Below 2^21 keys the tiles are of 4096 keys: tiles of 8192 would leave most
-// of the 256 CUs idle (1M keys: 123 tiles). On the 1M-face heightfield build
-// 214 vs 224 us; on 10M keys the larger tiles are faster (1.73 vs 1.80 ms).
-constexpr size_t kSmallTilesBelow = size_t(1) << 21;
+constexpr int kItems = RK_SCATTER_ITEMS;    // keys per lane, at most
+// Keys per tile: 8192 from 2^21 keys on, 4096 below (8192 would leave most of
+// the 256 CUs idle on 1M keys: 214 against 224 us per build; 10M keys 1.73 ms
+// with 8192 against 1.80), 2048 below 2^19 (a 180K-face build 97.7 against
+// 104.5 us, the 20,480-face icosphere 64 against 70; 1M 156.5 against 155.6).
+constexpr int kItemsMid = 8, kItemsSmall = 4;
+constexpr size_t kMidTilesBelow = size_t(1) << 21, kSmallTilesBelow = size_t(1) << 19;
 static_assert(kThreads >= 256, "one thread per digit");
 constexpr uint32_t kAgg = 1u << 30;
 constexpr uint32_t kInc = 2u << 30;
 constexpr uint32_t kCountMask = (1u << 30) - 1u;
 constexpr uint32_t kSpinLimit = 1u << 20;
 constexpr int kMaxPasses = 8;
+constexpr uint32_t kOneMax = 4096;  // up to this many keys one workgroup sorts them in LDS
 #ifndef RK_SORT_LOOK
 #define RK_SORT_LOOK 8
 #endif
 constexpr int kLook = RK_SORT_LOOK;  // look-back status loads in flight per digit
 
-// Exclusive scan over the first 256 threads of the block (one value per
-// digit); every thread of the block calls it, threads 256.. get no result.
-__device__ __forceinline__ uint32_t block_excl_scan256(uint32_t v, uint32_t* s_tmp /*>= 4*/) {
+constexpr uint32_t kGroup = 16;  // tiles per look-back group
+
+// Exclusive scan over a block of kT threads of kPer consecutive values each.
+template <int kT, int kPer>
+__device__ __forceinline__ void block_excl_scan(const uint32_t (&v)[kPer], uint32_t (&ex)[kPer],
+                                                uint32_t* s_tmp /*>= kT / 64*/) {
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  uint32_t incl = v;
+  uint32_t sum = 0;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) sum += v[u];
+  uint32_t incl = sum;
 #pragma unroll
   for (int off = 1; off < 64; off <<= 1) {
     uint32_t y = __shfl_up(incl, off, 64);
     if (lane >= (uint32_t)off) incl += y;
   }
-  if (lane == 63 && wave < 4) s_tmp[wave] = incl;
+  if (lane == 63) s_tmp[wave] = incl;
   __syncthreads();
-  uint32_t wprefix = 0;
+  uint32_t run = incl - sum;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) wprefix += (w < (int)wave) ? s_tmp[w] : 0u;
+  for (int w = 0; w < kT / 64; ++w) run += (w < (int)wave) ? s_tmp[w] : 0u;
   __syncthreads();
-  return wprefix + incl - v;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    ex[u] = run;
+    run += v[u];
+  }
 }
 
 // Digit counts of every pass in one read. Block b counts keys
 // [b * chunk, (b + 1) * chunk), eight loads in flight per thread; a wave whose
 // 64 keys share a digit (the high digits of spatially ordered keys) adds them
-// with one LDS atomic instead of 64 to the same address.
+// with one LDS atomic instead of 64 to the same address. Each block adds to one
+// of 'copies' copies of the counts, so that fewer meet on one address.
 constexpr int kHistUnroll = 8;
 constexpr uint32_t kHistMaxBlocks = 1024;
-#ifndef RK_HIST_KEYS_PER_BLOCK
-#define RK_HIST_KEYS_PER_BLOCK (256 * kHistUnroll * 2)
-#endif
-constexpr size_t kHistKeysPerBlock = RK_HIST_KEYS_PER_BLOCK;
+constexpr size_t kHistKeysPerBlock = 256 * kHistUnroll * 2;
 
-// Also zeroes the look-back status words of the passes that follow (zero,
-// zero_words), which saves a fill launch per sort.
+// Also zeroes the look-back words of the first pass (zero, zero_words), which
+// saves a fill launch per sort.
 template <typename K>
-__global__ __launch_bounds__(256) void k_rs_hist(const K* __restrict__ keys, uint32_t n, int passes, int first_pass,
-                                                 uint32_t chunk, uint32_t* __restrict__ hist,
+__global__ __launch_bounds__(256) void k_rs_hist(const K* __restrict__ keys, uint32_t n, int passes, uint32_t chunk,
+                                                 uint32_t* __restrict__ hist, uint32_t copies,
                                                  uint32_t* __restrict__ zero, size_t zero_words) {
-  __shared__ uint32_t s[kMaxPasses * 256];
+  constexpr uint32_t D = 256;
+  __shared__ uint32_t s[kMaxPasses * D];
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < zero_words; i += (size_t)gridDim.x * 256) zero[i] = 0u;
-  for (int i = threadIdx.x; i < passes * 256; i += 256) s[i] = 0;
+  for (uint32_t i = threadIdx.x; i < (uint32_t)passes * D; i += 256) s[i] = 0;
   __syncthreads();
   const size_t b0 = (size_t)blockIdx.x * chunk;
   const size_t b1 = b0 + chunk < (size_t)n ? b0 + chunk : (size_t)n;
@@ -107,20 +131,51 @@ __global__ __launch_bounds__(256) void k_rs_hist(const K* __restrict__ keys, uin
       const uint64_t active = __ballot(ok[u]);
       if (!ok[u]) continue;
       for (int p = 0; p < passes; ++p) {
-        const uint32_t d = (uint32_t)(k[u] >> (8 * (p + first_pass))) & 0xFFu;
+        const uint32_t d = (uint32_t)(k[u] >> (8 * p)) & (D - 1u);
         const uint32_t d0 = __builtin_amdgcn_readfirstlane(d);
         if (__ballot(d == d0) == active) {
-          if (__lane_id() == (uint32_t)__builtin_ctzll(active)) atomicAdd(&s[p * 256 + d0], (uint32_t)__popcll(active));
+          if (__lane_id() == (uint32_t)__builtin_ctzll(active)) atomicAdd(&s[p * D + d0], (uint32_t)__popcll(active));
         } else {
-          atomicAdd(&s[p * 256 + d], 1u);
+          atomicAdd(&s[p * D + d], 1u);
         }
       }
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < passes * 256; i += 256) {
+  uint32_t* g = hist + (size_t)(blockIdx.x % copies) * passes * D;
+  for (uint32_t i = threadIdx.x; i < (uint32_t)passes * D; i += 256) {
     uint32_t c = s[i];
-    if (c) atomicAdd(&hist[i], c);
+    if (c) atomicAdd(&g[i], c);
+  }
+}
+
+// Stable ranks of a wave's keys (kIt per lane, iteration j of lane l being the
+// wave's key 64 j + l) among its keys of the same digit, and the wave's digit
+// counts in cnt (zero before). Each lane ORs its bit into its digit's mask and
+// reads it back: the lanes that share the digit. The last of them advances the
+// digit's counter and clears the mask. wmask: the wave's 256 zero words, left zero.
+template <typename K, int kIt>
+__device__ __forceinline__ void wave_ranks(const K (&key)[kIt], const bool (&valid)[kIt], int shift,
+                                           uint64_t* __restrict__ wmask, uint32_t* __restrict__ cnt,
+                                           uint32_t (&rank)[kIt]) {
+  const uint64_t my_bit = 1ull << __lane_id(), lower_lanes = my_bit - 1;
+#pragma unroll
+  for (int j = 0; j < kIt; ++j) {
+    const uint32_t d = (uint32_t)(key[j] >> shift) & 0xFFu;
+    if (valid[j]) __hip_atomic_fetch_or(wmask + d, my_bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    __builtin_amdgcn_wave_barrier();
+    const uint64_t peers =
+        valid[j] ? __hip_atomic_load(wmask + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0ull;
+    const uint32_t lower = (uint32_t)__popcll(peers & lower_lanes);
+    const uint32_t all = (uint32_t)__popcll(peers);
+    const uint32_t old = cnt[d];
+    rank[j] = old + lower;
+    __builtin_amdgcn_wave_barrier();
+    if (valid[j] && lower + 1 == all) {
+      cnt[d] = old + all;
+      __hip_atomic_store(wmask + d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -129,131 +184,145 @@ __global__ __launch_bounds__(256) void k_rs_hist(const K* __restrict__ keys, uin
 // the look-back, so their registers are free while it waits; the values are
 // loaded during the look-back and follow through the same LDS buffer once the
 // keys are out, so a workgroup holds a tile of keys in LDS, not keys and values.
-template <typename K, bool kVals, int kIt>
+// kGroups (fewer than 2^21 keys): status holds a row of words per tile, then
+// one per group of tiles, all tagged with the pass, so that what the pass
+// before left counts as unpublished. Otherwise a row per tile, and next is the
+// other buffer, which this pass zeroes for the next (NULL after the last).
+template <typename K, bool kVals, int kIt, bool kGroups>
 __global__ __launch_bounds__(kThreads) void k_rs_scatter(const K* __restrict__ kin, const uint32_t* __restrict__ vin,
                                                          K* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n,
-                                                         int shift, const uint32_t* __restrict__ hist,
-                                                         uint32_t* __restrict__ status, uint32_t* __restrict__ err) {
+                                                         int pass, const uint32_t* __restrict__ hist,
+                                                         uint32_t copies, uint32_t copy_words,
+                                                         uint32_t* __restrict__ status, uint32_t* __restrict__ next,
+                                                         uint32_t* __restrict__ err) {
   constexpr int kTileT = kThreads * kIt, kWaveTileT = 64 * kIt;  // keys per tile and per wave
-  __shared__ uint32_t s_cnt[kWaves][256];
-  __shared__ uint32_t s_gbase[256];
-  __shared__ uint32_t s_tmp[8];
-  __shared__ K s_buf[kTileT];
+  constexpr uint32_t D = 256;
+  // words: flag (2 bits), with kGroups the pass's tag (4 bits, not 0), count
+  constexpr uint32_t kCount = kGroups ? (1u << 26) - 1u : kCountMask;
+  const uint32_t tag = kGroups ? (uint32_t)(pass + 1) << 26 : 0u;
+  const int shift = 8 * pass;
+  __shared__ uint32_t s_cnt[kWaves][D];
+  __shared__ uint32_t s_gbase[D];
+  __shared__ uint32_t s_tmp[kWaves];
+  // while ranking, s_buf holds 256 64-bit lane masks per wave
+  constexpr int kBuf = sizeof(K) * kTileT >= sizeof(uint64_t) * kWaves * D ? kTileT
+                                                                          : (int)(sizeof(uint64_t) * kWaves * D / sizeof(K));
+  __shared__ K s_buf[kBuf];
 
   const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  // While ranking, s_buf holds one 64-bit lane mask per (wave, digit): the
-  // lanes of the current 64 keys that carry that digit.
-  static_assert(sizeof(K) * kTileT >= sizeof(uint64_t) * kWaves * 256, "digit masks fit in the tile buffer");
   uint64_t* s_mask = reinterpret_cast<uint64_t*>(s_buf);
-  for (int i = tid; i < kWaves * 256; i += kThreads) {
+  for (uint32_t i = tid; i < kWaves * D; i += kThreads) {
     (&s_cnt[0][0])[i] = 0;
     s_mask[i] = 0;
   }
-  __syncthreads();
-  const uint32_t tile = blockIdx.x;
+  const uint32_t tile = blockIdx.x, group = tile / kGroup, place = tile % kGroup;
   const size_t base = (size_t)tile * kTileT;
   const size_t wbase = base + (size_t)wave * kWaveTileT;
-
+  uint32_t* gstatus = status + (size_t)gridDim.x * D;
+  if (!kGroups && next && tid < D) next[(size_t)tile * D + tid] = 0u;
   K key[kIt];
+  bool valid[kIt];
   uint32_t rank[kIt];
 #pragma unroll
   for (int j = 0; j < kIt; ++j) {
     size_t idx = wbase + (size_t)j * 64 + lane;
-    key[j] = idx < n ? kin[idx] : (K)0;
+    valid[j] = idx < n;
+    key[j] = valid[j] ? kin[idx] : (K)0;
   }
-  // Stable in-tile ranking: iteration j of wave w covers keys
-  // [wbase + 64j, wbase + 64j + 64) in lane order, so (w, j, lane) is memory order.
-  // Each lane ORs its bit into its digit's mask; reading the mask back gives
-  // the lanes that share the digit, so the lane's rank among them is the
-  // count of lower lanes. The group's last lane advances the digit's counter
-  // and clears the mask for the next 64 keys.
-  const uint64_t my_bit = 1ull << lane;
-  const uint64_t lower_lanes = my_bit - 1;
-  uint64_t* wmask = s_mask + wave * 256;
-#pragma unroll
-  for (int j = 0; j < kIt; ++j) {
-    size_t idx = wbase + (size_t)j * 64 + lane;
-    bool valid = idx < n;
-    uint32_t d = (uint32_t)(key[j] >> shift) & 0xFFu;
-    if (valid) __hip_atomic_fetch_or(wmask + d, my_bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    __builtin_amdgcn_wave_barrier();
-    const uint64_t peers =
-        valid ? __hip_atomic_load(wmask + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) : 0ull;
-    const uint32_t lower = (uint32_t)__popcll(peers & lower_lanes);
-    const uint32_t cnt = (uint32_t)__popcll(peers);
-    const uint32_t old = s_cnt[wave][d];
-    rank[j] = old + lower;
-    __builtin_amdgcn_wave_barrier();
-    if (valid && lower + 1 == cnt) {
-      s_cnt[wave][d] = old + cnt;
-      __hip_atomic_store(wmask + d, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    }
-    __builtin_amdgcn_wave_barrier();
-  }
+  __syncthreads();
+  wave_ranks<K, kIt>(key, valid, shift, s_mask + wave * 256, s_cnt[wave], rank);
   __syncthreads();
 
   // Per digit (thread d < 256): the tile's count, published at once for the
   // look-back of later tiles, and each wave's start within the digit's run.
   const uint32_t d = tid;
-  uint32_t total = 0;
-  if (tid < 256) {
+  const bool mine = tid < D;
+  uint32_t total[1] = {0u}, local[1], counted[1] = {0u}, global[1];
+  if (mine) {
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) {
-      uint32_t c = s_cnt[w][d];
-      s_cnt[w][d] = total;
-      total += c;
+      const uint32_t c = s_cnt[w][d];
+      s_cnt[w][d] = total[0];
+      total[0] += c;
     }
-    rk::atomic_store_relaxed(status + (size_t)tile * 256 + d, (tile == 0 ? kInc : kAgg) | total);
+    rk::atomic_store_relaxed(status + (size_t)tile * D + d, (!kGroups && tile == 0 ? kInc : kAgg) | tag | total[0]);
+    for (uint32_t c = 0; c < copies; ++c) counted[0] += hist[(size_t)c * copy_words + d];
   }
-  const uint32_t local_excl = block_excl_scan256(total, s_tmp);
-  if (tid < 256) {
+  block_excl_scan<kThreads, 1>(total, local, s_tmp);
+  if (mine) {
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) s_cnt[w][d] += local_excl;
+    for (int w = 0; w < kWaves; ++w) s_cnt[w][d] += local[0];
   }
   __syncthreads();
 #pragma unroll
   for (int j = 0; j < kIt; ++j) {
-    size_t idx = wbase + (size_t)j * 64 + lane;
-    if (idx < n) {
-      const uint32_t dd = (uint32_t)(key[j] >> shift) & 0xFFu;
-      rank[j] += s_cnt[wave][dd];  // position in the tile's digit order
+    if (valid[j]) {
+      rank[j] += s_cnt[wave][(uint32_t)(key[j] >> shift) & 0xFFu];  // position in the tile's digit order
       s_buf[rank[j]] = key[j];
     }
   }
   uint32_t val[kIt];
   if (kVals) {
 #pragma unroll
-    for (int j = 0; j < kIt; ++j) {
-      size_t idx = wbase + (size_t)j * 64 + lane;
-      val[j] = idx < n ? vin[idx] : 0u;
-    }
+    for (int j = 0; j < kIt; ++j) val[j] = valid[j] ? vin[wbase + (size_t)j * 64 + lane] : 0u;
   }
-  const uint32_t global_excl = block_excl_scan256(tid < 256 ? hist[tid & 255] : 0u, s_tmp);
+  block_excl_scan<kThreads, 1>(counted, global, s_tmp);
 
-  // Decoupled look-back, kLook predecessors' status words per round trip:
-  // add counts from tile j down until an inclusive prefix; stop the round at
-  // a tile that has published nothing yet and reload from there.
-  if (tid < 256) {
-    uint32_t prefix = 0;
-    if (tile > 0) {
-      int32_t j = (int32_t)tile - 1;
-      uint32_t spins = 0;
+  if (mine) {
+    // a word of this pass: its flag (0: not published yet)
+    auto flag_of = [&](uint32_t w) { return ((w ^ tag) & ~(kAgg | kInc | kCount)) == 0u ? w & (kAgg | kInc) : 0u; };
+    uint32_t prefix = 0, spins = 0;
+    if (kGroups && place > 0u) {
+      // the tiles before this one in its group, all in flight; again until all are published
+      for (;;) {
+        uint32_t sv[kGroup - 1];
+#pragma unroll
+        for (uint32_t w = 0; w < kGroup - 1; ++w)
+          sv[w] = w < place ? rk::atomic_load_relaxed(status + (size_t)(group * kGroup + w) * D + d) : kAgg | tag;
+        bool ready = true;
+        prefix = 0;
+#pragma unroll
+        for (uint32_t w = 0; w < kGroup - 1; ++w) {
+          ready = ready && flag_of(sv[w]) != 0u;
+          prefix += sv[w] & kCount;
+        }
+        if (ready) break;
+        if (++spins > kSpinLimit) {
+          atomicOr(err, (uint32_t)RK_FLAG_SPIN_LIMIT);
+          break;
+        }
+        __builtin_amdgcn_s_sleep(1);
+      }
+    }
+    // The rows looked back over: the groups', or the tiles'. The inclusive
+    // prefix goes out for a group by its last tile, or for every tile.
+    const uint32_t* rows = kGroups ? gstatus : status;
+    const uint32_t row = kGroups ? group : tile;
+    const bool publish = !kGroups || place == kGroup - 1u;
+    uint32_t* out = (kGroups ? gstatus : status) + (size_t)row * D + d;
+    if (kGroups && publish)
+      rk::atomic_store_relaxed(out, (group == 0u ? kInc : kAgg) | tag | ((prefix + total[0]) & kCount));
+    // Decoupled look-back, kLook predecessors' words per round trip: add counts
+    // from row j down until an inclusive prefix; stop the round at a row that
+    // has published nothing yet and reload from there.
+    if (row > 0u) {
+      int32_t j = (int32_t)row - 1;
       for (;;) {
         uint32_t sv[kLook];
 #pragma unroll
         for (int w = 0; w < kLook; ++w)
-          sv[w] = (j - w >= 0) ? rk::atomic_load_relaxed(status + (size_t)(j - w) * 256 + d) : kInc;
+          sv[w] = (j - w >= 0) ? rk::atomic_load_relaxed(rows + (size_t)(j - w) * D + d) : kInc | tag;
         int used = 0;
         bool inc = false, stalled = false;
 #pragma unroll
         for (int w = 0; w < kLook; ++w) {
           if (inc || stalled) continue;
-          const uint32_t flag = sv[w] & ~kCountMask;
+          const uint32_t flag = flag_of(sv[w]);
           if (flag == 0) {
             stalled = true;
             continue;
           }
-          prefix += sv[w] & kCountMask;
+          prefix += sv[w] & kCount;
           ++used;
           if (flag == kInc) inc = true;
         }
@@ -267,9 +336,9 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const K* __restrict__ k
           __builtin_amdgcn_s_sleep(1);
         }
       }
-      rk::atomic_store_relaxed(status + (size_t)tile * 256 + d, kInc | ((prefix + total) & kCountMask));
+      if (publish) rk::atomic_store_relaxed(out, kInc | tag | ((prefix + total[0]) & kCount));
     }
-    s_gbase[d] = global_excl + prefix - local_excl;
+    s_gbase[d] = global[0] + prefix - local[0];
   }
   __syncthreads();
 
@@ -294,8 +363,7 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const K* __restrict__ k
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < kIt; ++j) {
-      size_t idx = wbase + (size_t)j * 64 + lane;
-      if (idx < n) s_val[rank[j]] = val[j];
+      if (valid[j]) s_val[rank[j]] = val[j];
     }
     __syncthreads();
 #pragma unroll
@@ -304,6 +372,97 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const K* __restrict__ k
       if (i < tile_n && opos[m] != 0xFFFFFFFFu) vout[opos[m]] = s_val[i];
     }
   }
+}
+
+// All passes of a small sort in one workgroup: its keys and values stay in
+// registers and change places through LDS, with the scatter kernel's stable
+// ranks. 16 waves, kIt keys per lane. In place when kin is kout (every load
+// comes before every store). clear (may be NULL) is set to 0.
+constexpr int kOneThreads = 1024, kOneWaves = kOneThreads / 64;
+template <typename K, bool kVals, int kIt>
+__global__ __launch_bounds__(kOneThreads) void k_sort_one(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout,
+                                                          uint32_t n, int passes, uint32_t* clear) {
+  constexpr uint32_t D = 256;
+  __shared__ uint32_t s_cnt[kOneWaves][D];
+  __shared__ uint32_t s_tmp[kOneWaves];
+  __shared__ K s_buf[kOneThreads * kIt];
+  __shared__ uint64_t s_mask[kOneWaves * D];  // zero between the passes
+  uint32_t* s_val = reinterpret_cast<uint32_t*>(s_buf);
+  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  if (clear && tid == 0) *clear = 0u;
+  for (uint32_t i = tid; i < kOneWaves * D; i += kOneThreads) s_mask[i] = 0;
+  const uint32_t first = wave * (64u * kIt) + lane;
+  K key[kIt];
+  uint32_t val[kIt], rank[kIt];
+  bool valid[kIt];
+#pragma unroll
+  for (int j = 0; j < kIt; ++j) {
+    const uint32_t i = first + 64u * j;
+    valid[j] = i < n;
+    key[j] = valid[j] ? kin[i] : (K)0;
+    val[j] = kVals && valid[j] ? vin[i] : 0u;
+  }
+  for (int p = 0; p < passes; ++p) {
+    const int shift = p * 8;
+    for (uint32_t i = tid; i < kOneWaves * D; i += kOneThreads) (&s_cnt[0][0])[i] = 0;
+    __syncthreads();
+    wave_ranks<K, kIt>(key, valid, shift, s_mask + wave * D, s_cnt[wave], rank);
+    __syncthreads();
+    uint32_t total[1] = {0u}, excl[1];
+    if (tid < D) {
+#pragma unroll
+      for (int w = 0; w < kOneWaves; ++w) total[0] += s_cnt[w][tid];
+    }
+    block_excl_scan<kOneThreads, 1>(total, excl, s_tmp);
+    if (tid < D) {
+      uint32_t run = excl[0];
+#pragma unroll
+      for (int w = 0; w < kOneWaves; ++w) {
+        const uint32_t c = s_cnt[w][tid];
+        s_cnt[w][tid] = run;
+        run += c;
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kIt; ++j) {
+      if (valid[j]) {
+        rank[j] += s_cnt[wave][(uint32_t)(key[j] >> shift) & (D - 1u)];
+        s_buf[rank[j]] = key[j];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < kIt; ++j)
+      if (valid[j]) key[j] = s_buf[first + 64u * j];
+    if (kVals) {
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kIt; ++j)
+        if (valid[j]) s_val[rank[j]] = val[j];
+      __syncthreads();
+#pragma unroll
+      for (int j = 0; j < kIt; ++j)
+        if (valid[j]) val[j] = s_val[first + 64u * j];
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int j = 0; j < kIt; ++j) {
+    if (valid[j]) {
+      kout[first + 64u * j] = key[j];
+      if (kVals) vout[first + 64u * j] = val[j];
+    }
+  }
+}
+
+__global__ __launch_bounds__(256) void k_sort_clear(uint32_t* __restrict__ head, size_t head_words,
+                                                    uint32_t* __restrict__ status, size_t status_words,
+                                                    uint32_t* __restrict__ info) {
+  const size_t stride = (size_t)gridDim.x * 256, t = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (info && t < RK_INFO_WORDS) info[t] = 0u;
+  for (size_t i = t; i < head_words; i += stride) head[i] = 0u;
+  for (size_t i = t; i < status_words; i += stride) status[i] = 0u;
 }
 
 template <typename K, bool kVals>
@@ -390,7 +549,9 @@ __global__ __launch_bounds__(256) void k_iota(uint32_t* __restrict__ v, uint32_t
   for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += stride) v[i] = (uint32_t)i;
 }
 
-inline int items_of(uint32_t n) { return (size_t)n < kSmallTilesBelow ? kItemsSmall : kItems; }
+inline int items_of(uint32_t n) {
+  return (size_t)n < kSmallTilesBelow ? kItemsSmall : ((size_t)n < kMidTilesBelow ? kItemsMid : kItems);
+}
 inline uint32_t tiles_of(uint32_t n) {
   const uint32_t tile = (uint32_t)(kThreads * items_of(n));
   return (uint32_t)(((size_t)n + tile - 1) / tile);
@@ -420,96 +581,141 @@ inline unsigned grid_for(size_t n, size_t per_block, unsigned cap) {
 // Size of the workspace for a sort of 'length' keys of 'key_bytes' bytes.
 extern "C" size_t rk_sort_workspace_size(uint32_t length, uint32_t key_bytes) {
   size_t n = length ? length : 1;
-  size_t T = tiles_of((uint32_t)n);
+  const size_t tile = (size_t)kThreads * (n < kMidTilesBelow ? kItemsMid : kItems), T = (n + tile - 1) / tile;
   size_t P = key_bytes >= 8 ? 8 : 4;
   return rk_align_up(P * 256 * 4 + P * 4 + 4 + P * T * 256 * 4) + rk_align_up(n * (key_bytes >= 8 ? 8 : 4)) +
          rk_align_up(n * 4) + 1024;
 }
 
-// Sort keys (and values) stably on digits first_pass .. first_pass+passes-1.
-// 'err' (device, may be NULL) receives RK_FLAG_SPIN_LIMIT on a look-back
-// timeout; when it is NULL the first word of 'ws' does, cleared by this call.
-// The look-back status words count keys in 30 bits, so n < 2^30.
-// head_cleared: the caller has zeroed the first rk_sort_head_words(passes)
-// words of ws (error word and digit counts) in an earlier kernel on 'st', so
-// no fill runs here.
-// digit_counts (may be NULL): receives the device address of the first pass's
-// 256 digit counts, valid once the sort has run on 'st' (NULL when n <= 1).
+// The look-back words count keys in 30 bits, so n < 2^30.
 template <typename K>
-rk_status rk_radix_sort_impl(hipStream_t st, K* keys, uint32_t* vals, uint32_t n, int first_pass, int passes,
-                             void* ws, size_t ws_bytes, uint32_t* err, bool head_cleared = false,
-                             const uint32_t** digit_counts = nullptr) {
-  if (digit_counts) *digit_counts = nullptr;
+rk_status rk_sort_plan(uint32_t n, int bits, bool anywhere, K* keys, uint32_t* vals, void* ws, size_t ws_bytes,
+                       RkSortPlan<K>& p) {
   if (n >= kAgg) return RK_ERROR_UNSUPPORTED;
-  if (n <= 1 || passes <= 0) return err ? RK_SUCCESS : clear_ws_flags(st, ws, ws_bytes);
-  if (!keys || passes > kMaxPasses) return RK_ERROR_INVALID_VALUE;
-  const uint32_t T = tiles_of(n);
+  if (!keys || bits <= 0 || bits > (int)sizeof(K) * 8) return RK_ERROR_INVALID_VALUE;
+  p.n = n;
+  p.one = n <= kOneMax;
+  p.passes = (bits + 7) / 8;
+  p.tiles = tiles_of(n);
+  // rk_sort_workspace_size has one count and one status row per pass and tile of
+  // 4096 or 8192 keys: room for these copies of the counts and rows
+  const bool groups = items_of(n) != kItems;
+  p.copies = std::min<uint32_t>(8u, 1u + p.tiles / 8u);
+  p.head_words = p.one ? 1 : 1 + (size_t)p.copies * p.passes * 256;
+  p.status_words = p.one ? 0 : ((size_t)p.tiles + (groups ? (p.tiles + kGroup - 1) / kGroup : 0)) * 256;
   RkArena ar(ws, ws_bytes);
-  const size_t ctl_words = 1 + (size_t)passes * 256 + (size_t)passes * T * 256;
-  uint32_t* ctl = ar.take<uint32_t>(ctl_words);  // first in ws: ctl[0] is the error word
-  K* kalt = ar.take<K>(n);
-  uint32_t* valt = vals ? ar.take<uint32_t>(n) : nullptr;
-  if (!ctl || !kalt || (vals && !valt)) return RK_ERROR_WORKSPACE;
-  uint32_t* werr = ctl;
-  uint32_t* hist = ctl + 1;
-  uint32_t* status = hist + (size_t)passes * 256;
-  if (!err) err = werr;
-  if (digit_counts) *digit_counts = hist;
-
-  if (!head_cleared) {
-    rk_status s = rk_fill_u32(reinterpret_cast<rk_stream>(st), ctl, 1 + (size_t)passes * 256, 0u);
-    if (s != RK_SUCCESS) return s;
+  p.head = ar.take<uint32_t>(p.head_words + (groups || p.passes < 2 ? 1 : 2) * p.status_words);
+  p.status = p.head + p.head_words;
+  p.dst = p.src = keys;
+  p.vdst = p.vsrc = vals;
+  if (!p.head) return RK_ERROR_WORKSPACE;
+  if (p.one) return RK_SUCCESS;
+  p.alt = ar.take<K>(n);
+  p.valt = vals ? ar.take<uint32_t>(n) : nullptr;
+  if (!p.alt || (vals && !p.valt)) return RK_ERROR_WORKSPACE;
+  if (anywhere && (p.passes & 1)) {
+    p.src = p.alt;
+    p.vsrc = p.valt;
   }
-  const unsigned hist_blocks = grid_for(n, kHistKeysPerBlock, kHistMaxBlocks);
-  const uint32_t chunk = (uint32_t)(((size_t)n + hist_blocks - 1) / hist_blocks);
-  hipLaunchKernelGGL(k_rs_hist<K>, dim3(hist_blocks), dim3(256), 0, st, keys, n, passes, first_pass, chunk, hist,
-                     status, (size_t)passes * T * 256);
+  return RK_SUCCESS;
+}
+
+template <typename K>
+rk_status rk_sort_clear(hipStream_t st, const RkSortPlan<K>& p, uint32_t* info) {
+  const size_t words = p.head_words + p.status_words;
+  hipLaunchKernelGGL(k_sort_clear, dim3(grid_for(words, 256 * 4, 1024)), dim3(256), 0, st, p.head, p.head_words,
+                     p.status, p.status_words, info);
   RK_CHECK_LAUNCH();
-  K* ks = keys;
-  K* kd = kalt;
-  uint32_t* vs = vals;
-  uint32_t* vd = valt;
-  for (int p = 0; p < passes; ++p) {
-    int shift = 8 * (p + first_pass);
-    const bool small = items_of(n) == kItemsSmall;
-    if (vals) {
-      if (small)
-        hipLaunchKernelGGL((k_rs_scatter<K, true, kItemsSmall>), dim3(T), dim3(kThreads), 0, st, ks, vs, kd, vd, n,
-                           shift, hist + (size_t)p * 256, status + (size_t)p * T * 256, err);
-      else
-        hipLaunchKernelGGL((k_rs_scatter<K, true, kItems>), dim3(T), dim3(kThreads), 0, st, ks, vs, kd, vd, n, shift,
-                           hist + (size_t)p * 256, status + (size_t)p * T * 256, err);
+  return RK_SUCCESS;
+}
+
+namespace {
+
+template <typename K>
+rk_status launch_one(hipStream_t st, const RkSortPlan<K>& p, uint32_t* clear) {
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kOneThreads), 0, st, p.src, p.vsrc, p.dst, p.vdst, p.n, p.passes, clear);
+  };
+  static_assert(kOneMax == 4 * kOneThreads, "4 keys per thread at most");
+  const bool two = p.n <= 2 * kOneThreads;
+  if (p.vsrc) go(two ? k_sort_one<K, true, 2> : k_sort_one<K, true, 4>);
+  else go(two ? k_sort_one<K, false, 2> : k_sort_one<K, false, 4>);
+  RK_CHECK_LAUNCH();
+  return RK_SUCCESS;
+}
+
+}  // namespace
+
+template <typename K>
+rk_status rk_sort_run(hipStream_t st, const RkSortPlan<K>& p, bool counted, uint32_t* err) {
+  if (p.one) return launch_one<K>(st, p, err || counted ? nullptr : p.head);
+  uint32_t* hist = p.head + 1;
+  if (!counted) {
+    rk_status s = rk_fill_u32(reinterpret_cast<rk_stream>(st), p.head, p.head_words, 0u);
+    if (s != RK_SUCCESS) return s;
+    const unsigned blocks = grid_for(p.n, kHistKeysPerBlock, kHistMaxBlocks);
+    const uint32_t chunk = (uint32_t)(((size_t)p.n + blocks - 1) / blocks);
+    hipLaunchKernelGGL(k_rs_hist<K>, dim3(blocks), dim3(256), 0, st, p.src, p.n, p.passes, chunk, hist, p.copies,
+                       p.status, p.status_words);
+    RK_CHECK_LAUNCH();
+  }
+  if (!err) err = p.head;
+  K *ks = p.src, *kd = p.src == p.dst ? p.alt : p.dst;
+  uint32_t *vs = p.vsrc, *vd = p.vsrc == p.vdst ? p.valt : p.vdst;
+  for (int i = 0; i < p.passes; ++i) {
+    const int items = items_of(p.n);
+    const bool groups = items != kItems;
+    uint32_t* status = p.status + (groups ? 0 : (i & 1) * p.status_words);
+    uint32_t* next = !groups && i + 1 < p.passes ? p.status + ((i + 1) & 1) * p.status_words : nullptr;
+    auto go = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, dim3(p.tiles), dim3(kThreads), 0, st, ks, vs, kd, vd, p.n, i, hist + (size_t)i * 256,
+                         p.copies, (uint32_t)p.passes * 256u, status, next, err);
+    };
+    if (p.vsrc) {
+      if (items == kItemsSmall) go(k_rs_scatter<K, true, kItemsSmall, true>);
+      else if (groups) go(k_rs_scatter<K, true, kItemsMid, true>);
+      else go(k_rs_scatter<K, true, kItems, false>);
     } else {
-      if (small)
-        hipLaunchKernelGGL((k_rs_scatter<K, false, kItemsSmall>), dim3(T), dim3(kThreads), 0, st, ks,
-                           (const uint32_t*)nullptr, kd, (uint32_t*)nullptr, n, shift, hist + (size_t)p * 256,
-                           status + (size_t)p * T * 256, err);
-      else
-        hipLaunchKernelGGL((k_rs_scatter<K, false, kItems>), dim3(T), dim3(kThreads), 0, st, ks,
-                           (const uint32_t*)nullptr, kd, (uint32_t*)nullptr, n, shift, hist + (size_t)p * 256,
-                           status + (size_t)p * T * 256, err);
+      if (items == kItemsSmall) go(k_rs_scatter<K, false, kItemsSmall, true>);
+      else if (groups) go(k_rs_scatter<K, false, kItemsMid, true>);
+      else go(k_rs_scatter<K, false, kItems, false>);
     }
     RK_CHECK_LAUNCH();
     std::swap(ks, kd);
     std::swap(vs, vd);
   }
-  if (passes & 1) {
-    if (vals) {
-      hipLaunchKernelGGL((k_copy_back<K, true>), dim3(grid_for(n, 256 * 8, 4096)), dim3(256), 0, st, ks, vs, keys,
-                         vals, n);
-    } else {
-      hipLaunchKernelGGL((k_copy_back<K, false>), dim3(grid_for(n, 256 * 8, 4096)), dim3(256), 0, st, ks,
-                         (const uint32_t*)nullptr, keys, (uint32_t*)nullptr, n);
-    }
+  if (ks != p.dst) {
+    if (p.vsrc)
+      hipLaunchKernelGGL((k_copy_back<K, true>), dim3(grid_for(p.n, 256 * 8, 4096)), dim3(256), 0, st, ks, vs, p.dst,
+                         p.vdst, p.n);
+    else
+      hipLaunchKernelGGL((k_copy_back<K, false>), dim3(grid_for(p.n, 256 * 8, 4096)), dim3(256), 0, st, ks,
+                         (const uint32_t*)nullptr, p.dst, (uint32_t*)nullptr, p.n);
     RK_CHECK_LAUNCH();
   }
   return RK_SUCCESS;
 }
 
-template rk_status rk_radix_sort_impl<uint32_t>(hipStream_t, uint32_t*, uint32_t*, uint32_t, int, int, void*,
-                                                size_t, uint32_t*, bool, const uint32_t**);
-template rk_status rk_radix_sort_impl<uint64_t>(hipStream_t, uint64_t*, uint32_t*, uint32_t, int, int, void*,
-                                                size_t, uint32_t*, bool, const uint32_t**);
+#define RK_SORT_INSTANCES(K)                                                                                      \
+  template rk_status rk_sort_plan<K>(uint32_t, int, bool, K*, uint32_t*, void*, size_t, RkSortPlan<K>&);          \
+  template rk_status rk_sort_clear<K>(hipStream_t, const RkSortPlan<K>&, uint32_t*);                              \
+  template rk_status rk_sort_run<K>(hipStream_t, const RkSortPlan<K>&, bool, uint32_t*);
+RK_SORT_INSTANCES(uint32_t)
+RK_SORT_INSTANCES(uint64_t)
+#undef RK_SORT_INSTANCES
+
+// Sorts keys (and values, when not NULL) stably on their low 'bits' bits. 'err'
+// (device, may be NULL) receives RK_FLAG_SPIN_LIMIT on a look-back timeout; when
+// it is NULL the first word of 'ws' does, cleared by this call.
+template <typename K>
+static rk_status sort_keys(hipStream_t st, K* keys, uint32_t* vals, uint32_t n, int bits, void* ws, size_t ws_bytes,
+                           uint32_t* err) {
+  if (n >= kAgg) return RK_ERROR_UNSUPPORTED;
+  if (n <= 1) return err ? RK_SUCCESS : clear_ws_flags(st, ws, ws_bytes);
+  RkSortPlan<K> p;
+  rk_status s = rk_sort_plan<K>(n, bits, false, keys, vals, ws, ws_bytes, p);
+  return s == RK_SUCCESS ? rk_sort_run<K>(st, p, false, err) : s;
+}
 
 // The reference tie order of CUDA_radixSortGeneral (CUDA_radixSortGeneral.cu:397-482):
 //  length <= 512 (bubble, CUDA_bubbleSort512.cu): stable by key;
@@ -532,9 +738,9 @@ rk_status rk_sort_general_impl(hipStream_t st, uint32_t* keys, uint32_t* indices
   if (length <= byte_depth * 8192u) {
     hipLaunchKernelGGL(k_bitonic_chunks, dim3((length + 127) / 128), dim3(128), 0, st, keys, indices, length);
     RK_CHECK_LAUNCH();
-    return rk_radix_sort_impl<uint32_t>(st, keys, indices, length, 0, 4, ws, ws_bytes, err);
+    return sort_keys<uint32_t>(st, keys, indices, length, 32, ws, ws_bytes, err);
   }
-  return rk_radix_sort_impl<uint32_t>(st, keys, indices, length, 0, (int)byte_depth, ws, ws_bytes, err);
+  return sort_keys<uint32_t>(st, keys, indices, length, 8 * (int)byte_depth, ws, ws_bytes, err);
 }
 
 extern "C" rk_status rk_radix_sort_general(rk_stream stream, uint32_t* keys, uint32_t* indices, uint32_t length,
@@ -555,15 +761,14 @@ extern "C" rk_status rk_radix_sort(rk_stream stream, uint32_t* values, uint32_t 
     return launch_small_sort(rk_hip_stream(stream), values, nullptr, length, 0, ws_flags_word(ws, ws_bytes));
   const uint32_t byte_depth = 1 + (bit_depth - 1) / 8;
   int passes = (length <= byte_depth * 8192u) ? 4 : (int)byte_depth;
-  return rk_radix_sort_impl<uint32_t>(rk_hip_stream(stream), values, nullptr, length, 0, passes, ws, ws_bytes,
-                                      nullptr);
+  return sort_keys<uint32_t>(rk_hip_stream(stream), values, nullptr, length, 8 * passes, ws, ws_bytes, nullptr);
 }
 
 extern "C" rk_status rk_radix_sort_pairs_u64(rk_stream stream, uint64_t* keys, uint32_t* values, uint32_t length,
                                              uint32_t bit_depth, void* ws, size_t ws_bytes) {
   if (bit_depth == 0 || bit_depth > 64) return RK_ERROR_INVALID_VALUE;
   int passes = (int)(1 + (bit_depth - 1) / 8);
-  return rk_radix_sort_impl<uint64_t>(rk_hip_stream(stream), keys, values, length, 0, passes, ws, ws_bytes, nullptr);
+  return sort_keys<uint64_t>(rk_hip_stream(stream), keys, values, length, 8 * passes, ws, ws_bytes, nullptr);
 }
 
 // template <typename T> void CUDA_bitonicSort(T* values, uint length),
@@ -576,7 +781,7 @@ extern "C" rk_status rk_bitonic_sort(rk_stream stream, uint32_t* values, uint32_
   if (length > 1 && !values) return RK_ERROR_INVALID_VALUE;
   hipStream_t st = rk_hip_stream(stream);
   if (length <= kSmallSort) return launch_small_sort(st, values, nullptr, length, 0, ws_flags_word(ws, ws_bytes));
-  return rk_radix_sort_impl<uint32_t>(st, values, nullptr, length, 0, 4, ws, ws_bytes, nullptr);
+  return sort_keys<uint32_t>(st, values, nullptr, length, 32, ws, ws_bytes, nullptr);
 }
 
 // template <typename K, typename V> void CUDA_bitonicSortGeneral(K* keys, V* values, uint length),
@@ -596,7 +801,7 @@ extern "C" rk_status rk_bitonic_sort_general(rk_stream stream, uint32_t* keys, u
   hipLaunchKernelGGL(k_bitonic_chunks, dim3((length + 127) / 128), dim3(128), 0, st, keys, values, length);
   RK_CHECK_LAUNCH();
   if (length <= 128) return clear_ws_flags(st, ws, ws_bytes);
-  return rk_radix_sort_impl<uint32_t>(st, keys, values, length, 0, 4, ws, ws_bytes, nullptr);
+  return sort_keys<uint32_t>(st, keys, values, length, 32, ws, ws_bytes, nullptr);
 }
 
 // void CUDA_bubbleSort512(uint* keys, uint* indices, uint length, bool init_indices),

@@ -1,0 +1,113 @@
+"""The sort and the hierarchy pass at the sizes where their launches change: tiles
+and groups of tiles of the sort, the one-workgroup sort, runs and groups of runs of
+the hierarchy."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SORT_SIZES = [2, 513, 2048, 2049, 4096, 4097, 16 * 2048, 16 * 2048 + 1, (1 << 19) - 1, 1 << 19, (1 << 21) - 1, 1 << 21]
+
+
+@pytest.mark.parametrize("n", SORT_SIZES)
+def test_sorts_at_tile_edges(n):
+    """32-bit and 64-bit pairs with many equal keys, odd and even numbers of
+    passes, against numpy's stable sort."""
+    import torch
+
+    from cudart_amd import device as dev
+    rng = np.random.default_rng(n)
+    for bits in (8, 24, 32, 40, 64):
+        wide = bits > 32
+        k = rng.integers(0, 1 << min(bits, 63), n, dtype=np.uint64) & rng.integers(0, 1 << min(bits, 63), n, dtype=np.uint64)
+        k = k if wide else k.astype(np.uint32)
+        v = np.arange(n, dtype=np.uint32)[::-1].copy()
+        kt = torch.from_numpy(k.view(np.int64 if wide else np.int32).copy()).cuda()
+        vt = torch.from_numpy(v.view(np.int32)).cuda()
+        if wide:
+            dev.sort_pairs_u64(kt, vt, bits)
+        elif n > 32768 or n <= 512:  # between, the reference's bitonic chunks order equal keys
+            dev.sort_general(kt, vt, bits)
+        else:
+            dev.sort_values(kt, bits)
+        order = np.argsort(k, kind="stable")
+        np.testing.assert_array_equal(kt.cpu().numpy().view(k.dtype), k[order])
+        if wide or n > 32768 or n <= 512:
+            np.testing.assert_array_equal(vt.cpu().numpy().view(np.uint32), v[order])
+
+
+def _split(keys, i):
+    x = int(keys[i]) ^ int(keys[i + 1])
+    return (x | 1 << 63) if x else (i ^ (i + 1))
+
+
+def _expected(keys):
+    """{record: (left ref, right ref, left count, right count)} of the binary radix
+    tree over sorted keys, one face per leaf, from a stack of the splits' keys."""
+    n = len(keys)
+    up = [_split(keys, i) for i in range(n - 1)]
+    first = [0] * (n - 1)
+    last = [n - 1] * (n - 1)
+    stack = []  # each split's range ends at the nearest larger split on either side
+    for i, k in enumerate(up):
+        while stack and up[stack[-1]] < k:
+            last[stack.pop()] = i
+        first[i] = stack[-1] + 1 if stack else 0
+        stack.append(i)
+
+    def record(l, r):
+        if l == r:
+            return 0x80000000 | l << 4
+        if (l, r) == (0, n - 1):
+            return 0
+        left = l == 0 or (r + 1 < n and up[r] < up[l - 1])
+        return r if left else l
+    return {record(first[p], last[p]): (record(first[p], p), record(p + 1, last[p]), p - first[p] + 1, last[p] - p)
+            for p in range(n - 1)}
+
+
+@pytest.mark.parametrize("n", [2, 3, 511, 512, 513, 1024, 1025, 64 * 512, 64 * 512 + 1, 70001])
+@pytest.mark.parametrize("kind", ["soup30", "soup63", "equal", "chain"])
+def test_hierarchy_topology_at_run_edges(rk, n, kind):
+    """Every record of the tree against the tree computed from the sorted keys:
+    random faces, all faces with one key, and keys whose splits form a chain that
+    leaves over as many subtrees per run as the key length allows."""
+    import torch
+    V, F = rk.soup(n, seed=n)
+    if kind == "equal":
+        F = np.repeat(F[:1], n, axis=0)
+    elif kind == "chain":  # centroids halve towards one corner, over and over
+        c = np.float32(0.5) ** np.arange(n, dtype=np.float32).clip(0, 20)
+        V = V.reshape(n, 3, 4)
+        V[:, :, :3] = c[:, None, None] * np.float32(1.0)
+        V = np.ascontiguousarray(V.reshape(-1, 4))
+    hb = rk.hitbox(V)
+    mode = rk.RK_MORTON_63 if kind == "soup63" else rk.RK_MORTON_30
+    L = rk.lib()
+    Ft, Vt = torch.from_numpy(F.view(np.int32)).cuda(), torch.from_numpy(V).cuda()
+    nodes = torch.zeros((n, 16), dtype=torch.int32, device="cuda")
+    tris = torch.zeros((n, 12), dtype=torch.float32, device="cuda")
+    order = torch.zeros(n, dtype=torch.int32, device="cuda")
+    keys = torch.zeros(n, dtype=torch.int64 if kind == "soup63" else torch.int32, device="cuda")
+    info = torch.zeros(8, dtype=torch.int32, device="cuda")
+    ws = torch.empty(L.rk_fast_build_workspace_size(n, mode), dtype=torch.uint8, device="cuda")
+    desc = rk.FastBVH(nodes.data_ptr(), tris.data_ptr(), order.data_ptr(), None, n, 0)
+    box = rk.aabox(hb)
+    rk.check(L.rk_fast_build_keyed(None, Ft.data_ptr(), Vt.data_ptr(), n, C.byref(box), mode, 1, C.byref(desc),
+                                   info.data_ptr(), keys.data_ptr(), ws.data_ptr(), ws.numel()), "build")
+    torch.cuda.synchronize()
+    k = keys.cpu().numpy().view(np.uint64 if kind == "soup63" else np.uint32)
+    assert (np.diff(k.astype(np.float64)) >= 0).all()
+    np.testing.assert_array_equal(np.sort(order.cpu().numpy()), np.arange(n))
+    got = nodes.cpu().numpy().view(np.uint32)
+    boxes = got[:, :12].copy().view(np.float32)
+    expect = _expected(k)
+    idx = np.fromiter(expect, np.int64)
+    np.testing.assert_array_equal(got[idx, 12:], np.array(list(expect.values()), np.uint32))
+    # the root's two boxes hold every vertex
+    lo = np.minimum(boxes[0, [0, 2, 8]], boxes[0, [4, 6, 10]])
+    hi = np.maximum(boxes[0, [1, 3, 9]], boxes[0, [5, 7, 11]])
+    P = V[F[:, :3]].reshape(-1, 4)[:, :3]
+    assert (lo <= P.min(0)).all() and (hi >= P.max(0)).all()
