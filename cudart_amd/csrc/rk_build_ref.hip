@@ -7,6 +7,7 @@
 //   k_topo_ref       the host recursion of :309-455, level-synchronous (A13, A14)
 //   k_leaf_boxes     leaf boxes, one wave per leaf (A15, pass 0)
 //   k_refit_ref      internal boxes with the z-extent rule (A15, passes 1..)
+//   k_emit_ref       node ids and records
 //   reorder          faces'[i] = faces[indices[i]] (A16)
 // No step goes through the host: the reference's device->host copies
 // (:428, :651) and its host recursion are gone.
@@ -133,15 +134,16 @@ __global__ __launch_bounds__(kBoxThreads) void k_boxes_morton32(const uint4* __r
   }
 }
 
-// Zeroes the build's info words and level counts, and two runs of words.
+// Zeroes the build's info words and level counts, and three runs of words.
 __global__ __launch_bounds__(256) void k_lbvh_clear(uint32_t* __restrict__ info, uint32_t* __restrict__ level_count,
                                                     uint32_t* __restrict__ a, size_t na, uint32_t* __restrict__ b,
-                                                    size_t nb) {
+                                                    size_t nb, uint32_t* __restrict__ c, size_t nc) {
   const size_t stride = (size_t)gridDim.x * 256, t = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (t < RK_INFO_WORDS) info[t] = 0u;
   if (t < 64) level_count[t] = 0u;
   for (size_t i = t; i < na; i += stride) a[i] = 0u;
   for (size_t i = t; i < nb; i += stride) b[i] = 0u;
+  for (size_t i = t; i < nc; i += stride) c[i] = 0u;
 }
 
 __global__ __launch_bounds__(256) void k_morton(const Box* __restrict__ boxes, uint32_t n, float4 rmin, float4 rmax,
@@ -158,20 +160,22 @@ __global__ __launch_bounds__(256) void k_morton(const Box* __restrict__ boxes, u
 // codes with code[s]^code[s+1] != 0, level = clz (0 = bit 31). Here every
 // position gets a key (32 = no split) so one stable 8-bit pass groups the
 // splits by level, ascending within a level.
-// Counts the levels as it goes: into level_count (33 of its words), and into
-// the sort's digit counts when it takes them (digits, may be NULL).
-constexpr uint32_t kSplitPer = 8;  // positions per thread
-__global__ __launch_bounds__(256) void k_split_levels(const uint32_t* __restrict__ codes, uint32_t n,
-                                                      uint32_t* __restrict__ lev, uint32_t* __restrict__ pos,
-                                                      uint32_t* __restrict__ level_count,
-                                                      uint32_t* __restrict__ digits, uint32_t copies) {
+// Counts the levels as it goes, into the sort's digit counts when it takes
+// them, else into level_count (counts, copies, 256 words per copy). Few
+// workgroups, since each adds its counts to the same words: with 245 of 256
+// threads those atomics took 5 us of 9.8 on 1M codes.
+constexpr uint32_t kSplitPer = 16, kSplitThreads = 1024;  // positions per thread
+__global__ __launch_bounds__(kSplitThreads) void k_split_levels(const uint32_t* __restrict__ codes, uint32_t n,
+                                                                uint32_t* __restrict__ lev,
+                                                                uint32_t* __restrict__ pos,
+                                                                uint32_t* __restrict__ counts, uint32_t copies) {
   constexpr uint32_t kCopies = 16;  // most splits share a few levels: lanes count into copies
   __shared__ uint32_t s_count[kCopies][33];
-  for (uint32_t i = threadIdx.x; i < kCopies * 33; i += 256) (&s_count[0][0])[i] = 0u;
+  for (uint32_t i = threadIdx.x; i < kCopies * 33; i += kSplitThreads) (&s_count[0][0])[i] = 0u;
   __syncthreads();
 #pragma unroll 4
   for (uint32_t u = 0; u < kSplitPer; ++u) {
-    const uint32_t s = (blockIdx.x * kSplitPer + u) * 256 + threadIdx.x;
+    const uint32_t s = (blockIdx.x * kSplitPer + u) * kSplitThreads + threadIdx.x;
     if (s + 1 < n) {
       uint32_t diff = codes[s] ^ codes[s + 1];
       uint32_t level = diff ? (uint32_t)__clz((int)diff) : 32u;
@@ -184,49 +188,76 @@ __global__ __launch_bounds__(256) void k_split_levels(const uint32_t* __restrict
   if (threadIdx.x < 33) {
     uint32_t c = 0;
     for (uint32_t i = 0; i < kCopies; ++i) c += s_count[i][threadIdx.x];
-    if (c) {
-      atomicAdd(&level_count[threadIdx.x], c);
-      if (digits) atomicAdd(&digits[(size_t)(blockIdx.x % copies) * 256 + threadIdx.x], c);
-    }
+    if (c) atomicAdd(&counts[(size_t)(blockIdx.x % copies) * 256 + threadIdx.x], c);
   }
 }
 
 constexpr uint32_t kTopoThreads = 1024;
 constexpr uint32_t kMaxLevels = 96;
-constexpr uint32_t kKindMedian = 2u;  // rec flag bit 1: median-split subtree
-constexpr uint32_t kInternal = 1u;    // rec flag bit 0: internal node
+constexpr uint32_t kTopoFront = 5120;   // records of a level kept in LDS
+constexpr uint32_t kTopoLists = 16384;  // splits kept in LDS
+constexpr uint32_t kMedian = 0x80000000u;  // in rb: a median-split subtree
+constexpr uint8_t kInternal = 1u;          // in rmeta; the left turns on the path from the root above it
 
+// The tree's records, level by level, each level in ascending range order; a
+// node's children are records rchild and rchild + 1.
 struct TopoWs {
-  uint32_t* ra;      // range start (sorted position)
-  uint32_t* rb;      // range end
-  uint32_t* rflag;   // kInternal | kKindMedian | level << 8
-  uint32_t* rchild;  // record index of the left child (right = +1)
-  uint32_t* rcnt;    // internal nodes in the subtree
-  uint32_t* rrank;   // preorder rank among internal nodes
-  uint32_t* rid;     // node id
+  uint32_t* ra;         // range start (sorted position)
+  uint32_t* rb;         // range end
+  uint32_t* rchild;
+  uint8_t* rmeta;
+  float* rbox;          // six per record
   uint32_t* lev_begin;  // kMaxLevels + 1 record offsets
-  uint32_t* leaf_ids;   // node ids of leaves
+  uint32_t* bits;       // a bit per position: a node splits there
+  uint32_t* ranks;      // per kRankWords words, the bits before them
   uint32_t cap;
 };
+constexpr uint32_t kRankWords = 16;
 
-__device__ __forceinline__ uint32_t upper_bound(const uint32_t* __restrict__ A, uint32_t lo, uint32_t hi, uint32_t a) {
+// A barrier for what goes through LDS: stores to memory stay in flight.
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// The first of A[lo, hi) (ascending) above a, or hi.
+__device__ __forceinline__ uint32_t upper_bound(const uint32_t* A, uint32_t lo, uint32_t hi, uint32_t a) {
   while (lo < hi) {
-    uint32_t mid = (lo + hi) >> 1;
-    if (A[mid] <= a) lo = mid + 1; else hi = mid;
+    const uint32_t mid = (lo + hi) >> 1;
+    if (A[mid] <= a) lo = mid + 1u;
+    else hi = mid;
   }
   return lo;
 }
 
 // Where the reference's level-L split pointer stops when every level-L split
 // is <= a: it walks on through the (ascending) lists of levels L+1, L+2, ...
-// and stops at the first entry > a (CUDA_buildMeshTreeLBVH.cu:381-392).
-__device__ uint32_t chain_walk(const uint32_t* __restrict__ A, const uint32_t* s_idx, uint32_t L, uint32_t a,
-                               uint32_t S) {
+// and stops at the first entry > a (CUDA_buildMeshTreeLBVH.cu:381-392). That
+// entry's list: [lo, hi), or [S, S) past them all. s_last: each list's last
+// entry (0: empty list).
+__device__ __forceinline__ void chain_list(const uint32_t* s_idx, const uint32_t* s_last, uint32_t L, uint32_t a,
+                                           uint32_t S, uint32_t& lo, uint32_t& hi) {
   for (uint32_t k = L + 1; k < 32; ++k) {
-    uint32_t lo = s_idx[k], hi = s_idx[k + 1];
-    if (hi > lo && A[hi - 1] > a) return upper_bound(A, lo, hi, a);
+    if (s_last[k] > a) {
+      lo = s_idx[k];
+      hi = s_idx[k + 1];
+      return;
+    }
   }
-  return S;
+  lo = hi = S;
+}
+
+// The first of P[lo, hi) (ascending) above a, or hi, by a whole wave.
+__device__ __forceinline__ uint32_t wave_upper_bound(const uint32_t* P, uint32_t lo, uint32_t hi, uint32_t a,
+                                                     uint32_t lane) {
+  while (hi - lo > 64u) {
+    const uint32_t step = (hi - lo + 63u) / 64u, i = lo + lane * step;
+    const uint32_t c = (uint32_t)__popcll(__ballot(i < hi && P[i] <= a));
+    if (lo + c * step < hi) hi = lo + c * step;
+    if (c) lo += (c - 1u) * step + 1u;
+  }
+  return lo + (uint32_t)__popcll(__ballot(lo + lane < hi && P[lo + lane] <= a));
 }
 
 __device__ __forceinline__ uint32_t block_excl_scan1024(uint32_t v, uint32_t* s_tmp /*16*/, uint32_t* total) {
@@ -238,14 +269,14 @@ __device__ __forceinline__ uint32_t block_excl_scan1024(uint32_t v, uint32_t* s_
     if (lane >= (uint32_t)off) incl += y;
   }
   if (lane == 63) s_tmp[wave] = incl;
-  __syncthreads();
+  lds_barrier();
   uint32_t wprefix = 0, tot = 0;
   for (uint32_t w = 0; w < kTopoThreads / 64; ++w) {
     uint32_t c = s_tmp[w];
     wprefix += (w < wave) ? c : 0u;
     tot += c;
   }
-  __syncthreads();
+  lds_barrier();
   *total = tot;
   return wprefix + incl - v;
 }
@@ -261,165 +292,196 @@ __device__ __forceinline__ uint32_t block_excl_scan1024(uint32_t v, uint32_t* s_
 //    the start of level L+1's list, every later suffix node meets the entry test
 //    ptr == idx[L+1] (:375) and is a leaf; otherwise each later node stops at
 //    chain_walk(a).
-// Preorder ranks follow from per-subtree internal-node counts; an internal node
-// of rank r has children 2r+1, 2r+2 (:325-326, :394-395).
+// What bounds it is the chain from level to level on one CU, so the chain runs
+// in LDS: the first kTopoLists splits (the lists of the top levels, which hold
+// at most 2^L), and the current and the next level's records; memory is read for
+// what lies beyond, and written without waiting. One node per
+// lane and no work in waves without one: instruction issue is most of a level
+// (with 2 and 4 nodes per lane, searches interleaved, 76 and 104 us). Depth-12 tree of 1M faces: 154 us through memory, with
+// subtree counts up and down the levels for the node ids (k_emit_ref's ranks
+// now); 59 us so.
 __global__ __launch_bounds__(1024) void k_topo_ref(const uint32_t* __restrict__ A,
-                                                   const uint32_t* __restrict__ level_count, uint32_t n, uint32_t d,
-                                                   int complete, TopoWs w, Node* __restrict__ nodes,
-                                                   uint32_t* __restrict__ info) {
-  __shared__ uint32_t s_idx[34];
+                                                   const uint32_t* __restrict__ counts, uint32_t copies, uint32_t n,
+                                                   uint32_t d, int complete, TopoWs w, uint32_t* __restrict__ info) {
+  __shared__ uint32_t s_list[kTopoLists];
+  __shared__ uint32_t s_a[2][kTopoFront], s_b[2][kTopoFront];
+  __shared__ uint8_t s_meta[2][kTopoFront];
+  __shared__ uint32_t s_idx[34], s_cnt[33], s_last[33];
   __shared__ uint32_t s_lev[kMaxLevels + 2];
-  __shared__ uint32_t s_tmp[16];
-  __shared__ uint32_t s_j0, s_q0, s_flags, s_maxleaf, s_nleaves;
+  __shared__ __attribute__((aligned(16))) uint32_t s_sum[2][kTopoThreads / 64];
+  __shared__ uint32_t s_j0, s_flags;
   const uint32_t tid = threadIdx.x;
+  for (uint32_t i = tid; i < kTopoLists && i + 1 < n; i += kTopoThreads) s_list[i] = A[i];
+  if (tid < 64) {
+    uint32_t c = 0;
+    if (tid < 33)
+      for (uint32_t k = 0; k < copies; ++k) c += counts[(size_t)k * 256 + tid];
+    uint32_t incl = c;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(incl, off, 64);
+      if (tid >= (uint32_t)off) incl += y;
+    }
+    if (tid < 33) {
+      s_cnt[tid] = c;
+      s_idx[tid + 1] = incl;
+      s_last[tid] = tid < 32 && c ? A[incl - 1] : 0u;
+    }
+  }
   if (tid == 0) {
     s_idx[0] = 0;
-    for (int k = 0; k < 33; ++k) s_idx[k + 1] = s_idx[k] + level_count[k];
     s_flags = 0;
-    s_maxleaf = 0;
-    s_nleaves = 0;
-    w.ra[0] = 0;
-    w.rb[0] = n;
-    w.rflag[0] = 0;
+    s_j0 = 0xFFFFFFFFu;
+    s_a[0][0] = 0;
+    s_b[0][0] = n;
+    s_meta[0][0] = 0;
     s_lev[0] = 0;
   }
   __syncthreads();
   const uint32_t S = s_idx[32];
   const uint32_t past_depth = s_idx[d + 1 < 33 ? d + 1 : 32];
-  uint32_t cur = 0, end = 1, L = 0;
+  const uint32_t lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  uint32_t cur = 0, end = 1, L = 0, leaves = 0, turn = 0;
   while (cur < end) {
     if (L >= kMaxLevels) {
       if (tid == 0) s_flags |= 0x80000000u;
       break;
     }
-    const uint32_t cntL = L < 32 ? level_count[L] : 0u;
+    const uint32_t now = L & 1u, next = now ^ 1u;
+    const uint32_t cntL = L < 32 ? s_cnt[L] : 0u;
     const uint32_t EL = L < 32 ? s_idx[L + 1] : S;
-    const uint32_t lastA = cntL ? A[EL - 1] : 0u;
-    if (tid == 0) s_j0 = 0xFFFFFFFFu;
-    __syncthreads();
-    for (uint32_t r = cur + tid; r < end; r += kTopoThreads) {
-      uint32_t a = w.ra[r], b = w.rb[r], f = w.rflag[r];
-      bool walker = !(f & kKindMedian) && (b - a) >= 16 && L < d;
-      if (walker && (cntL == 0 || a >= lastA)) atomicMin(&s_j0, r);
+    const uint32_t lastA = cntL ? s_last[L] : 0u;
+    uint32_t j0 = 0xFFFFFFFFu;  // the first node whose walk leaves the level's list
+    if (cntL != 0u && L < d) {
+      for (uint32_t base = cur + wave * 64u; base < end; base += kTopoThreads) {
+        const uint32_t r = base + lane, i = r - cur;
+        bool leaves_list = false;
+        if (r < end) {
+          const uint32_t a = i < kTopoFront ? s_a[now][i] : w.ra[r], b = i < kTopoFront ? s_b[now][i] : w.rb[r];
+          leaves_list = !(b & kMedian) && b - a >= 16 && a >= lastA;
+        }
+        const unsigned long long m = __ballot(leaves_list);
+        if (m) {
+          if (lane == 0) atomicMin(&s_j0, base + (uint32_t)__builtin_ctzll(m));
+          break;
+        }
+      }
+      lds_barrier();
+      j0 = s_j0;
     }
-    __syncthreads();
-    if (tid == 0) {
-      uint32_t q0 = S;
-      if (s_j0 != 0xFFFFFFFFu && cntL != 0) q0 = chain_walk(A, s_idx, L, w.ra[s_j0], S);
-      s_q0 = q0;
-    }
-    __syncthreads();
-    const uint32_t j0 = s_j0, q0 = s_q0;
     uint32_t out = end;
     for (uint32_t chunk = cur; chunk < end; chunk += kTopoThreads) {
-      const uint32_t r = chunk + tid;
-      const bool in = r < end;
-      uint32_t internal = 0, split = 0, ckind = 0, a = 0, b = 0, f = 0;
-      if (in) {
-        a = w.ra[r]; b = w.rb[r]; f = w.rflag[r];
-        const uint32_t size = b - a;
-        if (f & kKindMedian) {  // createNode(median), :314-339
-          if (size >= 224) { internal = 1; split = (a + b) >> 1; ckind = kKindMedian; }
-        } else {                 // createNode(split), :360-411
-          bool leafish = true;
-          if (size >= 16 && L < d) {
-            uint32_t q = S;
-            bool entry_leaf = false;
-            if (cntL == 0) entry_leaf = true;
-            else if (a < lastA) q = upper_bound(A, s_idx[L], EL, a);
-            else if (r == j0) q = q0;
-            else if (q0 == EL) entry_leaf = true;
-            else q = chain_walk(A, s_idx, L, a, S);
-            if (!entry_leaf) {
-              if (q >= S) {
-                atomicOr(&s_flags, (uint32_t)RK_FLAG_WALK_PAST_END);
-              } else {
-                if (q >= past_depth) atomicOr(&s_flags, (uint32_t)RK_FLAG_WALK_PAST_DEPTH);
-                uint32_t sp = A[q];
-                if (sp < b) { leafish = false; internal = 1; split = sp; ckind = 0; }
-              }
+      const uint32_t w0 = chunk + wave * 64u, r = w0 + lane;
+      uint32_t a = 0, b = 0, meta = 0, split = 0, before = 0, mine = 0;
+      bool median = false, internal = false;
+      if (w0 < end) {  // a wave without records leaves its SIMD to the others
+        if (r < end) {
+          const uint32_t i = r - cur;
+          if (i < kTopoFront) {
+            a = s_a[now][i];
+            b = s_b[now][i];
+            meta = s_meta[now][i];
+            w.ra[r] = a;
+            w.rb[r] = b;
+          } else {
+            a = w.ra[r];
+            b = w.rb[r];
+            meta = w.rmeta[r];
+          }
+          median = (b & kMedian) != 0u;
+          b &= ~kMedian;
+        }
+        const uint32_t size = b - a;  // 0 past the end: a leaf
+        if (cntL != 0u && L < d) {    // createNode(split), :360-411
+          uint32_t q0 = S;
+          if (j0 < w0 + 64u) {  // where the walk that leaves the list stops
+            const uint32_t j = j0 - cur, aj = j < kTopoFront ? s_a[now][j] : w.ra[j0];
+            uint32_t l, h;
+            chain_list(s_idx, s_last, L, aj, S, l, h);
+            q0 = wave_upper_bound(h <= kTopoLists ? s_list : A, l, h, aj, lane);
+          }
+          bool search = !median && size >= 16u;
+          uint32_t lo = s_idx[L], hi = EL;
+          if (search && a >= lastA) {
+            if (r == j0) lo = hi = q0;
+            else if (q0 == EL) search = false;  // the entry test (:375): a leaf
+            else chain_list(s_idx, s_last, L, a, S, lo, hi);
+          }
+          if (search) {
+            const uint32_t q = __any(lo < hi && hi > kTopoLists) ? upper_bound(A, lo, hi, a) : upper_bound(s_list, lo, hi, a);
+            if (q >= S) {
+              atomicOr(&s_flags, (uint32_t)RK_FLAG_WALK_PAST_END);
+            } else {
+              if (q >= past_depth) atomicOr(&s_flags, (uint32_t)RK_FLAG_WALK_PAST_DEPTH);
+              split = q < kTopoLists ? s_list[q] : A[q];
+              internal = split < b;
             }
           }
-          // createLeaf, :341-358: a complete tree splits oversized leaves at the median.
-          if (leafish && complete && size > 224) { internal = 1; split = (a + b) >> 1; ckind = kKindMedian; }
         }
-        if (!internal) atomicMax(&s_maxleaf, L);
+        // createNode(median), :314-339; createLeaf, :341-358: a complete tree
+        // splits oversized leaves at the median
+        if (!internal && (median ? size >= 224u : complete && size > 224u)) {
+          internal = median = true;
+          split = (a + b) >> 1;
+        }
+        const unsigned long long m = __ballot(internal);
+        before = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        mine = (uint32_t)__popcll(m);
+        if (r < end) w.rmeta[r] = (uint8_t)(meta | (internal ? kInternal : 0u));
       }
-      uint32_t total;
-      uint32_t excl = block_excl_scan1024(internal * 2u, s_tmp, &total);
-      if (in) {
-        w.rflag[r] = (f & kKindMedian) | internal | (L << 8);
-        if (internal) {
-          uint32_t pos = out + excl;
-          if (pos + 2 <= w.cap) {
-            w.rchild[r] = pos;
-            w.ra[pos] = a; w.rb[pos] = split; w.rflag[pos] = ckind;
-            w.ra[pos + 1] = split; w.rb[pos + 1] = b; w.rflag[pos + 1] = ckind;
+      if (lane == 0) s_sum[turn][wave] = mine;
+      lds_barrier();
+      uint32_t total = 0, first = 0;
+#pragma unroll
+      for (uint32_t k = 0; k < kTopoThreads / 64; ++k) {
+        const uint32_t c = s_sum[turn][k];
+        first += k < wave ? c : 0u;
+        total += c;
+      }
+      turn ^= 1u;
+      if (internal) {
+        const uint32_t pos = out + 2u * (first + before), i = pos - end;
+        if (pos + 2 <= w.cap) {
+          const uint32_t kind = median ? kMedian : 0u;
+          w.rchild[r] = pos;
+          if (i + 1 < kTopoFront) {  // i is even: both or neither
+            s_a[next][i] = a;
+            s_b[next][i] = split | kind;
+            s_meta[next][i] = (uint8_t)(meta + 2u);  // one more left turn
+            s_a[next][i + 1] = split;
+            s_b[next][i + 1] = b | kind;
+            s_meta[next][i + 1] = (uint8_t)meta;
           } else {
-            atomicOr(&s_flags, 0x40000000u);
+            w.ra[pos] = a;
+            w.rb[pos] = split | kind;
+            w.rmeta[pos] = (uint8_t)(meta + 2u);
+            w.ra[pos + 1] = split;
+            w.rb[pos + 1] = b | kind;
+            w.rmeta[pos + 1] = (uint8_t)meta;
           }
+          atomicOr(&w.bits[split >> 5], 1u << (split & 31u));
+        } else {
+          atomicOr(&s_flags, 0x40000000u);
         }
       }
-      out += total;
-      __syncthreads();
+      out += 2u * total;
     }
+    leaves += end - cur - (out - end) / 2u;
     cur = end;
     end = out < w.cap ? out : w.cap;
     ++L;
-    if (tid == 0) s_lev[L] = cur;
-    __syncthreads();
+    if (tid == 0) {
+      s_lev[L] = cur;
+      s_j0 = 0xFFFFFFFFu;
+    }
+    if (end - cur > kTopoFront) __syncthreads();
+    else lds_barrier();
   }
   const uint32_t nlev = L;
   const uint32_t R = end;
   if (tid == 0) s_lev[nlev] = R;
   __syncthreads();
-  // Internal-node counts per subtree, bottom-up.
-  for (int lv = (int)nlev - 1; lv >= 0; --lv) {
-    for (uint32_t r = s_lev[lv] + tid; r < s_lev[lv + 1]; r += kTopoThreads) {
-      uint32_t c = 0;
-      if (w.rflag[r] & kInternal) {
-        uint32_t lc = w.rchild[r];
-        c = 1 + ((w.rflag[lc] & kInternal) ? w.rcnt[lc] : 0u) + ((w.rflag[lc + 1] & kInternal) ? w.rcnt[lc + 1] : 0u);
-      }
-      w.rcnt[r] = c;
-    }
-    __syncthreads();
-  }
-  // Preorder ranks and ids, top-down.
-  if (tid == 0) { w.rrank[0] = 0; w.rid[0] = 0; }
-  __syncthreads();
-  for (uint32_t lv = 0; lv < nlev; ++lv) {
-    for (uint32_t r = s_lev[lv] + tid; r < s_lev[lv + 1]; r += kTopoThreads) {
-      if (w.rflag[r] & kInternal) {
-        uint32_t R0 = w.rrank[r], lc = w.rchild[r];
-        w.rid[lc] = 2 * R0 + 1;
-        w.rid[lc + 1] = 2 * R0 + 2;
-        if (w.rflag[lc] & kInternal) w.rrank[lc] = R0 + 1;
-        if (w.rflag[lc + 1] & kInternal) w.rrank[lc + 1] = R0 + 1 + ((w.rflag[lc] & kInternal) ? w.rcnt[lc] : 0u);
-      }
-    }
-    __syncthreads();
-  }
-  // Emit bvnodes (make_node / make_leaf, :85-109) with empty boxes.
-  for (uint32_t r = tid; r < R; r += kTopoThreads) {
-    uint32_t f = w.rflag[r], id = w.rid[r];
-    Node nd;
-    if (f & kInternal) {
-      nd.w0 = (((f >> 8) % 3u) & 3u) << 1;
-      nd.w1 = 2 * w.rrank[r] + 1;
-    } else {
-      uint32_t a = w.ra[r], b = w.rb[r];
-      nd.w0 = 1u | ((b - a) << 1);
-      nd.w1 = a;
-      uint32_t li = atomicAdd(&s_nleaves, 1u);
-      w.leaf_ids[li] = id;
-    }
-    nd.bmin[0] = nd.bmin[1] = nd.bmin[2] = RK_HUGE;
-    nd.bmax[0] = nd.bmax[1] = nd.bmax[2] = -RK_HUGE;
-    nodes[id] = nd;
-  }
   for (uint32_t k = tid; k <= nlev; k += kTopoThreads) w.lev_begin[k] = s_lev[k];
-  __syncthreads();
   if (tid == 0) {
     uint32_t flags = s_flags & 0xFFFFu;
     if (R > n) flags |= RK_FLAG_NODES_GT_N;
@@ -430,35 +492,38 @@ __global__ __launch_bounds__(1024) void k_topo_ref(const uint32_t* __restrict__ 
     auto merge2x_oob = [](uint32_t c) { return ((c + 127) / 128) % 2 == 0 && (c % 128) != 0; };
     if (n > 512 && n <= 32768 && merge2x_oob(n)) flags |= RK_FLAG_MERGE2X_OOB;
     for (uint32_t k = 1; k <= d; ++k) {
-      uint32_t c = level_count[k];
+      uint32_t c = s_cnt[k];
       if (c > 128 && c <= 32768 && merge2x_oob(c)) flags |= RK_FLAG_MERGE2X_OOB;
     }
     info[RK_INFO_NODE_COUNT] = R;
-    info[RK_INFO_REAL_DEPTH] = s_maxleaf + 1;
+    info[RK_INFO_REAL_DEPTH] = nlev;  // the last level is all leaves
     atomicOr(&info[RK_INFO_FLAGS], flags | (s_flags & 0xC0000000u));
     info[RK_INFO_SPLITS] = S;
-    info[RK_INFO_LEAVES] = s_nleaves;
+    info[RK_INFO_LEAVES] = leaves;
     info[5] = nlev;
   }
 }
 
+__device__ __forceinline__ void store_rbox(float* __restrict__ p, const float (&mn)[3], const float (&mx)[3]) {
+  float2* o = reinterpret_cast<float2*>(p);  // 24 B per record: 8-B aligned
+  o[0] = make_float2(mn[0], mn[1]);
+  o[1] = make_float2(mn[2], mx[0]);
+  o[2] = make_float2(mx[1], mx[2]);
+}
+
 // Leaf boxes (kernel_calcBoundingBoxes pass 0, CUDA_buildMeshTreeLBVH.cu:246-268):
-// merge of the leaf's triangle boxes via indices. One wave per leaf.
-__global__ __launch_bounds__(256) void k_leaf_boxes(const uint32_t* __restrict__ leaf_ids, uint32_t n,
-                                                    const uint32_t* __restrict__ info,
-                                                    const uint32_t* __restrict__ indices, const Box* __restrict__ boxes,
-                                                    Node* __restrict__ nodes) {
-  const uint32_t nleaves = info[RK_INFO_LEAVES];
+// merge of the leaf's triangle boxes via indices. One wave per record.
+__global__ __launch_bounds__(256) void k_leaf_boxes(TopoWs w, uint32_t n, const uint32_t* __restrict__ info,
+                                                    const uint32_t* __restrict__ indices,
+                                                    const Box* __restrict__ boxes) {
+  const uint32_t R = info[RK_INFO_NODE_COUNT];
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t wave_global = (blockIdx.x * 256 + threadIdx.x) >> 6;
   const uint32_t nwaves = (gridDim.x * 256) >> 6;
-  for (uint32_t li = wave_global; li < nleaves; li += nwaves) {
-    const uint32_t id = leaf_ids[li];
-    const uint32_t w0 = nodes[id].w0, first = nodes[id].w1;
-    uint32_t cnt = rk::leaf_count(w0);
-    if (first >= n) cnt = 0;
-    else if (cnt > n - first) cnt = n - first;
-    float mnx = RK_HUGE, mny = RK_HUGE, mnz = RK_HUGE, mxx = -RK_HUGE, mxy = -RK_HUGE, mxz = -RK_HUGE;
+  for (uint32_t r = wave_global; r < R; r += nwaves) {
+    if (w.rmeta[r] & kInternal) continue;
+    const uint32_t first = w.ra[r], cnt = (w.rb[r] & ~kMedian) - first;
+    float mn[3] = {RK_HUGE, RK_HUGE, RK_HUGE}, mx[3] = {-RK_HUGE, -RK_HUGE, -RK_HUGE};
     // Faces lane, lane + 64, lane + 128, ... in that order, kLeafFetch at a
     // time with all their loads issued first: a face costs two dependent loads
     // (its index, then its box), and the leaves of an incomplete tree (the
@@ -472,52 +537,179 @@ __global__ __launch_bounds__(256) void k_leaf_boxes(const uint32_t* __restrict__
       for (uint32_t k = 0; k < kLeafFetch; ++k) {
         if (i0 + 64 * k < cnt) {
           const Box b = rk::load_box(boxes + ix[k]);
-          mnx = rk::fmn(mnx, b.mn.x); mny = rk::fmn(mny, b.mn.y); mnz = rk::fmn(mnz, b.mn.z);
-          mxx = rk::fmx(mxx, b.mx.x); mxy = rk::fmx(mxy, b.mx.y); mxz = rk::fmx(mxz, b.mx.z);
+          mn[0] = rk::fmn(mn[0], b.mn.x); mn[1] = rk::fmn(mn[1], b.mn.y); mn[2] = rk::fmn(mn[2], b.mn.z);
+          mx[0] = rk::fmx(mx[0], b.mx.x); mx[1] = rk::fmx(mx[1], b.mx.y); mx[2] = rk::fmx(mx[2], b.mx.z);
         }
       }
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) {
-      mnx = rk::fmn(mnx, __shfl_xor(mnx, off, 64)); mny = rk::fmn(mny, __shfl_xor(mny, off, 64));
-      mnz = rk::fmn(mnz, __shfl_xor(mnz, off, 64)); mxx = rk::fmx(mxx, __shfl_xor(mxx, off, 64));
-      mxy = rk::fmx(mxy, __shfl_xor(mxy, off, 64)); mxz = rk::fmx(mxz, __shfl_xor(mxz, off, 64));
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        mn[q] = rk::fmn(mn[q], __shfl_xor(mn[q], off, 64));
+        mx[q] = rk::fmx(mx[q], __shfl_xor(mx[q], off, 64));
+      }
     }
-    if (lane == 0) {
-      Node* nd = nodes + id;
-      nd->bmin[0] = mnx; nd->bmin[1] = mny; nd->bmin[2] = mnz;
-      nd->bmax[0] = mxx; nd->bmax[1] = mxy; nd->bmax[2] = mxz;
-    }
+    if (lane == 0) store_rbox(w.rbox + 6 * (size_t)r, mn, mx);
   }
 }
 
 // Internal boxes, bottom-up by level in one workgroup. The fixpoint of the
 // reference's real_depth racy passes (CUDA_buildMeshTreeLBVH.cu:269-301): a node
 // takes the union of its children only if both have z-extent > 0, else it
-// stays EMPTY (and so does every ancestor).
-__global__ __launch_bounds__(1024) void k_refit_ref(const uint32_t* __restrict__ rflag,
-                                                    const uint32_t* __restrict__ rid,
-                                                    const uint32_t* __restrict__ lev_begin,
-                                                    const uint32_t* __restrict__ info, Node* __restrict__ nodes) {
+// stays EMPTY (and so does every ancestor). Boxes are by record, so a level
+// costs one dependent load (the children's two boxes, side by side), from LDS
+// where the children's level fits, with the next level's kinds, children and leaf
+// boxes loaded meanwhile. (By node id, three loads from memory per level: 50 us
+// for the depth-12 tree of 1M faces; one: 33; 27 so.)
+// Also counts the split bits before each kRankWords words, for k_emit_ref.
+constexpr uint32_t kRefitPer = 3, kRefitLevel = kRefitPer * 1024;  // levels up to this size go through LDS
+__global__ __launch_bounds__(1024) void k_refit_ref(TopoWs w, uint32_t n, const uint32_t* __restrict__ info) {
+  __shared__ __attribute__((aligned(16))) float s_box[2][6 * kRefitLevel];
+  __shared__ uint32_t s_tmp[16];
+  __shared__ uint32_t s_lev[kMaxLevels + 2];
   const uint32_t nlev = info[5];
-  const uint32_t M = info[RK_INFO_NODE_COUNT];
-  for (int lv = (int)nlev - 1; lv >= 0; --lv) {
-    const uint32_t b0 = lev_begin[lv], b1 = lev_begin[lv + 1];
-    for (uint32_t r = b0 + threadIdx.x; r < b1; r += 1024) {
-      if (!(rflag[r] & kInternal)) continue;
-      Node* nd = nodes + rid[r];
-      if (nd->w1 + 1 >= M) continue;
-      const Node* l = nodes + nd->w1;
-      const Node* q = nodes + nd->w1 + 1;
-      if (l->bmax[2] - l->bmin[2] > 0.0f && q->bmax[2] - q->bmin[2] > 0.0f) {
+  uint32_t run = 0;
+  const uint32_t groups = n / 32u / kRankWords + 1u;
+  for (uint32_t g0 = 0; g0 < groups; g0 += 1024) {
+    const uint32_t g = g0 + threadIdx.x;
+    uint32_t c = 0;
+    if (g < groups) {
+      const uint4* p = reinterpret_cast<const uint4*>(w.bits + (size_t)g * kRankWords);
 #pragma unroll
-        for (int a = 0; a < 3; ++a) {
-          nd->bmin[a] = rk::fmn(l->bmin[a], q->bmin[a]);
-          nd->bmax[a] = rk::fmx(l->bmax[a], q->bmax[a]);
-        }
+      for (uint32_t k = 0; k < kRankWords / 4; ++k) {
+        const uint4 v = p[k];
+        c += __popc(v.x) + __popc(v.y) + __popc(v.z) + __popc(v.w);
       }
     }
-    __syncthreads();
+    uint32_t total;
+    const uint32_t ex = block_excl_scan1024(c, s_tmp, &total);
+    if (g < groups) w.ranks[g] = run + ex;
+    run += total;
+  }
+  for (uint32_t k = threadIdx.x; k <= nlev; k += 1024) s_lev[k] = w.lev_begin[k];
+  __syncthreads();
+  uint32_t meta[kRefitPer], child[kRefitPer];
+  float2 own[kRefitPer][3];
+  // kinds, children and boxes (a leaf's; an internal node's is not there yet) of a level
+  auto fetch = [&](int lv) {
+    const uint32_t b0 = s_lev[lv], b1 = s_lev[lv + 1];
+#pragma unroll
+    for (uint32_t u = 0; u < kRefitPer; ++u) {
+      const uint32_t r = b0 + u * 1024 + threadIdx.x;
+      if (r < b1) {
+        meta[u] = w.rmeta[r];
+        child[u] = w.rchild[r];
+        const float2* p = reinterpret_cast<const float2*>(w.rbox + 6 * (size_t)r);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) own[u][q] = p[q];
+      }
+    }
+  };
+  auto merge = [](const float2* p, float (&mn)[3], float (&mx)[3]) {
+    const float2 l0 = p[0], l1 = p[1], l2 = p[2], q0 = p[3], q1 = p[4], q2 = p[5];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      mn[q] = RK_HUGE;
+      mx[q] = -RK_HUGE;
+    }
+    if (l2.y - l1.x > 0.0f && q2.y - q1.x > 0.0f) {
+      mn[0] = rk::fmn(l0.x, q0.x); mn[1] = rk::fmn(l0.y, q0.y); mn[2] = rk::fmn(l1.x, q1.x);
+      mx[0] = rk::fmx(l1.y, q1.y); mx[1] = rk::fmx(l2.x, q2.x); mx[2] = rk::fmx(l2.y, q2.y);
+    }
+  };
+  bool fetched = false, below = false;  // below: the level below is in s_box
+  for (int lv = (int)nlev - 1; lv >= 0; --lv) {
+    const uint32_t b0 = s_lev[lv], b1 = s_lev[lv + 1];
+    if (b1 - b0 <= kRefitLevel) {
+      if (!fetched) fetch(lv);
+      float* to = s_box[lv & 1];
+      const float* from = s_box[(lv & 1) ^ 1];
+#pragma unroll
+      for (uint32_t u = 0; u < kRefitPer; ++u) {
+        const uint32_t i = u * 1024 + threadIdx.x;
+        if (b0 + i >= b1) continue;
+        float mn[3], mx[3];
+        if (meta[u] & kInternal) {
+          merge(reinterpret_cast<const float2*>(below ? from + 6 * (child[u] - b1) : w.rbox + 6 * (size_t)child[u]),
+                mn, mx);
+          store_rbox(w.rbox + 6 * (size_t)(b0 + i), mn, mx);
+        } else {
+          mn[0] = own[u][0].x; mn[1] = own[u][0].y; mn[2] = own[u][1].x;
+          mx[0] = own[u][1].y; mx[1] = own[u][2].x; mx[2] = own[u][2].y;
+        }
+        store_rbox(to + 6 * i, mn, mx);
+      }
+      fetched = lv > 0 && b0 - s_lev[lv - 1] <= kRefitLevel;
+      if (fetched) fetch(lv - 1);
+      below = true;
+      if (fetched || lv == 0) lds_barrier();
+      else __syncthreads();
+    } else {
+      for (uint32_t r = b0 + threadIdx.x; r < b1; r += 1024) {
+        if (!(w.rmeta[r] & kInternal)) continue;
+        float mn[3], mx[3];
+        merge(reinterpret_cast<const float2*>(w.rbox + 6 * (size_t)w.rchild[r]), mn, mx);
+        store_rbox(w.rbox + 6 * (size_t)r, mn, mx);
+      }
+      fetched = below = false;
+      __syncthreads();
+    }
+  }
+}
+
+// The node records (make_node / make_leaf, :85-109), by the reference's ids:
+// the internal node of preorder rank R gets children 2R+1, 2R+2 (:325-326,
+// :394-395). R counts the internal nodes before it in preorder: those whose
+// split is at or before its start a (in order, as many as leaves before a),
+// and its ancestors it lies to the left of. So each record finds its own.
+__global__ __launch_bounds__(256) void k_emit_ref(TopoWs w, const uint32_t* __restrict__ info,
+                                                  Node* __restrict__ nodes) {
+  __shared__ uint32_t s_lev[kMaxLevels + 2];
+  const uint32_t R = info[RK_INFO_NODE_COUNT], nlev = info[5];
+  for (uint32_t k = threadIdx.x; k <= nlev; k += 256) s_lev[k] = w.lev_begin[k];
+  __syncthreads();
+  auto rank_of = [&](uint32_t a, uint32_t meta) {
+    const uint32_t word = a >> 5, g = word / kRankWords;
+    uint32_t c = w.ranks[g] + (meta >> 1);
+#pragma unroll
+    for (uint32_t k = 0; k < kRankWords; ++k) {
+      const uint32_t i = g * kRankWords + k;
+      const uint32_t v = w.bits[i];
+      c += __popc(i < word ? v : (i == word ? v & (0xFFFFFFFFu >> (31u - (a & 31u))) : 0u));
+    }
+    return c;
+  };
+  auto emit = [&](uint32_t r, uint32_t id, uint32_t level) {
+    const uint32_t a = w.ra[r], meta = w.rmeta[r];
+    Node nd;
+    if (meta & kInternal) {
+      nd.w0 = ((level % 3u) & 3u) << 1;
+      nd.w1 = 2 * rank_of(a, meta) + 1;
+    } else {
+      nd.w0 = 1u | (((w.rb[r] & ~kMedian) - a) << 1);
+      nd.w1 = a;
+    }
+    const float* b = w.rbox + 6 * (size_t)r;
+    for (int q = 0; q < 3; ++q) {
+      nd.bmin[q] = b[q];
+      nd.bmax[q] = b[3 + q];
+    }
+    nodes[id] = nd;
+  };
+  for (uint32_t r = blockIdx.x * 256 + threadIdx.x; r < R; r += gridDim.x * 256) {
+    if (r == 0) emit(0, 0, 0);
+    const uint32_t meta = w.rmeta[r];
+    if (!(meta & kInternal)) continue;
+    uint32_t lo = 0, hi = nlev;  // the last level that starts at or before r
+    while (lo + 1 < hi) {
+      const uint32_t mid = (lo + hi) >> 1;
+      if (s_lev[mid] <= r) lo = mid;
+      else hi = mid;
+    }
+    const uint32_t id = 2 * rank_of(w.ra[r], meta) + 1, c = w.rchild[r];
+    emit(c, id, lo + 1);
+    emit(c + 1, id + 1, lo + 1);
   }
 }
 
@@ -583,9 +775,9 @@ extern "C" size_t rk_build_lbvh_workspace_size(uint32_t face_count) {
   b += rk_align_up(n * 4);            // codes
   b += rk_align_up(n * 4) * 2;        // level keys, positions
   b += rk_align_up(64 * 4);           // level counts
-  b += rk_align_up(cap * 4) * 7;      // topology records
+  b += rk_align_up(cap * 4) * 7;      // topology records: 24-B boxes, range starts
   b += rk_align_up((kMaxLevels + 2) * 4);
-  b += rk_align_up(n * 4);            // leaf ids
+  b += rk_align_up(n * 4);            // record kinds, split bits and their ranks
   b += rk_align_up(n * 16);           // face reorder temp
   b += rk_sort_workspace_size((uint32_t)n, 4);
   return b + 4096;
@@ -608,18 +800,28 @@ extern "C" rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_f
   uint32_t* pos = ar.take<uint32_t>(n);
   uint32_t* level_count = ar.take<uint32_t>(64);
   TopoWs tw;
-  tw.ra = ar.take<uint32_t>(cap); tw.rb = ar.take<uint32_t>(cap); tw.rflag = ar.take<uint32_t>(cap);
-  tw.rchild = ar.take<uint32_t>(cap); tw.rcnt = ar.take<uint32_t>(cap); tw.rrank = ar.take<uint32_t>(cap);
-  tw.rid = ar.take<uint32_t>(cap);
+  const size_t rec_bytes = 7 * rk_align_up(cap * 4);
+  char* rec = ar.take<char>(rec_bytes);
   tw.lev_begin = ar.take<uint32_t>(kMaxLevels + 2);
-  tw.leaf_ids = ar.take<uint32_t>(n);
+  char* marks = ar.take<char>((size_t)n * 4);
   tw.cap = (uint32_t)cap;
   uint4* ftmp = ar.take<uint4>(n);
   size_t sort_bytes = rk_sort_workspace_size(n, 4);
   void* sort_ws = ar.take<char>(sort_bytes);
-  if (!codes || !lev || !pos || !level_count || !tw.ra || !tw.rb || !tw.rflag || !tw.rchild || !tw.rcnt ||
-      !tw.rrank || !tw.rid || !tw.lev_begin || !tw.leaf_ids || !ftmp || !sort_ws)
+  if (!codes || !lev || !pos || !level_count || !rec || !tw.lev_begin || !marks || !ftmp || !sort_ws)
     return RK_ERROR_WORKSPACE;
+  // The records: boxes and range starts in rec, which the sort of the splits
+  // by level has as its workspace before; ends and children in the code sort's
+  // and in codes and lev, done with by then; one byte each, the split bits and
+  // their ranks in marks.
+  const uint32_t groups = n / 32u / kRankWords + 1u;
+  tw.rbox = reinterpret_cast<float*>(rec);
+  tw.ra = reinterpret_cast<uint32_t*>(rec + 6 * rk_align_up(cap * 4));
+  tw.rb = reinterpret_cast<uint32_t*>(sort_ws);  // at least 8 bytes per face
+  tw.rchild = codes;
+  tw.rmeta = reinterpret_cast<uint8_t*>(marks);
+  tw.bits = reinterpret_cast<uint32_t*>(marks + ((cap + 63) & ~(size_t)63));
+  tw.ranks = tw.bits + (size_t)groups * kRankWords;  // ends within marks, a multiple of 256 B, for every n
 
   rk_status s;
   const float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
@@ -632,14 +834,15 @@ extern "C" rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_f
   RkSortPlan<uint32_t> codes_plan, levels_plan;
   if (plain && (s = rk_sort_plan<uint32_t>(n, 32, false, codes, indices, sort_ws, sort_bytes, codes_plan)) != RK_SUCCESS)
     return s;
-  if (n > 1 && (s = rk_sort_plan<uint32_t>(n - 1, 8, true, lev, pos, tw.ra, 7 * rk_align_up(cap * 4), levels_plan)) !=
+  if (n > 1 && (s = rk_sort_plan<uint32_t>(n - 1, 8, true, lev, pos, rec, rec_bytes, levels_plan)) !=
                    RK_SUCCESS)
     return s;
   const bool counted = n > 1 && !levels_plan.one;  // the levels are counted where they are found
   const size_t clear_a = plain ? codes_plan.head_words + codes_plan.status_words : 0;
   const size_t clear_b = counted ? levels_plan.head_words + levels_plan.status_words : 0;
   hipLaunchKernelGGL(k_lbvh_clear, dim3(std::min<unsigned>(1024u, blocks_for((uint32_t)(clear_a + clear_b + 64), 1024))),
-                     dim3(256), 0, st, info, level_count, codes_plan.head, clear_a, levels_plan.head, clear_b);
+                     dim3(256), 0, st, info, level_count, codes_plan.head, clear_a, levels_plan.head, clear_b, tw.bits,
+                     groups * kRankWords);
   RK_CHECK_LAUNCH();
   // 4 faces per thread from 2^18 on, where that still leaves a workgroup for most CUs
   const uint32_t per = n >= (1u << 18) ? 4u : 1u;
@@ -652,22 +855,25 @@ extern "C" rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_f
             : rk_sort_general_impl(st, codes, indices, n, 32, 0, sort_ws, sort_bytes, info + RK_INFO_FLAGS);
   if (s != RK_SUCCESS) return s;
   if (n > 1) {
-    hipLaunchKernelGGL(k_split_levels, dim3(blocks_for(n - 1, 256 * kSplitPer)), dim3(256), 0, st, codes, n,
-                       levels_plan.src, levels_plan.vsrc, level_count,
-                       counted ? levels_plan.head + 1 : (uint32_t*)nullptr, levels_plan.copies);
+    hipLaunchKernelGGL(k_split_levels, dim3(blocks_for(n - 1, kSplitThreads * kSplitPer)), dim3(kSplitThreads), 0, st,
+                       codes, n, levels_plan.src, levels_plan.vsrc, counted ? levels_plan.head + 1 : level_count,
+                       counted ? levels_plan.copies : 1u);
     RK_CHECK_LAUNCH();
     s = rk_sort_run<uint32_t>(st, levels_plan, counted, info + RK_INFO_FLAGS);
     if (s != RK_SUCCESS) return s;
   }
-  hipLaunchKernelGGL(k_topo_ref, dim3(1), dim3(kTopoThreads), 0, st, pos, level_count, n, tree_depth, tree_complete,
-                     tw, reinterpret_cast<Node*>(nodes), info);
+  hipLaunchKernelGGL(k_topo_ref, dim3(1), dim3(kTopoThreads), 0, st, pos,
+                     counted ? levels_plan.head + 1 : level_count, counted ? levels_plan.copies : 1u, n, tree_depth,
+                     tree_complete, tw, info);
   RK_CHECK_LAUNCH();
   unsigned lb = blocks_for(n, 64 * 4);
   if (lb > 2048) lb = 2048;
-  hipLaunchKernelGGL(k_leaf_boxes, dim3(lb), dim3(256), 0, st, tw.leaf_ids, n, info, indices,
-                     reinterpret_cast<const Box*>(boxes), reinterpret_cast<Node*>(nodes));
+  hipLaunchKernelGGL(k_leaf_boxes, dim3(lb), dim3(256), 0, st, tw, n, info, indices,
+                     reinterpret_cast<const Box*>(boxes));
   RK_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_refit_ref, dim3(1), dim3(1024), 0, st, tw.rflag, tw.rid, tw.lev_begin, info,
+  hipLaunchKernelGGL(k_refit_ref, dim3(1), dim3(1024), 0, st, tw, n, info);
+  RK_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_emit_ref, dim3(std::min(2048u, blocks_for(n, 8 * 256))), dim3(256), 0, st, tw, info,
                      reinterpret_cast<Node*>(nodes));
   RK_CHECK_LAUNCH();
   if (tree_complete) {  // CUDA_reorderMeshFaces, CUDA_buildMeshTreeLBVH.cu:669-676

@@ -1,6 +1,7 @@
 """The sort and the hierarchy pass at the sizes where their launches change: tiles
 and groups of tiles of the sort, the one-workgroup sort, runs and groups of runs of
-the hierarchy."""
+the hierarchy; and the reference topology where a level or the split lists stop
+fitting in LDS."""
 import ctypes as C
 
 import numpy as np
@@ -111,3 +112,31 @@ def test_hierarchy_topology_at_run_edges(rk, n, kind):
     hi = np.maximum(boxes[0, [1, 3, 9]], boxes[0, [5, 7, 11]])
     P = V[F[:, :3]].reshape(-1, 4)[:, :3]
     assert (lo <= P.min(0)).all() and (hi >= P.max(0)).all()
+
+
+# faces: groups of 512 split bits; 16384 splits and levels of 3072 and 5120
+# records (LDS). "same": one code, so every split is a median's, by levels of 2^L.
+@pytest.mark.parametrize("n,depth,complete,same", [
+    (1, 12, True, False), (2, 31, True, False), (225, 12, True, True), (511, 31, True, False), (512, 31, True, False),
+    (513, 31, False, False), (16385, 31, True, False), (16386, 31, True, False), (60001, 31, True, False),
+    (150000, 31, True, False), (150000, 14, False, False), (1200000, 12, True, True)])
+def test_reference_topology_at_lds_edges(rk, ora, n, depth, complete, same):
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = rk.soup(n, seed=n)
+    if same:
+        F = np.repeat(F[:1], n, axis=0)
+    hb = rk.hitbox(V)
+    ref = ora.build_lbvh_ref(F, V, hb, depth, complete)
+    Ft = torch.from_numpy(F.view(np.int32).copy()).cuda()
+    tree = dev.build_lbvh(Ft, torch.from_numpy(V).cuda(), hb, depth, complete)
+    info = tree.host_info()
+    m = int(info[rk.RK_INFO_NODE_COUNT])
+    assert m == ref.node_count and int(info[rk.RK_INFO_REAL_DEPTH]) == ref.real_depth
+    assert int(info[rk.RK_INFO_FLAGS]) & 0xFF == ref.flags
+    np.testing.assert_array_equal(tree.indices.cpu().numpy().view(np.uint32), ref.indices)
+    np.testing.assert_array_equal(Ft.cpu().numpy().view(np.uint32), ref.faces)
+    nodes = tree.nodes.cpu().numpy().view(np.uint32)[:m].copy().view(ora.NODE_DTYPE).reshape(m)
+    for name in ("w0", "w1", "bmin", "bmax"):  # boxes as floats: -0 == +0
+        assert np.array_equal(nodes[name], ref.nodes[name]), name
