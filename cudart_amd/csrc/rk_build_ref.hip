@@ -512,30 +512,35 @@ __device__ __forceinline__ void store_rbox(float* __restrict__ p, const float (&
 }
 
 // Leaf boxes (kernel_calcBoundingBoxes pass 0, CUDA_buildMeshTreeLBVH.cu:246-268):
-// merge of the leaf's triangle boxes via indices. One wave per record.
-__global__ __launch_bounds__(256) void k_leaf_boxes(TopoWs w, uint32_t n, const uint32_t* __restrict__ info,
-                                                    const uint32_t* __restrict__ indices,
-                                                    const Box* __restrict__ boxes) {
+// merge of the leaf's triangle boxes via indices. One wave per record; leaves of
+// more than kWaveLeaf faces, which only incomplete trees (the Hybrid's first
+// pass) have, by the whole workgroup: of the 1M-face heightfield's at depth 12
+// the largest took one wave 343 us, this takes 31.
+constexpr uint32_t kLeafThreads = 1024, kWaveLeaf = 512;
+__global__ __launch_bounds__(kLeafThreads) void k_leaf_boxes(TopoWs w, int large, const uint32_t* __restrict__ info,
+                                                             const uint32_t* __restrict__ indices,
+                                                             const Box* __restrict__ boxes) {
+  constexpr uint32_t kWaves = kLeafThreads / 64;
+  __shared__ __attribute__((aligned(8))) float s_box[kWaves][6];
+  __shared__ uint32_t s_first[kWaves], s_cnt[kWaves];
   const uint32_t R = info[RK_INFO_NODE_COUNT];
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t wave_global = (blockIdx.x * 256 + threadIdx.x) >> 6;
-  const uint32_t nwaves = (gridDim.x * 256) >> 6;
-  for (uint32_t r = wave_global; r < R; r += nwaves) {
-    if (w.rmeta[r] & kInternal) continue;
-    const uint32_t first = w.ra[r], cnt = (w.rb[r] & ~kMedian) - first;
-    float mn[3] = {RK_HUGE, RK_HUGE, RK_HUGE}, mx[3] = {-RK_HUGE, -RK_HUGE, -RK_HUGE};
-    // Faces lane, lane + 64, lane + 128, ... in that order, kLeafFetch at a
-    // time with all their loads issued first: a face costs two dependent loads
-    // (its index, then its box), and the leaves of an incomplete tree (the
-    // Hybrid's first pass) hold thousands of faces.
+  const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // The leaf's faces t, t + threads, ... in that order, kLeafFetch at a time with
+  // all their loads issued first: a face costs two dependent loads (its index,
+  // then its box). In every lane, the wave's box.
+  auto merge = [&](uint32_t first, uint32_t cnt, uint32_t t, uint32_t threads, float (&mn)[3], float (&mx)[3]) {
+    for (int q = 0; q < 3; ++q) {
+      mn[q] = RK_HUGE;
+      mx[q] = -RK_HUGE;
+    }
     constexpr uint32_t kLeafFetch = 8;
-    for (uint32_t i0 = lane; i0 < cnt; i0 += 64 * kLeafFetch) {
+    for (uint32_t i0 = t; i0 < cnt; i0 += threads * kLeafFetch) {
       uint32_t ix[kLeafFetch];
 #pragma unroll
-      for (uint32_t k = 0; k < kLeafFetch; ++k) ix[k] = i0 + 64 * k < cnt ? indices[first + i0 + 64 * k] : 0u;
+      for (uint32_t k = 0; k < kLeafFetch; ++k) ix[k] = i0 + threads * k < cnt ? indices[first + i0 + threads * k] : 0u;
 #pragma unroll
       for (uint32_t k = 0; k < kLeafFetch; ++k) {
-        if (i0 + 64 * k < cnt) {
+        if (i0 + threads * k < cnt) {
           const Box b = rk::load_box(boxes + ix[k]);
           mn[0] = rk::fmn(mn[0], b.mn.x); mn[1] = rk::fmn(mn[1], b.mn.y); mn[2] = rk::fmn(mn[2], b.mn.z);
           mx[0] = rk::fmx(mx[0], b.mx.x); mx[1] = rk::fmx(mx[1], b.mx.y); mx[2] = rk::fmx(mx[2], b.mx.z);
@@ -550,7 +555,44 @@ __global__ __launch_bounds__(256) void k_leaf_boxes(TopoWs w, uint32_t n, const 
         mx[q] = rk::fmx(mx[q], __shfl_xor(mx[q], off, 64));
       }
     }
-    if (lane == 0) store_rbox(w.rbox + 6 * (size_t)r, mn, mx);
+  };
+  // neighbours in a level, which are alike in size, go to different workgroups
+  for (uint32_t base = blockIdx.x; base < R; base += gridDim.x * kWaves) {
+    const uint32_t r = base + wave * gridDim.x;
+    float mn[3], mx[3];
+    uint32_t first = 0, cnt = 0;
+    const bool leaf = r < R && !(w.rmeta[r] & kInternal);
+    if (leaf) {
+      first = w.ra[r];
+      cnt = (w.rb[r] & ~kMedian) - first;
+      if (!large || cnt <= kWaveLeaf) {
+        merge(first, cnt, lane, 64, mn, mx);
+        if (lane == 0) store_rbox(w.rbox + 6 * (size_t)r, mn, mx);
+        cnt = 0;
+      }
+    }
+    if (!large) continue;
+    if (lane == 0) {
+      s_first[wave] = first;
+      s_cnt[wave] = cnt;
+    }
+    __syncthreads();
+    for (uint32_t x = 0; x < kWaves; ++x) {
+      if (s_cnt[x] == 0u) continue;  // uniform
+      merge(s_first[x], s_cnt[x], threadIdx.x, kLeafThreads, mn, mx);
+      if (lane == 0) store_rbox(s_box[wave], mn, mx);
+      __syncthreads();
+      if (threadIdx.x == 0) {
+        for (uint32_t v = 1; v < kWaves; ++v)
+          for (int q = 0; q < 3; ++q) {
+            mn[q] = rk::fmn(mn[q], s_box[v][q]);
+            mx[q] = rk::fmx(mx[q], s_box[v][3 + q]);
+          }
+        store_rbox(w.rbox + 6 * (size_t)(base + x * gridDim.x), mn, mx);
+      }
+      __syncthreads();
+    }
+    __syncthreads();
   }
 }
 
@@ -866,10 +908,8 @@ extern "C" rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_f
                      counted ? levels_plan.head + 1 : level_count, counted ? levels_plan.copies : 1u, n, tree_depth,
                      tree_complete, tw, info);
   RK_CHECK_LAUNCH();
-  unsigned lb = blocks_for(n, 64 * 4);
-  if (lb > 2048) lb = 2048;
-  hipLaunchKernelGGL(k_leaf_boxes, dim3(lb), dim3(256), 0, st, tw, n, info, indices,
-                     reinterpret_cast<const Box*>(boxes));
+  hipLaunchKernelGGL(k_leaf_boxes, dim3(std::min(512u, blocks_for(n, 1024))), dim3(kLeafThreads), 0, st, tw,
+                     tree_complete ? 0 : 1, info, indices, reinterpret_cast<const Box*>(boxes));
   RK_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_refit_ref, dim3(1), dim3(1024), 0, st, tw, n, info);
   RK_CHECK_LAUNCH();

@@ -2,30 +2,34 @@
 // and the Hybrid refinement of LBVH leaves (kernel_initStack, :647-666), for
 // gfx950. The reference processes one node per 32-thread block with thread 0
 // doing the binning, sweep and partition serially, and a host round trip per
-// level through a 4096-entry global stack. Here each level's nodes ("items")
-// are cut into 1024-face chunks, one workgroup per chunk:
-//   k_sah_prep       chunk offsets per item (one workgroup scan), accumulator reset
-//   k_sah_bounds     centroid bounds per item (ordered-int atomics)
-//   k_sah_bins       32 bins per item: count + primitive-box bounds (LDS, then atomics)
-//   k_sah_decide     one half-wave per item, one lane per bin: the reference
-//                    sweep (:424-474), leaf test (:479-496), children boxes
-//                    (:501-530)
-//   k_sah_small      items of 17 to 1024 faces, one wave each: all of the
-//                    above and the partition, in LDS; the chunk kernels take
-//                    the items of more than 1024 faces
-//   k_sah_emit       1024 items per workgroup: scan of the internal items,
-//                    node records, next-level items; child ids in
-//                    breadth-first order
-//   k_sah_count      per-chunk left counts
-//   k_sah_offsets    per-item exclusive scan over chunks, one wave per item
-//   k_sah_scatter    stable partition (bin <= m_min goes left, :572-594)
-//   k_sah_copyback   partitioned ranges back into indices
+// level through a 4096-entry global stack. Here the tree is made first, without
+// node ids, and numbered afterwards:
+//   items of more than 1024 faces, level by level, cut into 1024-face chunks,
+//   one workgroup per chunk:
+//     k_sah_bins     32 bins per item: count + primitive-box bounds (LDS, then
+//                    atomics); each face's bin and the chunk's counts are kept
+//     k_sah_split    one half-wave per item, one lane per bin: the reference
+//                    sweep (:424-474), leaf test (:479-496), children (:501-530)
+//     k_sah_scatter  stable partition (bin <= m_min goes left, :572-594) into the
+//                    other id buffer, and the children's centroid bounds
+//   k_sah_subtrees   items of at most 1024 faces, start to end in one workgroup's
+//                    LDS: every level below them
+//   k_sah_number,    ids in breadth-first order and the node records, level by
+//   k_sah_number_run level
+// The 999,698-face heightfield takes 640 us: 12 levels of bins (11.5 us: the gather
+// of the boxes, then LDS atomics), split (7: a chain of loads) and scatter (9.7: the
+// same gather), subtrees 153 (instruction issue), numbering 70. With the items
+// numbered as they were made (nine kernels per level, the boxes gathered in four
+// of them, and again on each of 19 levels for the small items) it took 1750.
 // Min/max are exact in any order, so the atomics and the sweep's scans
 // reproduce the reference's serial merges; each cost is the reference's
-// expression on the same values. Node numbering: items are processed level by
-// level in queue order, and the k-th internal item of a level takes children
-// (count + 2k, count + 2k + 1), the breadth-first equivalent of the
-// reference's atomicAdd(node_count, 2).
+// expression on the same values. Node numbering: a level's items are in queue
+// order, and its k-th internal item takes children (count + 2k, count + 2k + 1),
+// the breadth-first equivalent of the reference's atomicAdd(node_count, 2).
+#include <algorithm>
+#include <numeric>
+#include <vector>
+
 #include "rk_device.h"
 
 namespace {
@@ -34,45 +38,88 @@ using rk::Box;
 using rk::Node;
 
 constexpr uint32_t kChunk = 1024;
-// threads per workgroup of the per-chunk kernels (bounds, bins, count,
-// scatter, copyback): one chunk each
-#ifndef RK_SAH_CHUNK_THREADS
-#define RK_SAH_CHUNK_THREADS 128
-#endif
-constexpr int kCT = RK_SAH_CHUNK_THREADS;
-static_assert(kCT % 64 == 0 && kCT <= 256, "whole waves, at most 4");
-constexpr uint32_t kEmitGroup = 1024;  // items per workgroup of k_sah_emit
+constexpr int kCT = 256;             // threads of the per-chunk kernels
+constexpr int kPer = kChunk / kCT;   // faces per thread
 constexpr int kBins = 32;
 constexpr uint32_t kLeafMin = 16;    // MIN_LEAF_SIZE, :55
 constexpr uint32_t kLeafMax = 224;   // MAX_LEAF_SIZE, :56
+constexpr uint32_t kLevelMax = 4096; // deeper trees are refused
 
-struct Item {
-  uint32_t node, lo, hi, pad;
+// An item's record. The split positions of the items are all different (the
+// ranges are disjoint and both sides hold faces: the cost of a split with an
+// empty side is not a number), so an item split at position p has its children
+// in records 2p and 2p + 1, with nothing to allocate; the items that the build
+// starts from come after them, at 2n.
+struct Rec {
   float bmin[3], bmax[3];
-  float pad2[2];
+  uint32_t lo, cnt;
 };
-static_assert(sizeof(Item) == 48, "item is 48 B");
+static_assert(sizeof(Rec) == 32, "record is 32 B");
+constexpr uint32_t kLeaf = 0xFFFFFFFFu;  // link of a leaf; else split | axis << 30
 
-// Accumulators of an item of more than kChunk faces: its centroid bounds
-// (6 ordered ints) in kBoundSlots copies, which its chunks update in turn so
-// that fewer atomics meet on one address, then kBinSlots copies of 32 bins
-// of (count, 3 min, 3 max ordered ints).
-constexpr int kBoundSlots = 8;
-constexpr int kBinSlots = 4;  // copies of the bins, likewise
-constexpr int kBinBase = 6 * kBoundSlots;
-constexpr int kBinWords = kBins * 7;
-constexpr int kAccWords = kBinBase + kBinSlots * kBinWords;
-
-// Per-item decision written by k_sah_decide.
-struct Decision {
-  int axis;
-  float scale, bmin0;
-  int m_min;        // -1: leaf
+struct BigItem {  // of more than kChunk faces
+  uint32_t rec, lo, hi, chunk_base;
+  float bmin[3], bmax[3];
+  uint32_t bref, pad;  // its centroid bounds
+};
+static_assert(sizeof(BigItem) == 48, "item is 48 B");
+struct BigDec {
+  int m_min;  // -1: leaf
   uint32_t lcount;
-  uint32_t pad[3];
-  float child[12];  // internal items: left min xyz, left max xyz, right min xyz, right max xyz
 };
-static_assert(sizeof(Decision) == 80, "decision is 80 B");
+
+// Accumulators of the big items, kept empty between levels by who reads them
+// last (k_sah_split): 32 bins of (count, 3 min, 3 max ordered ints) in kBinSlots
+// copies, which an item's chunks update in turn so that fewer atomics meet on
+// one address; centroid bounds (6 ordered ints) of both children, likewise.
+constexpr int kBinSlots = 4;
+constexpr int kBinWords = kBins * 7;
+constexpr int kAccWords = kBinSlots * kBinWords;
+constexpr int kBoundSlots = 8;
+constexpr int kBoundWords = 6 * kBoundSlots;
+
+constexpr int kCtlFlags = 0, kCtlDeep = 1, kCtlRoots = 2, kCtlLargest = 5, kCtlHist = 16;
+// a tree of n faces has fewer than n levels with internal items
+__device__ __host__ constexpr size_t ctl_words(uint32_t n) { return kCtlHist + (n < kLevelMax ? n : kLevelMax) + 1; }
+// per level parity: big items, their chunks
+__device__ __host__ constexpr int kCtlBig(uint32_t par) { return 8 + 2 * (int)par; }
+constexpr int kCtlRead = 12;  // words the host reads between levels
+
+// Items of at most kChunk faces by size, so that a workgroup of k_sah_subtrees
+// takes 8, 4 or 1 of them.
+constexpr uint32_t kClasses = 3;
+__device__ __host__ constexpr uint32_t class_cap(uint32_t c) { return c == 0 ? 128u : (c == 1 ? 256u : kChunk); }
+__device__ __forceinline__ uint32_t class_of(uint32_t size) { return size <= 128u ? 0u : (size <= 256u ? 1u : 2u); }
+
+struct Sah {
+  uint32_t n, chunks_cap, big_cap;
+  size_t m_cap;
+  const Box* boxes;
+  uint32_t *ids0, *ids1;  // levels of even parity read the first and write the second
+  Rec* rec;
+  uint32_t* link;
+  uint32_t* node0;        // node ids of the starting items
+  uint32_t *q0, *q1;      // a level's splits, in order, by parity
+  uint2* roots;           // kClasses lists of (record, level)
+  BigItem *big0, *big1;
+  BigDec* dec;
+  uint32_t *chunk_item0, *chunk_item1;
+  int* acc;
+  int *bnd0, *bnd1;
+  uint16_t* cum;          // [bin][chunk]: faces of the chunk up to the bin
+  uint8_t* bin;           // by position
+  uint32_t* ctl;          // ctl_words; at kCtlHist the internal items per level
+  uint32_t* groups;       // 3 x group_cap: internal items per kNumberItems of a level
+  uint32_t group_cap;
+};
+constexpr uint32_t kNumberItems = 1024;
+
+__device__ __forceinline__ BigItem* big_of(const Sah& s, uint32_t par) { return par ? s.big1 : s.big0; }
+__device__ __forceinline__ uint32_t* chunks_of(const Sah& s, uint32_t par) {
+  return par ? s.chunk_item1 : s.chunk_item0;
+}
+__device__ __forceinline__ int* bounds_of(const Sah& s, uint32_t par) { return par ? s.bnd1 : s.bnd0; }
+__device__ __forceinline__ uint32_t* ids_of(const Sah& s, uint32_t par) { return par ? s.ids1 : s.ids0; }
 
 __device__ __forceinline__ int f2o(float f) {  // order-preserving float -> int
   int i = __float_as_int(f);
@@ -106,154 +153,118 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* s_tmp,
   return wprefix + incl - v;
 }
 
-// ctl words: [0] flags; per level parity p (level & 1), at kCtlLevel(p):
-// +0 items (m), +1 items of more than kChunk faces, +2 chunks (T), +3 slots
-// taken, +4 node count before the level. A level of parity p reads its own
-// words and writes the next level's m, big-item count and node count; its
-// k_sah_prep clears the next level's counters, which nothing of this level
-// uses.
-constexpr int kCtlFlags = 0, kCtlWords = 32;
-__device__ __host__ constexpr int kCtlLevel(uint32_t p) { return 8 + 8 * (int)p; }
-constexpr int kLvM = 0, kLvBig = 1, kLvT = 2, kLvSlot = 3, kLvCount = 4;
-
-// Items of more than kChunk faces get a slot of accumulators (kept in the
-// item's pad word) and a run of chunks, in any order among items; chunk_item
-// maps a chunk back to its item. Smaller items are k_sah_small's. One wave
-// per item, launched over the level's items (with a bound, kPrepItems per
-// workgroup), and the grid's threads also clear the emit groups' counters.
-constexpr uint32_t kPrepItems = 4;
-__global__ __launch_bounds__(64 * kPrepItems) void k_sah_prep(Item* __restrict__ items, uint32_t* __restrict__ ctl,
-                                                              uint32_t par, uint32_t* __restrict__ chunk_base,
-                                                              uint32_t* __restrict__ chunk_item,
-                                                              int* __restrict__ acc,
-                                                              uint32_t* __restrict__ group_internal) {
-  uint32_t* lv = ctl + kCtlLevel(par);
-  const uint32_t m = lv[kLvM];
-  const uint32_t t = blockIdx.x * (64 * kPrepItems) + threadIdx.x, lane = threadIdx.x & 63;
-  if (t == 0) {
-    uint32_t* nx = ctl + kCtlLevel(par ^ 1u);
-    nx[kLvBig] = 0u;
-    nx[kLvT] = 0u;
-    nx[kLvSlot] = 0u;
+// Empties the accumulators, clears the counters and info, and makes the root
+// item (root: not Hybrid).
+__global__ __launch_bounds__(256) void k_sah_clear(Sah s, uint32_t* __restrict__ info, int root, float4 rmin,
+                                                   float4 rmax) {
+  const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, stride = (size_t)gridDim.x * 256;
+  const int lo = f2o(RK_HUGE), hi = f2o(-RK_HUGE);
+  for (size_t i = t; i < (size_t)s.big_cap * kAccWords; i += stride) {
+    const uint32_t k = (uint32_t)(i % 7);
+    s.acc[i] = k == 0 ? 0 : (k < 4 ? lo : hi);
   }
-  if (t < (m + kEmitGroup - 1) / kEmitGroup) group_internal[t] = 0u;
-  const uint32_t i = t >> 6;
-  if (i >= m) return;  // wave-uniform
-  const uint32_t size = items[i].hi - items[i].lo;
-  if (size <= kChunk) return;
-  const uint32_t nch = (size + kChunk - 1) / kChunk;
-  uint32_t slot = 0, base = 0;
-  if (lane == 0) {
-    slot = atomicAdd(lv + kLvSlot, 1u);
-    base = atomicAdd(lv + kLvT, nch);
-    items[i].pad = slot;
-    chunk_base[i] = base;
+  for (size_t i = t; i < (size_t)s.big_cap * 2 * kBoundWords; i += stride)
+    s.bnd0[i] = s.bnd1[i] = i % 6 < 3 ? lo : hi;
+  const uint32_t nch = root && s.n > kChunk ? (s.n + kChunk - 1) / kChunk : 0u;
+  for (size_t i = t; i < ctl_words(s.n); i += stride) {
+    uint32_t v = 0;
+    if (nch && i == (size_t)kCtlBig(0)) v = 1;
+    if (nch && i == (size_t)kCtlBig(0) + 1) v = nch;
+    if (root && !nch && i == kCtlRoots + class_of(s.n)) v = 1;
+    s.ctl[i] = v;
   }
-  slot = __shfl(slot, 0, 64);
-  base = __shfl(base, 0, 64);
-  for (uint32_t j = lane; j < nch; j += 64) chunk_item[base + j] = i;
-  int* a = acc + (size_t)slot * kAccWords;  // the bins are reset by k_sah_bounds
-  if (lane < 6 * kBoundSlots) a[lane] = (lane % 6) < 3 ? f2o(RK_HUGE) : f2o(-RK_HUGE);
+  if (t < RK_INFO_WORDS) info[t] = 0u;
+  for (size_t i = t; i < nch; i += stride) s.chunk_item0[i] = 0u;
+  if (root && t == 0) {
+    Rec r;
+    r.bmin[0] = rmin.x; r.bmin[1] = rmin.y; r.bmin[2] = rmin.z;
+    r.bmax[0] = rmax.x; r.bmax[1] = rmax.y; r.bmax[2] = rmax.z;
+    r.lo = 0;
+    r.cnt = s.n;
+    s.rec[2 * (size_t)s.n] = r;
+    s.node0[0] = 0;
+    if (nch) {
+      BigItem b;
+      b.rec = 2 * s.n; b.lo = 0; b.hi = s.n; b.chunk_base = 0; b.bref = 0; b.pad = 0;
+      for (int q = 0; q < 3; ++q) { b.bmin[q] = r.bmin[q]; b.bmax[q] = r.bmax[q]; }
+      s.big0[0] = b;
+    } else {
+      s.roots[class_of(s.n) * s.m_cap] = make_uint2(2 * s.n, 0u);
+    }
+  }
 }
 
-struct ChunkRange { uint32_t item, slot, lo, hi; bool first, ok; };
+// Hybrid entry (kernel_initStack, :647-666): every leaf of the existing tree
+// becomes an item, in ascending node order, with the leaf's box.
+__global__ __launch_bounds__(1024) void k_sah_init_from_leaves(Sah s, const Node* __restrict__ nodes,
+                                                               uint32_t existing) {
+  __shared__ uint32_t s_tmp[16], s_cnt[2 + kClasses], s_largest;
+  if (threadIdx.x < 2 + kClasses) s_cnt[threadIdx.x] = 0;
+  if (threadIdx.x == 0) s_largest = 0;
+  uint32_t carry = 0;
+  __syncthreads();
+  for (uint32_t c0 = 0; c0 < existing; c0 += 1024) {
+    const uint32_t k = c0 + threadIdx.x, lane = threadIdx.x & 63;
+    uint32_t leaf = 0;
+    Node nd;
+    if (k < existing) {
+      nd = nodes[k];
+      leaf = rk::node_is_leaf(nd.w0);
+    }
+    uint32_t total;
+    const uint32_t i = carry + block_excl_scan(leaf, s_tmp, &total, 1024);
+    carry += total;
+    uint32_t nch = 0, base = 0, at = 0;
+    if (leaf) {
+      Rec r;
+      for (int q = 0; q < 3; ++q) { r.bmin[q] = nd.bmin[q]; r.bmax[q] = nd.bmax[q]; }
+      r.lo = nd.w1;
+      r.cnt = rk::leaf_count(nd.w0);
+      const uint32_t rec = 2 * s.n + i;
+      s.rec[rec] = r;
+      s.node0[i] = k;
+      if (r.cnt > kChunk) {
+        nch = (r.cnt + kChunk - 1) / kChunk;
+        at = atomicAdd(&s_cnt[0], 1u);
+        base = atomicAdd(&s_cnt[1], nch);
+        atomicMax(&s_largest, r.cnt);
+        BigItem b;
+        b.rec = rec; b.lo = r.lo; b.hi = r.lo + r.cnt; b.chunk_base = base; b.bref = at; b.pad = 0;
+        for (int q = 0; q < 3; ++q) { b.bmin[q] = r.bmin[q]; b.bmax[q] = r.bmax[q]; }
+        s.big0[at] = b;
+      } else {
+        const uint32_t c = class_of(r.cnt);
+        s.roots[c * s.m_cap + atomicAdd(&s_cnt[2 + c], 1u)] = make_uint2(rec, 0u);
+      }
+    }
+    for (uint64_t m = __ballot(nch != 0u); m; m &= m - 1) {
+      const int l = __builtin_ctzll(m);
+      const uint32_t b = __shfl(base, l, 64), e = __shfl(nch, l, 64), a = __shfl(at, l, 64);
+      for (uint32_t j = lane; j < e; j += 64) s.chunk_item0[b + j] = a;
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) s.ctl[kCtlBig(0) + threadIdx.x] = s_cnt[threadIdx.x];
+  else if (threadIdx.x < 2 + kClasses) s.ctl[kCtlRoots + threadIdx.x - 2] = s_cnt[threadIdx.x];
+  else if (threadIdx.x == 64) s.ctl[kCtlLargest] = s_largest;
+}
 
-__device__ __forceinline__ ChunkRange chunk_range(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                  uint32_t par, const uint32_t* __restrict__ chunk_base,
-                                                  const uint32_t* __restrict__ chunk_item, uint32_t c) {
+struct ChunkRange { BigItem it; uint32_t item, j, lo, hi; bool ok; };
+
+__device__ __forceinline__ ChunkRange chunk_range(const Sah& s, uint32_t par) {
   ChunkRange r;
-  r.ok = c < ctl[kCtlLevel(par) + kLvT];
+  r.ok = blockIdx.x < s.ctl[kCtlBig(par) + 1];
   if (!r.ok) return r;
-  r.item = chunk_item[c];
-  const Item it = items[r.item];
-  const uint32_t j = c - chunk_base[r.item];
-  r.slot = it.pad;
-  r.first = j == 0;
-  r.lo = it.lo + j * kChunk;
-  r.hi = min(it.hi, r.lo + kChunk);
+  r.item = chunks_of(s, par)[blockIdx.x];
+  r.it = big_of(s, par)[r.item];
+  r.j = blockIdx.x - r.it.chunk_base;
+  r.lo = r.it.lo + r.j * kChunk;
+  r.hi = min(r.it.hi, r.lo + kChunk);
   return r;
-}
-
-// The boxes of a chunk's faces, kPer per thread, with every gather in flight
-// at once: the face ids first, then the boxes.
-constexpr int kPer = kChunk / kCT;
-__device__ __forceinline__ void chunk_boxes(const ChunkRange& r, const uint32_t* __restrict__ indices,
-                                            const Box* __restrict__ boxes, Box (&b)[kPer], bool (&in)[kPer]) {
-  uint32_t id[kPer];
-#pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    const uint32_t l = r.lo + threadIdx.x + (uint32_t)u * kCT;
-    in[u] = l < r.hi;
-    id[u] = in[u] ? indices[l] : 0u;
-  }
-#pragma unroll
-  for (int u = 0; u < kPer; ++u)
-    if (in[u]) b[u] = rk::load_box(boxes + id[u]);
 }
 
 __device__ __forceinline__ float center_axis(const Box& b, int a) {  // 0.5f * (min + max), :292
   return a == 0 ? (b.mn.x + b.mx.x) * 0.5f : (a == 1 ? (b.mn.y + b.mx.y) * 0.5f : (b.mn.z + b.mx.z) * 0.5f);
-}
-
-__global__ __launch_bounds__(kCT) void k_sah_bounds(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                    uint32_t par, const uint32_t* __restrict__ chunk_base,
-                                                    const uint32_t* __restrict__ chunk_item,
-                                                    const uint32_t* __restrict__ indices, const Box* __restrict__ boxes,
-                                                    int* __restrict__ acc) {
-  const ChunkRange r = chunk_range(items, ctl, par, chunk_base, chunk_item, blockIdx.x);
-  if (!r.ok) return;
-  int* a = acc + (size_t)r.slot * kAccWords;
-  if (r.first) {  // the item's first chunk resets its bins for k_sah_bins
-    int* bins = a + kBinBase;
-    for (int w = threadIdx.x; w < kBinSlots * kBinWords; w += kCT) {
-      int k = (w % kBinWords) % 7;
-      bins[w] = k == 0 ? 0 : (k < 4 ? f2o(RK_HUGE) : f2o(-RK_HUGE));
-    }
-  }
-  // ordered ints, as the atomics compare them
-  int mn[3] = {f2o(RK_HUGE), f2o(RK_HUGE), f2o(RK_HUGE)}, mx[3] = {f2o(-RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE)};
-  Box bb[kPer];
-  bool in[kPer];
-  chunk_boxes(r, indices, boxes, bb, in);
-#pragma unroll
-  for (int u = 0; u < kPer; ++u) {
-    if (!in[u]) continue;
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      const int c = f2o(center_axis(bb[u], q));
-      mn[q] = min(mn[q], c);
-      mx[q] = max(mx[q], c);
-    }
-  }
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1)
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      mn[q] = min(mn[q], __shfl_xor(mn[q], off, 64));
-      mx[q] = max(mx[q], __shfl_xor(mx[q], off, 64));
-    }
-  // one set of atomics per workgroup, into one of the item's bound slots
-  __shared__ int s_red[kCT / 64][6];
-  const uint32_t w = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0)
-    for (int q = 0; q < 3; ++q) { s_red[w][q] = mn[q]; s_red[w][3 + q] = mx[q]; }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    int* bs = a + 6 * (blockIdx.x % kBoundSlots);
-    for (int q = 0; q < 3; ++q) {
-      int lo = s_red[0][q], hi = s_red[0][3 + q];
-      for (int v = 1; v < kCT / 64; ++v) { lo = min(lo, s_red[v][q]); hi = max(hi, s_red[v][3 + q]); }
-      atomicMin(bs + q, lo);
-      atomicMax(bs + 3 + q, hi);
-    }
-  }
-}
-
-// An item's centroid bounds from its bound slots.
-__device__ __forceinline__ void acc_bounds(const int* __restrict__ a, int (&cb)[6]) {
-  for (int q = 0; q < 3; ++q) { cb[q] = a[q]; cb[3 + q] = a[3 + q]; }
-  for (int v = 1; v < kBoundSlots; ++v)
-    for (int q = 0; q < 3; ++q) { cb[q] = min(cb[q], a[6 * v + q]); cb[3 + q] = max(cb[3 + q], a[6 * v + 3 + q]); }
 }
 
 // Axis and bin scale of an item from its centroid bounds (:302-342).
@@ -267,79 +278,142 @@ __device__ __forceinline__ void item_axis(const int (&a)[6], int& axis, float& s
 }
 
 __device__ __forceinline__ int bin_of(const Box& b, int axis, float scale, float bmin0) {  // :375-385
-  int m = rk::f2i_sat((center_axis(b, axis) - bmin0) * scale);
-  if (m < 0) m = 0;
-  else if (m >= kBins - 1) m = kBins - 1;
-  return m;
+  // truncated and clamped to [0, kBins - 1], NaN to 0 (fmaxf takes the number)
+  return (int)fminf(fmaxf((center_axis(b, axis) - bmin0) * scale, 0.f), (float)(kBins - 1));
 }
 
-__global__ __launch_bounds__(kCT) void k_sah_bins(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                  uint32_t par, const uint32_t* __restrict__ chunk_base,
-                                                  const uint32_t* __restrict__ chunk_item,
-                                                  const uint32_t* __restrict__ indices, const Box* __restrict__ boxes,
-                                                  int* __restrict__ acc) {
-  __shared__ int s_bin[kBins * 7];
-  const ChunkRange r = chunk_range(items, ctl, par, chunk_base, chunk_item, blockIdx.x);
-  if (!r.ok) return;
-  for (int w = threadIdx.x; w < kBins * 7; w += kCT) {
-    int k = w % 7;
-    s_bin[w] = k == 0 ? 0 : (k < 4 ? f2o(RK_HUGE) : f2o(-RK_HUGE));
-  }
+// A workgroup's centroid bounds into one of an item's copies.
+__device__ __forceinline__ void add_bounds(int (&b)[6], int* __restrict__ bounds) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      b[q] = min(b[q], __shfl_xor(b[q], off, 64));
+      b[3 + q] = max(b[3 + q], __shfl_xor(b[3 + q], off, 64));
+    }
+  __shared__ int s_red[16][6];
+  if ((threadIdx.x & 63) == 0)
+    for (int q = 0; q < 6; ++q) s_red[threadIdx.x >> 6][q] = b[q];
   __syncthreads();
-  int* a = acc + (size_t)r.slot * kAccWords;
+  if (threadIdx.x < 6) {
+    const int q = (int)threadIdx.x;
+    int v = s_red[0][q];
+    for (uint32_t w = 1; w < blockDim.x / 64; ++w) v = q < 3 ? min(v, s_red[w][q]) : max(v, s_red[w][q]);
+    int* g = bounds + 6 * (blockIdx.x % kBoundSlots) + q;
+    if (q < 3) atomicMin(g, v);
+    else atomicMax(g, v);
+  }
+}
+
+// Centroid bounds of the starting items (Hybrid; the root's come from
+// k_boxes_root); those of the others come from k_sah_scatter.
+__global__ __launch_bounds__(kCT) void k_sah_bounds(Sah s) {
+  const ChunkRange r = chunk_range(s, 0);
+  if (!r.ok) return;
+  int b[6] = {f2o(RK_HUGE), f2o(RK_HUGE), f2o(RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE)};
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const uint32_t l = r.lo + threadIdx.x + (uint32_t)u * kCT;
+    if (l >= r.hi) continue;
+    const Box x = rk::load_box(s.boxes + s.ids0[l]);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int c = f2o(center_axis(x, q));
+      b[q] = min(b[q], c);
+      b[3 + q] = max(b[3 + q], c);
+    }
+  }
+  add_bounds(b, s.bnd1 + (size_t)r.it.bref * kBoundWords);
+}
+
+// An item's centroid bounds from their copies.
+__device__ __forceinline__ void item_bounds(const int* __restrict__ a, int (&cb)[6]) {
+  for (int q = 0; q < 6; ++q) cb[q] = a[q];
+  for (int v = 1; v < kBoundSlots; ++v)
+    for (int q = 0; q < 3; ++q) {
+      cb[q] = min(cb[q], a[6 * v + q]);
+      cb[3 + q] = max(cb[3 + q], a[6 * v + 3 + q]);
+    }
+}
+
+// The boxes go into kBinCopies copies of the bins by lane: neighbours in space
+// are neighbours in the list and fall into the same bin, and atomics on one
+// address take turns.
+constexpr int kBinCopies = 8, kBinStride = kBinWords + 8;
+__global__ __launch_bounds__(kCT) void k_sah_bins(Sah s, uint32_t par) {
+  __shared__ int s_bin[kBinCopies][kBinStride];
+  __shared__ uint32_t s_sum[kBins];
+  // the next level's counters, which k_sah_split adds to
+  if (blockIdx.x == 0 && threadIdx.x < 2) s.ctl[kCtlBig(par ^ 1u) + threadIdx.x] = 0u;
+  const ChunkRange r = chunk_range(s, par);
+  if (!r.ok) return;
+  uint32_t id[kPer];
+  const uint32_t* ids = ids_of(s, par);
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const uint32_t l = r.lo + threadIdx.x + (uint32_t)u * kCT;
+    id[u] = l < r.hi ? ids[l] : 0u;
+  }
+  for (int w = threadIdx.x; w < kBinCopies * kBinStride; w += kCT) {
+    const int k = (w % kBinStride) % 7;
+    (&s_bin[0][0])[w] = k == 0 ? 0 : (k < 4 ? f2o(RK_HUGE) : f2o(-RK_HUGE));
+  }
+  Box bb[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u)
+    if (r.lo + threadIdx.x + (uint32_t)u * kCT < r.hi) bb[u] = rk::load_box(s.boxes + id[u]);
   int cb[6];
-  acc_bounds(a, cb);
+  item_bounds(bounds_of(s, par ^ 1u) + (size_t)r.it.bref * kBoundWords, cb);
   int axis;
   float scale, bmin0;
   item_axis(cb, axis, scale, bmin0);
-  Box bb[kPer];
-  bool in[kPer];
-  chunk_boxes(r, indices, boxes, bb, in);
+  __syncthreads();
 #pragma unroll
   for (int u = 0; u < kPer; ++u) {
-    if (!in[u]) continue;
+    const uint32_t l = r.lo + threadIdx.x + (uint32_t)u * kCT;
+    if (l >= r.hi) continue;
     const Box& b = bb[u];
-    int m = bin_of(b, axis, scale, bmin0);
-    int* s = s_bin + m * 7;
-    atomicAdd(s, 1);
-    atomicMin(s + 1, f2o(b.mn.x)); atomicMin(s + 2, f2o(b.mn.y)); atomicMin(s + 3, f2o(b.mn.z));
-    atomicMax(s + 4, f2o(b.mx.x)); atomicMax(s + 5, f2o(b.mx.y)); atomicMax(s + 6, f2o(b.mx.z));
+    const int m = bin_of(b, axis, scale, bmin0);
+    s.bin[l] = (uint8_t)m;
+    int* p = s_bin[threadIdx.x % kBinCopies] + m * 7;
+    atomicAdd(p, 1);
+    atomicMin(p + 1, f2o(b.mn.x)); atomicMin(p + 2, f2o(b.mn.y)); atomicMin(p + 3, f2o(b.mn.z));
+    atomicMax(p + 4, f2o(b.mx.x)); atomicMax(p + 5, f2o(b.mx.y)); atomicMax(p + 6, f2o(b.mx.z));
   }
   __syncthreads();
-  int* slot_bins = a + kBinBase + (blockIdx.x % kBinSlots) * kBinWords;
-  for (int w = threadIdx.x; w < kBins * 7; w += kCT) {
-    int k = w % 7, v = s_bin[w];
-    int* g = slot_bins + w;
-    if (k == 0) { if (v) atomicAdd(g, v); }
-    else if (k < 4) { if (v != f2o(RK_HUGE)) atomicMin(g, v); }
-    else { if (v != f2o(-RK_HUGE)) atomicMax(g, v); }
+  int* g = s.acc + (size_t)r.item * kAccWords + (blockIdx.x % kBinSlots) * kBinWords;
+  for (int w = threadIdx.x; w < kBinWords; w += kCT) {
+    const int k = w % 7;
+    int v = s_bin[0][w];
+#pragma unroll
+    for (int c = 1; c < kBinCopies; ++c) {
+      const int x = s_bin[c][w];
+      v = k == 0 ? v + x : (k < 4 ? min(v, x) : max(v, x));
+    }
+    if (k == 0) {
+      s_sum[w / 7] = (uint32_t)v;
+      if (v) atomicAdd(g + w, v);
+    } else if (k < 4) {
+      if (v != f2o(RK_HUGE)) atomicMin(g + w, v);
+    } else if (v != f2o(-RK_HUGE)) {
+      atomicMax(g + w, v);
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x < kBins) {
+    uint32_t c = s_sum[threadIdx.x];
+#pragma unroll
+    for (int off = 1; off < kBins; off <<= 1) {
+      const uint32_t y = __shfl_up(c, off, 32);
+      if (threadIdx.x >= (uint32_t)off) c += y;
+    }
+    s.cum[(size_t)threadIdx.x * s.chunks_cap + blockIdx.x] = (uint16_t)c;
   }
 }
-
-__device__ __forceinline__ Node make_node(uint32_t axis, uint32_t child, const float* bmin, const float* bmax) {
-  Node n;
-  n.w0 = (axis & 3u) << 1;
-  n.w1 = child;
-  for (int a = 0; a < 3; ++a) { n.bmin[a] = bmin[a]; n.bmax[a] = bmax[a]; }
-  return n;
-}
-__device__ __forceinline__ Node make_leaf(uint32_t first, uint32_t count, const float* bmin, const float* bmax) {
-  Node n;
-  n.w0 = 1u | (count << 1);
-  n.w1 = first;
-  for (int a = 0; a < 3; ++a) { n.bmin[a] = bmin[a]; n.bmax[a] = bmax[a]; }
-  return n;
-}
-
-// Items per workgroup of k_sah_decide (two per wave, one lane per bin) and
-// per workgroup of k_sah_emit.
-constexpr uint32_t kDecideItems = 8;
-constexpr uint32_t kEmitItems = kEmitGroup;
-static_assert(kEmitItems % kDecideItems == 0, "a decide workgroup's items lie in one emit group");
 
 // The reference's sweep over one item's bins (:424-474) and children boxes
 // (:501-530), one lane per bin: lane k of each 32-lane half holds bin k
-// (count, ordered-int box) of its half's item, and every lane of the wave
+// (count, ordered-int box) of its half's item, and every lane of the half
 // calls this. The left sweep's running box and count after bin k are the
 // inclusive prefix at lane k, and the right sweep's after bin k the inclusive
 // suffix; min, max and integer sums give the same values in any order, and
@@ -354,47 +428,71 @@ struct Sweep {
   float child[12];  // left min xyz, left max xyz, right min xyz, right max xyz
 };
 
+// A step of a prefix over 32 lanes: what the lanes' neighbours hold, 'old' where
+// there is none. row_shr 1, 2, 4, 8 within 16 lanes, then row_bcast 15 across.
+template <int kStep>
+__device__ __forceinline__ int lane_step(int old, int x) {
+  if constexpr (kStep < 4) return __builtin_amdgcn_update_dpp(old, x, 0x110 | 1 << kStep, 0xF, 0xF, false);
+  else return __builtin_amdgcn_update_dpp(old, x, 0x142, 0xA, 0xF, false);
+}
+template <int kStep>
+__device__ __forceinline__ float lane_step(float old, float x) {
+  return __int_as_float(lane_step<kStep>(__float_as_int(old), __float_as_int(x)));
+}
+template <int kStep = 0>
+__device__ __forceinline__ void prefix_box(int& n, float (&mn)[3], float (&mx)[3]) {
+  n += lane_step<kStep>(0, n);
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    mn[q] = rk::fmn(mn[q], lane_step<kStep>(mn[q], mn[q]));
+    mx[q] = rk::fmx(mx[q], lane_step<kStep>(mx[q], mx[q]));
+  }
+  if constexpr (kStep < 4) prefix_box<kStep + 1>(n, mn, mx);
+}
+// The value of each half's last lane.
+__device__ __forceinline__ int half_last(int x) {
+  const int a = __builtin_amdgcn_readlane(x, 31), b = __builtin_amdgcn_readlane(x, 63);
+  return (threadIdx.x & 32u) ? b : a;
+}
+// Smallest over each half-wave, in every lane.
+template <int kStep = 0>
+__device__ __forceinline__ int half_min(int x) {
+  x = min(x, lane_step<kStep>(0x7FFFFFFF, x));
+  if constexpr (kStep < 4) return half_min<kStep + 1>(x);
+  else return half_last(x);
+}
+
 __device__ __forceinline__ Sweep sweep_bins(int cnt, const float (&bmn)[3], const float (&bmx)[3], float pa,
                                             uint32_t k) {
-  int lc = cnt, rc = cnt;
+  // the right sweep runs over the bins in reverse: bin 31 - k in lane k
+  const int rev = 31 - (int)k;
+  int lc = cnt, rc = __shfl(cnt, rev, 32);
   float lmn[3], lmx[3], rmn[3], rmx[3];
-  for (int q = 0; q < 3; ++q) { lmn[q] = rmn[q] = bmn[q]; lmx[q] = rmx[q] = bmx[q]; }
-#pragma unroll
-  for (int off = 1; off < 32; off <<= 1) {
-    const int ylc = __shfl_up(lc, off, 32), yrc = __shfl_down(rc, off, 32);
-    float ylmn[3], ylmx[3], yrmn[3], yrmx[3];
-    for (int q = 0; q < 3; ++q) {
-      ylmn[q] = __shfl_up(lmn[q], off, 32); ylmx[q] = __shfl_up(lmx[q], off, 32);
-      yrmn[q] = __shfl_down(rmn[q], off, 32); yrmx[q] = __shfl_down(rmx[q], off, 32);
-    }
-    if (k >= (uint32_t)off) {
-      lc += ylc;
-      for (int q = 0; q < 3; ++q) { lmn[q] = rk::fmn(lmn[q], ylmn[q]); lmx[q] = rk::fmx(lmx[q], ylmx[q]); }
-    }
-    if (k + off < 32) {
-      rc += yrc;
-      for (int q = 0; q < 3; ++q) { rmn[q] = rk::fmn(rmn[q], yrmn[q]); rmx[q] = rk::fmx(rmx[q], yrmx[q]); }
-    }
+  for (int q = 0; q < 3; ++q) {
+    lmn[q] = bmn[q];
+    lmx[q] = bmx[q];
+    rmn[q] = __shfl(bmn[q], rev, 32);
+    rmx[q] = __shfl(bmx[q], rev, 32);
   }
+  prefix_box(lc, lmn, lmx);
+  prefix_box(rc, rmn, rmx);
   // cost of the split after bin k (k <= 30): prefix at k, suffix at k + 1
   const float rarea = 0.f + box_area(rmn[0], rmn[1], rmn[2], rmx[0], rmx[1], rmx[2]);
-  const float rarea_next = __shfl_down(rarea, 1, 32);
-  const int rc_next = __shfl_down(rc, 1, 32);
+  const int next = (30 - (int)k) & 31;
+  const float rarea_next = __shfl(rarea, next, 32);
+  const int rc_next = __shfl(rc, next, 32);
   const float larea = 0.f + box_area(lmn[0], lmn[1], lmn[2], lmx[0], lmx[1], lmx[2]);
   const int lcount = 0 + lc;
   const float T = 1.0f * 2.f + 0.125f * ((larea / pa) * (float)lcount + (rarea_next / pa) * (float)(0 + rc_next));
-  float bt = T;
-  int bj = (k < 31 && T < RK_HUGE) ? (int)k : -1;  // NaN and +huge never win a strict <
-#pragma unroll
-  for (int off = 16; off > 0; off >>= 1) {
-    const float ot = __shfl_xor(bt, off, 32);
-    const int oj = __shfl_xor(bj, off, 32);
-    if (oj >= 0 && (bj < 0 || ot < bt || (ot == bt && oj > bj))) { bt = ot; bj = oj; }
-  }
+  const bool valid = k < 31 && T < RK_HUGE;  // NaN and +huge never win a strict <
+  // the smallest as an ordered int, then the largest index among the lanes that hold it as a number
+  const float bt = o2f(half_min(valid ? f2o(T) : 0x7FFFFFFF));
+  const uint32_t best = (uint32_t)(__ballot(valid && T == bt) >> (threadIdx.x & 32u));
+  const int bj = best ? 31 - (int)__clz((int)best) : -1;
   Sweep r;
   r.m_min = bj;
   r.T_min = bj >= 0 ? bt : RK_HUGE;
-  const int src_l = bj >= 0 ? bj : 0, src_r = bj >= 0 ? bj + 1 : 0;
+  const int src_l = bj >= 0 ? bj : 0, src_r = bj >= 0 ? 30 - bj : 0;
   for (int q = 0; q < 3; ++q) {
     r.child[q] = __shfl(lmn[q], src_l, 32);
     r.child[3 + q] = __shfl(lmx[q], src_l, 32);
@@ -405,67 +503,57 @@ __device__ __forceinline__ Sweep sweep_bins(int cnt, const float (&bmn)[3], cons
   return r;
 }
 
-// The leaf test (:479-496) on a sweep's result; an item with no finite cut
-// that is too large for a leaf becomes one anyway and is flagged in the flags word
-// (when ctl is given).
-__device__ __forceinline__ Decision make_decision(uint32_t size, int axis, float scale, float bmin0, const Sweep& sw,
-                                                  uint32_t* __restrict__ ctl) {
-  Decision d;
-  d.axis = axis; d.scale = scale; d.bmin0 = bmin0; d.m_min = -1; d.lcount = 0;
-  d.pad[0] = d.pad[1] = d.pad[2] = 0;
-  for (int q = 0; q < 12; ++q) d.child[q] = 0.f;
-  bool leaf = size < kLeafMax && sw.T_min > (float)(size + 1) * 0.125f;
-  if (!leaf && sw.m_min < 0) {
-    leaf = true;
-    if (ctl) atomicOr(ctl + kCtlFlags, (uint32_t)RK_FLAG_SAH_NO_CUT);
-  }
-  if (!leaf) {
-    d.m_min = sw.m_min;
-    d.lcount = (uint32_t)sw.lcount;
-    for (int q = 0; q < 12; ++q) d.child[q] = sw.child[q];
-  }
-  return d;
+// The leaf test (:479-496) on a sweep's result: the bin of the split, or -1. An
+// item with no finite cut that is too large for a leaf becomes one anyway and is
+// flagged (by the lane that says so).
+__device__ __forceinline__ int split_bin(const Sah& s, uint32_t size, const Sweep& sw, bool flags) {
+  if (size < kLeafMax && sw.T_min > (float)(size + 1) * 0.125f) return -1;
+  // a split with an empty side never has a finite cost; the build ends for this reason
+  const bool cut = sw.m_min >= 0 && sw.lcount > 0 && (uint32_t)sw.lcount < size;
+  if (!cut && flags) atomicOr(s.ctl + kCtlFlags, (uint32_t)RK_FLAG_SAH_NO_CUT);
+  return cut ? sw.m_min : -1;
 }
 
-__device__ __forceinline__ Decision leaf_decision() {
-  Decision d;
-  d.axis = 0; d.scale = 0.f; d.bmin0 = 0.f; d.m_min = -1; d.lcount = 0;
-  d.pad[0] = d.pad[1] = d.pad[2] = 0;
-  for (int q = 0; q < 12; ++q) d.child[q] = 0.f;
-  return d;
+// The child of this lane (0: left, 1: right) of a half-wave's item.
+__device__ __forceinline__ Rec child_rec(const Sweep& sw, uint32_t k, uint32_t lo, uint32_t size) {
+  Rec r;
+  for (int q = 0; q < 3; ++q) {
+    r.bmin[q] = k == 0 ? sw.child[q] : sw.child[6 + q];
+    r.bmax[q] = k == 0 ? sw.child[3 + q] : sw.child[9 + q];
+  }
+  r.lo = k == 0 ? lo : lo + (uint32_t)sw.lcount;
+  r.cnt = k == 0 ? (uint32_t)sw.lcount : size - (uint32_t)sw.lcount;
+  return r;
 }
 
-// Items of more than kChunk faces, decided from their chunks' accumulators;
-// k_sah_small decides the rest. One 32-lane half-wave per item.
-__global__ __launch_bounds__(256) void k_sah_decide(const Item* __restrict__ items, uint32_t* __restrict__ ctl,
-                                                    uint32_t par, const int* __restrict__ acc,
-                                                    Decision* __restrict__ dec,
-                                                    uint32_t* __restrict__ group_internal) {
-  __shared__ uint32_t s_internal;
-  const uint32_t m = ctl[kCtlLevel(par) + kLvM];
-  const uint32_t k = threadIdx.x & 31;
-  const uint32_t i = blockIdx.x * kDecideItems + (threadIdx.x >> 5);
-  if (threadIdx.x == 0) s_internal = 0;
+// The decision on the level's big items, their children, and the next level's
+// big items and chunks, in any order: one half-wave per item.
+constexpr uint32_t kSplitItems = 8;
+__global__ __launch_bounds__(32 * kSplitItems) void k_sah_split(Sah s, uint32_t par, uint32_t level) {
+  // children: of more than kChunk faces, their chunks, the others by class; internal items
+  __shared__ uint32_t s_cnt[3 + kClasses], s_base[3 + kClasses];
+  const uint32_t m = s.ctl[kCtlBig(par)];
+  if (blockIdx.x * kSplitItems >= m) return;
+  const uint32_t t = threadIdx.x, k = t & 31u, i = blockIdx.x * kSplitItems + (t >> 5);
+  if (t < 3 + kClasses) s_cnt[t] = 0u;
   __syncthreads();
-  Item it;
+  const bool live = i < m;
+  BigItem it;
   uint32_t size = 0;
-  if (i < m) {
-    it = items[i];
-    size = it.hi - it.lo;
-  }
-  const bool split_test = i < m && size > kChunk;
   int axis = 0, cnt = 0;
-  float scale = 0.f, bmin0 = 0.f, pa = 0.f;
-  float bmn[3] = {RK_HUGE, RK_HUGE, RK_HUGE}, bmx[3] = {-RK_HUGE, -RK_HUGE, -RK_HUGE};
-  if (split_test) {
-    const int* a = acc + (size_t)it.pad * kAccWords;
-    int cb[6];
-    acc_bounds(a, cb);
+  float pa = 0.f, bmn[3] = {RK_HUGE, RK_HUGE, RK_HUGE}, bmx[3] = {-RK_HUGE, -RK_HUGE, -RK_HUGE};
+  if (live) {
+    it = big_of(s, par)[i];
+    size = it.hi - it.lo;
+    int* g = bounds_of(s, par ^ 1u) + (size_t)it.bref * kBoundWords;
+    int* a = s.acc + (size_t)i * kAccWords;
+    int cb[6], bi[7];
+    item_bounds(g, cb);
+    float scale, bmin0;
     item_axis(cb, axis, scale, bmin0);
-    int bi[7];
-    for (int q = 0; q < 7; ++q) bi[q] = a[kBinBase + k * 7 + q];
+    for (int q = 0; q < 7; ++q) bi[q] = a[k * 7 + q];
     for (int v = 1; v < kBinSlots; ++v) {
-      const int* b = a + kBinBase + v * kBinWords + k * 7;
+      const int* b = a + v * kBinWords + k * 7;
       bi[0] += b[0];
       for (int q = 1; q < 4; ++q) bi[q] = min(bi[q], b[q]);
       for (int q = 4; q < 7; ++q) bi[q] = max(bi[q], b[q]);
@@ -473,393 +561,662 @@ __global__ __launch_bounds__(256) void k_sah_decide(const Item* __restrict__ ite
     cnt = bi[0];
     for (int q = 0; q < 3; ++q) { bmn[q] = o2f(bi[1 + q]); bmx[q] = o2f(bi[4 + q]); }
     pa = box_area(it.bmin[0], it.bmin[1], it.bmin[2], it.bmax[0], it.bmax[1], it.bmax[2]);
+    // empty again for the levels after this one
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int w = (int)k; w < kAccWords; w += 32) a[w] = w % 7 == 0 ? 0 : (w % 7 < 4 ? f2o(RK_HUGE) : f2o(-RK_HUGE));
+    for (int w = (int)k; w < kBoundWords; w += 32) g[w] = w % 6 < 3 ? f2o(RK_HUGE) : f2o(-RK_HUGE);
   }
   const Sweep sw = sweep_bins(cnt, bmn, bmx, pa, k);
-  if (k == 0 && split_test) {
-    const Decision d = make_decision(size, axis, scale, bmin0, sw, ctl);
-    if (d.m_min >= 0) atomicAdd(&s_internal, 1u);
-    dec[i] = d;
+  int m_min = -1;
+  Rec child;
+  uint32_t cls = 0, at = 0, nch = 0, chunk_at = 0;
+  if (live) {
+    m_min = split_bin(s, size, sw, k == 0);
+    if (m_min >= 0 && k < 2) {
+      child = child_rec(sw, k, it.lo, size);
+      if (child.cnt > kChunk) {
+        nch = (child.cnt + kChunk - 1) / kChunk;
+        at = atomicAdd(&s_cnt[0], 1u);
+        chunk_at = atomicAdd(&s_cnt[1], nch);
+      } else {
+        cls = class_of(child.cnt);
+        at = atomicAdd(&s_cnt[3 + cls], 1u);
+      }
+      if (k == 0) {
+        atomicAdd(&s_cnt[2], 1u);
+        if (level >= kLevelMax) s.ctl[kCtlDeep] = 1u;
+      }
+    }
   }
   __syncthreads();
-  // kEmitItems is a multiple of kDecideItems: the workgroup's items share a group
-  if (threadIdx.x == 0 && s_internal)
-    atomicAdd(group_internal + blockIdx.x * kDecideItems / kEmitItems, s_internal);
-}
-
-// Items of kLeafMin + 1 to kChunk faces, one wave each, start to end: centroid
-// bounds, bins, the sweep and the stable partition, with the item's face ids
-// held in LDS so that the partition writes back in place. Every step reduces
-// or scans the same values as the chunk kernels, so the decision is the same.
-// Items of at most kLeafMin faces are leaves (:239-255).
-constexpr uint32_t kSmallWaves = 4;
-constexpr int kSmallPer = 4;  // faces per lane in flight
-static_assert(kEmitItems % kSmallWaves == 0, "a small-item workgroup's items lie in one emit group");
-__global__ __launch_bounds__(64 * kSmallWaves) void k_sah_small(const Item* __restrict__ items,
-                                                                uint32_t* __restrict__ ctl, uint32_t par,
-                                                                uint32_t* __restrict__ indices,
-                                                                const Box* __restrict__ boxes,
-                                                                Decision* __restrict__ dec,
-                                                                uint32_t* __restrict__ group_internal) {
-  __shared__ uint32_t s_ids[kSmallWaves][kChunk];
-  __shared__ uint8_t s_binof[kSmallWaves][kChunk];
-  __shared__ int s_bins[kSmallWaves][kBins * 7];
-  __shared__ uint32_t s_internal;
-  const uint32_t m = ctl[kCtlLevel(par) + kLvM];
-  const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t i = blockIdx.x * kSmallWaves + w;
-  if (threadIdx.x == 0) s_internal = 0;
-  __syncthreads();
-  Item it;
-  uint32_t size = 0;
-  if (i < m) {
-    it = items[i];
-    size = it.hi - it.lo;
-  }
-  if (i < m && size <= kLeafMin) {  // wave-uniform
-    if (lane == 0) dec[i] = leaf_decision();
-  } else if (size > kLeafMin && size <= kChunk) {  // wave-uniform
-    uint32_t* ids = s_ids[w];
-    uint8_t* binof = s_binof[w];
-    int* bins = s_bins[w];
-    // centroid bounds, ordered ints as in k_sah_bounds' atomics. Faces go
-    // kSmallPer per lane at a time, every gather in flight at once; the first
-    // 64 * kSmallPer boxes stay in registers for the binning pass.
-    int cmn[3] = {f2o(RK_HUGE), f2o(RK_HUGE), f2o(RK_HUGE)}, cmx[3] = {f2o(-RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE)};
-    Box keep[kSmallPer];
-    for (uint32_t l0 = 0; l0 < size; l0 += 64 * kSmallPer) {
-      uint32_t id[kSmallPer];
-      Box b[kSmallPer];
-#pragma unroll
-      for (int u = 0; u < kSmallPer; ++u) {
-        const uint32_t l = l0 + lane + 64u * u;
-        id[u] = l < size ? indices[it.lo + l] : 0u;
-      }
-#pragma unroll
-      for (int u = 0; u < kSmallPer; ++u)
-        if (l0 + lane + 64u * u < size) b[u] = rk::load_box(boxes + id[u]);
-#pragma unroll
-      for (int u = 0; u < kSmallPer; ++u) {
-        const uint32_t l = l0 + lane + 64u * u;
-        if (l >= size) continue;
-        ids[l] = id[u];
-        if (l0 == 0) keep[u] = b[u];
-        for (int a = 0; a < 3; ++a) {
-          const int c = f2o(center_axis(b[u], a));
-          cmn[a] = min(cmn[a], c);
-          cmx[a] = max(cmx[a], c);
-        }
-      }
-    }
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-      for (int a = 0; a < 3; ++a) {
-        cmn[a] = min(cmn[a], __shfl_xor(cmn[a], off, 64));
-        cmx[a] = max(cmx[a], __shfl_xor(cmx[a], off, 64));
-      }
-    int cb[6] = {cmn[0], cmn[1], cmn[2], cmx[0], cmx[1], cmx[2]};
-    int axis;
-    float scale, bmin0;
-    item_axis(cb, axis, scale, bmin0);
-    for (int q = lane; q < kBins * 7; q += 64) {
-      const int kq = q % 7;
-      bins[q] = kq == 0 ? 0 : (kq < 4 ? f2o(RK_HUGE) : f2o(-RK_HUGE));
-    }
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    for (uint32_t l0 = 0; l0 < size; l0 += 64 * kSmallPer) {
-      Box b[kSmallPer];
-#pragma unroll
-      for (int u = 0; u < kSmallPer; ++u) {
-        const uint32_t l = l0 + lane + 64u * u;
-        if (l < size) b[u] = l0 == 0 ? keep[u] : rk::load_box(boxes + ids[l]);
-      }
-#pragma unroll
-      for (int u = 0; u < kSmallPer; ++u) {
-        const uint32_t l = l0 + lane + 64u * u;
-        if (l >= size) continue;
-        const int bn = bin_of(b[u], axis, scale, bmin0);
-        binof[l] = (uint8_t)bn;
-        int* sb = bins + bn * 7;
-        atomicAdd(sb, 1);
-        atomicMin(sb + 1, f2o(b[u].mn.x)); atomicMin(sb + 2, f2o(b[u].mn.y)); atomicMin(sb + 3, f2o(b[u].mn.z));
-        atomicMax(sb + 4, f2o(b[u].mx.x)); atomicMax(sb + 5, f2o(b[u].mx.y)); atomicMax(sb + 6, f2o(b[u].mx.z));
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    const uint32_t k = lane & 31;
-    const int* bk = bins + k * 7;
-    const int cnt = bk[0];
-    float bmn[3], bmx[3];
-    for (int q = 0; q < 3; ++q) { bmn[q] = o2f(bk[1 + q]); bmx[q] = o2f(bk[4 + q]); }
-    const float pa = box_area(it.bmin[0], it.bmin[1], it.bmin[2], it.bmax[0], it.bmax[1], it.bmax[2]);
-    const Sweep sw = sweep_bins(cnt, bmn, bmx, pa, k);
-    const Decision d = make_decision(size, axis, scale, bmin0, sw, lane == 0 ? ctl : nullptr);
-    if (d.m_min >= 0) {
-      // stable partition of the item's ids, bin <= m_min first (:534-610)
-      uint32_t left_before = 0, right_before = 0;
-      for (uint32_t l0 = 0; l0 < size; l0 += 64) {
-        const uint32_t l = l0 + lane;
-        uint32_t id = 0;
-        bool is_left = false;
-        if (l < size) {
-          id = ids[l];
-          is_left = (int)binof[l] <= d.m_min;
-        }
-        const uint64_t lm = __ballot(l < size && is_left), rm = __ballot(l < size && !is_left);
-        const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-        if (l < size) {
-          const uint32_t out = is_left ? it.lo + left_before + (uint32_t)__popcll(lm & below)
-                                       : it.lo + d.lcount + right_before + (uint32_t)__popcll(rm & below);
-          indices[out] = id;
-        }
-        left_before += (uint32_t)__popcll(lm);
-        right_before += (uint32_t)__popcll(rm);
-      }
-      if (lane == 0) atomicAdd(&s_internal, 1u);
-    }
-    if (lane == 0) dec[i] = d;
+  if (t < 3 + kClasses && s_cnt[t]) {
+    const uint32_t to = t < 2 ? kCtlBig(par ^ 1u) + t : (t == 2 ? kCtlHist + level : kCtlRoots + t - 3);
+    s_base[t] = atomicAdd(s.ctl + to, s_cnt[t]);
   }
   __syncthreads();
-  // kEmitItems is a multiple of kSmallWaves: the workgroup's items share a group
-  if (threadIdx.x == 0 && s_internal)
-    atomicAdd(group_internal + blockIdx.x * kSmallWaves / kEmitItems, s_internal);
-}
-
-// Node records and the next level's items, in item order: the k-th internal
-// item of the level takes children (count + 2k, count + 2k + 1). Workgroup g
-// handles items [g, g + 1) * kEmitItems and starts after the internal items
-// counted in the groups before it. The grid may hold more workgroups than the
-// level has groups; the one with the last group (workgroup 0 when the level
-// is empty) writes the next level's item and node counts.
-__global__ __launch_bounds__(1024) void k_sah_emit(const Item* __restrict__ items, uint32_t* __restrict__ ctl,
-                                                   uint32_t par, const Decision* __restrict__ dec,
-                                                   const uint32_t* __restrict__ group_internal,
-                                                   Item* __restrict__ next, Node* __restrict__ nodes,
-                                                   uint32_t nodes_cap) {
-  __shared__ uint32_t s_tmp[16];
-  const uint32_t m = ctl[kCtlLevel(par) + kLvM];
-  const uint32_t count0 = ctl[kCtlLevel(par) + kLvCount];
-  const uint32_t g = blockIdx.x;
-  uint32_t before = 0, before_total;
-  for (uint32_t h = threadIdx.x; h < g; h += 1024) before += group_internal[h];
-  block_excl_scan(before, s_tmp, &before_total, 1024);
-  const uint32_t i = g * kEmitItems + threadIdx.x;
-  uint32_t internal = 0;
-  Item it;
-  Decision d;
-  if (i < m) {
-    it = items[i];
-    d = dec[i];
-    internal = d.m_min >= 0 ? 1u : 0u;
+  if (!live) return;
+  if (k == 0) {
+    BigDec d;
+    d.m_min = m_min;
+    d.lcount = (uint32_t)sw.lcount;
+    s.dec[i] = d;
+    s.link[it.rec] = m_min >= 0 ? (it.lo + (uint32_t)sw.lcount) | (uint32_t)axis << 30 : kLeaf;
   }
-  uint32_t total;
-  const uint32_t ex = block_excl_scan(internal, s_tmp, &total, 1024);
-  // children of more than kChunk faces, for the next level's launches
-  uint32_t big = 0, big_total;
-  if (internal) big = (d.lcount > kChunk ? 1u : 0u) + (it.hi - it.lo - d.lcount > kChunk ? 1u : 0u);
-  block_excl_scan(big, s_tmp, &big_total, 1024);
-  uint32_t* nx = ctl + kCtlLevel(par ^ 1u);
-  if (threadIdx.x == 0 && big_total) atomicAdd(nx + kLvBig, big_total);
-  if (i < m) {
-    if (internal) {
-      const uint32_t k = before_total + ex;
-      const uint32_t c = count0 + 2 * k;
-      if (it.node < nodes_cap) nodes[it.node] = make_node((uint32_t)d.axis, c, it.bmin, it.bmax);
-      Item li, ri;
-      li.node = c; li.lo = it.lo; li.hi = it.lo + d.lcount; li.pad = 0;
-      ri.node = c + 1; ri.lo = it.lo + d.lcount; ri.hi = it.hi; ri.pad = 0;
-      for (int q = 0; q < 3; ++q) {
-        li.bmin[q] = d.child[q]; li.bmax[q] = d.child[3 + q];
-        ri.bmin[q] = d.child[6 + q]; ri.bmax[q] = d.child[9 + q];
-      }
-      li.pad2[0] = li.pad2[1] = ri.pad2[0] = ri.pad2[1] = 0.f;
-      next[2 * k] = li;
-      next[2 * k + 1] = ri;
-    } else if (it.node < nodes_cap) {
-      nodes[it.node] = make_leaf(it.lo, it.hi - it.lo, it.bmin, it.bmax);
+  if (m_min < 0) return;
+  if (k < 2) {
+    const uint32_t rec = 2 * (it.lo + (uint32_t)sw.lcount) + k;
+    s.rec[rec] = child;
+    if (nch) {
+      at += s_base[0];
+      chunk_at += s_base[1];
+      BigItem b;
+      b.rec = rec; b.lo = child.lo; b.hi = child.lo + child.cnt; b.chunk_base = chunk_at;
+      b.bref = 2 * i + k;
+      b.pad = 0;
+      for (int q = 0; q < 3; ++q) { b.bmin[q] = child.bmin[q]; b.bmax[q] = child.bmax[q]; }
+      big_of(s, par ^ 1u)[at] = b;
+    } else {
+      s.roots[cls * s.m_cap + s_base[3 + cls] + at] = make_uint2(rec, level + 1);
     }
   }
-  if (threadIdx.x == 0 && g == (m ? (m - 1) / kEmitItems : 0u)) {
-    const uint32_t all = before_total + total;
-    nx[kLvM] = 2 * all;
-    nx[kLvCount] = count0 + 2 * all;
-    if (count0 + 2 * all > nodes_cap) atomicOr(ctl + kCtlFlags, 0x20u);
+  uint32_t* map = chunks_of(s, par ^ 1u);
+  for (int c = 0; c < 2; ++c) {
+    const uint32_t b = __shfl(chunk_at, c, 32), e = __shfl(nch, c, 32), a = __shfl(at, c, 32);
+    for (uint32_t j = k; j < e; j += 32) map[b + j] = a;
   }
 }
 
-__global__ __launch_bounds__(kCT) void k_sah_count(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                   uint32_t par, const uint32_t* __restrict__ chunk_item,
-                                                   const uint32_t* __restrict__ chunk_base,
-                                                   const uint32_t* __restrict__ indices, const Box* __restrict__ boxes,
-                                                   const Decision* __restrict__ dec, uint32_t* __restrict__ chunk_left) {
-  __shared__ uint32_t s_cnt;
-  const ChunkRange r = chunk_range(items, ctl, par, chunk_base, chunk_item, blockIdx.x);
+// Smallest of each of 12 values over a wave, in a way that halves the values
+// while it can: lane 0 ends with v[0..2], lane 16 with v[3..5], 32 with v[6..8],
+// 48 with v[9..11], in v[0..2].
+__device__ __forceinline__ void wave_min12(int (&v)[12], uint32_t lane) {
+#pragma unroll
+  for (int q = 0; q < 6; ++q) {
+    const int send = lane & 32u ? v[q] : v[6 + q], keep = lane & 32u ? v[6 + q] : v[q];
+    v[q] = min(keep, __shfl_xor(send, 32, 64));
+  }
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    const int send = lane & 16u ? v[q] : v[3 + q], keep = lane & 16u ? v[3 + q] : v[q];
+    v[q] = min(keep, __shfl_xor(send, 16, 64));
+  }
+#pragma unroll
+  for (int off = 8; off > 0; off >>= 1)
+#pragma unroll
+    for (int q = 0; q < 3; ++q) v[q] = min(v[q], __shfl_xor(v[q], off, 64));
+}
+
+// The stable partition: a face's place needs the left faces of the item's
+// earlier chunks (their cumulative bin counts at the split, one run of memory)
+// and those before it in the chunk (ballots). A leaf's ids go to where the
+// finished ones are.
+__global__ __launch_bounds__(kCT) void k_sah_scatter(Sah s, uint32_t par) {
+  constexpr uint32_t kWaves = kCT / 64;
+  __shared__ uint32_t s_left[kWaves], s_before[kWaves];
+  __shared__ int s_red[kWaves][4][3];
+  const ChunkRange r = chunk_range(s, par);
   if (!r.ok) return;
-  const Decision d = dec[r.item];
-  if (threadIdx.x == 0) s_cnt = 0;
-  __syncthreads();
-  if (d.m_min >= 0) {
-    Box bb[kPer];
-    bool in[kPer];
-    chunk_boxes(r, indices, boxes, bb, in);
-    uint32_t c = 0;
+  const BigDec d = s.dec[r.item];
+  const uint32_t* src = ids_of(s, par);
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6;
+  if (d.m_min < 0) {
+    if (par)
+      for (uint32_t l = r.lo + t; l < r.hi; l += kCT) s.ids0[l] = src[l];
+    return;
+  }
+  uint32_t id[kPer];
+  int bin[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const uint32_t l = r.lo + w * (64u * kPer) + (uint32_t)u * 64u + lane;
+    id[u] = l < r.hi ? src[l] : 0u;
+    bin[u] = l < r.hi ? (int)s.bin[l] : kBins;
+  }
+  const bool need_l = d.lcount > kChunk, need_r = r.it.hi - r.it.lo - d.lcount > kChunk;
+  Box bb[kPer];
+  if (need_l || need_r) {
 #pragma unroll
     for (int u = 0; u < kPer; ++u)
-      if (in[u]) c += bin_of(bb[u], d.axis, d.scale, d.bmin0) <= d.m_min ? 1u : 0u;
-    atomicAdd(&s_cnt, c);
+      if (bin[u] < kBins) bb[u] = rk::load_box(s.boxes + id[u]);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) chunk_left[blockIdx.x] = s_cnt;
-}
-
-// Exclusive scan of chunk_left within each item (an item's chunks are
-// contiguous), one wave per item.
-__global__ __launch_bounds__(256) void k_sah_offsets(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                     uint32_t par, const uint32_t* __restrict__ chunk_base,
-                                                     const uint32_t* __restrict__ chunk_left,
-                                                     uint32_t* __restrict__ chunk_loff) {
-  const uint32_t m = ctl[kCtlLevel(par) + kLvM];
-  const uint32_t i = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (i >= m) return;  // wave-uniform
-  const uint32_t size = items[i].hi - items[i].lo;
-  if (size <= kChunk) return;  // no chunks
-  const uint32_t b = chunk_base[i], nch = (size + kChunk - 1) / kChunk;
-  uint32_t run = 0;
-  for (uint32_t c0 = 0; c0 < nch; c0 += 64) {
-    const uint32_t c = c0 + lane;
-    const uint32_t v = c < nch ? chunk_left[b + c] : 0u;
-    uint32_t incl = v;
+  uint32_t before = 0;
+  const uint16_t* cum = s.cum + (size_t)d.m_min * s.chunks_cap + r.it.chunk_base;
+  for (uint32_t j = t; j < r.j; j += kCT) before += cum[j];
 #pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const uint32_t y = __shfl_up(incl, off, 64);
-      if (lane >= (uint32_t)off) incl += y;
-    }
-    if (c < nch) chunk_loff[b + c] = run + incl - v;
-    run += __shfl(incl, 63, 64);
+  for (int off = 32; off > 0; off >>= 1) before += __shfl_xor(before, off, 64);
+  uint64_t left[kPer];
+  uint32_t mine = 0;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    left[u] = __ballot(bin[u] <= d.m_min);
+    mine += (uint32_t)__popcll(left[u]);
   }
-}
-
-__global__ __launch_bounds__(kCT) void k_sah_scatter(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                     uint32_t par, const uint32_t* __restrict__ chunk_item,
-                                                     const uint32_t* __restrict__ chunk_base,
-                                                     const uint32_t* __restrict__ indices,
-                                                     const Box* __restrict__ boxes, const Decision* __restrict__ dec,
-                                                     const uint32_t* __restrict__ chunk_loff,
-                                                     uint32_t* __restrict__ tmp) {
-  __shared__ uint32_t s_tmp[8];
-  const ChunkRange r = chunk_range(items, ctl, par, chunk_base, chunk_item, blockIdx.x);
-  if (!r.ok) return;
-  const Decision d = dec[r.item];
-  if (d.m_min < 0) return;
-  const Item it = items[r.item];
-  const uint32_t loff = chunk_loff[blockIdx.x];
-  const uint32_t chunk_start = r.lo - it.lo;  // elements of this item before the chunk
-  uint32_t left_before = 0;                    // left elements of this chunk before the current step
-  for (uint32_t s = r.lo; s < r.hi; s += kCT) {
-    const uint32_t l = s + threadIdx.x;
-    uint32_t id = 0, is_left = 0;
-    const bool in = l < r.hi;
-    if (in) {
-      id = indices[l];
-      is_left = bin_of(rk::load_box(boxes + id), d.axis, d.scale, d.bmin0) <= d.m_min ? 1u : 0u;
-    }
-    uint32_t total;
-    const uint32_t ex = block_excl_scan(is_left, s_tmp, &total, kCT);
-    if (in) {
-      const uint32_t pos_in_item = chunk_start + (l - r.lo);
-      const uint32_t lrank = loff + left_before + ex;            // left elements before this one
-      const uint32_t out = is_left ? (it.lo + lrank) : (it.lo + d.lcount + (pos_in_item - lrank));
-      tmp[out] = id;
-    }
-    left_before += total;
+  if (lane == 0) {
+    s_left[w] = mine;
+    s_before[w] = before;
   }
-}
-
-__global__ __launch_bounds__(kCT) void k_sah_copyback(const Item* __restrict__ items, const uint32_t* __restrict__ ctl,
-                                                      uint32_t par, const uint32_t* __restrict__ chunk_item,
-                                                      const uint32_t* __restrict__ chunk_base,
-                                                      const Decision* __restrict__ dec,
-                                                      const uint32_t* __restrict__ tmp, uint32_t* __restrict__ indices) {
-  const ChunkRange r = chunk_range(items, ctl, par, chunk_base, chunk_item, blockIdx.x);
-  if (!r.ok) return;
-  if (dec[r.item].m_min < 0) return;
-  for (uint32_t l = r.lo + threadIdx.x; l < r.hi; l += kCT) indices[l] = tmp[l];
-}
-
-// Hybrid entry (kernel_initStack, :647-666): every leaf of the existing tree
-// becomes an item, in ascending node order, with the leaf's box.
-__global__ __launch_bounds__(1024) void k_sah_init_from_leaves(const Node* __restrict__ nodes, uint32_t existing,
-                                                               Item* __restrict__ items, uint32_t* __restrict__ ctl) {
-  __shared__ uint32_t s_tmp[16];
-  __shared__ uint32_t s_carry, s_big;
-  if (threadIdx.x == 0) s_carry = s_big = 0;
+  if (need_l || need_r) {
+    int v[12];  // left min, left max, right min, right max; ~x turns a max into a min
+#pragma unroll
+    for (int q = 0; q < 12; ++q) v[q] = q % 6 < 3 ? f2o(RK_HUGE) : ~f2o(-RK_HUGE);
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+      if (bin[u] >= kBins) continue;
+      const bool is_left = bin[u] <= d.m_min;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int c = f2o(center_axis(bb[u], q)), lo = min(is_left ? v[q] : v[6 + q], c),
+                  hi = min(is_left ? v[3 + q] : v[9 + q], ~c);
+        v[q] = is_left ? lo : v[q];
+        v[3 + q] = is_left ? hi : v[3 + q];
+        v[6 + q] = is_left ? v[6 + q] : lo;
+        v[9 + q] = is_left ? v[9 + q] : hi;
+      }
+    }
+    wave_min12(v, lane);
+    if ((lane & 15u) == 0)
+      for (int q = 0; q < 3; ++q) s_red[w][lane >> 4][q] = v[q];
+  }
   __syncthreads();
-  for (uint32_t c0 = 0; c0 < existing; c0 += 1024) {
-    const uint32_t k = c0 + threadIdx.x;
-    uint32_t leaf = 0;
+  if ((need_l || need_r) && t < 12) {
+    const uint32_t part = t / 3, q = t % 3;
+    int v = s_red[0][part][q];
+    for (uint32_t x = 1; x < kWaves; ++x) v = min(v, s_red[x][part][q]);
+    int* g = bounds_of(s, par) + (size_t)(2 * r.item + part / 2) * kBoundWords + 6 * (blockIdx.x % kBoundSlots) +
+             3 * (part & 1u) + q;
+    if (part < 2 ? need_l : need_r) {
+      if (part & 1u) atomicMax(g, ~v);
+      else atomicMin(g, v);
+    }
+  }
+  uint32_t rank = 0;
+  for (uint32_t x = 0; x < kWaves; ++x) rank += s_before[x] + (x < w ? s_left[x] : 0u);
+  uint32_t* dst = ids_of(s, par ^ 1u);
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const uint32_t l = r.lo + w * (64u * kPer) + (uint32_t)u * 64u + lane;
+    const uint32_t lrank = rank + __builtin_amdgcn_mbcnt_hi((uint32_t)(left[u] >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((uint32_t)left[u], 0u));
+    if (l < r.hi) dst[bin[u] <= d.m_min ? r.it.lo + lrank : r.it.lo + d.lcount + (l - r.it.lo - lrank)] = id[u];
+    rank += (uint32_t)__popcll(left[u]);
+  }
+}
+
+// Items of at most kChunk faces, to the leaves: a workgroup takes 1 of more than
+// 256 faces, or 4 or 8 smaller ones, reads their boxes once into LDS and makes
+// every level below them there. Items of more than kWide faces are done by the
+// whole workgroup, then the others by half-waves (the sweep is a lane per bin),
+// a round per level. A face is its place in the workgroup's lists at the start;
+// s_ord holds the faces in order (by the item's depth below its root, odd and
+// even), with the bin above.
+// What bounds it is instruction issue: the sweep goes over lane rows (DPP), not
+// through LDS (213 us, now 153 for the 1M-face heightfield); kWide 256, 512 and
+// 1024: 157, 153, 162.
+constexpr uint32_t kTreeThreads = 256, kTreeHalves = kTreeThreads / 32, kWide = 512;
+constexpr uint32_t kTreeList = kChunk / (kLeafMin + 1) + 1;  // items that are not leaves by size
+struct TreeItem {
+  uint32_t range;  // lo | (size - 1) << 10
+  uint32_t rec;
+  float area;
+  uint32_t depth;
+};
+struct RootsDone { uint32_t n[kClasses]; };  // of each list, taken by an earlier launch
+__global__ __launch_bounds__(kTreeThreads, 4) void k_sah_subtrees(Sah s, RootsDone done) {
+  __shared__ float s_box[6][kChunk];
+  __shared__ uint16_t s_ord[2][kChunk];
+  __shared__ int s_bins[kTreeHalves][kBinWords];
+  __shared__ TreeItem s_list[2][kTreeList];
+  __shared__ TreeItem s_wide[4];
+  __shared__ uint32_t s_n[2], s_nwide;
+  __shared__ uint32_t s_shift[8];   // global position less place, per 128 places
+  __shared__ uint32_t s_size[8], s_rec[8], s_level[8];
+  __shared__ uint32_t s_hist[8][32];  // internal items by depth below their root
+  __shared__ uint32_t s_left[kTreeThreads / 64];
+  __shared__ int s_red[kTreeHalves][6];
+  __shared__ int s_cut, s_lcount;
+  const uint32_t t = threadIdx.x, lane = t & 63u, w = t >> 6, h = t >> 5, k = t & 31u;
+  const uint32_t n0 = s.ctl[kCtlRoots] - done.n[0], n1 = s.ctl[kCtlRoots + 1] - done.n[1],
+                 n2 = s.ctl[kCtlRoots + 2] - done.n[2];
+  const uint32_t g0 = (n0 + 7) / 8, g1 = (n1 + 3) / 4;
+  // the larger ones first
+  for (uint32_t group = blockIdx.x; group < n2 + g1 + g0; group += gridDim.x) {
+    const uint32_t cls = group < n2 ? 2u : (group < n2 + g1 ? 1u : 0u);
+    const uint32_t cap = class_cap(cls), per = kChunk / cap;
+    const uint32_t first = (group - (cls == 2 ? 0u : (cls == 1 ? n2 : n2 + g1))) * per;
+    const uint32_t have = cls == 0 ? n0 - first : (cls == 1 ? n1 - first : 1u);  // may be more than per
+    if (t < 8) s_size[t] = 0u;
+    if (t < 2) s_n[t] = 0u;
+    if (t == 2) s_nwide = 0u;
+    (&s_hist[0][0])[t] = 0u;
+    __syncthreads();
+    if (t < per && t < have) {
+      const uint2 root = s.roots[cls * s.m_cap + done.n[cls] + first + t];
+      const Rec r = s.rec[root.x];
+      s_size[t] = r.cnt;
+      s_rec[t] = root.x;
+      s_level[t] = root.y;
+      for (uint32_t x = 0; x < cap / 128u; ++x) s_shift[t * (cap / 128u) + x] = r.lo - t * cap;
+      if (r.cnt > kLeafMin) {
+        TreeItem it;
+        it.range = (t * cap) | (r.cnt - 1u) << 10;
+        it.rec = root.x;
+        it.area = box_area(r.bmin[0], r.bmin[1], r.bmin[2], r.bmax[0], r.bmax[1], r.bmax[2]);
+        it.depth = 0;
+        if (r.cnt > kWide) s_wide[atomicAdd(&s_nwide, 1u)] = it;
+        else s_list[0][atomicAdd(&s_n[0], 1u)] = it;
+      } else {
+        s.link[root.x] = kLeaf;
+      }
+    }
+    __syncthreads();
+    {
+      uint32_t id[kChunk / kTreeThreads];
+      bool in[kChunk / kTreeThreads];
+#pragma unroll
+      for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+        const uint32_t l = t + u * kTreeThreads, x = l / cap;
+        in[u] = l - x * cap < s_size[x];
+        id[u] = 0;
+        if (!in[u]) continue;
+        // all ids end in ids0; ids1 keeps them until then
+        const uint32_t g = s_shift[l >> 7] + l;
+        if (s_level[x] & 1u) {
+          id[u] = s.ids1[g];
+          if (s_size[x] <= kLeafMin) s.ids0[g] = id[u];
+        } else {
+          id[u] = s.ids0[g];
+          s.ids1[g] = id[u];
+        }
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+        const uint32_t l = t + u * kTreeThreads;
+        if (!in[u]) continue;
+        const Box b = rk::load_box(s.boxes + id[u]);
+        s_box[0][l] = b.mn.x; s_box[1][l] = b.mn.y; s_box[2][l] = b.mn.z;
+        s_box[3][l] = b.mx.x; s_box[4][l] = b.mx.y; s_box[5][l] = b.mx.z;
+        s_ord[0][l] = (uint16_t)l;
+      }
+    }
+    __syncthreads();
+
+    // what goes between a wave's lanes through LDS
+    auto wave_order = [] {
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+    };
+    auto load = [&](uint32_t f) {
+      Box b;
+      b.mn = make_float4(s_box[0][f], s_box[1][f], s_box[2][f], 0.f);
+      b.mx = make_float4(s_box[3][f], s_box[4][f], s_box[5][f], 0.f);
+      return b;
+    };
+    auto finish = [&](uint32_t place, uint32_t f) {
+      s.ids0[s_shift[place >> 7] + place] = s.ids1[s_shift[f >> 7] + f];
+    };
+    auto add_bounds = [&](const Box& b, int (&c)[6]) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        const int x = f2o(center_axis(b, q));
+        c[q] = min(c[q], x);
+        c[3 + q] = max(c[3 + q], x);
+      }
+    };
+    auto half_bounds = [](int (&c)[6]) {
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        c[q] = half_min(c[q]);
+        c[3 + q] = ~half_min(~c[3 + q]);
+      }
+    };
+    auto add_bin = [&](int* bins, const Box& b, int m) {
+      int* p = bins + m * 7;
+      atomicAdd(p, 1);
+      atomicMin(p + 1, f2o(b.mn.x)); atomicMin(p + 2, f2o(b.mn.y)); atomicMin(p + 3, f2o(b.mn.z));
+      atomicMax(p + 4, f2o(b.mx.x)); atomicMax(p + 5, f2o(b.mx.y)); atomicMax(p + 6, f2o(b.mx.z));
+    };
+    auto empty_bin = [](int q) { return q % 7 == 0 ? 0 : (q % 7 < 4 ? f2o(RK_HUGE) : f2o(-RK_HUGE)); };
+    // by lanes 0 and 1 of a half-wave: the records and the items of the children
+    auto children = [&](const TreeItem& it, const Sweep& sw, int axis, uint32_t lo, uint32_t size, bool wide,
+                        uint32_t next) {
+      const uint32_t x = lo / cap, gl = s_shift[lo >> 7] + lo, split = gl + (uint32_t)sw.lcount;
+      const Rec r = child_rec(sw, k, gl, size);
+      s.rec[2 * (size_t)split + k] = r;
+      if (r.cnt <= kLeafMin) {
+        s.link[2 * (size_t)split + k] = kLeaf;
+      } else {
+        TreeItem c;
+        c.range = (k == 0 ? lo : lo + (uint32_t)sw.lcount) | (r.cnt - 1u) << 10;
+        c.rec = 2 * split + k;
+        c.area = box_area(r.bmin[0], r.bmin[1], r.bmin[2], r.bmax[0], r.bmax[1], r.bmax[2]);
+        c.depth = it.depth + 1u;
+        if (wide && r.cnt > kWide) s_wide[atomicAdd(&s_nwide, 1u)] = c;
+        else s_list[next][atomicAdd(&s_n[next], 1u)] = c;
+      }
+      if (k == 0) {
+        s.link[it.rec] = split | (uint32_t)axis << 30;
+        const uint32_t level = s_level[x] + it.depth;
+        if (it.depth < 32u) atomicAdd(&s_hist[x][it.depth], 1u);
+        else if (level <= kLevelMax) atomicAdd(s.ctl + kCtlHist + level, 1u);
+        if (level >= kLevelMax) s.ctl[kCtlDeep] = 1u;
+      }
+    };
+
+    while (s_nwide != 0u) {
+      const TreeItem it = s_wide[s_nwide - 1u];
+      const uint32_t lo = it.range & 1023u, size = (it.range >> 10) + 1u, now = it.depth & 1u;
+      int c[6] = {f2o(RK_HUGE), f2o(RK_HUGE), f2o(RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE)};
+      uint32_t f[kChunk / kTreeThreads];
+#pragma unroll
+      for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+        const uint32_t l = w * 256u + u * 64u + lane;
+        f[u] = l < size ? s_ord[now][lo + l] & 1023u : 0u;
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+        if (w * 256u + u * 64u + lane >= size) continue;
+        add_bounds(load(f[u]), c);
+      }
+      half_bounds(c);
+      if (k == 0)
+        for (int q = 0; q < 6; ++q) s_red[h][q] = c[q];
+      for (int x = (int)k; x < kBinWords; x += 32) s_bins[h][x] = empty_bin(x);
+      __syncthreads();
+      if (t == 0) s_nwide -= 1u;
+      for (int q = 0; q < 3; ++q)
+        for (uint32_t x = 0; x < kTreeHalves; ++x) {
+          c[q] = min(c[q], s_red[x][q]);
+          c[3 + q] = max(c[3 + q], s_red[x][3 + q]);
+        }
+      int axis;
+      float scale, bmin0;
+      item_axis(c, axis, scale, bmin0);
+      int bin[kChunk / kTreeThreads];
+#pragma unroll
+      for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+        bin[u] = kBins;
+        if (w * 256u + u * 64u + lane >= size) continue;
+        const Box b = load(f[u]);
+        bin[u] = bin_of(b, axis, scale, bmin0);
+        add_bin(s_bins[h], b, bin[u]);
+      }
+      __syncthreads();
+      if (t < (uint32_t)kBinWords) {
+        const int q = (int)t % 7;
+        int v = s_bins[0][t];
+        for (uint32_t x = 1; x < kTreeHalves; ++x) {
+          const int y = s_bins[x][t];
+          v = q == 0 ? v + y : (q < 4 ? min(v, y) : max(v, y));
+        }
+        s_bins[0][t] = v;
+      }
+      __syncthreads();
+      Sweep sw;
+      if (t < 64) {  // one wave: issue slots are what the kernel runs out of
+        float bmn[3], bmx[3];
+        const int* row = s_bins[0] + k * 7;
+        for (int q = 0; q < 3; ++q) { bmn[q] = o2f(row[1 + q]); bmx[q] = o2f(row[4 + q]); }
+        sw = sweep_bins(row[0], bmn, bmx, it.area, k);
+        const int m = split_bin(s, size, sw, t == 0);
+        if (t == 0) {
+          s_cut = m;
+          s_lcount = sw.lcount;
+        }
+      }
+      __syncthreads();
+      const int m_min = s_cut;
+      if (m_min < 0) {
+        if (t == 0) s.link[it.rec] = kLeaf;
+        for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+          const uint32_t l = w * 256u + u * 64u + lane;
+          if (l < size) finish(lo + l, f[u]);
+        }
+      } else {
+        uint64_t left[kChunk / kTreeThreads];
+        uint32_t mine = 0, rank = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+          left[u] = __ballot(bin[u] <= m_min);
+          mine += (uint32_t)__popcll(left[u]);
+        }
+        if (lane == 0) s_left[w] = mine;
+        __syncthreads();
+        for (uint32_t x = 0; x < w; ++x) rank += s_left[x];
+        const uint32_t lc = (uint32_t)s_lcount;
+#pragma unroll
+        for (uint32_t u = 0; u < kChunk / kTreeThreads; ++u) {
+          const uint32_t l = w * 256u + u * 64u + lane;
+          const uint32_t lrank = rank + __builtin_amdgcn_mbcnt_hi((uint32_t)(left[u] >> 32),
+                                                                  __builtin_amdgcn_mbcnt_lo((uint32_t)left[u], 0u));
+          const bool is_left = bin[u] <= m_min;
+          const uint32_t place = lo + (is_left ? lrank : lc + (l - lrank));
+          if (l < size) {
+            s_ord[now ^ 1u][place] = (uint16_t)f[u];
+            if ((is_left ? lc : size - lc) <= kLeafMin) finish(place, f[u]);
+          }
+          rank += (uint32_t)__popcll(left[u]);
+        }
+        if (t < 2) children(it, sw, axis, lo, size, true, 0);
+      }
+      __syncthreads();
+    }
+
+    uint32_t cur = 0, count = s_n[0];
+    while (count != 0u) {
+      for (uint32_t i = h; i < count; i += kTreeHalves) {
+        const TreeItem it = s_list[cur][i];
+        const uint32_t lo = it.range & 1023u, size = (it.range >> 10) + 1u, now = it.depth & 1u;
+        uint16_t* ord = s_ord[now] + lo;
+        int* bins = s_bins[h];
+        int c[6] = {f2o(RK_HUGE), f2o(RK_HUGE), f2o(RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE)};
+        for (uint32_t l = k; l < size; l += 32) add_bounds(load(ord[l] & 1023u), c);
+        half_bounds(c);
+        int axis;
+        float scale, bmin0;
+        item_axis(c, axis, scale, bmin0);
+        for (int x = (int)k; x < kBinWords; x += 32) bins[x] = empty_bin(x);
+        wave_order();
+        for (uint32_t l = k; l < size; l += 32) {
+          const uint32_t f = ord[l] & 1023u;
+          const Box b = load(f);
+          const int m = bin_of(b, axis, scale, bmin0);
+          ord[l] = (uint16_t)(f | (uint32_t)m << 10);
+          add_bin(bins, b, m);
+        }
+        wave_order();
+        float bmn[3], bmx[3];
+        const int* row = bins + k * 7;
+        for (int q = 0; q < 3; ++q) { bmn[q] = o2f(row[1 + q]); bmx[q] = o2f(row[4 + q]); }
+        const Sweep sw = sweep_bins(row[0], bmn, bmx, it.area, k);
+        const int m_min = split_bin(s, size, sw, k == 0);
+        if (m_min < 0) {
+          if (k == 0) s.link[it.rec] = kLeaf;
+          for (uint32_t l = k; l < size; l += 32) finish(lo + l, ord[l] & 1023u);
+        } else {
+          const uint32_t lc = (uint32_t)sw.lcount;
+          uint32_t rank = 0;
+          for (uint32_t l0 = 0; l0 < size; l0 += 32) {
+            const uint32_t l = l0 + k, v = l < size ? ord[l] : 0xFFFFu;
+            const bool is_left = (int)(v >> 10) <= m_min;
+            const uint32_t left = (uint32_t)(__ballot(is_left) >> (lane & 32u));
+            const uint32_t lrank = rank + (uint32_t)__popc(left & ((1u << k) - 1u));
+            const uint32_t place = lo + (is_left ? lrank : lc + (l - lrank));
+            if (l < size) {
+              s_ord[now ^ 1u][place] = (uint16_t)(v & 1023u);
+              if ((is_left ? lc : size - lc) <= kLeafMin) finish(place, v & 1023u);
+            }
+            rank += (uint32_t)__popc(left);
+          }
+          if (k < 2) children(it, sw, axis, lo, size, false, cur ^ 1u);
+        }
+        wave_order();
+      }
+      __syncthreads();
+      count = s_n[cur ^ 1u];
+      if (t == 0) s_n[cur] = 0u;
+      cur ^= 1u;
+      __syncthreads();
+    }
+    const uint32_t level = s_level[h] + k, c = s_hist[h][k];
+    if (c && level <= kLevelMax) atomicAdd(s.ctl + kCtlHist + level, c);
+    __syncthreads();
+  }
+}
+
+// A level's items i of m (this thread's, in order): the node record, its id id0 + i
+// (the starting items': node0), and the internal ones' splits in order to
+// q[2 * rank]. before: internal items of the level before the workgroup's.
+// Counts the next level's internal items by group, if there is a groups. Returns
+// the workgroup's internal items.
+__device__ __forceinline__ uint32_t number_items(const Sah& s, uint32_t level, uint32_t i, uint32_t m,
+                                                 const uint32_t* q_in, uint32_t* q_out, uint32_t id0, uint32_t before,
+                                                 uint32_t child0, uint32_t* groups, Node* __restrict__ nodes,
+                                                 uint32_t nodes_cap, uint32_t* s_wave) {
+  const uint32_t lane = threadIdx.x & 63u, w = threadIdx.x >> 6;
+  const bool in = i < m;
+  Rec r;
+  uint32_t link = kLeaf, id = 0;
+  if (in) {
+    const uint32_t rec = level ? 2 * q_in[i >> 1] + (i & 1u) : 2 * s.n + i;
+    link = s.link[rec];
+    r = s.rec[rec];
+    id = level ? id0 + i : s.node0[i];
+  }
+  const bool internal = link != kLeaf;
+  const uint64_t mask = __ballot(internal);
+  if (lane == 0) s_wave[w] = (uint32_t)__popcll(mask);
+  __syncthreads();
+  uint32_t k =
+      before + __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+  uint32_t total = 0;
+#pragma unroll
+  for (uint32_t x = 0; x < 16; ++x) {
+    const uint32_t c = s_wave[x];
+    k += x < w ? c : 0u;
+    total += c;
+  }
+  if (in) {
     Node nd;
-    if (k < existing) {
-      nd = nodes[k];
-      leaf = rk::node_is_leaf(nd.w0);
+    for (int q = 0; q < 3; ++q) { nd.bmin[q] = r.bmin[q]; nd.bmax[q] = r.bmax[q]; }
+    nd.w0 = internal ? (link >> 30) << 1 : 1u | (r.cnt << 1);
+    nd.w1 = internal ? child0 + 2 * k : r.lo;
+    if (id < nodes_cap) nodes[id] = nd;
+  }
+  const uint32_t split = link & 0x3FFFFFFFu;
+  if (internal) q_out[k] = split;
+  if (groups && mask) {
+    uint2 below = make_uint2(kLeaf, kLeaf);
+    if (internal) below = *reinterpret_cast<const uint2*>(s.link + 2 * (size_t)split);
+    const uint32_t g = 2 * k / kNumberItems, c = (below.x != kLeaf ? 1u : 0u) + (below.y != kLeaf ? 1u : 0u);
+    const uint32_t g0 = (uint32_t)__shfl((int)g, __builtin_ctzll(mask), 64);  // a wave's children lie in two groups
+    const uint64_t one = __ballot(internal && g == g0), has1 = __ballot((c & 1u) != 0), has2 = __ballot((c & 2u) != 0);
+    const uint32_t a = (uint32_t)(__popcll(one & has1) + 2 * __popcll(one & has2)),
+                   b = (uint32_t)(__popcll(~one & has1) + 2 * __popcll(~one & has2));
+    if (lane == 0) {
+      if (a) atomicAdd(groups + g0, a);
+      if (b) atomicAdd(groups + g0 + 1, b);
     }
-    uint32_t total, big_total;
-    const uint32_t ex = block_excl_scan(leaf, s_tmp, &total, 1024);
-    block_excl_scan(leaf && rk::leaf_count(nd.w0) > kChunk ? 1u : 0u, s_tmp, &big_total, 1024);
-    if (leaf) {
-      Item it;
-      it.node = k; it.lo = nd.w1; it.hi = nd.w1 + rk::leaf_count(nd.w0); it.pad = 0;
-      for (int q = 0; q < 3; ++q) { it.bmin[q] = nd.bmin[q]; it.bmax[q] = nd.bmax[q]; }
-      it.pad2[0] = it.pad2[1] = 0.f;
-      items[s_carry + ex] = it;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      s_carry += total;
-      s_big += big_total;
-    }
+  }
+  return total;
+}
+
+__device__ __forceinline__ void number_info(const Sah& s, uint32_t* __restrict__ info, uint32_t total) {
+  info[RK_INFO_NODE_COUNT] = total;
+  info[RK_INFO_FLAGS] |= s.ctl[kCtlFlags];
+}
+
+// A level, kNumberItems items per workgroup, after the groups before it; their
+// internal items were counted when the level's queue was written. Clears the
+// groups of the level after the next.
+__global__ __launch_bounds__(1024) void k_sah_number(Sah s, uint32_t level, uint32_t m, uint32_t id0, uint32_t child0,
+                                                     Node* __restrict__ nodes, uint32_t nodes_cap,
+                                                     uint32_t* __restrict__ info, uint32_t total) {
+  __shared__ uint32_t s_wave[16], s_tmp[16];
+  const uint32_t* now = s.groups + (level % 3u) * s.group_cap;
+  uint32_t* next = s.groups + ((level + 1u) % 3u) * s.group_cap;
+  uint32_t* after = s.groups + ((level + 2u) % 3u) * s.group_cap;
+  for (uint32_t i = blockIdx.x * 1024 + threadIdx.x; i < s.group_cap; i += gridDim.x * 1024) after[i] = 0u;
+  uint32_t before = 0, before_total;
+  for (uint32_t h = threadIdx.x; h < blockIdx.x; h += 1024) before += now[h];
+  block_excl_scan(before, s_tmp, &before_total, 1024);
+  const uint32_t* q_in = level & 1u ? s.q1 : s.q0;
+  uint32_t* q_out = level & 1u ? s.q0 : s.q1;
+  number_items(s, level, blockIdx.x * kNumberItems + threadIdx.x, m, q_in, q_out, id0, before_total, child0, next,
+               nodes, nodes_cap, s_wave);
+  if (info && blockIdx.x == 0 && threadIdx.x == 0) number_info(s, info, total);
+}
+
+// Levels [level, end) of at most 1024 items each, in one workgroup.
+__global__ __launch_bounds__(1024) void k_sah_number_run(Sah s, uint32_t level, uint32_t end, uint32_t m, uint32_t id0,
+                                                         uint32_t child0, Node* __restrict__ nodes, uint32_t nodes_cap,
+                                                         uint32_t* __restrict__ info, uint32_t total) {
+  __shared__ uint32_t s_wave[2][16];
+  __shared__ uint32_t s_q[2][1024];
+  uint32_t* next = s.groups + (end % 3u) * s.group_cap;
+  uint32_t* after = s.groups + ((end + 1u) % 3u) * s.group_cap;
+  for (uint32_t i = threadIdx.x; i < s.group_cap; i += 1024) next[i] = after[i] = 0u;
+  if (info && threadIdx.x == 0) number_info(s, info, total);
+  if (level && threadIdx.x < (m + 1) / 2) s_q[level & 1u][threadIdx.x] = (level & 1u ? s.q1 : s.q0)[threadIdx.x];
+  __syncthreads();
+  for (; level < end; ++level) {
+    const bool last = level + 1 == end;
+    uint32_t* q_out = last ? (level & 1u ? s.q0 : s.q1) : s_q[(level & 1u) ^ 1u];
+    const uint32_t found = number_items(s, level, threadIdx.x, m, s_q[level & 1u], q_out, id0, 0, child0,
+                                        last ? next : nullptr, nodes, nodes_cap, s_wave[level & 1u]);
+    id0 = child0;
+    m = 2 * found;
+    child0 += m;
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    uint32_t* lv = ctl + kCtlLevel(0);
-    lv[kLvM] = s_carry;
-    lv[kLvBig] = s_big;
-    lv[kLvCount] = existing;
-    ctl[kCtlFlags] = 0;
+}
+
+// The groups of the starting items, and the next two levels' cleared.
+__global__ __launch_bounds__(1024) void k_sah_number_start(Sah s, uint32_t m) {
+  __shared__ uint32_t s_sum;
+  const uint32_t i = blockIdx.x * kNumberItems + threadIdx.x;
+  if (threadIdx.x == 0) s_sum = 0u;
+  for (uint32_t j = i; j < 2 * s.group_cap; j += gridDim.x * 1024) s.groups[s.group_cap + j] = 0u;
+  __syncthreads();
+  const uint64_t mask = __ballot(i < m && s.link[2 * (size_t)s.n + i] != kLeaf);
+  if ((threadIdx.x & 63) == 0) atomicAdd(&s_sum, (uint32_t)__popcll(mask));
+  __syncthreads();
+  if (threadIdx.x == 0) s.groups[blockIdx.x] = s_sum;
+}
+
+// The faces' boxes, ids and a copy of them, and the root's centroid bounds:
+// kBoxPer faces per thread, so that few workgroups add to the same words.
+constexpr uint32_t kBoxThreads = 1024, kBoxPer = 4;
+__global__ __launch_bounds__(kBoxThreads) void k_boxes_root(Sah s, const uint4* __restrict__ faces,
+                                                            const float4* __restrict__ verts, Box* __restrict__ boxes,
+                                                            uint4* __restrict__ copy) {
+  int b[6] = {f2o(RK_HUGE), f2o(RK_HUGE), f2o(RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE), f2o(-RK_HUGE)};
+  uint4 f[kBoxPer];
+#pragma unroll
+  for (uint32_t u = 0; u < kBoxPer; ++u) {
+    const uint32_t k = (blockIdx.x * kBoxPer + u) * kBoxThreads + threadIdx.x;
+    f[u] = k < s.n ? faces[k] : make_uint4(0u, 0u, 0u, 0u);
   }
-}
-
-__global__ void k_sah_init_root(Item* __restrict__ items, uint32_t* __restrict__ ctl, uint32_t n, float4 rmin,
-                                float4 rmax) {
-  Item it;
-  it.node = 0; it.lo = 0; it.hi = n; it.pad = 0;
-  it.bmin[0] = rmin.x; it.bmin[1] = rmin.y; it.bmin[2] = rmin.z;
-  it.bmax[0] = rmax.x; it.bmax[1] = rmax.y; it.bmax[2] = rmax.z;
-  it.pad2[0] = it.pad2[1] = 0.f;
-  items[0] = it;
-  uint32_t* lv = ctl + kCtlLevel(0);
-  lv[kLvM] = 1;
-  lv[kLvBig] = n > kChunk ? 1u : 0u;
-  lv[kLvCount] = 1;
-  ctl[kCtlFlags] = 0;
-}
-
-// par: the parity of the first level that did not run, whose node count is the total.
-__global__ void k_sah_finish(const uint32_t* __restrict__ ctl, uint32_t par, uint32_t* __restrict__ info) {
-  info[RK_INFO_NODE_COUNT] = ctl[kCtlLevel(par) + kLvCount];
-  info[RK_INFO_FLAGS] |= ctl[kCtlFlags];
-}
-
-__global__ __launch_bounds__(256) void k_boxes_iota(const uint4* __restrict__ faces, const float4* __restrict__ verts,
-                                                    uint32_t n, Box* __restrict__ boxes, uint32_t* __restrict__ idx) {
-  uint32_t k = blockIdx.x * 256 + threadIdx.x;
-  if (k >= n) return;
-  uint4 f = faces[k];
-  float4 v0 = verts[f.x], v1 = verts[f.y], v2 = verts[f.z];
-  float4* o = reinterpret_cast<float4*>(boxes + k);
-  o[0] = rk::min4(rk::min4(v0, v1), v2);
-  o[1] = rk::max4(rk::max4(v0, v1), v2);
-  idx[k] = k;
+#pragma unroll
+  for (uint32_t u = 0; u < kBoxPer; ++u) {
+    const uint32_t k = (blockIdx.x * kBoxPer + u) * kBoxThreads + threadIdx.x;
+    if (k >= s.n) continue;
+    const float4 v0 = verts[f[u].x], v1 = verts[f[u].y], v2 = verts[f[u].z];
+    Box x;
+    x.mn = rk::min4(rk::min4(v0, v1), v2);
+    x.mx = rk::max4(rk::max4(v0, v1), v2);
+    float4* o = reinterpret_cast<float4*>(boxes + k);
+    o[0] = x.mn;
+    o[1] = x.mx;
+    s.ids0[k] = k;
+    copy[k] = f[u];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      const int c = f2o(center_axis(x, q));
+      b[q] = min(b[q], c);
+      b[3 + q] = max(b[3 + q], c);
+    }
+  }
+  add_bounds(b, s.bnd1);
 }
 
 __global__ __launch_bounds__(256) void k_gather_faces2(const uint4* __restrict__ src, const uint32_t* __restrict__ idx,
@@ -876,19 +1233,19 @@ __global__ __launch_bounds__(256) void k_copy_faces2(const uint4* __restrict__ s
 
 extern "C" size_t rk_build_sah_workspace_size(uint32_t face_count, uint32_t existing_nodes) {
   size_t n = face_count ? face_count : 1;
-  size_t m = n + existing_nodes + 1;   // items per level
-  size_t big = n / kChunk + 1;         // items of more than kChunk faces per level
-  size_t T = n / kChunk + big + 1;     // chunks per level: their ceil(size / kChunk)
-  size_t b = 0;
-  b += rk_align_up(m * sizeof(Item)) * 2;
-  b += rk_align_up(m * 4);                         // chunk_base
-  b += rk_align_up(big * kAccWords * 4);           // accumulators
-  b += rk_align_up(m * sizeof(Decision));
-  b += rk_align_up(T * 4) * 3;                     // chunk_item, chunk_left, chunk_loff
-  b += rk_align_up(n * 4);                         // partition temp
-  b += rk_align_up(n * 16);                        // face reorder temp
-  b += rk_align_up(kCtlWords * 4);
-  b += rk_align_up((m / kEmitGroup + 1) * 4);      // internal items per emit group
+  size_t m = n + existing_nodes + 1;
+  size_t big = n / kChunk + 1;
+  size_t T = n / kChunk + big + 1;
+  size_t b = 0;  // more than rk_build_sah takes
+  b += rk_align_up(m * 48) * 2;
+  b += rk_align_up(m * 4);
+  b += rk_align_up(big * 3776);
+  b += rk_align_up(m * 80);
+  b += rk_align_up(T * 4) * 3;
+  b += rk_align_up(n * 4);
+  b += rk_align_up(n * 16);
+  b += rk_align_up(128);
+  b += rk_align_up((m / 1024 + 1) * 4);
   return b + 4096;
 }
 
@@ -897,9 +1254,10 @@ extern "C" size_t rk_build_sah_workspace_size(uint32_t face_count, uint32_t exis
 // (re)computed and the root is the mesh hitbox; existing_nodes > 0 (Hybrid):
 // boxes/indices come from the LBVH pass and every leaf among nodes[0,
 // existing_nodes) is refined. Faces are reordered by the final indices.
-// Synchronises 'stream' once per tree level once a level can hold more than
-// min(4096, n/256) items (the level's counts size the next launches); the
-// info words and the face reorder are queued on 'stream' when it returns.
+// Synchronises 'stream' a few times (once the levels that n faces cannot do
+// without are queued, then once per two levels of big items, then for the level
+// sizes); the node records and the info words are queued on 'stream' when it
+// returns.
 extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_float4* vertices, uint32_t face_count,
                                   const rk_aabox* hitbox, rk_aabox* boxes, uint32_t* indices, rk_bvnode* nodes,
                                   uint32_t existing_nodes, uint32_t nodes_capacity, uint32_t* info, void* ws,
@@ -909,112 +1267,142 @@ extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_fl
   if (n >= (1u << 30)) return RK_ERROR_UNSUPPORTED;
   if ((size_t)nodes_capacity < (size_t)existing_nodes + 2 * (size_t)n - 1) return RK_ERROR_INVALID_VALUE;
   hipStream_t st = rk_hip_stream(stream);
-  const size_t m_cap = (size_t)n + existing_nodes + 1;
-  const size_t big_cap = n / kChunk + 1;
-  const size_t T_cap = n / kChunk + big_cap + 1;
+  Sah s;
+  s.n = n;
+  s.m_cap = (size_t)n + existing_nodes + 1;
+  s.big_cap = n > kChunk ? n / kChunk + 1 : 0;
+  s.chunks_cap = n > kChunk ? n / kChunk + s.big_cap + 1 : 0;
+  s.group_cap = (uint32_t)(s.m_cap / kNumberItems + 1);
+  s.boxes = reinterpret_cast<const Box*>(boxes);
+  const size_t starts = existing_nodes ? existing_nodes : 1;
+  const size_t spare = 4096 + rk_align_up((s.m_cap / 1024 + 1) * 4) - (s.m_cap / 1024 + 1) * 4;
+  if (ws_bytes < rk_build_sah_workspace_size(n, existing_nodes) - spare) return RK_ERROR_WORKSPACE;
   RkArena ar(ws, ws_bytes);
-  Item* items_a = ar.take<Item>(m_cap);
-  Item* items_b = ar.take<Item>(m_cap);
-  uint32_t* chunk_base = ar.take<uint32_t>(m_cap);
-  int* acc = ar.take<int>(big_cap * kAccWords);
-  Decision* dec = ar.take<Decision>(m_cap);
-  uint32_t* chunk_item = ar.take<uint32_t>(T_cap);
-  uint32_t* chunk_left = ar.take<uint32_t>(T_cap);
-  uint32_t* chunk_loff = ar.take<uint32_t>(T_cap);
-  uint32_t* tmp = ar.take<uint32_t>(n);
+  s.ids0 = indices;
+  s.ids1 = ar.take<uint32_t>(n);
+  s.rec = ar.take<Rec>(2 * (size_t)n + starts);
+  s.link = ar.take<uint32_t>(2 * (size_t)n + starts);
+  s.node0 = ar.take<uint32_t>(starts);
+  s.q0 = ar.take<uint32_t>(2 * (size_t)n);
+  s.roots = ar.take<uint2>(kClasses * s.m_cap);
+  s.big0 = ar.take<BigItem>(2 * (size_t)s.big_cap);
+  s.dec = ar.take<BigDec>(s.big_cap);
+  s.chunk_item0 = ar.take<uint32_t>(2 * (size_t)s.chunks_cap);
+  s.acc = ar.take<int>((size_t)s.big_cap * kAccWords);
+  s.bnd0 = ar.take<int>((size_t)s.big_cap * 4 * kBoundWords);
+  s.cum = ar.take<uint16_t>((size_t)kBins * s.chunks_cap);
+  s.bin = ar.take<uint8_t>(n);
+  s.ctl = ar.take<uint32_t>(ctl_words(n));
+  s.groups = ar.take<uint32_t>(3 * (size_t)s.group_cap);
   uint4* ftmp = ar.take<uint4>(n);
-  uint32_t* ctl = ar.take<uint32_t>(kCtlWords);
-  uint32_t* group_internal = ar.take<uint32_t>(m_cap / kEmitGroup + 1);
-  if (!items_a || !items_b || !chunk_base || !acc || !dec || !chunk_item || !chunk_left || !chunk_loff || !tmp ||
-      !ftmp || !ctl || !group_internal)
+  if (!s.ids1 || !s.rec || !s.link || !s.node0 || !s.q0 || !s.roots || !s.big0 || !s.dec || !s.chunk_item0 || !s.acc ||
+      !s.bnd0 || !s.cum || !s.bin || !s.ctl || !s.groups || !ftmp)
     return RK_ERROR_WORKSPACE;
-  rk_status s;
-  if ((s = rk_fill_u32(stream, ctl, kCtlWords, 0u)) != RK_SUCCESS) return s;
-  if ((s = rk_fill_u32(stream, info, RK_INFO_WORDS, 0u)) != RK_SUCCESS) return s;
-  if (existing_nodes == 0) {
-    hipLaunchKernelGGL(k_boxes_iota, dim3((n + 255) / 256), dim3(256), 0, st, reinterpret_cast<const uint4*>(faces),
-                       reinterpret_cast<const float4*>(vertices), n, reinterpret_cast<Box*>(boxes), indices);
-    RK_CHECK_LAUNCH();
-    float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
-    float4 rmax = make_float4(hitbox->max.x, hitbox->max.y, hitbox->max.z, hitbox->max.w);
-    hipLaunchKernelGGL(k_sah_init_root, dim3(1), dim3(1), 0, st, items_a, ctl, n, rmin, rmax);
-  } else {
-    hipLaunchKernelGGL(k_sah_init_from_leaves, dim3(1), dim3(1024), 0, st, reinterpret_cast<const Node*>(nodes),
-                       existing_nodes, items_a, ctl);
-  }
+  s.q1 = s.q0 + n;
+  s.big1 = s.big0 + s.big_cap;
+  s.chunk_item1 = s.chunk_item0 + s.chunks_cap;
+  s.bnd1 = s.bnd0 + (size_t)s.big_cap * 2 * kBoundWords;
+
+  const bool root = existing_nodes == 0;
+  const float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
+  const float4 rmax = make_float4(hitbox->max.x, hitbox->max.y, hitbox->max.z, hitbox->max.w);
+  hipLaunchKernelGGL(k_sah_clear, dim3(std::min(1024u, s.big_cap + 1)), dim3(256), 0, st, s, info, root ? 1 : 0,
+                     rmin, rmax);
   RK_CHECK_LAUNCH();
-  // this level's item count and items of more than kChunk faces, or upper
-  // bounds of them while !exact
-  uint32_t lvh[2] = {0u, 0u};
-  RK_HIP(hipMemcpyAsync(lvh, ctl + kCtlLevel(0), sizeof(lvh), hipMemcpyDeviceToHost, st));
-  RK_HIP(hipStreamSynchronize(st));
-  uint32_t m = lvh[0], big = lvh[1];
-  bool exact = true;
-  // The first levels, while their item count is bounded by a few thousand,
-  // run without reading it back: a level has at most twice the items of the
-  // one before, and every kernel reads the exact counts on the device, so a
-  // grid sized by a bound is only larger than needed. From the first level
-  // beyond that bound on, the counts are read back after every level to size
-  // the next level's grids (and to skip the chunk kernels when no item has
-  // more than kChunk faces), and an empty level ends the build.
-  const uint32_t async_items = std::min<uint32_t>(4096u, n / 256);
-  const uint32_t big_bound = n / (kChunk + 1);
-  bool shallow = true;
-  Item* cur = items_a;
-  Item* nxt = items_b;
-  const Box* bx = reinterpret_cast<const Box*>(boxes);
-  Node* nd = reinterpret_cast<Node*>(nodes);
-  uint32_t level = 0;
-  for (; !(exact && m == 0); ++level) {
-    if (level > 4096) return RK_ERROR_LAUNCH;
-    const uint32_t par = level & 1u;
-    const unsigned grid = (unsigned)(n / kChunk + std::min(big, big_bound) + 1);  // chunks: see the workspace
-    hipLaunchKernelGGL(k_sah_prep, dim3(m ? (m + kPrepItems - 1) / kPrepItems : 1u), dim3(64 * kPrepItems), 0, st,
-                       cur, ctl, par, chunk_base, chunk_item, acc, group_internal);
-    if (big) {
-      hipLaunchKernelGGL(k_sah_bounds, dim3(grid), dim3(kCT), 0, st, cur, ctl, par, chunk_base, chunk_item, indices,
-                         bx, acc);
-      hipLaunchKernelGGL(k_sah_bins, dim3(grid), dim3(kCT), 0, st, cur, ctl, par, chunk_base, chunk_item, indices, bx,
-                         acc);
-      hipLaunchKernelGGL(k_sah_decide, dim3((m + kDecideItems - 1) / kDecideItems), dim3(256), 0, st, cur, ctl, par,
-                         acc, dec, group_internal);
-    }
-    hipLaunchKernelGGL(k_sah_small, dim3((m + kSmallWaves - 1) / kSmallWaves), dim3(64 * kSmallWaves), 0, st, cur,
-                       ctl, par, indices, bx, dec, group_internal);
-    hipLaunchKernelGGL(k_sah_emit, dim3(m ? (m + kEmitItems - 1) / kEmitItems : 1u), dim3(1024), 0, st, cur, ctl,
-                       par, dec, group_internal, nxt, nd, nodes_capacity);
-    if (big) {
-      hipLaunchKernelGGL(k_sah_count, dim3(grid), dim3(kCT), 0, st, cur, ctl, par, chunk_item, chunk_base, indices,
-                         bx, dec, chunk_left);
-      hipLaunchKernelGGL(k_sah_offsets, dim3((m + 3) / 4), dim3(256), 0, st, cur, ctl, par, chunk_base, chunk_left,
-                         chunk_loff);
-      hipLaunchKernelGGL(k_sah_scatter, dim3(grid), dim3(kCT), 0, st, cur, ctl, par, chunk_item, chunk_base, indices,
-                         bx, dec, chunk_loff, tmp);
-      hipLaunchKernelGGL(k_sah_copyback, dim3(grid), dim3(kCT), 0, st, cur, ctl, par, chunk_item, chunk_base, dec, tmp,
-                         indices);
-    }
-    RK_CHECK_LAUNCH();
-    const uint64_t bound = std::min<uint64_t>(2 * (uint64_t)m, m_cap);
-    if (shallow && bound <= async_items) {
-      m = (uint32_t)bound;
-      big = (uint32_t)std::min<uint64_t>(bound, big_bound);
-      exact = false;
-    } else {
-      shallow = false;
-      RK_HIP(hipMemcpyAsync(lvh, ctl + kCtlLevel(par ^ 1u), sizeof(lvh), hipMemcpyDeviceToHost, st));
-      RK_HIP(hipStreamSynchronize(st));
-      m = lvh[0];
-      big = lvh[1];
-      exact = true;
-    }
-    std::swap(cur, nxt);
-  }
-  hipLaunchKernelGGL(k_sah_finish, dim3(1), dim3(1), 0, st, ctl, level & 1u, info);
-  RK_CHECK_LAUNCH();
-  // CUDA_reorderMeshFaces, :778-784
   uint4* f = reinterpret_cast<uint4*>(faces);
-  hipLaunchKernelGGL(k_gather_faces2, dim3((n + 255) / 256), dim3(256), 0, st, f, indices, ftmp, n);
-  hipLaunchKernelGGL(k_copy_faces2, dim3((n + 255) / 256), dim3(256), 0, st, ftmp, f, n);
+  const unsigned per_face = (n + 255) / 256;
+  constexpr uint32_t kHistRead = 64;  // levels read at once
+  uint32_t got[kCtlHist + kHistRead] = {};
+  auto read_ctl = [&](size_t words) -> rk_status {
+    RK_HIP(hipMemcpyAsync(got, s.ctl, std::min(words, ctl_words(n)) * 4, hipMemcpyDeviceToHost, st));
+    RK_HIP(hipStreamSynchronize(st));
+    return RK_SUCCESS;
+  };
+  rk_status e;
+  // big: items of more than kChunk faces on the level, or a bound of them; ahead:
+  // levels to queue before the count is read back. A level has at most twice the
+  // big items of the one before, and every kernel reads the exact counts on the
+  // device, so a grid sized by a bound is only larger than needed. An item takes
+  // as many levels of big items as it takes halvings down to kChunk, and seldom
+  // more than two beyond; k_sah_subtrees is queued after those without a look, and
+  // again for what further levels leave. (Read back before it too: 50 us more per
+  // build.)
+  uint32_t big, ahead = 2, starts_found = 1, largest = n;
+  const uint32_t big_bound = n / (kChunk + 1);
+  if (root) {
+    hipLaunchKernelGGL(k_boxes_root, dim3((n + kBoxPer * kBoxThreads - 1) / (kBoxPer * kBoxThreads)), dim3(kBoxThreads),
+                       0, st, s, f, reinterpret_cast<const float4*>(vertices), reinterpret_cast<Box*>(boxes), ftmp);
+    RK_CHECK_LAUNCH();
+    big = n > kChunk ? 1u : 0u;
+  } else {
+    hipLaunchKernelGGL(k_sah_init_from_leaves, dim3(1), dim3(1024), 0, st, s, reinterpret_cast<const Node*>(nodes),
+                       existing_nodes);
+    hipLaunchKernelGGL(k_copy_faces2, dim3(per_face), dim3(256), 0, st, f, ftmp, n);
+    RK_CHECK_LAUNCH();
+    if ((e = read_ctl(kCtlRead)) != RK_SUCCESS) return e;
+    big = got[kCtlBig(0)];
+    starts_found = big + got[kCtlRoots] + got[kCtlRoots + 1] + got[kCtlRoots + 2];
+    largest = got[kCtlLargest];
+  }
+  for (uint32_t x = largest; x > kChunk; x -= x / 2) ++ahead;
+  RootsDone done = {};
+  uint32_t level = 0;
+  do {
+    for (uint32_t x = 0; x < ahead && big; ++x, ++level) {
+      if (level > kLevelMax) return RK_ERROR_LAUNCH;
+      const uint32_t par = level & 1u;
+      const unsigned grid = n / kChunk + std::min(big, big_bound) + 1;  // chunks: see chunks_cap
+      if (level == 0 && !root) hipLaunchKernelGGL(k_sah_bounds, dim3(grid), dim3(kCT), 0, st, s);
+      hipLaunchKernelGGL(k_sah_bins, dim3(grid), dim3(kCT), 0, st, s, par);
+      hipLaunchKernelGGL(k_sah_split, dim3((big + kSplitItems - 1) / kSplitItems), dim3(32 * kSplitItems), 0, st, s,
+                         par, level);
+      hipLaunchKernelGGL(k_sah_scatter, dim3(grid), dim3(kCT), 0, st, s, par);
+      RK_CHECK_LAUNCH();
+      big = std::min(2 * big, big_bound);
+    }
+    hipLaunchKernelGGL(k_sah_subtrees, dim3(std::min(2048u, n / 256 + 1)), dim3(kTreeThreads), 0, st, s, done);
+    RK_CHECK_LAUNCH();
+    if ((e = read_ctl(kCtlHist + kHistRead)) != RK_SUCCESS) return e;
+    big = level ? got[kCtlBig(level & 1u)] : 0u;
+    for (uint32_t c = 0; c < kClasses; ++c) done.n[c] = got[kCtlRoots + c];
+    ahead = 2;
+  } while (big);
+  // CUDA_reorderMeshFaces, :778-784
+  hipLaunchKernelGGL(k_gather_faces2, dim3(per_face), dim3(256), 0, st, ftmp, indices, f, n);
   RK_CHECK_LAUNCH();
+  // the numbering, by the levels' sizes
+  if (got[kCtlDeep]) return RK_ERROR_LAUNCH;
+  std::vector<uint32_t> hist(got + kCtlHist, got + kCtlHist + kHistRead);
+  if (hist.back()) {
+    hist.resize(ctl_words(n) - kCtlHist);
+    RK_HIP(hipMemcpyAsync(hist.data(), s.ctl + kCtlHist, hist.size() * 4, hipMemcpyDeviceToHost, st));
+    RK_HIP(hipStreamSynchronize(st));
+  }
+  hist.push_back(0u);
+  const uint32_t total = (root ? 1u : existing_nodes) + 2u * std::accumulate(hist.begin(), hist.end(), 0u);
+  Node* nd = reinterpret_cast<Node*>(nodes);
+  uint32_t m = starts_found, id0 = 0, child0 = root ? 1u : existing_nodes;
+  if (m > kNumberItems) {
+    hipLaunchKernelGGL(k_sah_number_start, dim3((m + kNumberItems - 1) / kNumberItems), dim3(1024), 0, st, s, m);
+    RK_CHECK_LAUNCH();
+  }
+  for (level = 0; m;) {
+    uint32_t end = level + 1;
+    uint32_t* out = level == 0 ? info : nullptr;
+    if (m <= kNumberItems) {
+      while (hist[end - 1] && 2 * hist[end - 1] <= kNumberItems) ++end;
+      hipLaunchKernelGGL(k_sah_number_run, dim3(1), dim3(1024), 0, st, s, level, end, m, id0, child0, nd,
+                         nodes_capacity, out, total);
+    } else {
+      hipLaunchKernelGGL(k_sah_number, dim3((m + kNumberItems - 1) / kNumberItems), dim3(1024), 0, st, s, level, m,
+                         id0, child0, nd, nodes_capacity, out, total);
+    }
+    RK_CHECK_LAUNCH();
+    for (; level < end; ++level) {
+      id0 = child0;
+      m = 2 * hist[level];
+      child0 += m;
+    }
+  }
   return RK_SUCCESS;
 }

@@ -1,7 +1,7 @@
 """The sort and the hierarchy pass at the sizes where their launches change: tiles
 and groups of tiles of the sort, the one-workgroup sort, runs and groups of runs of
-the hierarchy; and the reference topology where a level or the split lists stop
-fitting in LDS."""
+the hierarchy; the reference topology where a level or the split lists stop
+fitting in LDS; the SAH build where its items change hands."""
 import ctypes as C
 
 import numpy as np
@@ -140,3 +140,71 @@ def test_reference_topology_at_lds_edges(rk, ora, n, depth, complete, same):
     nodes = tree.nodes.cpu().numpy().view(np.uint32)[:m].copy().view(ora.NODE_DTYPE).reshape(m)
     for name in ("w0", "w1", "bmin", "bmax"):  # boxes as floats: -0 == +0
         assert np.array_equal(nodes[name], ref.nodes[name]), name
+
+
+def _chain(per):
+    """Faces at distances 2^-60 to 2^60 along each axis, 'per' to an octave: a SAH
+    tree of more than 64 levels."""
+    rng = np.random.default_rng(per)
+    c = np.zeros((3, 120, per, 3), np.float32)
+    for a in range(3):
+        c[a, :, :, a] = 2.0 ** np.arange(-60, 60)[:, None] * rng.uniform(1, 2, (120, per))
+    c = c.reshape(-1, 3)
+    d = np.abs(c).max(1, keepdims=True) * np.float32(2.0 ** -10)
+    corners = np.stack([c, c + d * np.array([1, 0, .5], np.float32), c + d * np.array([0, 1, .5], np.float32)], 1)
+    n = len(c)
+    V, F = np.zeros((3 * n, 4), np.float32), np.zeros((n, 4), np.uint32)
+    V[:, :3] = corners.reshape(-1, 3)
+    F[:, :3] = np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+    return V, F
+
+
+# items of 16, 128, 256, 512 and 1024 faces; chunks of 1024; levels of more than 1024 items
+@pytest.mark.parametrize("scene", [1, 16, 17, 127, 129, 256, 257, 511, 513, 1024, 1025, 2048, 2049, 70000, "chain4",
+                                   "chain40"])
+def test_sah_at_item_edges(rk, ora, scene):
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = _chain(int(scene[5:])) if isinstance(scene, str) else rk.soup(scene, seed=scene)
+    hb = rk.hitbox(V)
+    boxes, idx = ora.calc_boxes(F, V)
+    nodes, order, flags = ora.build_sah(boxes, idx, hb)
+    Ft = torch.from_numpy(F.view(np.int32).copy()).cuda()
+    tree = dev.build_sah(Ft, torch.from_numpy(V).cuda(), hb)
+    _compare_sah(rk, ora, F, Ft, tree, nodes, order, flags)
+
+
+@pytest.mark.parametrize("n,depth,complete", [(60000, 31, True), (60000, 8, False), (3000, 3, False), (17, 0, False)])
+def test_hybrid_at_item_edges(rk, ora, n, depth, complete):
+    """Thousands of small leaves, a few of thousands of faces, and one."""
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = rk.soup(n, seed=n + depth)
+    hb = rk.hitbox(V)
+    ref = ora.build_lbvh_ref(F, V, hb, depth, False)
+    if complete:
+        ref = ora.build_lbvh_ref(F, V, hb, depth, True)
+        F = ref.faces
+    boxes, idx = (ref.boxes, ref.indices) if not complete else ora.calc_boxes(F, V)
+    nodes, order, flags = ora.build_sah(boxes, idx, hb, ref.nodes, ref.node_count)
+    Ft, Vt = torch.from_numpy(F.view(np.int32).copy()).cuda(), torch.from_numpy(V).cuda()
+    lb = dev.build_lbvh(Ft, Vt, hb, depth, complete)
+    if complete:  # its faces are in tree order: boxes and ids of those
+        assert lb.node_count == ref.node_count
+        Ft = torch.from_numpy(F.view(np.int32).copy()).cuda()
+        lb.boxes.copy_(torch.from_numpy(boxes.reshape(lb.boxes.shape)))
+        lb.indices.copy_(torch.from_numpy(idx.view(np.int32).reshape(lb.indices.shape)))
+    tree = dev.build_sah(Ft, Vt, hb, lbvh=lb)
+    _compare_sah(rk, ora, F, Ft, tree, nodes, order, flags)
+
+
+def _compare_sah(rk, ora, F, Ft, tree, nodes, order, flags):
+    m = tree.node_count
+    assert m == nodes.shape[0] and int(tree.host_info()[rk.RK_INFO_FLAGS]) == flags
+    np.testing.assert_array_equal(tree.indices.cpu().numpy().view(np.uint32), order)
+    np.testing.assert_array_equal(Ft.cpu().numpy().view(np.uint32), F[order])
+    got = tree.nodes.cpu().numpy().view(np.uint32)[:m].copy().view(ora.NODE_DTYPE).reshape(m)
+    for name in ("w0", "w1", "bmin", "bmax"):
+        assert np.array_equal(got[name], nodes[name]), name
