@@ -494,8 +494,16 @@ __global__ __launch_bounds__(kChunk) void k_fast_hierarchy(const K* __restrict__
 // become the items of one run, completed as above; what is left over goes to
 // the group's first chunk. More items than threads are taken in steps, each
 // with the subtrees the one before left over in front.
-constexpr uint32_t kReduceFan = 64, kReduceThreads = 1024;
-template <typename K, bool kBatch>
+//
+// 1024 threads take 128 VGPRs each, so the workgroup waits for a whole CU to fall
+// free, which on a GPU full of another stream's traces takes as long as the traces
+// (a served frame's pass: 188 us of waiting). Few enough runs (kReduceSmall chunks
+// with about 12 subtrees each, kReduceSmallGroups groups with about 25) that 512
+// threads take them in one step as fast have half of that: 32 requests served in
+// 3.45 ms, with 1024 threads for all 3.58-3.74; with 512 for all the 1M-face build
+// takes 180 us, not 158.
+constexpr uint32_t kReduceFan = 64, kReduceSmall = 40, kReduceSmallGroups = 16;
+template <typename K, bool kBatch, uint32_t kReduceThreads>
 __global__ __launch_bounds__(kReduceThreads) void k_hier_reduce(const K* __restrict__ keys, uint32_t n,
                                                                 uint32_t leaf_max, uint32_t chunks, uint32_t stride,
                                                                 FNode* __restrict__ nodes,
@@ -606,8 +614,10 @@ constexpr int kStack = RK_TRACE_STACK;
 #define RK_LDS_STACK 8
 #endif
 // Stack entries per lane kept in LDS: 8 x 8 B x 64 lanes x 32 waves = 128 KB,
-// so the traces still run 32 waves per CU.
-constexpr int kLdsStack = RK_LDS_STACK;
+// so the traces still run 32 waves per CU. Incoherent rays go deeper: 9 entries,
+// which with the exchange are 5 KB per wave, just leave room for 32 waves and
+// are 2% faster on the 10M soup (12 entries and 25 waves: 8% slower than 9).
+constexpr int kLdsStack = RK_LDS_STACK, kDeepLdsStack = 9;
 
 // intersectTriRay, CUDA_raytraceMeshTree.cu:57-89, with vert0.w = edge1.w =
 // edge2.w = 0 (:174-176) and the reference's four-term dot products. eps is
@@ -684,8 +694,9 @@ struct RayHit {
 // an LDS access takes a fraction of the time of a scratch access that misses
 // the L1 (the scratch of thousands of resident lanes does not fit in it).
 // LDS words per wave for the exchange of pending subtrees: reference, entry
-// distance, owner lane and donor lane of each of up to 64 donations.
-constexpr int kXchgWords = 4 * 64;
+// distance, owner lane and donor lane of each donation. A step has at most 32: a
+// lane is a donor or idle, not both.
+constexpr int kXchg = 32, kXchgWords = 4 * kXchg;
 
 // kOldest: a donor hands out its oldest pending entry (the bottom of its
 // stack: the subtree nearest the root, the largest) instead of its newest, as
@@ -814,18 +825,18 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
           st_get(sp, r0, t0);
         }
         __hip_atomic_store(xchg + rd, r0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __hip_atomic_store(xchg + 64 + rd, __float_as_uint(t0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __hip_atomic_store(xchg + 128 + rd, (uint32_t)owner, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        __hip_atomic_store(xchg + 192 + rd, lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __hip_atomic_store(xchg + kXchg + rd, __float_as_uint(t0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __hip_atomic_store(xchg + 2 * kXchg + rd, (uint32_t)owner, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        __hip_atomic_store(xchg + 3 * kXchg + rd, lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
       }
       __builtin_amdgcn_wave_barrier();
       const bool take = !working && ri < nd;
       uint32_t g_ref = 0, g_t = 0, g_own = lane, g_don = lane;
       if (take) {
         g_ref = __hip_atomic_load(xchg + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        g_t = __hip_atomic_load(xchg + 64 + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        g_own = __hip_atomic_load(xchg + 128 + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-        g_don = __hip_atomic_load(xchg + 192 + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        g_t = __hip_atomic_load(xchg + kXchg + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        g_own = __hip_atomic_load(xchg + 2 * kXchg + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        g_don = __hip_atomic_load(xchg + 3 * kXchg + ri, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
       }
       __builtin_amdgcn_wave_barrier();
       // Every lane takes part in the exchange. The donor's job is a subtree of
@@ -1041,11 +1052,24 @@ constexpr int kTraceWG = RK_TRACE_WG;
 constexpr int kTraceDonateMin = RK_TRACE_DONATE_MIN;
 static_assert(kTraceWG % 64 == 0 && kTraceWG <= 1024, "whole waves");
 
+// Sorted rays of a tree that the eight L2s cannot hold between them: workgroups are
+// dealt to the XCDs in turn, so consecutive ones would fetch the same nodes into all
+// eight L2s. With kXcdRuns an XCD takes runs of kXcdRun consecutive workgroups of the
+// order. 16M rays on the 10M soup, with runs of 1, 32, 128, 512 and an eighth of
+// all: 29.3, 27.6, 27.0, 26.6 and 28.1 ms; 2M on 300k faces (34 MB): 1.668 and 1.627
+// with 1 and 512; 1M on 100k: 0.870 and 0.883.
+constexpr uint32_t kXcdRun = 512, kXcdFaces = 1u << 18;
+// And from this many faces on, where what bounds the trace is fetching nodes past
+// the L2, idle lanes take subtrees (which the owner might have culled) only on steps
+// where half the wave is idle: 16M rays on the 10M soup 26.6 -> 24.0 ms, 8M on 3M
+// faces 9.52 -> 9.01, 4M on 1M 3.83 -> 3.80; 2M on 300k 1.63 -> 1.65.
+constexpr uint32_t kFetchBoundFaces = 1u << 20;
+
 // kWG threads per workgroup, runs of kRun rays per band (spread_ray; 0: 64
 // consecutive rays per wave), kLds stack entries per lane in LDS. The
 // defaults above are one variant; rk_fast_autotune chooses among several.
 template <bool kCount, int kWG, uint32_t kRun, int kLds, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
-          int kBoundEvery = 1>
+          int kBoundEvery = 1, bool kXcdRuns = false>
 __global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
                                                       uint32_t n_tris, const float4* __restrict__ origins,
                                                       const float4* __restrict__ dirs, uint32_t n_rays,
@@ -1053,7 +1077,12 @@ __global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ 
                                                       float* __restrict__ depths, float eps,
                                                       unsigned long long* __restrict__ counters,
                                                       const uint32_t* __restrict__ order, uint32_t flags) {
-  const uint32_t t = blockIdx.x * kWG + threadIdx.x;
+  uint32_t block = blockIdx.x;
+  if (kXcdRuns) {
+    const uint32_t group = block / (8u * kXcdRun) * (8u * kXcdRun), i = block - group;
+    if (group + 8u * kXcdRun <= gridDim.x) block = group + (i & 7u) * kXcdRun + (i >> 3);
+  }
+  const uint32_t t = block * kWG + threadIdx.x;
   const bool reset = (flags & RK_TRACE_RESET_DEPTH) != 0u;
   const uint32_t l = order ? (t < n_rays ? order[t] : n_rays) : rk::band_ray<kRun>(t, n_rays);
   const bool has_ray = l < n_rays;
@@ -1114,9 +1143,14 @@ rk_status launch_hierarchy(hipStream_t st, const K* keys, const uint32_t* order,
   RK_CHECK_LAUNCH();
   uint32_t stride = 1;
   for (uint32_t groups = chunks; groups > 1; stride *= kReduceFan) {
+    const bool small = groups <= (stride == 1 ? kReduceSmall : kReduceSmallGroups);
     groups = blocks_for(groups, kReduceFan);
-    hipLaunchKernelGGL((k_hier_reduce<K, kBatch>), dim3(groups), dim3(kReduceThreads), 0, st, keys, n, leaf_max,
-                       chunks, stride, nodes, w.items, w.counts);
+    if (small)
+      hipLaunchKernelGGL((k_hier_reduce<K, kBatch, 512>), dim3(groups), dim3(512), 0, st, keys, n, leaf_max, chunks,
+                         stride, nodes, w.items, w.counts);
+    else
+      hipLaunchKernelGGL((k_hier_reduce<K, kBatch, 1024>), dim3(groups), dim3(1024), 0, st, keys, n, leaf_max, chunks,
+                         stride, nodes, w.items, w.counts);
     RK_CHECK_LAUNCH();
   }
   return RK_SUCCESS;
@@ -1369,7 +1403,7 @@ __device__ __forceinline__ void batch_trace_one(const rk_batch_mesh* __restrict_
   const uint32_t root = has_ray ? meshes[mesh_of_ray(meshes, mesh_count, r)].face_offset : 0u;
   const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   uint32_t nb = 0, nt = 0;
-  const RayHit h = trace_ray_shared<false, kStackN, kLdsStack, kWG, false, 0, kDM>(
+  const RayHit h = trace_ray_shared<false, kStackN, kDeepLdsStack, kWG, false, 0, kDM>(
       nodes, tris, n_tris, root, has_ray, has_ray ? origins[r] : zero4, has_ray ? dirs[r] : zero4,
       has_ray ? depths[r] : 0.0f, eps, nb, nt, lds_stack, xchg);
   if (has_ray && h.pos != 0xFFFFFFFFu) {
@@ -1391,7 +1425,7 @@ __global__ __launch_bounds__(kWG) void k_batch_trace_grid(const rk_batch_mesh* _
                                                           const uint32_t* __restrict__ order) {
   const uint32_t t = blockIdx.x * kWG + threadIdx.x;
   const uint32_t r = t < n_rays ? (order ? order[t] : t) : n_rays;
-  __shared__ uint2 s_stack[kLdsStack * kWG];
+  __shared__ uint2 s_stack[kDeepLdsStack * kWG];
   __shared__ uint32_t s_xchg[kWG / 64][kXchgWords];
   batch_trace_one<kStackN, kWG, kDM>(meshes, mesh_count, nodes, tris, n_tris, origins, dirs, r, n_rays, faces_id, coords,
                                 depths, eps, s_stack, s_xchg[threadIdx.x >> 6]);
@@ -1413,7 +1447,7 @@ __global__ __launch_bounds__(kWG) void k_batch_trace_queue(const rk_batch_mesh* 
                                                            float2* __restrict__ coords, float* __restrict__ depths,
                                                            float eps, uint32_t* __restrict__ queues,
                                                            const uint32_t* __restrict__ order) {
-  __shared__ uint2 s_stack[kLdsStack * kWG];
+  __shared__ uint2 s_stack[kDeepLdsStack * kWG];
   __shared__ uint32_t s_xchg[kWG / 64][kXchgWords];
   const uint32_t lane = threadIdx.x & 63;
   const uint32_t n_tiles = (n_rays + 63) / 64;
@@ -1556,8 +1590,12 @@ extern "C" rk_status rk_batch_trace(rk_stream stream, const rk_batch_mesh* meshe
     int dev = 0, cus = 0;
     RK_HIP(hipGetDevice(&dev));
     RK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    // 16 waves per CU, a multiple of the eight XCDs
-    grid_persistent = (uint32_t)cus * 16u * 64u / config->trace_wg;
+    // As many waves as are resident at once (32 per CU: the kernel waits on memory;
+    // the 1024-mesh batch takes 4.40 ms, with 16 per CU 5.12, 24 4.48), no more than
+    // there are tiles (100 meshes of at most 4096 rays: 0.39 ms, with 16 per CU 0.42,
+    // 32 0.47), in a multiple of the eight XCDs.
+    const uint32_t waves = std::min((uint32_t)cus * 32u, blocks_for(ray_count, 64));
+    grid_persistent = blocks_for(waves, config->trace_wg / 64);
     grid_persistent = (grid_persistent + kQueues - 1) / kQueues * kQueues;
   }
   const FNode* nodes = static_cast<const FNode*>(bvh->nodes);
@@ -2257,7 +2295,15 @@ extern "C" rk_status rk_fast_trace_sorted(rk_stream stream, const rk_fast_bvh* b
   s = rk_sort_run<uint32_t>(st, plan, false, nullptr);
   if (s != RK_SUCCESS) return s;
   // the variant's workgroup, stack and exchange settings; the order replaces its ray runs
-  hipLaunchKernelGGL(tv->kernel, dim3(blocks_for(n_rays, tv->wg)), dim3(tv->wg), 0, st, nodes,
+  const bool by_rule = !options || options->config == 0;
+  const TraceKernel kernel =
+      !by_rule ? tv->kernel
+      : bvh->face_count >= kFetchBoundFaces
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, 32, 1, true>
+      : bvh->face_count >= kXcdFaces
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, true>
+          : k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin>;
+  hipLaunchKernelGGL(kernel, dim3(blocks_for(n_rays, tv->wg)), dim3(tv->wg), 0, st, nodes,
                      static_cast<const float4*>(bvh->tris), bvh->face_count, o,
                      reinterpret_cast<const float4*>(directions), n_rays, faces_id, reinterpret_cast<float2*>(coords),
                      depths, det_eps_of(options), (unsigned long long*)nullptr, (const uint32_t*)order,

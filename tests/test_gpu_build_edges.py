@@ -69,7 +69,7 @@ def _expected(keys):
             for p in range(n - 1)}
 
 
-@pytest.mark.parametrize("n", [2, 3, 511, 512, 513, 1024, 1025, 64 * 512, 64 * 512 + 1, 70001])
+@pytest.mark.parametrize("n", [2, 3, 511, 512, 513, 1024, 1025, 40 * 512, 40 * 512 + 1, 64 * 512, 64 * 512 + 1, 70001])
 @pytest.mark.parametrize("kind", ["soup30", "soup63", "equal", "chain"])
 def test_hierarchy_topology_at_run_edges(rk, n, kind):
     """Every record of the tree against the tree computed from the sorted keys:
