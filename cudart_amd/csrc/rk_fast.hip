@@ -613,11 +613,13 @@ constexpr int kStack = RK_TRACE_STACK;
 #ifndef RK_LDS_STACK
 #define RK_LDS_STACK 8
 #endif
-// Stack entries per lane kept in LDS: 8 x 8 B x 64 lanes x 32 waves = 128 KB,
-// so the traces still run 32 waves per CU. Incoherent rays go deeper: 9 entries,
-// which with the exchange are 5 KB per wave, just leave room for 32 waves and
-// are 2% faster on the 10M soup (12 entries and 25 waves: 8% slower than 9).
-constexpr int kLdsStack = RK_LDS_STACK, kDeepLdsStack = 9;
+// Stack entries per lane kept in LDS: 8 x 8 B x 64 lanes is 4 KB per wave,
+// far within the 20 or 24 waves per CU that the traces' registers allow. Incoherent
+// rays go deeper: 12 entries in batches and sorted traces (1024-mesh batch with 9,
+// 12, 15, 19: 4.01, 3.96, 4.07, 4.09 ms; 1M rays on the 100k soup: 0.824, 0.788,
+// 0.823, 0.848), 15, all that 20 waves leave room for, on trees past the L2 (16M rays on
+// the 10M soup: 24.3, 24.8, 23.2, 23.7 ms).
+constexpr int kLdsStack = RK_LDS_STACK, kDeepLdsStack = 12, kDeepestLdsStack = 15;
 
 // intersectTriRay, CUDA_raytraceMeshTree.cu:57-89, with vert0.w = edge1.w =
 // edge2.w = 0 (:174-176) and the reference's four-term dot products. eps is
@@ -720,30 +722,31 @@ constexpr int kXchg = 32, kXchgWords = 4 * kXchg;
 // best (j_*), kept only if it can beat the owner's best as of this step (dmax,
 // d_hit). Ties on t go to the smaller original id. A macro, not a function: the
 // best-hit variables stay in registers only if no reference to them is taken.
-#define RK_LEAF_HITS(ref)                                                                              \
+#define RK_TRI_HIT(r0, e1, e2, position)                                                               \
   do {                                                                                                 \
-    const uint32_t first_ = ((ref) & ~kLeafBit) >> 4;                                                 \
-    const uint32_t cnt_ = first_ < n_tris ? min(((ref) & 15u) + 1, n_tris - first_) : 0u;             \
-    for (uint32_t k = 0; k < cnt_; ++k) {                                                              \
-      const float4 r0 = tris[3 * (size_t)(first_ + k) + 0];                                            \
-      float4 v0 = r0;                                                                                  \
-      v0.w = 0.0f;                                                                                     \
-      const float4 e1 = tris[3 * (size_t)(first_ + k) + 1], e2 = tris[3 * (size_t)(first_ + k) + 2];   \
-      float t, u, v;                                                                                   \
-      if (kCount) ++n_tri;                                                                             \
-      if (tri_ray(jo, jd, v0, e1, e2, eps, t, u, v)) {                                                 \
-        const uint32_t oid = __float_as_uint(r0.w);                                                    \
-        if (own) {                                                                                     \
-          if (t < o_t || (o_pos != 0xFFFFFFFFu && t == o_t && oid < o_oid)) {                          \
-            o_t = t; o_pos = first_ + k; o_oid = oid; o_u = u; o_v = v;                                \
-          }                                                                                            \
-        } else if ((t < dmax || (d_hit && t == dmax)) &&                                               \
-                   (j_pos == 0xFFFFFFFFu || t < j_t || (t == j_t && oid < j_oid))) {                   \
-          j_t = t; j_pos = first_ + k; j_oid = oid; j_u = u; j_v = v;                                  \
+    float4 v0 = r0;                                                                                    \
+    v0.w = 0.0f;                                                                                       \
+    float t, u, v;                                                                                     \
+    if (kCount) ++n_tri;                                                                               \
+    if (tri_ray(jo, jd, v0, e1, e2, eps, t, u, v)) {                                                   \
+      const uint32_t oid = __float_as_uint((r0).w);                                                    \
+      if (own) {                                                                                       \
+        if (t < o_t || (o_pos != 0xFFFFFFFFu && t == o_t && oid < o_oid)) {                            \
+          o_t = t; o_pos = (position); o_oid = oid; o_u = u; o_v = v;                                  \
         }                                                                                              \
+      } else if ((t < dmax || (d_hit && t == dmax)) &&                                                 \
+                 (j_pos == 0xFFFFFFFFu || t < j_t || (t == j_t && oid < j_oid))) {                     \
+        j_t = t; j_pos = (position); j_oid = oid; j_u = u; j_v = v;                                    \
       }                                                                                                \
     }                                                                                                  \
   } while (0)
+// Faces from..cnt - 1 of the leaf at position 'first'.
+#define RK_LEAF_HITS(first, from, cnt)                                                                 \
+  for (uint32_t k = (from); k < (cnt); ++k) {                                                          \
+    const float4* tri_ = tris + 3 * (size_t)((first) + k);                                             \
+    const float4 a_ = tri_[0], b_ = tri_[1], c_ = tri_[2];                                             \
+    RK_TRI_HIT(a_, b_, c_, (first) + k);                                                               \
+  }
 
 //
 // kBoundEvery: helpers read their owner's best so far on every kBoundEvery-th
@@ -870,6 +873,27 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
       }
     }
     const bool own = owner == (int)lane;
+    // This step's record, a node or a leaf's first triangle, is fetched here for
+    // both kinds of lanes, with one wait where there would be one in each branch,
+    // and meanwhile the owner's bound is read. It takes 86 registers, not 64, and
+    // 20 waves per CU that wait once are faster than 32 that wait twice: the
+    // 1024-mesh batch 4.35 -> 4.01 ms, the 256x256 icosphere frame 71 -> 62 us (more so
+    // the fewer waves there are), 32 served requests 3.50 -> 3.10 ms. The 1920x1080
+    // heightfield frame: 192 us -> 190, and 179 with 80 registers and 24 waves
+    // (k_fast_trace_v's bounds; there the others are slower: batch 4.7 ms).
+    const bool at_leaf = (cur & kLeafBit) != 0u;
+    const uint32_t first = (cur & ~kLeafBit) >> 4;
+    const uint32_t cnt = at_leaf && first < n_tris ? min((cur & 15u) + 1u, n_tris - first) : 0u;
+    const bool leaf_now = kLeafBatch == 0 && cnt != 0u;
+    float4 q0, q1, q2;
+    float2 q3;
+    if (owner >= 0 && (at_leaf ? leaf_now : cur < n_tris)) {
+      const float4* rec = at_leaf ? tris + 3 * (size_t)first : reinterpret_cast<const float4*>(nodes + cur);
+      q0 = rec[0];
+      q1 = rec[1];
+      q2 = rec[2];
+      if (!at_leaf) q3 = *reinterpret_cast<const float2*>(rec + 3);
+    }
     // the owner's best so far bounds a helper's subtree
     float dmax = o_t;
     bool d_hit = o_pos != 0xFFFFFFFFu;
@@ -900,11 +924,15 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
       if (++visits > max_visits) {
         job_end = true;
         pend = 0u;
-      } else if (!(cur & kLeafBit)) {
+      } else if (!at_leaf) {
         if (cur >= n_tris) {
           job_end = true;  // never taken for a tree built here
         } else {
-          const FNode nd = nodes[cur];
+          FNode nd;
+          nd.a = q0;
+          nd.b = q1;
+          nd.c = q2;
+          nd.d = make_uint4(__float_as_uint(q3.x), __float_as_uint(q3.y), 0u, 0u);
           const Slab2 sl = slab2(nd, ix, iy, iz, ox, oy, oz, bound);
           const float tmin0 = sl.tmin0, tmin1 = sl.tmin1;
           const bool h0 = sl.h0, h1 = sl.h1;
@@ -925,7 +953,10 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
           }
         }
       } else if (kLeafBatch == 0) {
-        RK_LEAF_HITS(cur);
+        if (leaf_now) {
+          RK_TRI_HIT(q0, q1, q2, first);
+          RK_LEAF_HITS(first, 1u, cnt);
+        }
         need_pop = true;
       } else if (pend == 0u) {
         pend = cur;  // postponed: go on to the next pending subtree
@@ -962,7 +993,9 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
       const uint64_t pm = __ballot(pend != 0u);
       if (pm != 0ull && (__ballot(flush_me) != 0ull || __popcll(pm) >= kLeafBatch)) {
         if (pend != 0u) {
-          RK_LEAF_HITS(pend);
+          const uint32_t p_first = (pend & ~kLeafBit) >> 4;
+          const uint32_t p_cnt = p_first < n_tris ? min((pend & 15u) + 1u, n_tris - p_first) : 0u;
+          RK_LEAF_HITS(p_first, 0u, p_cnt);
           pend = 0u;
         }
         if (end_after) job_end = true;
@@ -986,6 +1019,7 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
   return RayHit{o_pos, o_t, o_u, o_v};
 }
 #undef RK_LEAF_HITS
+#undef RK_TRI_HIT
 
 // Sort key of a ray: the 30-bit Morton code of its origin in the tree's root
 // box (the union of the root record's two child boxes), clamped to the box.
@@ -1070,7 +1104,7 @@ constexpr uint32_t kFetchBoundFaces = 1u << 20;
 // defaults above are one variant; rk_fast_autotune chooses among several.
 template <bool kCount, int kWG, uint32_t kRun, int kLds, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
           int kBoundEvery = 1, bool kXcdRuns = false>
-__global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
+__global__ __launch_bounds__(kWG, kLds > kLdsStack ? 5 : 6) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
                                                       uint32_t n_tris, const float4* __restrict__ origins,
                                                       const float4* __restrict__ dirs, uint32_t n_rays,
                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
@@ -1868,8 +1902,16 @@ __device__ __forceinline__ bool camera_pixel(int width, int height, int& x, int&
 // reference's CUDA_calcPrimaryRays.cu:43-55 formula: origin, and direction
 // (dir - x * step_x) - y * step_y), so a frame reads no ray arrays. Every pixel is written:
 // a miss gives face ~0, coords (0, 0), depth FLT_MAX.
-template <int kWG, int kBands, bool kXcd, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1>
-__global__ __launch_bounds__(kWG) void k_fast_trace_camera_v(const FNode* __restrict__ nodes,
+//
+// kWaves: waves per SIMD to leave registers for. 6 (80 registers) for the variants
+// and frames of more than kSmallFrame pixels, 5 (86) for those whose waves all fit at
+// 5: the 256x256 icosphere frame 59.6 us with 5, 61.5 with 6, 512x512 heightfield 65.5
+// and 67.1, 1280x720 98.6 and 96.7, 1920x1080 184.9 and 177.9, 1280x720 icosphere 110.2
+// and 100.3.
+constexpr uint64_t kSmallFrame = 5 * 1024 * 64;
+template <int kWG, int kBands, bool kXcd, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
+          int kWaves = 6>
+__global__ __launch_bounds__(kWG, kWaves) void k_fast_trace_camera_v(const FNode* __restrict__ nodes,
                                                              const float4* __restrict__ tris, uint32_t n_tris,
                                                              float4 ro, float4 rd, float4 rx, float4 ry, int width,
                                                              int height, uint32_t* __restrict__ faces_id,
@@ -1900,8 +1942,8 @@ __global__ __launch_bounds__(kWG) void k_fast_trace_camera_v(const FNode* __rest
 // theirs. faces: the mesh's faces in the tree's leaf order (faces[position]),
 // as the reference's builds leave them. faces_id, coords and depths, when not
 // NULL, receive what k_fast_trace_camera_v writes.
-template <int kWG, int kBands, int kDM>
-__global__ __launch_bounds__(kWG) void k_fast_render_camera(
+template <int kWG, int kBands, int kDM, int kWaves>
+__global__ __launch_bounds__(kWG, kWaves) void k_fast_render_camera(
     const FNode* __restrict__ nodes, const float4* __restrict__ tris, uint32_t n_tris, float4 ro, float4 rd,
     float4 rx, float4 ry, int width, int height, const uint4* __restrict__ faces, const float4* __restrict__ verts,
     const float4* __restrict__ norms, float4 back, float4 cam, uint32_t* __restrict__ pixels, int pitch,
@@ -2187,7 +2229,10 @@ extern "C" rk_status rk_fast_trace_camera(rk_stream stream, const rk_fast_bvh* b
   const CameraVariant* cv = camera_variant(options ? options->config : 0u);
   if (!cv) return RK_ERROR_INVALID_VALUE;
   dim3 grid(camera_blocks(width, height, (int)cv->wg, (int)cv->bands, cv->xcd != 0));
-  hipLaunchKernelGGL(cv->kernel, grid, dim3(cv->wg), 0, rk_hip_stream(stream), static_cast<const FNode*>(bvh->nodes),
+  const bool small = (!options || options->config == 0) && (uint64_t)width * (uint64_t)height <= kSmallFrame;
+  const CameraKernel kernel =
+      small ? k_fast_trace_camera_v<kTraceWG, kCamBands, false, false, 0, kTraceDonateMin, 5> : cv->kernel;
+  hipLaunchKernelGGL(kernel, grid, dim3(cv->wg), 0, rk_hip_stream(stream), static_cast<const FNode*>(bvh->nodes),
                      static_cast<const float4*>(bvh->tris), bvh->face_count, f4(camera->origin),
                      f4(camera->direction), f4(camera->step_x), f4(camera->step_y), width, height, faces_id,
                      reinterpret_cast<float2*>(coords), depths, det_eps_of(options));
@@ -2208,7 +2253,10 @@ extern "C" rk_status rk_fast_render_camera(rk_stream stream, const rk_fast_bvh* 
     return RK_ERROR_UNSUPPORTED;
   auto f4 = [](const rk_float4& v) { return make_float4(v.x, v.y, v.z, v.w); };
   dim3 grid(camera_blocks(width, height, kTraceWG, kCamBands, false));
-  hipLaunchKernelGGL((k_fast_render_camera<kTraceWG, kCamBands, kTraceDonateMin>), grid, dim3(kTraceWG), 0,
+  const auto kernel = (uint64_t)width * (uint64_t)height <= kSmallFrame
+                          ? k_fast_render_camera<kTraceWG, kCamBands, kTraceDonateMin, 5>
+                          : k_fast_render_camera<kTraceWG, kCamBands, kTraceDonateMin, 6>;
+  hipLaunchKernelGGL(kernel, grid, dim3(kTraceWG), 0,
                      rk_hip_stream(stream), static_cast<const FNode*>(bvh->nodes),
                      static_cast<const float4*>(bvh->tris), bvh->face_count, f4(camera->origin),
                      f4(camera->direction), f4(camera->step_x), f4(camera->step_y), width, height,
@@ -2299,7 +2347,7 @@ extern "C" rk_status rk_fast_trace_sorted(rk_stream stream, const rk_fast_bvh* b
   const TraceKernel kernel =
       !by_rule ? tv->kernel
       : bvh->face_count >= kFetchBoundFaces
-          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, 32, 1, true>
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32, 1, true>
       : bvh->face_count >= kXcdFaces
           ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, true>
           : k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin>;
