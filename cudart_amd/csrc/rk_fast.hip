@@ -1624,11 +1624,10 @@ extern "C" rk_status rk_batch_trace(rk_stream stream, const rk_batch_mesh* meshe
     int dev = 0, cus = 0;
     RK_HIP(hipGetDevice(&dev));
     RK_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-    // As many waves as are resident at once (32 per CU: the kernel waits on memory;
-    // the 1024-mesh batch takes 4.40 ms, with 16 per CU 5.12, 24 4.48), no more than
-    // there are tiles (100 meshes of at most 4096 rays: 0.39 ms, with 16 per CU 0.42,
-    // 32 0.47), in a multiple of the eight XCDs.
-    const uint32_t waves = std::min((uint32_t)cus * 32u, blocks_for(ray_count, 64));
+    // As many waves as are resident at once (20 per CU; the 1024-mesh batch takes 3.99
+    // ms, with 16 per CU 4.12, 32 3.99), no more than there are tiles (100 meshes of at
+    // most 4096 rays: without this limit 0.06 ms more), in a multiple of the eight XCDs.
+    const uint32_t waves = std::min((uint32_t)cus * 20u, blocks_for(ray_count, 64));
     grid_persistent = blocks_for(waves, config->trace_wg / 64);
     grid_persistent = (grid_persistent + kQueues - 1) / kQueues * kQueues;
   }

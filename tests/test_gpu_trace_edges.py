@@ -1,7 +1,8 @@
 """Traces where their launches change. Sorted: at 2^18 faces an XCD takes runs of
 512 workgroups (groups of 8 runs, 262144 rays; a remainder in plain order), at 2^20
 idle lanes help later. Camera frames: at 327680 pixels. The closest hit does not
-depend on any: bit-equal to the trace in ray order."""
+depend on any: bit-equal to the trace in ray order. The reference's per-ray walk:
+tiles of 16 x 4 rays, whole, cut at an edge, and refused for too many idle lanes."""
 import numpy as np
 import pytest
 
@@ -40,3 +41,22 @@ def test_camera_equals_rays(rk, w, h, leaf_max):
     hit = b[2] < torch.finfo(torch.float32).max
     assert torch.equal(a[2], b[2]) and (w == 1 or bool(hit.any()))
     assert torch.equal(a[0][hit], b[0][hit]) and torch.equal(a[1][hit], b[1][hit])
+
+
+@pytest.mark.parametrize("w,h", [(64, 48), (120, 64), (128, 50), (67, 50), (16, 4), (15, 4), (1000, 1), (1, 1000)])
+def test_reference_rays_in_tiles(rk, ora, w, h):
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = rk.soup(3000, seed=w, mu=float(np.log(0.1)))
+    hb = rk.hitbox(V)
+    ref = ora.build_lbvh_ref(F, V, hb, 12, True)
+    Ft, Vt = torch.from_numpy(F.view(np.int32)).cuda(), torch.from_numpy(V).cuda()
+    tree = dev.build_lbvh(Ft, Vt, hb, 12, True)
+    O, D = rk.random_rays(w * h, seed=h)
+    of, ouv, od, _ = ora.trace_ref_ray(ref.nodes, ref.faces, V, O, D)
+    out = dev.trace_ref(tree, Vt, torch.from_numpy(O).cuda(), torch.from_numpy(D).cuda(), w, h, False)
+    got = [t.cpu().numpy() for t in out]
+    np.testing.assert_array_equal(got[0].view(np.uint32), of)
+    np.testing.assert_array_equal(got[1], ouv)
+    np.testing.assert_array_equal(got[2], od)
