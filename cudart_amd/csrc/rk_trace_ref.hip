@@ -598,24 +598,23 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
   }
 }
 
-// Clears the head's counters and the groups' pops.
-__global__ __launch_bounds__(256) void k_handoff_clear(uint32_t* __restrict__ handoff, unsigned long long* __restrict__ pops,
-                                                       uint32_t groups) {
-  const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-  if (t < kHandoffHead) handoff[t] = 0u;
-  if (t < groups) pops[t] = 0ull;
-}
-
 // The cut: one workgroup per octant expands the tree level by level, in walk
 // order, down to kUnitLevel; a leaf or a child out of range ends where it is.
 // The reference's stack holds, after it pops a node, one far child for every
-// near step on the path to it.
+// near step on the path to it. The workgroups after the first eight clear the
+// head's counters and the groups' pops.
 __global__ __launch_bounds__(256) void k_units_cut(const rk::Node* __restrict__ nodes, uint32_t node_count,
-                                                   const uint32_t* __restrict__ handoff, UnitCut* __restrict__ cut) {
+                                                   UnitCut* __restrict__ cut, uint32_t* __restrict__ handoff,
+                                                   unsigned long long* __restrict__ pops, uint32_t groups) {
   static_assert(kUnits <= 256, "one thread per subtree");
   __shared__ uint32_t s_node[kUnits], s_sp[kUnits], s_wave[4];
   constexpr uint32_t kDone = 0x80000000u;
-  if (handoff[1] == 0u && handoff[2] == 0u) return;  // nothing to walk
+  if (blockIdx.x >= 8u) {
+    const uint32_t i = (blockIdx.x - 8u) * 256 + threadIdx.x;
+    if (i < kHandoffHead) handoff[i] = 0u;
+    if (i < groups) pops[i] = 0ull;
+    return;
+  }
   const uint32_t o = blockIdx.x, t = threadIdx.x, lane = t & 63u, wv = t >> 6;
   uint32_t n = 1, tops = 0;
   if (t == 0) {
@@ -1083,6 +1082,30 @@ __global__ __launch_bounds__(64) void k_units_merge(uint32_t node_count, uint32_
 // back on top, sp and the visits before that leaf's pop (so that the second
 // pass, given the record as resume, makes the same pops from there). Returns
 // whether it was.
+//
+// Leaves of at most kPlainLeaf faces: the second pass tests a part's share of the
+// faces as they are. Finding the groups of faces a ray is near costs one more round
+// trip to memory per leaf, and round trips are what a pass over few packets is made
+// of: a 93x52 frame of a small heightfield takes 1.50 ms with the groups, 1.09 so
+// (loads of 2 faces in flight; 4: 1.15), the 1920x1080 frame the same with both. The
+// first pass, which has many packets, does so for leaves of at most a group (a
+// 1528x859 frame of the 1,280-face sphere: 218 -> 201 us; 24 and 48 faces: no gain).
+constexpr uint32_t kPlainLeaf = 96, kPlainBatch = 2;
+__device__ __forceinline__ void plain_leaf(const RefMesh& mesh, uint32_t f, uint32_t end, float4 o, float4 d,
+                                           float& depth, uint32_t& fid, float2& coord) {
+  for (; f < end; f += kPlainBatch) {
+    float4 v0[kPlainBatch], e1[kPlainBatch], e2[kPlainBatch];
+#pragma unroll
+    for (uint32_t b = 0; b < kPlainBatch; ++b) tri_get(mesh, min(f + b, end - 1u), v0[b], e1[b], e2[b]);
+#pragma unroll
+    for (uint32_t b = 0; b < kPlainBatch; ++b) {
+      float t, u, v;
+      if (f + b < end && tri_ray(o, d, v0[b], e1[b], e2[b], t, u, v)) {
+        if (t < depth) { fid = f + b; coord = make_float2(u, v); depth = t; }
+      }
+    }
+  }
+}
 template <int kS>
 __device__ __forceinline__ bool trace_packet_job(
     const rk::Node* __restrict__ nodes, RefMesh mesh,
@@ -1198,19 +1221,23 @@ __device__ __forceinline__ bool trace_packet_job(
         }
       }
       if (kS == 1) {
-        if (in_image) lane_leaf(mesh, tri_id, cnt, orig, dir, cr, depth, fid, coord);
+        if (in_image) {
+          if (cnt <= kGroup) plain_leaf(mesh, tri_id, tri_id + cnt, orig, dir, depth, fid, coord);
+          else lane_leaf(mesh, tri_id, cnt, orig, dir, cr, depth, fid, coord);
+        }
       } else {
-        // part p: an equal run of the leaf's groups of faces
-        const uint32_t end = tri_id + cnt, g_first = tri_id / kGroup;
-        const uint32_t ng = cnt ? (end - 1u) / kGroup + 1u - g_first : 0u, q = (ng + kS - 1) / kS;
+        // part p: an equal run of the leaf's faces, or of its groups of faces
+        const uint32_t end = tri_id + cnt, unit = cnt <= kPlainLeaf ? 1u : kGroup, g_first = tri_id / unit;
+        const uint32_t ng = cnt ? (end - 1u) / unit + 1u - g_first : 0u, q = (ng + kS - 1) / kS;
         const uint32_t ga = min((uint32_t)part * q, ng), gb = min(ga + q, ng);
         float pt = depth;
         float2 puv = make_float2(0.0f, 0.0f);
         uint32_t pk = 0xffffffffu;  // none
         if (in_image && ga < gb) {
-          const uint32_t a = max(tri_id, (g_first + ga) * kGroup);
-          const uint32_t m = gb == ng ? end - a : (g_first + gb) * kGroup - a;
-          lane_leaf(mesh, a, m, orig, dir, cr, pt, pk, puv);
+          const uint32_t a = max(tri_id, (g_first + ga) * unit);
+          const uint32_t m = gb == ng ? end - a : (g_first + gb) * unit - a;
+          if (unit == 1u) plain_leaf(mesh, a, a + m, orig, dir, pt, pk, puv);
+          else lane_leaf(mesh, a, m, orig, dir, cr, pt, pk, puv);
         }
         s_pt[threadIdx.x] = pt;
         s_pu[threadIdx.x] = puv.x;
@@ -1407,11 +1434,12 @@ static hipMemPool_t handoff_pool() {
 }
 
 // The hand-off buffer of one call (words 32-bit words), its counters and its
-// groups' pops (at word pops_off) cleared:
+// groups' pops (at word pops_off) cleared, the tree's cut made (at cut_off):
 // a stream-ordered allocation, so that calls on other streams have their own.
 // Without it (nullptr) every ray or packet stays in the first pass, with the
 // same results.
-static uint32_t* handoff_alloc(hipStream_t st, size_t words, size_t pops_off, uint32_t groups, uint32_t faces) {
+static uint32_t* handoff_alloc(hipStream_t st, size_t words, size_t pops_off, uint32_t groups, size_t cut_off,
+                               const rk_bvnode* nodes, uint32_t node_count, uint32_t faces) {
   uint32_t* ho = nullptr;
   if (faces == kNoHandoff || words <= kHandoffHead) return nullptr;
   hipMemPool_t pool = handoff_pool();
@@ -1422,7 +1450,8 @@ static uint32_t* handoff_alloc(hipStream_t st, size_t words, size_t pops_off, ui
     (void)hipGetLastError();
     return nullptr;
   }
-  hipLaunchKernelGGL(k_handoff_clear, dim3((std::max(groups, kHandoffHead) + 255) / 256), dim3(256), 0, st, ho,
+  hipLaunchKernelGGL(k_units_cut, dim3(8 + (std::max(groups, kHandoffHead) + 255) / 256), dim3(256), 0, st,
+                     reinterpret_cast<const rk::Node*>(nodes), node_count, reinterpret_cast<UnitCut*>(ho + cut_off), ho,
                      reinterpret_cast<unsigned long long*>(ho + pops_off), groups);
   return ho;
 }
@@ -1483,8 +1512,8 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
     const size_t cut_off = flist_off + (2ull + kPT) * fcap;
     const size_t hits_off = cut_off + sizeof(UnitCut) / 4;
     const uint32_t hit_cap = kHitsPerSlot * kPT * fcap;
-    uint32_t* ho = handoff_alloc(st, hits_off + hit_cap * (sizeof(UnitHit) / 4), pops_off, kPGroups * fcap,
-                                 faces_limit);
+    uint32_t* ho = handoff_alloc(st, hits_off + hit_cap * (sizeof(UnitHit) / 4), pops_off, kPGroups * fcap, cut_off,
+                                 nodes, node_count, faces_limit);
     UnitArgs ua{};
     PacketArgs pa{width, height, (int)gx, cap, ho ? ho + flist_off : nullptr};
     if (ho) {
@@ -1506,7 +1535,6 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
                        face_count, faces_id, uv, depths, ho, ho ? cap : 0u, faces_limit, ho ? ho + flist_off : nullptr,
                        ua);
     if (ho) {
-      hipLaunchKernelGGL(k_units_cut, dim3(8), dim3(256), 0, st, nd, node_count, ho, ua.cut);
       hipLaunchKernelGGL(k_unit_walk<true>, dim3(kUnitGrid), dim3(64), 0, st, nd, mesh, org, drs, depths, node_count,
                          face_count, ho, ua, pa);
       hipLaunchKernelGGL(k_packet_commit, dim3(fcap), dim3(kPT), 0, st, node_count, drs, ho, ua, pa, faces_id, uv,
@@ -1532,7 +1560,8 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
     const size_t cut_off = list_off + 12ull * ucap;
     const size_t hits_off = cut_off + sizeof(UnitCut) / 4;
     const uint32_t hit_cap = kHitsPerRay * ucap;
-    uint32_t* ho = handoff_alloc(st, hits_off + hit_cap * (sizeof(UnitHit) / 4), pops_off, groups, faces_limit);
+    uint32_t* ho = handoff_alloc(st, hits_off + hit_cap * (sizeof(UnitHit) / 4), pops_off, groups, cut_off, nodes,
+                                 node_count, faces_limit);
     UnitArgs ua{};
     if (ho) {
       uint32_t* p = ho + list_off;
@@ -1559,7 +1588,6 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
                        (uint32_t)height, tiles_x, node_count, face_count, faces_id, uv, depths, ho, ho ? cap : 0u,
                        faces_limit, ua);
     if (ho) {
-      hipLaunchKernelGGL(k_units_cut, dim3(8), dim3(256), 0, st, nd, node_count, ho, ua.cut);
       hipLaunchKernelGGL(k_unit_walk<false>, dim3(kUnitGrid), dim3(64), 0, st, nd, mesh, org, drs, depths, node_count,
                          face_count, ho, ua, PacketArgs{});
       hipLaunchKernelGGL(k_units_merge, dim3((ucap + 63) / 64), dim3(64), 0, st, node_count, ho, ua, faces_id, uv,
