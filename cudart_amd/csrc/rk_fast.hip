@@ -614,7 +614,7 @@ constexpr int kStack = RK_TRACE_STACK;
 #define RK_LDS_STACK 8
 #endif
 // Stack entries per lane kept in LDS: 8 x 8 B x 64 lanes is 4 KB per wave,
-// far within the 20 or 24 waves per CU that the traces' registers allow. Incoherent
+// far within the 20 waves per CU that the traces' registers allow. Incoherent
 // rays go deeper: 12 entries in batches and sorted traces (1024-mesh batch with 9,
 // 12, 15, 19: 4.01, 3.96, 4.07, 4.09 ms; 1M rays on the 100k soup: 0.824, 0.788,
 // 0.823, 0.848), 15, all that 20 waves leave room for, on trees past the L2 (16M rays on
@@ -770,7 +770,7 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
   float ix = safe_inv(jd.x), iy = safe_inv(jd.y), iz = safe_inv(jd.z);
   float ox = jo.x * ix, oy = jo.y * iy, oz = jo.z * iz;
   uint32_t j_pos = 0xFFFFFFFFu, j_oid = 0xFFFFFFFFu;
-  float j_t = 0.0f, j_u = 0.0f, j_v = 0.0f;
+  float j_t = RK_HUGE, j_u = 0.0f, j_v = 0.0f;
   uint32_t cur = root, visits = 0;
   uint32_t pend = 0u;  // a postponed leaf (a leaf reference always has kLeafBit set; 0: none)
   uint32_t step = 0;   // loop steps so far (the same in every lane)
@@ -869,26 +869,28 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
         sb = 0;
         visits = 0;
         j_pos = 0xFFFFFFFFu;
+        j_t = RK_HUGE;
         j_oid = 0xFFFFFFFFu;
       }
     }
     const bool own = owner == (int)lane;
     // This step's record, a node or a leaf's first triangle, is fetched here for
     // both kinds of lanes, with one wait where there would be one in each branch,
-    // and meanwhile the owner's bound is read. It takes 86 registers, not 64, and
-    // 20 waves per CU that wait once are faster than 32 that wait twice: the
-    // 1024-mesh batch 4.35 -> 4.01 ms, the 256x256 icosphere frame 71 -> 62 us (more so
-    // the fewer waves there are), 32 served requests 3.50 -> 3.10 ms. The 1920x1080
-    // heightfield frame: 192 us -> 190, and 179 with 80 registers and 24 waves
-    // (k_fast_trace_v's bounds; there the others are slower: batch 4.7 ms).
+    // and meanwhile the owner's bound is read; its address is computed without a
+    // branch. It takes 86 registers, not 64, and 20 waves per CU that wait once are
+    // faster than 32 that wait twice: the 1024-mesh batch 4.35 -> 3.95 ms, the 1920x1080
+    // heightfield frame 192 -> 167 us (179 with branches for the address, and then the
+    // 1380x1035 frame of a small heightfield 82 -> 90; 24 waves: no better), the
+    // 256x256 icosphere frame 63 -> 55, 32 served requests 3.50 -> 3.03 ms.
     const bool at_leaf = (cur & kLeafBit) != 0u;
     const uint32_t first = (cur & ~kLeafBit) >> 4;
-    const uint32_t cnt = at_leaf && first < n_tris ? min((cur & 15u) + 1u, n_tris - first) : 0u;
-    const bool leaf_now = kLeafBatch == 0 && cnt != 0u;
+    const uint32_t idx = at_leaf ? first : cur;
+    const bool in_tree = idx < n_tris;
     float4 q0, q1, q2;
     float2 q3;
-    if (owner >= 0 && (at_leaf ? leaf_now : cur < n_tris)) {
-      const float4* rec = at_leaf ? tris + 3 * (size_t)first : reinterpret_cast<const float4*>(nodes + cur);
+    if (owner >= 0 && in_tree && (kLeafBatch == 0 || !at_leaf)) {
+      const uint64_t base = at_leaf ? reinterpret_cast<uint64_t>(tris) : reinterpret_cast<uint64_t>(nodes);
+      const float4* rec = reinterpret_cast<const float4*>(base + (uint64_t)idx * (at_leaf ? 48u : 64u));
       q0 = rec[0];
       q1 = rec[1];
       q2 = rec[2];
@@ -919,43 +921,43 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
     ++step;
     bool job_end = false, flush_me = false, end_after = false;
     if (owner >= 0) {
-      float bound = own ? o_t : (j_pos != 0xFFFFFFFFu ? fminf(dmax, j_t) : dmax);
+      // an owner's dmax is its o_t; its j_t, and a helper's without a hit, are RK_HUGE
+      float bound = j_t < dmax ? j_t : dmax;
       bool need_pop = false;
-      if (++visits > max_visits) {
-        job_end = true;
+      if (++visits > max_visits || !(in_tree || at_leaf)) {
+        job_end = true;  // never taken for a tree built here
         pend = 0u;
       } else if (!at_leaf) {
-        if (cur >= n_tris) {
-          job_end = true;  // never taken for a tree built here
-        } else {
-          FNode nd;
-          nd.a = q0;
-          nd.b = q1;
-          nd.c = q2;
-          nd.d = make_uint4(__float_as_uint(q3.x), __float_as_uint(q3.y), 0u, 0u);
-          const Slab2 sl = slab2(nd, ix, iy, iz, ox, oy, oz, bound);
-          const float tmin0 = sl.tmin0, tmin1 = sl.tmin1;
-          const bool h0 = sl.h0, h1 = sl.h1;
-          if (kCount) n_box += 2;
-          if (h0 && h1) {
-            const bool first0 = tmin0 <= tmin1;
-            if (sp < kStackN) {
-              st_set(sp, first0 ? nd.d.y : nd.d.x, first0 ? tmin1 : tmin0);
-              ++sp;
-            }
-            cur = first0 ? nd.d.x : nd.d.y;
-          } else if (h0) {
-            cur = nd.d.x;
-          } else if (h1) {
-            cur = nd.d.y;
-          } else {
-            need_pop = true;
+        FNode nd;
+        nd.a = q0;
+        nd.b = q1;
+        nd.c = q2;
+        nd.d = make_uint4(__float_as_uint(q3.x), __float_as_uint(q3.y), 0u, 0u);
+        const Slab2 sl = slab2(nd, ix, iy, iz, ox, oy, oz, bound);
+        const float tmin0 = sl.tmin0, tmin1 = sl.tmin1;
+        const bool h0 = sl.h0, h1 = sl.h1;
+        if (kCount) n_box += 2;
+        if (h0 && h1) {
+          const bool first0 = tmin0 <= tmin1;
+          if (sp < kStackN) {
+            st_set(sp, first0 ? nd.d.y : nd.d.x, first0 ? tmin1 : tmin0);
+            ++sp;
           }
+          cur = first0 ? nd.d.x : nd.d.y;
+        } else if (h0) {
+          cur = nd.d.x;
+        } else if (h1) {
+          cur = nd.d.y;
+        } else {
+          need_pop = true;
         }
       } else if (kLeafBatch == 0) {
-        if (leaf_now) {
+        if (in_tree) {
           RK_TRI_HIT(q0, q1, q2, first);
-          RK_LEAF_HITS(first, 1u, cnt);
+          if ((cur & 15u) != 0u) {
+            const uint32_t cnt = min((cur & 15u) + 1u, n_tris - first);
+            RK_LEAF_HITS(first, 1u, cnt);
+          }
         }
         need_pop = true;
       } else if (pend == 0u) {
@@ -966,7 +968,8 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
       }
       if (need_pop) {
         // the nearest pending entry that can still hold a closer hit
-        bound = own ? o_t : (j_pos != 0xFFFFFFFFu ? fminf(dmax, j_t) : dmax);
+        const float lim = own ? o_t : dmax;
+        bound = j_t < lim ? j_t : lim;
         bool found = false;
         while (sp > sb) {
           --sp;
@@ -1104,7 +1107,7 @@ constexpr uint32_t kFetchBoundFaces = 1u << 20;
 // defaults above are one variant; rk_fast_autotune chooses among several.
 template <bool kCount, int kWG, uint32_t kRun, int kLds, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
           int kBoundEvery = 1, bool kXcdRuns = false>
-__global__ __launch_bounds__(kWG, kLds > kLdsStack ? 5 : 6) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
+__global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
                                                       uint32_t n_tris, const float4* __restrict__ origins,
                                                       const float4* __restrict__ dirs, uint32_t n_rays,
                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
@@ -1901,16 +1904,8 @@ __device__ __forceinline__ bool camera_pixel(int width, int height, int& x, int&
 // reference's CUDA_calcPrimaryRays.cu:43-55 formula: origin, and direction
 // (dir - x * step_x) - y * step_y), so a frame reads no ray arrays. Every pixel is written:
 // a miss gives face ~0, coords (0, 0), depth FLT_MAX.
-//
-// kWaves: waves per SIMD to leave registers for. 6 (80 registers) for the variants
-// and frames of more than kSmallFrame pixels, 5 (86) for those whose waves all fit at
-// 5: the 256x256 icosphere frame 59.6 us with 5, 61.5 with 6, 512x512 heightfield 65.5
-// and 67.1, 1280x720 98.6 and 96.7, 1920x1080 184.9 and 177.9, 1280x720 icosphere 110.2
-// and 100.3.
-constexpr uint64_t kSmallFrame = 5 * 1024 * 64;
-template <int kWG, int kBands, bool kXcd, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
-          int kWaves = 6>
-__global__ __launch_bounds__(kWG, kWaves) void k_fast_trace_camera_v(const FNode* __restrict__ nodes,
+template <int kWG, int kBands, bool kXcd, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1>
+__global__ __launch_bounds__(kWG) void k_fast_trace_camera_v(const FNode* __restrict__ nodes,
                                                              const float4* __restrict__ tris, uint32_t n_tris,
                                                              float4 ro, float4 rd, float4 rx, float4 ry, int width,
                                                              int height, uint32_t* __restrict__ faces_id,
@@ -1941,8 +1936,8 @@ __global__ __launch_bounds__(kWG, kWaves) void k_fast_trace_camera_v(const FNode
 // theirs. faces: the mesh's faces in the tree's leaf order (faces[position]),
 // as the reference's builds leave them. faces_id, coords and depths, when not
 // NULL, receive what k_fast_trace_camera_v writes.
-template <int kWG, int kBands, int kDM, int kWaves>
-__global__ __launch_bounds__(kWG, kWaves) void k_fast_render_camera(
+template <int kWG, int kBands, int kDM>
+__global__ __launch_bounds__(kWG) void k_fast_render_camera(
     const FNode* __restrict__ nodes, const float4* __restrict__ tris, uint32_t n_tris, float4 ro, float4 rd,
     float4 rx, float4 ry, int width, int height, const uint4* __restrict__ faces, const float4* __restrict__ verts,
     const float4* __restrict__ norms, float4 back, float4 cam, uint32_t* __restrict__ pixels, int pitch,
@@ -2228,10 +2223,7 @@ extern "C" rk_status rk_fast_trace_camera(rk_stream stream, const rk_fast_bvh* b
   const CameraVariant* cv = camera_variant(options ? options->config : 0u);
   if (!cv) return RK_ERROR_INVALID_VALUE;
   dim3 grid(camera_blocks(width, height, (int)cv->wg, (int)cv->bands, cv->xcd != 0));
-  const bool small = (!options || options->config == 0) && (uint64_t)width * (uint64_t)height <= kSmallFrame;
-  const CameraKernel kernel =
-      small ? k_fast_trace_camera_v<kTraceWG, kCamBands, false, false, 0, kTraceDonateMin, 5> : cv->kernel;
-  hipLaunchKernelGGL(kernel, grid, dim3(cv->wg), 0, rk_hip_stream(stream), static_cast<const FNode*>(bvh->nodes),
+  hipLaunchKernelGGL(cv->kernel, grid, dim3(cv->wg), 0, rk_hip_stream(stream), static_cast<const FNode*>(bvh->nodes),
                      static_cast<const float4*>(bvh->tris), bvh->face_count, f4(camera->origin),
                      f4(camera->direction), f4(camera->step_x), f4(camera->step_y), width, height, faces_id,
                      reinterpret_cast<float2*>(coords), depths, det_eps_of(options));
@@ -2252,10 +2244,7 @@ extern "C" rk_status rk_fast_render_camera(rk_stream stream, const rk_fast_bvh* 
     return RK_ERROR_UNSUPPORTED;
   auto f4 = [](const rk_float4& v) { return make_float4(v.x, v.y, v.z, v.w); };
   dim3 grid(camera_blocks(width, height, kTraceWG, kCamBands, false));
-  const auto kernel = (uint64_t)width * (uint64_t)height <= kSmallFrame
-                          ? k_fast_render_camera<kTraceWG, kCamBands, kTraceDonateMin, 5>
-                          : k_fast_render_camera<kTraceWG, kCamBands, kTraceDonateMin, 6>;
-  hipLaunchKernelGGL(kernel, grid, dim3(kTraceWG), 0,
+  hipLaunchKernelGGL((k_fast_render_camera<kTraceWG, kCamBands, kTraceDonateMin>), grid, dim3(kTraceWG), 0,
                      rk_hip_stream(stream), static_cast<const FNode*>(bvh->nodes),
                      static_cast<const float4*>(bvh->tris), bvh->face_count, f4(camera->origin),
                      f4(camera->direction), f4(camera->step_x), f4(camera->step_y), width, height,

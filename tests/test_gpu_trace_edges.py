@@ -1,8 +1,9 @@
 """Traces where their launches change. Sorted: at 2^18 faces an XCD takes runs of
 512 workgroups (groups of 8 runs, 262144 rays; a remainder in plain order), at 2^20
-idle lanes help later. Camera frames: at 327680 pixels. The closest hit does not
-depend on any: bit-equal to the trace in ray order. The reference's per-ray walk:
-tiles of 16 x 4 rays, whole, cut at an edge, and refused for too many idle lanes."""
+idle lanes help later. Camera frames, with leaves of one and of several faces. The
+closest hit does not depend on any: bit-equal to the trace in ray order. The
+reference's per-ray walk: tiles of 16 x 4 rays, whole, cut at an edge, and refused
+for too many idle lanes."""
 import numpy as np
 import pytest
 
@@ -25,7 +26,7 @@ def test_sorted_equals_ray_order(rk, faces):
             assert torch.equal(x, y)
 
 
-@pytest.mark.parametrize("w,h", [(1, 1), (640, 512), (641, 512)])
+@pytest.mark.parametrize("w,h", [(1, 1), (641, 512)])
 @pytest.mark.parametrize("leaf_max", [1, 5, 16])
 def test_camera_equals_rays(rk, w, h, leaf_max):
     import torch
