@@ -1101,6 +1101,12 @@ constexpr uint32_t kXcdRun = 512, kXcdFaces = 1u << 18;
 // where half the wave is idle: 16M rays on the 10M soup 26.6 -> 24.0 ms, 8M on 3M
 // faces 9.52 -> 9.01, 4M on 1M 3.83 -> 3.80; 2M on 300k 1.63 -> 1.65.
 constexpr uint32_t kFetchBoundFaces = 1u << 20;
+// Rays in array order may be a picture's, whose rays share nodes and gain from early
+// help, so the same holds only from where the tree is beyond the 256 MB memory-side cache
+// too: 16M rays on the 10M soup 45.0 -> 38.7 ms; a 1920x1080 frame of a 3.9M-face heightfield
+// would go from 234 us to 289, as long as it took before nodes and leaves were
+// fetched together.
+constexpr uint32_t kMemoryFaces = 1u << 22;
 
 // kWG threads per workgroup, runs of kRun rays per band (spread_ray; 0: 64
 // consecutive rays per wave), kLds stack entries per lane in LDS. The
@@ -2209,7 +2215,10 @@ extern "C" rk_status rk_fast_trace(rk_stream stream, const rk_fast_bvh* bvh, con
   if (!origins || !directions || !faces_id || !coords || !depths) return RK_ERROR_INVALID_VALUE;
   const TraceVariant* tv = trace_variant(options ? options->config : 0u);
   if (!tv) return RK_ERROR_INVALID_VALUE;
-  return launch_trace_variant(rk_hip_stream(stream), *tv, bvh, origins, directions, n_rays, faces_id, coords, depths,
+  TraceVariant v = *tv;
+  if ((!options || options->config == 0) && bvh->face_count >= kMemoryFaces)
+    v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32>;
+  return launch_trace_variant(rk_hip_stream(stream), v, bvh, origins, directions, n_rays, faces_id, coords, depths,
                               det_eps_of(options), trace_flags_of(options));
 }
 

@@ -10,7 +10,7 @@ import pytest
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("faces", [(1 << 18) - 1, 1 << 18, (1 << 20) - 1, 1 << 20])
+@pytest.mark.parametrize("faces", [(1 << 18) - 1, 1 << 18, (1 << 20) - 1, 1 << 20, 1 << 22])
 def test_sorted_equals_ray_order(rk, faces):
     import torch
 
@@ -21,9 +21,10 @@ def test_sorted_equals_ray_order(rk, faces):
         O, D = rk.random_rays(n, seed=n)
         O, D = torch.from_numpy(O).cuda(), torch.from_numpy(D).cuda()
         a = dev.fast_trace_sorted(tree, O, D, det_epsilon=0.0)
-        b = dev.fast_trace(tree, O, D, det_epsilon=0.0)
-        for x, y in zip(a, b):
-            assert torch.equal(x, y)
+        b = dev.fast_trace(tree, O, D, det_epsilon=0.0)  # from 2^22 faces on, late help here too
+        c = dev.fast_trace(tree, O, D, det_epsilon=0.0, config=1)
+        for x, y, z in zip(a, b, c):
+            assert torch.equal(x, y) and torch.equal(x, z)
 
 
 @pytest.mark.parametrize("w,h", [(1, 1), (641, 512)])
