@@ -73,22 +73,20 @@ TRACE_TRAFFIC_BYTES = (107_351 * 2 + 10_576) * 1024
 # heightfield (`bench.py --profile-only`) and on the 10M soup (`--profile-soup`):
 # average duration (us) from --kernel-trace, HBM bytes read and written (KiB)
 # from --pmc FETCH_SIZE (x2, the factor a 256 MiB copy gives) and WRITE_SIZE
-# (profiles/fast_build_trace_heightfield708.md, profiles/soup10m_build_trace.md).
-# The heightfield's climbs through the splits that cross chunks run inside
-# k_fast_hierarchy (up to 2^21 faces); the soup's in k_fast_hierarchy_top.
+# (profiles/case_kernels.md).
 BUILD_KERNELS = {  # kernel: (us, HBM read KiB, HBM write KiB, launches per build)
     "heightfield": {
-        "k_fast_prep": (15.12, 32_289, 42_960, 1),
-        "k_rs_hist": (12.20, 3_992, 1_285, 1),
-        "k_rs_scatter": (16.46, 10_937, 10_366, 4),
-        "k_fast_hierarchy": (109.70, 51_675, 119_632, 1),
+        "k_fast_prep": (14.53, 26_740, 39_561, 1),
+        "k_rs_scatter": (16.44, 9_768, 10_169, 4),
+        "k_fast_hierarchy": (46.36, 47_530, 114_420, 1),
+        "k_hier_reduce": (16.61, 618, 777, 2),
     },
     "soup": {
-        "k_fast_prep": (211.5, 625_591, 468_775, 1),
-        "k_rs_hist": (66.08, 78_298, 18_713, 1),
-        "k_rs_scatter": (60.33, 132_323, 134_816, 8),
-        "k_fast_hierarchy": (854.0, 2_928_171, 1_192_198, 1),
-        "k_fast_hierarchy_top": (126.2, 51_644, 38_306, 1),
+        "k_fast_prep": (204.4, 625_130, 429_701, 1),
+        "k_rs_hist": (43.45, 78_300, 9_899, 1),
+        "k_rs_scatter": (63.01, 131_978, 135_924, 8),
+        "k_fast_hierarchy": (781.1, 2_926_534, 1_177_784, 1),
+        "k_hier_reduce": (20.42, 3_416, 4_688, 3),
     },
 }
 HBM_PEAK_GBS = 8000.0
