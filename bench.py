@@ -63,10 +63,10 @@ OPS_PER_TRI_TEST = 53   # algorithmic FP32 ops of one Moller-Trumbore test
 HEADLINE_DET_EPSILON = 1e-6  # the reference's absolute parallel-ray threshold (CUDA_raytraceMeshTree.cu:36)
 # HBM bytes per launch of the headline trace kernel (the default traversal
 # variant, tmax reset in the kernel), from two rocprofv3 --pmc runs of
-# `bench.py --profile-only` (profiles/fast_build_trace_heightfield708.md):
-# FETCH_SIZE 107,351 KiB, scaled x2 by a 256 MiB copy, plus WRITE_SIZE 10,576 KiB
+# `bench.py --profile-only` (profiles/case_kernels.md):
+# FETCH_SIZE 102,101 KiB, scaled x2 by a 256 MiB copy, plus WRITE_SIZE 10,575 KiB
 # (means of the two warm frames at the 1e-6 threshold).
-TRACE_TRAFFIC_BYTES = (107_351 * 2 + 10_576) * 1024
+TRACE_TRAFFIC_BYTES = (102_101 * 2 + 10_575) * 1024
 
 
 # The fast build's kernels, per launch, measured with rocprofv3 on the headline

@@ -1051,9 +1051,9 @@ __global__ __launch_bounds__(256) void k_ray_keys(const FNode* __restrict__ node
 // wave does not take 64 consecutive rays: it takes runs of kSpreadRun
 // consecutive rays (a 128-B line of origins and one of directions) from
 // 64 / kSpreadRun bands of the ray array, the run at the same place in each
-// band. Runs of 8 measured best on the 1920x1080 heightfield frame (0.224 ms
-// against 0.257 ms for 64 consecutive rays; 0.276 ms for runs of 4, 0.231
-// for runs of 16). 0 traces the rays in array order. Sorted traces keep
+// band. Runs of 8 measured best on the 1920x1080 heightfield frame (with help at
+// one idle lane 0.176 ms against 0.283 for 64 consecutive rays; 0.219 for runs of
+// 4, 0.200 for runs of 16). 0 traces the rays in array order. Sorted traces keep
 // their order.
 #ifndef RK_TRACE_SPREAD
 #define RK_TRACE_SPREAD 8
@@ -1068,10 +1068,11 @@ __device__ __forceinline__ uint32_t spread_ray(uint32_t t, uint32_t n_rays) {
 // order (may be NULL): thread t traces ray order[t], so rays that start near
 // each other run in the same wave; results still go to the ray's own slot.
 // Threads per workgroup of k_fast_trace and k_fast_trace_camera. One wave per
-// workgroup measured best on the 1920x1080 heightfield frame (rays 0.211 ms,
-// camera 0.199 ms; 128: 0.218 / 0.200; 256: 0.228 / 0.209; 512: 0.251 /
-// 0.230) and within 1% on the 10M soup's incoherent rays: a finished wave
-// frees its slot at once, where a larger workgroup waits for its slowest wave.
+// workgroup: a finished wave frees its slot at once, where a larger workgroup
+// waits for its slowest wave. On the 1920x1080 heightfield frame 64, 128 and 256
+// threads take 0.176, 0.175 and 0.181 ms (camera 0.173 and 0.171) with help at one
+// idle lane, and are within 1% on the 10M soup's incoherent rays. (Before a step
+// fetched in one place 64 was ahead: 0.211, 0.218, 0.228 ms.)
 #ifndef RK_TRACE_WG
 #define RK_TRACE_WG 64
 #endif
@@ -1080,9 +1081,8 @@ constexpr int kTraceWG = RK_TRACE_WG;
 // many lanes are idle (trace_ray_shared's kDonateMin): each exchange costs
 // every lane of the wave a dozen shuffles and two LDS round trips, and a lane
 // that waits a few steps for work costs less. 16 measured best on the
-// 1920x1080 heightfield frame (0.183 ms against 0.189 with 1 and 0.215 with
-// 32) and better than 1 on the 10M soup's incoherent rays (45.9 against 48.4
-// ms; 42.5 with 32, which the autotuner picks there).
+// 1920x1080 heightfield frame (0.166 ms against 0.177 with 1, 0.171 with 8 and
+// 0.190 with 32); trees past the L2 take 32 (kFetchBoundFaces, kMemoryFaces).
 #ifndef RK_TRACE_DONATE_MIN
 #define RK_TRACE_DONATE_MIN 16
 #endif
@@ -1711,10 +1711,8 @@ extern "C" rk_status rk_fast_trace_counted(rk_stream stream, const rk_fast_bvh* 
 namespace {
 
 // Bands of the camera kernel: 8 bands of 8-pixel runs measured best on the
-// 1920x1080 heightfield frame with the 64-VGPR traversal (0.181 ms; 16 bands
-// of 4-pixel runs 0.184, 4 bands 0.192). At 79 VGPRs 16 bands had been best
-// (0.212 ms; 8 bands 0.216, 32 bands 0.218, 64 bands of single pixels 0.231,
-// and 8x8 tiles per wave 0.249).
+// 1920x1080 heightfield frame (with help at one idle lane 0.173 ms; 16 bands of
+// 4-pixel runs 0.195, 4 bands 0.176; with the default's 16 idle lanes 0.163).
 #ifndef RK_CAM_BANDS
 #define RK_CAM_BANDS 8
 #endif
