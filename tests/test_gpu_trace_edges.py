@@ -3,7 +3,7 @@
 idle lanes help later. Camera frames, with leaves of one and of several faces. The
 closest hit does not depend on any: bit-equal to the trace in ray order. The
 reference's per-ray walk: tiles of 16 x 4 rays, whole, cut at an edge, and refused
-for too many idle lanes."""
+for too many idle lanes; and its hand-off limits on both sides of 12 rays per face."""
 import numpy as np
 import pytest
 
@@ -62,3 +62,26 @@ def test_reference_rays_in_tiles(rk, ora, w, h):
     np.testing.assert_array_equal(got[0].view(np.uint32), of)
     np.testing.assert_array_equal(got[1], ouv)
     np.testing.assert_array_equal(got[2], od)
+
+
+@pytest.mark.parametrize("coherency", [False, True])
+@pytest.mark.parametrize("faces,w,h", [(16384, 512, 384), (16385, 512, 384), (16384, 512, 383), (5461, 256, 256),
+                                       (5462, 256, 256)])
+def test_reference_handoff_limit_by_rays_per_face(rk, faces, w, h, coherency):
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = rk.soup(faces, seed=faces)
+    hb = rk.hitbox(V)
+    Ft, Vt = torch.from_numpy(F.view(np.int32)).cuda(), torch.from_numpy(V).cuda()
+    tree = dev.build_lbvh(Ft, Vt, hb, 12, True)
+    O, D = rk.random_rays(w * h, seed=h)
+    O, D = torch.from_numpy(O).cuda(), torch.from_numpy(D).cuda()
+    a = dev.trace_ref(tree, Vt, O, D, w, h, coherency)
+    try:
+        dev.set_ref_handoff(0xFFFFFFFF, 0xFFFFFFFF)  # no second passes
+        b = dev.trace_ref(tree, Vt, O, D, w, h, coherency)
+    finally:
+        dev.set_ref_handoff()
+    for x, y in zip(a, b):
+        assert torch.equal(x, y)
