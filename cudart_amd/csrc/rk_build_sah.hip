@@ -1183,7 +1183,7 @@ __global__ __launch_bounds__(1024) void k_sah_number_start(Sah s, uint32_t m) {
   if (threadIdx.x == 0) s.groups[blockIdx.x] = s_sum;
 }
 
-// The faces' boxes, ids and a copy of them, and the root's centroid bounds:
+// The faces' boxes, ids and a copy of them, and a large root's centroid bounds:
 // kBoxPer faces per thread, so that few workgroups add to the same words.
 constexpr uint32_t kBoxThreads = 1024, kBoxPer = 4;
 __global__ __launch_bounds__(kBoxThreads) void k_boxes_root(Sah s, const uint4* __restrict__ faces,
@@ -1216,7 +1216,8 @@ __global__ __launch_bounds__(kBoxThreads) void k_boxes_root(Sah s, const uint4* 
       b[3 + q] = max(b[3 + q], c);
     }
   }
-  add_bounds(b, s.bnd1);
+  // a root of at most kChunk faces is k_sah_subtrees': big_cap is 0, and there are no bounds
+  if (s.n > kChunk) add_bounds(b, s.bnd1);
 }
 
 __global__ __launch_bounds__(256) void k_gather_faces2(const uint4* __restrict__ src, const uint32_t* __restrict__ idx,

@@ -208,3 +208,26 @@ def _compare_sah(rk, ora, F, Ft, tree, nodes, order, flags):
     got = tree.nodes.cpu().numpy().view(np.uint32)[:m].copy().view(ora.NODE_DTYPE).reshape(m)
     for name in ("w0", "w1", "bmin", "bmax"):
         assert np.array_equal(got[name], nodes[name]), name
+
+
+@pytest.mark.parametrize("n", [1, 16, 1000, 1024])
+def test_sah_small_root_keeps_no_bounds(rk, n):
+    """A root that goes straight to the small items has no room for centroid bounds
+    in the workspace: theirs (as ordered ints, the bits of a positive float) are
+    nowhere in it, whatever it held before."""
+    import torch
+    V, F = rk.soup(n, seed=n, lo=1.0, hi=2.0)
+    hb = rk.aabox(rk.hitbox(V))
+    L = rk.lib()
+    Ft, Vt = torch.from_numpy(F.view(np.int32).copy()).cuda(), torch.from_numpy(V).cuda()
+    boxes = torch.zeros((n, 8), dtype=torch.float32, device="cuda")
+    ids = torch.zeros(n, dtype=torch.int32, device="cuda")
+    nodes = torch.zeros((2 * n, 8), dtype=torch.int32, device="cuda")
+    info = torch.zeros(8, dtype=torch.int32, device="cuda")
+    ws = torch.full((L.rk_build_sah_workspace_size(n, 0) // 4,), 0x7FFFFFFF, dtype=torch.int32, device="cuda")
+    rk.check(L.rk_build_sah(None, Ft.data_ptr(), Vt.data_ptr(), n, C.byref(hb), boxes.data_ptr(), ids.data_ptr(),
+                            nodes.data_ptr(), 0, 2 * n, info.data_ptr(), ws.data_ptr(), 4 * ws.numel()), "sah")
+    torch.cuda.synchronize()
+    T = V[F[:, :3], :3]
+    low = ((T.min(1) + T.max(1)) * np.float32(0.5)).min(0)
+    assert (low > 0).all() and not np.isin(low.view(np.int32), ws.cpu().numpy()).any()
