@@ -1368,11 +1368,11 @@ extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_fl
     for (uint32_t c = 0; c < kClasses; ++c) done.n[c] = got[kCtlRoots + c];
     ahead = 2;
   } while (big);
+  if (got[kCtlDeep]) return RK_ERROR_LAUNCH;  // refused: the faces stay as they are
   // CUDA_reorderMeshFaces, :778-784
   hipLaunchKernelGGL(k_gather_faces2, dim3(per_face), dim3(256), 0, st, ftmp, indices, f, n);
   RK_CHECK_LAUNCH();
   // the numbering, by the levels' sizes
-  if (got[kCtlDeep]) return RK_ERROR_LAUNCH;
   std::vector<uint32_t> hist(got + kCtlHist, got + kCtlHist + kHistRead);
   if (hist.back()) {
     hist.resize(ctl_words(n) - kCtlHist);

@@ -231,3 +231,47 @@ def test_sah_small_root_keeps_no_bounds(rk, n):
     T = V[F[:, :3], :3]
     low = ((T.min(1) + T.max(1)) * np.float32(0.5)).min(0)
     assert (low > 0).all() and not np.isin(low.view(np.int32), ws.cpu().numpy()).any()
+
+
+def _comb(n):
+    """n faces in parallel planes, so large that every split of them costs the same:
+    the SAH takes the last one, which holds the last face alone (the distances from
+    the first are those whose 31 / d * d does not round below 31). A face per level,
+    down to a leaf of 223: internal items on levels 0 to n - 224."""
+    d = np.arange(1, 4 * n, dtype=np.float32)
+    d = d[np.float32(31) / d * d >= 31][:n - 1]
+    assert len(d) == n - 1
+    V, F = np.zeros((n, 3, 4), np.float32), np.zeros((n, 4), np.uint32)
+    V[1:, :, 0] = d[:, None]
+    V[:, 1, 1] = V[:, 2, 2] = 1e15
+    F[:, :3] = np.arange(3 * n, dtype=np.uint32).reshape(n, 3)
+    return V.reshape(-1, 4), F
+
+
+def test_sah_at_the_depth_limit(rk, ora):
+    """The deepest tree the build takes, 4096 levels with internal items."""
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = _comb(4096 + 223)
+    hb = rk.hitbox(V)
+    boxes, idx = ora.calc_boxes(F, V)
+    nodes, order, flags = ora.build_sah(boxes, idx, hb)
+    assert nodes.shape[0] == 2 * 4096 + 1
+    Ft = torch.from_numpy(F.view(np.int32).copy()).cuda()
+    tree = dev.build_sah(Ft, torch.from_numpy(V).cuda(), hb)
+    _compare_sah(rk, ora, F, Ft, tree, nodes, order, flags)
+
+
+@pytest.mark.parametrize("n", [4096 + 224, 4096 + 1024 + 2])  # met by a small item, by a large one
+def test_sah_past_the_depth_limit_leaves_the_faces(rk, n):
+    import torch
+
+    from cudart_amd import device as dev
+    V, F = _comb(n)
+    F = F[np.random.default_rng(n).permutation(n)]
+    Ft = torch.from_numpy(F.view(np.int32).copy()).cuda()
+    with pytest.raises(rk.RkError, match=r"\(3\)"):
+        dev.build_sah(Ft, torch.from_numpy(V).cuda(), rk.hitbox(V))
+    torch.cuda.synchronize()
+    np.testing.assert_array_equal(Ft.cpu().numpy().view(np.uint32), F)
