@@ -1387,7 +1387,8 @@ extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_fl
     hipLaunchKernelGGL(k_sah_number_start, dim3((m + kNumberItems - 1) / kNumberItems), dim3(1024), 0, st, s, m);
     RK_CHECK_LAUNCH();
   }
-  for (level = 0; m;) {
+  level = 0;
+  do {  // level 0 writes the info words too, also with nothing on it
     uint32_t end = level + 1;
     uint32_t* out = level == 0 ? info : nullptr;
     if (m <= kNumberItems) {
@@ -1404,6 +1405,6 @@ extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_fl
       m = 2 * hist[level];
       child0 += m;
     }
-  }
+  } while (m);
   return RK_SUCCESS;
 }

@@ -275,3 +275,26 @@ def test_sah_past_the_depth_limit_leaves_the_faces(rk, n):
         dev.build_sah(Ft, torch.from_numpy(V).cuda(), rk.hitbox(V))
     torch.cuda.synchronize()
     np.testing.assert_array_equal(Ft.cpu().numpy().view(np.uint32), F)
+
+
+def test_hybrid_without_leaves_counts_the_nodes(rk):
+    """Existing nodes that hold no leaf leave nothing to refine: the node count is
+    theirs, and the faces follow the indices."""
+    import torch
+    n, existing = 40, 3
+    V, F = rk.soup(n, seed=n)
+    hb = rk.aabox(rk.hitbox(V))
+    L = rk.lib()
+    order = np.random.default_rng(n).permutation(n).astype(np.uint32)
+    Ft, Vt = torch.from_numpy(F.view(np.int32).copy()).cuda(), torch.from_numpy(V).cuda()
+    boxes = torch.zeros((n, 8), dtype=torch.float32, device="cuda")
+    ids = torch.from_numpy(order.view(np.int32)).cuda()
+    nodes = torch.zeros((existing + 2 * n, 8), dtype=torch.int32, device="cuda")
+    info = torch.full((8,), -1, dtype=torch.int32, device="cuda")
+    ws = torch.empty(L.rk_build_sah_workspace_size(n, existing), dtype=torch.uint8, device="cuda")
+    rk.check(L.rk_build_sah(None, Ft.data_ptr(), Vt.data_ptr(), n, C.byref(hb), boxes.data_ptr(), ids.data_ptr(),
+                            nodes.data_ptr(), existing, existing + 2 * n, info.data_ptr(), ws.data_ptr(),
+                            ws.numel()), "sah")
+    torch.cuda.synchronize()
+    assert info.cpu().tolist()[:3] == [existing, 0, 0] and not nodes.any()
+    np.testing.assert_array_equal(Ft.cpu().numpy().view(np.uint32), F[order])
