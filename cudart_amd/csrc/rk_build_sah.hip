@@ -27,8 +27,8 @@
 // order, and its k-th internal item takes children (count + 2k, count + 2k + 1),
 // the breadth-first equivalent of the reference's atomicAdd(node_count, 2).
 #include <algorithm>
+#include <iterator>
 #include <numeric>
-#include <vector>
 
 #include "rk_device.h"
 
@@ -1373,14 +1373,14 @@ extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_fl
   hipLaunchKernelGGL(k_gather_faces2, dim3(per_face), dim3(256), 0, st, ftmp, indices, f, n);
   RK_CHECK_LAUNCH();
   // the numbering, by the levels' sizes
-  std::vector<uint32_t> hist(got + kCtlHist, got + kCtlHist + kHistRead);
-  if (hist.back()) {
-    hist.resize(ctl_words(n) - kCtlHist);
-    RK_HIP(hipMemcpyAsync(hist.data(), s.ctl + kCtlHist, hist.size() * 4, hipMemcpyDeviceToHost, st));
+  uint32_t hist[kLevelMax + 2] = {};  // (not from the heap, whose exceptions a C entry must not let out)
+  std::copy_n(got + kCtlHist, kHistRead, hist);
+  if (hist[kHistRead - 1]) {
+    RK_HIP(hipMemcpyAsync(hist, s.ctl + kCtlHist, (ctl_words(n) - kCtlHist) * 4, hipMemcpyDeviceToHost, st));
     RK_HIP(hipStreamSynchronize(st));
   }
-  hist.push_back(0u);
-  const uint32_t total = (root ? 1u : existing_nodes) + 2u * std::accumulate(hist.begin(), hist.end(), 0u);
+  const uint32_t total =
+      (root ? 1u : existing_nodes) + 2u * std::accumulate(std::begin(hist), std::end(hist), 0u);
   Node* nd = reinterpret_cast<Node*>(nodes);
   uint32_t m = starts_found, id0 = 0, child0 = root ? 1u : existing_nodes;
   if (m > kNumberItems) {

@@ -3,6 +3,8 @@ and groups of tiles of the sort, the one-workgroup sort, runs and groups of runs
 the hierarchy; the reference topology where a level or the split lists stop
 fitting in LDS; the SAH build where its items change hands."""
 import ctypes as C
+import subprocess
+from pathlib import Path
 
 import numpy as np
 import pytest
@@ -298,3 +300,11 @@ def test_hybrid_without_leaves_counts_the_nodes(rk):
     torch.cuda.synchronize()
     assert info.cpu().tolist()[:3] == [existing, 0, 0] and not nodes.any()
     np.testing.assert_array_equal(Ft.cpu().numpy().view(np.uint32), F[order])
+
+
+def test_sah_lets_no_exception_out():
+    """The build with no C++ heap at hand (tests/cpp/no_heap.cpp)."""
+    exe = Path(__file__).resolve().parent / "cpp" / "_build" / "no_heap"
+    assert exe.exists(), "build() compiles tests/cpp first"
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "status 0" in r.stdout, r.stdout + r.stderr
