@@ -1153,9 +1153,9 @@ __global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ 
 
 inline unsigned blocks_for(uint32_t n, uint32_t per) { return (n + per - 1) / per; }
 
-// Workspace of the hierarchy passes over n positions. Its size has 8 B per
-// position more than the passes use, so that the workspace sizes and the
-// no-allocation build's face limits stay what callers know.
+// Workspace of the hierarchy passes over n positions. What callers know of it, its
+// size, the no-allocation build's face limits and what is refused as too small, has
+// two words per position that no pass uses: they are taken all the same.
 struct HierWs {
   HierItem* items;   // the subtrees each chunk, then each group of chunks, left over
   uint32_t* counts;  // per chunk, how many
@@ -1165,15 +1165,11 @@ inline size_t hier_ws_bytes(size_t n) {
          rk_align_up(((n + kChunk - 1) / kChunk) * 4);
 }
 inline bool take_hier_ws(RkArena& ar, uint32_t n, HierWs& w) {
+  const bool first = ar.take<uint32_t>(n) != nullptr;
   w.items = ar.take<HierItem>(n);
+  const bool second = ar.take<uint32_t>(n) != nullptr;
   w.counts = ar.take<uint32_t>((n + kChunk - 1) / kChunk);
-  return w.items && w.counts;
-}
-// What is left of the workspace.
-inline void* rest_of(const RkArena& ar, size_t& bytes) {
-  const size_t at = rk_align_up(ar.used);
-  bytes = at < ar.size ? ar.size - at : 0;
-  return ar.base ? ar.base + at : nullptr;
+  return first && w.items && second && w.counts;
 }
 // The chunk pass, then reductions of kReduceFan groups to one until one is left.
 template <typename K, bool kBatch>
@@ -1257,9 +1253,9 @@ static rk_status fast_build_common(rk_stream stream, const rk_uint4* faces, cons
   void* keys = wide ? (void*)ar.take<uint64_t>(n) : (void*)ar.take<uint32_t>(n);
   HierWs hw;
   const bool hw_ok = take_hier_ws(ar, n, hw);
-  size_t sort_bytes = 0;
-  void* sort_ws = rest_of(ar, sort_bytes);
-  if (!keys || !hw_ok) return RK_ERROR_WORKSPACE;
+  const size_t sort_bytes = rk_sort_workspace_size(n, wide ? 8 : 4);
+  void* sort_ws = ar.take<char>(sort_bytes);
+  if (!keys || !hw_ok || !sort_ws) return RK_ERROR_WORKSPACE;
   if (sorted_keys) keys = sorted_keys;
   float4 rmin = make_float4(hitbox->min.x, hitbox->min.y, hitbox->min.z, hitbox->min.w);
   float4 rmax = make_float4(hitbox->max.x, hitbox->max.y, hitbox->max.z, hitbox->max.w);
@@ -1562,9 +1558,9 @@ extern "C" rk_status rk_batch_build(rk_stream stream, const rk_batch_mesh* meshe
   uint64_t* keys = ar.take<uint64_t>(n);
   HierWs hw;
   const bool hw_ok = take_hier_ws(ar, n, hw);
-  size_t sort_bytes = 0;
-  void* sort_ws = rest_of(ar, sort_bytes);
-  if (!keys || !hw_ok) return RK_ERROR_WORKSPACE;
+  const size_t sort_bytes = rk_sort_workspace_size(n, 8);
+  void* sort_ws = ar.take<char>(sort_bytes);
+  if (!keys || !hw_ok || !sort_ws) return RK_ERROR_WORKSPACE;
   const uint4* f = reinterpret_cast<const uint4*>(faces);
   const float4* v = reinterpret_cast<const float4*>(vertices);
   uint32_t* order = bvh->indices;

@@ -10,8 +10,9 @@ template <typename K>
 struct RkSortPlan {
   uint32_t n = 0, tiles = 0, copies = 0;
   int passes = 0;              // of 8 bits
-  bool one = false;          // one workgroup sorts everything in LDS
-  uint32_t* head = nullptr;  // [0] error word, then copies x passes x 256 counts
+  int items = 0;               // keys per lane of the scatter kernel
+  bool one = false;            // one workgroup sorts everything in LDS
+  uint32_t* head = nullptr;    // [0] error word, then copies x passes x 256 counts
   uint32_t* status = nullptr;  // look-back words
   size_t head_words = 0, status_words = 0;  // status_words: of the first pass
   K* src = nullptr;            // where the unsorted keys and values go

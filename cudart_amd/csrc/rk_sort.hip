@@ -552,8 +552,8 @@ __global__ __launch_bounds__(256) void k_iota(uint32_t* __restrict__ v, uint32_t
 inline int items_of(uint32_t n) {
   return (size_t)n < kSmallTilesBelow ? kItemsSmall : ((size_t)n < kMidTilesBelow ? kItemsMid : kItems);
 }
-inline uint32_t tiles_of(uint32_t n) {
-  const uint32_t tile = (uint32_t)(kThreads * items_of(n));
+inline uint32_t tiles_of(uint32_t n, int items) {
+  const uint32_t tile = (uint32_t)(kThreads * items);
   return (uint32_t)(((size_t)n + tile - 1) / tile);
 }
 // The error word of a sort called with this workspace: its first 4 bytes.
@@ -596,23 +596,30 @@ rk_status rk_sort_plan(uint32_t n, int bits, bool anywhere, K* keys, uint32_t* v
   p.n = n;
   p.one = n <= kOneMax;
   p.passes = (bits + 7) / 8;
-  p.tiles = tiles_of(n);
-  // rk_sort_workspace_size has one count and one status row per pass and tile of
-  // 4096 or 8192 keys: room for these copies of the counts and rows
-  const bool groups = items_of(n) != kItems;
-  p.copies = std::min<uint32_t>(8u, 1u + p.tiles / 8u);
-  p.head_words = p.one ? 1 : 1 + (size_t)p.copies * p.passes * 256;
-  p.status_words = p.one ? 0 : ((size_t)p.tiles + (groups ? (p.tiles + kGroup - 1) / kGroup : 0)) * 256;
-  RkArena ar(ws, ws_bytes);
-  p.head = ar.take<uint32_t>(p.head_words + (groups || p.passes < 2 ? 1 : 2) * p.status_words);
-  p.status = p.head + p.head_words;
   p.dst = p.src = keys;
   p.vdst = p.vsrc = vals;
-  if (!p.head) return RK_ERROR_WORKSPACE;
+  // rk_sort_workspace_size has one count and one status row per pass and tile of
+  // 4096 or 8192 keys: room for these copies of the counts and rows. A caller's
+  // smaller workspace may still have room for fewer: one copy, tiles of 8192 keys
+  // and two rows each, which fit wherever 'least_ws' bytes do.
+  auto fits = [&](int items, bool copies) {
+    const bool groups = items != kItems;
+    p.items = items;
+    p.tiles = tiles_of(n, items);
+    p.copies = copies ? std::min<uint32_t>(8u, 1u + p.tiles / 8u) : 1u;
+    p.head_words = p.one ? 1 : 1 + (size_t)p.copies * p.passes * 256;
+    p.status_words = p.one ? 0 : ((size_t)p.tiles + (groups ? (p.tiles + kGroup - 1) / kGroup : 0)) * 256;
+    RkArena ar(ws, ws_bytes);
+    p.head = ar.take<uint32_t>(p.head_words + (groups || p.passes < 2 ? 1 : 2) * p.status_words);
+    if (!p.head) return false;
+    p.status = p.head + p.head_words;
+    if (p.one) return true;
+    p.alt = ar.take<K>(n);
+    p.valt = vals ? ar.take<uint32_t>(n) : nullptr;
+    return p.alt && (!vals || p.valt);
+  };
+  if (!fits(items_of(n), true) && !fits(kItems, false)) return RK_ERROR_WORKSPACE;
   if (p.one) return RK_SUCCESS;
-  p.alt = ar.take<K>(n);
-  p.valt = vals ? ar.take<uint32_t>(n) : nullptr;
-  if (!p.alt || (vals && !p.valt)) return RK_ERROR_WORKSPACE;
   if (anywhere && (p.passes & 1)) {
     p.src = p.alt;
     p.vsrc = p.valt;
@@ -663,8 +670,7 @@ rk_status rk_sort_run(hipStream_t st, const RkSortPlan<K>& p, bool counted, uint
   K *ks = p.src, *kd = p.src == p.dst ? p.alt : p.dst;
   uint32_t *vs = p.vsrc, *vd = p.vsrc == p.vdst ? p.valt : p.vdst;
   for (int i = 0; i < p.passes; ++i) {
-    const int items = items_of(p.n);
-    const bool groups = items != kItems;
+    const bool groups = p.items != kItems;
     uint32_t* status = p.status + (groups ? 0 : (i & 1) * p.status_words);
     uint32_t* next = !groups && i + 1 < p.passes ? p.status + ((i + 1) & 1) * p.status_words : nullptr;
     auto go = [&](auto kernel) {
@@ -672,11 +678,11 @@ rk_status rk_sort_run(hipStream_t st, const RkSortPlan<K>& p, bool counted, uint
                          p.copies, (uint32_t)p.passes * 256u, status, next, err);
     };
     if (p.vsrc) {
-      if (items == kItemsSmall) go(k_rs_scatter<K, true, kItemsSmall, true>);
+      if (p.items == kItemsSmall) go(k_rs_scatter<K, true, kItemsSmall, true>);
       else if (groups) go(k_rs_scatter<K, true, kItemsMid, true>);
       else go(k_rs_scatter<K, true, kItems, false>);
     } else {
-      if (items == kItemsSmall) go(k_rs_scatter<K, false, kItemsSmall, true>);
+      if (p.items == kItemsSmall) go(k_rs_scatter<K, false, kItemsSmall, true>);
       else if (groups) go(k_rs_scatter<K, false, kItemsMid, true>);
       else go(k_rs_scatter<K, false, kItems, false>);
     }
@@ -704,6 +710,15 @@ RK_SORT_INSTANCES(uint32_t)
 RK_SORT_INSTANCES(uint64_t)
 #undef RK_SORT_INSTANCES
 
+// The workspace that a sort of n > 1 keys asks for whichever way it goes, the
+// one-workgroup sort included: a count and a status row per pass and tile of 4096 or
+// 8192 keys, and the other halves of the keys and values.
+template <typename K>
+static size_t least_ws(uint32_t n, int passes, bool vals) {
+  const size_t T = tiles_of(n, n < kMidTilesBelow ? kItemsMid : kItems), P = (size_t)passes, keys = n * sizeof(K);
+  return rk_align_up((1 + P * 256 + P * T * 256) * 4) + (vals ? rk_align_up(keys) + (size_t)n * 4 : keys);
+}
+
 // Sorts keys (and values, when not NULL) stably on their low 'bits' bits. 'err'
 // (device, may be NULL) receives RK_FLAG_SPIN_LIMIT on a look-back timeout; when
 // it is NULL the first word of 'ws' does, cleared by this call.
@@ -714,6 +729,7 @@ static rk_status sort_keys(hipStream_t st, K* keys, uint32_t* vals, uint32_t n, 
   if (n <= 1) return err ? RK_SUCCESS : clear_ws_flags(st, ws, ws_bytes);
   RkSortPlan<K> p;
   rk_status s = rk_sort_plan<K>(n, bits, false, keys, vals, ws, ws_bytes, p);
+  if (s == RK_SUCCESS && ws_bytes < least_ws<K>(n, p.passes, vals != nullptr)) s = RK_ERROR_WORKSPACE;
   return s == RK_SUCCESS ? rk_sort_run<K>(st, p, false, err) : s;
 }
 
