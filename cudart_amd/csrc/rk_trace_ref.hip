@@ -1391,23 +1391,16 @@ static std::atomic<uint32_t> g_packet_faces{RK_HANDOFF_AUTO};
 // own finish sooner: on a 179k-face heightfield a 512x512 per-ray frame takes
 // 0.69 ms past 256 faces against 1.23 past 4096, a packet frame 0.87 past 512
 // against 1.17. On the 1M-face heightfield at 1920x1080 it is 3.33 against 1.83
-// and 3.78 against 3.27. A mesh with many rays per face is another matter: most
-// rays that hit pass 256 faces, close ones the same faces, and a wave each costs
-// more than the lanes of one (20k-face icosphere, 512x512: per-ray 1.02 against
-// 0.51 ms, packets 0.42 against 0.33). With few rays in all the first pass lasts
-// as long as its slowest wave all the same, so there is a least number of rays.
-// 256 against 4096 (512 for packets), time ratios, by rays per face: per-ray from
-// 3 x 2^16 rays on, below 9: 0.4-0.9; 9.6: 1.5 (icosphere); 12-15: 0.87-1.16
-// (heightfields), 2.0; 16 and more: 1.1-2.3. Packets, below 8: 0.64-1.07, from 12 on
-// 0.99-1.45.
-constexpr uint32_t kAutoRaysBelow = 1u << 19, kAutoRaysPerFace = 12;
+// and 3.78 against 3.27. Which is better below 2^19 rays depends on the view, which
+// a rule by sizes does not see (per-ray, 256 against 4096): the 20k-face icosphere at
+// 512x512 1.02 and 0.50 ms, from twice as far 0.57 and 0.71; 30,000 scattered faces at
+// 704x545 5.31 and 2.72, from twice as far 1.63 and 3.16. Early is never slower than
+// testing every face was; late at 12 rays per face or more was (the last: 2.06).
+constexpr uint32_t kAutoRaysBelow = 1u << 19;
 constexpr uint32_t kAutoSmallRayFaces = 256, kAutoSmallPacketFaces = 512;
-constexpr uint32_t kAutoManyRays = 3u << 16, kAutoManyPacketRays = 1u << 16;
-static uint32_t limit_of(uint32_t set, uint32_t n_rays, uint32_t n_faces, uint32_t many_rays, uint32_t small_limit,
-                         uint32_t large_limit) {
+static uint32_t limit_of(uint32_t set, uint32_t n_rays, uint32_t small_limit, uint32_t large_limit) {
   if (set != RK_HANDOFF_AUTO) return set;
-  const bool many = n_rays >= many_rays && n_rays / kAutoRaysPerFace >= n_faces;
-  return n_rays < kAutoRaysBelow && !many ? small_limit : large_limit;
+  return n_rays < kAutoRaysBelow ? small_limit : large_limit;
 }
 static std::atomic<uint32_t> g_list_cap{kHandoffCap};
 constexpr uint32_t kNoHandoff = 0xffffffffu;
@@ -1513,8 +1506,8 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
     // its rays test every face; at its first leaf), is traced on by the second
     // pass, kPacketSplit threads per ray, from where it was left.
     const uint32_t gx = (uint32_t)(width + kPW - 1) / kPW, gy = (uint32_t)(height + kPH - 1) / kPH;
-    const uint32_t faces_limit = limit_of(g_packet_faces.load(std::memory_order_relaxed), n, face_count,
-                                          kAutoManyPacketRays, kAutoSmallPacketFaces, RK_REF_PACKET_HANDOFF_FACES);
+    const uint32_t faces_limit = limit_of(g_packet_faces.load(std::memory_order_relaxed), n, kAutoSmallPacketFaces,
+                                          RK_REF_PACKET_HANDOFF_FACES);
     const uint32_t cap = std::min<uint32_t>(gx * gy, g_list_cap.load(std::memory_order_relaxed));
     const uint32_t fcap = std::min<uint32_t>(cap, kForcedCap);
     // [head | list | records | pops (2 words each) | forced list | diverged | slots' heads | cut | hit entries]
@@ -1560,8 +1553,8 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
     // A ray whose leaves pass g_ray_faces faces, or a ray that passes every
     // box test (at its first leaf), is traced again by the second pass, one
     // wave per ray.
-    const uint32_t faces_limit = limit_of(g_ray_faces.load(std::memory_order_relaxed), n, face_count, kAutoManyRays,
-                                          kAutoSmallRayFaces, RK_REF_HANDOFF_FACES);
+    const uint32_t faces_limit = limit_of(g_ray_faces.load(std::memory_order_relaxed), n, kAutoSmallRayFaces,
+                                          RK_REF_HANDOFF_FACES);
     const uint32_t cap = std::min<uint32_t>(n, g_list_cap.load(std::memory_order_relaxed));
     const uint32_t ucap = std::min<uint32_t>(cap, kCrossCap);
     // [head | list | pops (2 words each) | crossing rays: list, buckets (8), redo, diverged, heads | cut | hit entries]
