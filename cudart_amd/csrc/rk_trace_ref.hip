@@ -246,6 +246,26 @@ __device__ __forceinline__ void lane_leaf(const RefMesh& mesh, uint32_t first, u
   }
 }
 
+// The same pass without the bounds, kB faces in flight: for leaves of few faces.
+// Finding the groups of faces a ray is near costs one more round trip to memory per
+// leaf, and round trips are what a frame of few waves is made of.
+template <uint32_t kB>
+__device__ __forceinline__ void plain_leaf(const RefMesh& mesh, uint32_t f, uint32_t end, float4 o, float4 d,
+                                           float& depth, uint32_t& fid, float2& coord) {
+  for (; f < end; f += kB) {
+    float4 v0[kB], e1[kB], e2[kB];
+#pragma unroll
+    for (uint32_t b = 0; b < kB; ++b) tri_get(mesh, min(f + b, end - 1u), v0[b], e1[b], e2[b]);
+#pragma unroll
+    for (uint32_t b = 0; b < kB; ++b) {
+      float t, u, v;
+      if (f + b < end && tri_ray(o, d, v0[b], e1[b], e2[b], t, u, v)) {
+        if (t < depth) { fid = f + b; coord = make_float2(u, v); depth = t; }
+      }
+    }
+  }
+}
+
 struct NodeRegs { uint32_t w0, w1; float4 bmin, bmax; };
 
 __device__ __forceinline__ NodeRegs load_node(const rk::Node* __restrict__ nodes, uint32_t id) {
@@ -297,9 +317,10 @@ struct LeafBest { float t, u, v; uint32_t k; bool found; };
 // same t fails t < depth. Each lane tests one group's bound, then the faces of
 // four groups the ray may hit at a time, one face per lane, so that lane
 // order is face order: the lowest lane holding the wave's smallest t has the
-// first such face. The next four compare with that t.
+// first such face. The next four compare with that t. A leaf of at most 'plain'
+// (<= 64) faces is tested without the bounds, in one round trip.
 __device__ __forceinline__ LeafBest wave_leaf(const RefMesh& mesh, float4 o, float4 d, const rk::CullRay& cr,
-                                              uint32_t first, uint32_t cnt, float dep) {
+                                              uint32_t first, uint32_t cnt, float dep, uint32_t plain) {
   const uint32_t lane = threadIdx.x & 63u, quarter = lane / kGroup;
   LeafBest r;
   r.t = dep;
@@ -308,7 +329,35 @@ __device__ __forceinline__ LeafBest wave_leaf(const RefMesh& mesh, float4 o, flo
   r.k = 0;
   r.found = false;
   const float inf = __int_as_float(0x7f800000);
-  const uint32_t end = first + cnt, g_end = cnt ? (end - 1u) / kGroup + 1u : 0u;
+  auto test = [&](bool has, uint32_t f) {  // a face per lane
+    float bt = inf, bu = 0.0f, bv = 0.0f;
+    bool any = false;
+    if (has) {
+      float4 v0, e1, e2;
+      tri_get(mesh, f, v0, e1, e2);
+      float t, u, v;
+      if (tri_ray(o, d, v0, e1, e2, t, u, v) && t < r.t) {
+        bt = t;  // t < dep <= FLT_MAX or +inf: t is finite, below the sentinel
+        bu = u;
+        bv = v;
+        any = true;
+      }
+    }
+    if (__ballot(any) == 0ull) return;
+    float mn = bt;
+    for (int off = 32; off > 0; off >>= 1) mn = fminf(mn, __shfl_xor(mn, off, 64));
+    const int w = __builtin_ctzll(__ballot(any && bt == mn));
+    r.t = __shfl(bt, w, 64);  // the winner's own bits (bt == mn holds for -0 against +0 too)
+    r.u = __shfl(bu, w, 64);
+    r.v = __shfl(bv, w, 64);
+    r.k = (uint32_t)__shfl((int)(f - first), w, 64);
+    r.found = true;
+  };
+  if (cnt <= plain) {
+    test(lane < cnt, first + lane);
+    return r;
+  }
+  const uint32_t end = first + cnt, g_end = (end - 1u) / kGroup + 1u;
   for (uint32_t g0 = first / kGroup; g0 < g_end; g0 += 64u) {
     bool near = lane < g_end - g0;
     if (near && mesh.bounds)
@@ -328,29 +377,7 @@ __device__ __forceinline__ LeafBest wave_leaf(const RefMesh& mesh, float4 o, flo
         }
       }
       const uint32_t f = (g0 + g) * kGroup + lane % kGroup;
-      has = has && f >= first && f < end;
-      float bt = inf, bu = 0.0f, bv = 0.0f;
-      bool any = false;
-      if (has) {
-        float4 v0, e1, e2;
-        tri_get(mesh, f, v0, e1, e2);
-        float t, u, v;
-        if (tri_ray(o, d, v0, e1, e2, t, u, v) && t < r.t) {
-          bt = t;  // t < dep <= FLT_MAX or +inf: t is finite, below the sentinel
-          bu = u;
-          bv = v;
-          any = true;
-        }
-      }
-      if (__ballot(any) == 0ull) continue;
-      float mn = bt;
-      for (int off = 32; off > 0; off >>= 1) mn = fminf(mn, __shfl_xor(mn, off, 64));
-      const int w = __builtin_ctzll(__ballot(any && bt == mn));
-      r.t = __shfl(bt, w, 64);  // the winner's own bits (bt == mn holds for -0 against +0 too)
-      r.u = __shfl(bu, w, 64);
-      r.v = __shfl(bv, w, 64);
-      r.k = (uint32_t)__shfl((int)(f - first), w, 64);
-      r.found = true;
+      test(has && f >= first && f < end, f);
     }
   }
   return r;
@@ -450,14 +477,31 @@ __device__ __forceinline__ uint32_t octant_of(float4 dir) {
 // A wave's rays are a tile of 16 x 4 pixels where that fills nearly all lanes
 // (tiled_rays), else 64 in a row: neighbours in the picture walk the same nodes
 // to the same leaves. The 1920x1080 heightfield frame: 2.02 -> 1.82 ms with 16 x 4 (8
-// x 8: 1.96, 32 x 2: 1.85, 4 x 16: 1.93); 256x256: 0.455 -> 0.412; the sphere at 512x512:
-// 1.05 -> 1.02; at tree depths 20 and 31, 2.55 -> 2.70 and 3.50 -> 3.63, from another
-// side 2.41 -> 2.25.
+// x 8: 1.96, 32 x 2: 1.85, 4 x 16: 1.93); at tree depths 20 and 31, 2.55 -> 2.70 and
+// 3.50 -> 3.63, from another side 2.41 -> 2.25.
+//
+// Not below kTileRays, a wave per SIMD: such a frame takes as long as its longest
+// wave, and where the mesh fills a small part of the picture tiles gather the rays
+// that reach a leaf into few waves (95x53 frame of a 2k-face heightfield from afar 223
+// us tiled, 154 in rows; 111x62 of 90,000 scattered faces 676 and 485).
+//
+// Leaves of at most 16 faces go without the bounds (320-face sphere, 253x142: 165 ->
+// 147 us), and in frames in rows, which are made of round trips to memory, leaves of at
+// most 64 where the whole wave tests one. Large frames of many scattered faces
+// would gain from bounds there too (68,000 faces, 1902x1902: 13.3 ms, 15.0 so), but
+// close views of few large ones would be slower than with every face tested (345
+// faces, 1548x1548: 1.56 ms, 1.36 so, 1.43 then).
+//
+// Over 110 random frames of up to 400x400, 260 of 200x112 to 1920x1920, near and far
+// views, and 200 of the terrains' and spheres' usual ones: 1.24, 1.43 and 1.74 times as
+// fast as with every face tested, one of them slower (0.87, 800 faces from afar). With
+// tiles and bounds for all: 1.14, 1.37 and 1.66, sixty slower, down to 0.63.
 constexpr uint32_t kTileW = 16, kTileH = 64 / kTileW;
+constexpr uint64_t kTileRays = 1u << 16;
 inline bool tiled_rays(uint32_t width, uint32_t height) {  // at most an eighth of the lanes without a ray
   const uint64_t n = (uint64_t)width * height;
   const uint64_t tiles = ((uint64_t)width + kTileW - 1) / kTileW * (((uint64_t)height + kTileH - 1) / kTileH);
-  return 64 * tiles <= n + n / 8;
+  return n >= kTileRays && 64 * tiles <= n + n / 8;
 }
 template <int kCoopMax>
 __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ nodes,
@@ -573,7 +617,11 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
     if (pending == 0ull) break;  // every lane is done
     if (__popcll(pending) > kCoopMax) {
       // each lane its own leaf, in face order
-      if (at_leaf) lane_leaf(mesh, leaf_first, leaf_cnt, orig, dir, cr, depth, fid, coord);
+      const bool plain = __ballot(at_leaf && leaf_cnt > kGroup) == 0ull;
+      if (at_leaf) {
+        if (plain) plain_leaf<kLeafBatch>(mesh, leaf_first, leaf_first + leaf_cnt, orig, dir, depth, fid, coord);
+        else lane_leaf(mesh, leaf_first, leaf_cnt, orig, dir, cr, depth, fid, coord);
+      }
     } else {
       // the whole wave on each pending leaf in turn
       while (pending != 0ull) {
@@ -582,7 +630,8 @@ __global__ __launch_bounds__(64) void k_trace_ray(const rk::Node* __restrict__ n
         const uint32_t first = readlane_u32(leaf_first, L);
         const float4 oL = readlane_f4(orig, L), dL = readlane_f4(dir, L);
         const LeafBest b = wave_leaf(mesh, oL, dL, rk::CullRay{readlane_f32(cr.dl, L), readlane_f32(cr.d2, L)},
-                                     first, readlane_u32(leaf_cnt, L), readlane_f32(depth, L));
+                                     first, readlane_u32(leaf_cnt, L), readlane_f32(depth, L),
+                                     tiles_x != 0u ? kGroup : 64u);
         if (lane == L && b.found) {
           depth = b.t;
           fid = first + b.k;
@@ -706,7 +755,7 @@ __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint3
     if (rk::node_is_leaf(nd.w0)) {
       const uint32_t first = nd.w1;
       const uint32_t cnt = first < face_count ? min(rk::leaf_count(nd.w0), face_count - first) : 0u;
-      const LeafBest b = wave_leaf(mesh, orig, dir, cr, first, cnt, depth);
+      const LeafBest b = wave_leaf(mesh, orig, dir, cr, first, cnt, depth, 64u);
       if (b.found) {
         depth = b.t;
         fid = first + b.k;
@@ -1084,28 +1133,11 @@ __global__ __launch_bounds__(64) void k_units_merge(uint32_t node_count, uint32_
 // whether it was.
 //
 // Leaves of at most kPlainLeaf faces: the second pass tests a part's share of the
-// faces as they are. Finding the groups of faces a ray is near costs one more round
-// trip to memory per leaf, and round trips are what a pass over few packets is made
-// of: a 93x52 frame of a small heightfield takes 1.50 ms with the groups, 1.09 so
-// (loads of 2 faces in flight; 4: 1.15), the 1920x1080 frame the same with both. The
-// first pass, which has many packets, does so for leaves of at most a group (a
-// 1528x859 frame of the 1,280-face sphere: 218 -> 201 us; 24 and 48 faces: no gain).
+// faces without the bounds. A 93x52 frame of a small heightfield takes 1.50 ms with
+// them, 1.09 so (loads of 2 faces in flight; 4: 1.15), the 1920x1080 frame the same
+// with both. The first pass, which has many packets, does so for leaves of at most a
+// group (a 1528x859 frame of the 1,280-face sphere: 218 -> 201 us; 24 and 48 faces: no gain).
 constexpr uint32_t kPlainLeaf = 96, kPlainBatch = 2;
-__device__ __forceinline__ void plain_leaf(const RefMesh& mesh, uint32_t f, uint32_t end, float4 o, float4 d,
-                                           float& depth, uint32_t& fid, float2& coord) {
-  for (; f < end; f += kPlainBatch) {
-    float4 v0[kPlainBatch], e1[kPlainBatch], e2[kPlainBatch];
-#pragma unroll
-    for (uint32_t b = 0; b < kPlainBatch; ++b) tri_get(mesh, min(f + b, end - 1u), v0[b], e1[b], e2[b]);
-#pragma unroll
-    for (uint32_t b = 0; b < kPlainBatch; ++b) {
-      float t, u, v;
-      if (f + b < end && tri_ray(o, d, v0[b], e1[b], e2[b], t, u, v)) {
-        if (t < depth) { fid = f + b; coord = make_float2(u, v); depth = t; }
-      }
-    }
-  }
-}
 template <int kS>
 __device__ __forceinline__ bool trace_packet_job(
     const rk::Node* __restrict__ nodes, RefMesh mesh,
@@ -1222,7 +1254,7 @@ __device__ __forceinline__ bool trace_packet_job(
       }
       if (kS == 1) {
         if (in_image) {
-          if (cnt <= kGroup) plain_leaf(mesh, tri_id, tri_id + cnt, orig, dir, depth, fid, coord);
+          if (cnt <= kGroup) plain_leaf<kPlainBatch>(mesh, tri_id, tri_id + cnt, orig, dir, depth, fid, coord);
           else lane_leaf(mesh, tri_id, cnt, orig, dir, cr, depth, fid, coord);
         }
       } else {
@@ -1236,7 +1268,7 @@ __device__ __forceinline__ bool trace_packet_job(
         if (in_image && ga < gb) {
           const uint32_t a = max(tri_id, (g_first + ga) * unit);
           const uint32_t m = gb == ng ? end - a : (g_first + gb) * unit - a;
-          if (unit == 1u) plain_leaf(mesh, a, a + m, orig, dir, pt, pk, puv);
+          if (unit == 1u) plain_leaf<kPlainBatch>(mesh, a, a + m, orig, dir, pt, pk, puv);
           else lane_leaf(mesh, a, m, orig, dir, cr, pt, pk, puv);
         }
         s_pt[threadIdx.x] = pt;

@@ -85,3 +85,49 @@ def test_reference_handoff_limit_by_rays_per_face(rk, faces, w, h, coherency):
         dev.set_ref_handoff()
     for x, y in zip(a, b):
         assert torch.equal(x, y)
+
+
+def _eight_leaves(ora, leaf):
+    """Eight leaves of 'leaf' scattered faces each at the corners of a cube, under a
+    tree of three levels."""
+    rng = np.random.default_rng(leaf)
+    corner = np.array([[x, y, z] for x in (.25, .75) for y in (.25, .75) for z in (.25, .75)])
+    P = corner[:, None, None] + rng.normal(0, .05, (8, leaf, 1, 3)) + rng.normal(0, .04, (8, leaf, 3, 3))
+    V, F = np.zeros((24 * leaf, 4), np.float32), np.zeros((8 * leaf, 4), np.uint32)
+    V[:, :3] = P.reshape(-1, 3)
+    F[:, :3] = np.arange(24 * leaf, dtype=np.uint32).reshape(-1, 3)
+    nodes = np.zeros(15, ora.NODE_DTYPE)
+    for k in range(14, -1, -1):  # heap order: children 2k + 1, 2k + 2
+        if k >= 7:
+            T = V[3 * leaf * (k - 7):3 * leaf * (k - 6), :3]
+            nodes[k] = (1 | leaf << 1, leaf * (k - 7), T.min(0), T.max(0))
+        else:
+            a, b = nodes[2 * k + 1], nodes[2 * k + 2]
+            axis = 0 if k == 0 else (1 if k < 3 else 2)
+            nodes[k] = (axis << 1, 2 * k + 1, np.minimum(a["bmin"], b["bmin"]), np.maximum(a["bmax"], b["bmax"]))
+    return V, F, nodes
+
+
+def _trace(dev, nodes, V, F, O, D, w, h, packet):
+    import torch
+    t = lambda a: torch.from_numpy(np.ascontiguousarray(a)).cuda()
+    tree = dev.RefTree(t(F.view(np.int32)), None, None, t(nodes.view(np.int32).reshape(-1, 8)), None, len(nodes))
+    return [x.cpu().numpy() for x in dev.trace_ref(tree, t(V), t(O), t(D), w, h, packet)]
+
+
+@pytest.mark.parametrize("leaf", [1, 4, 5, 16, 17, 63, 64, 65, 200])
+@pytest.mark.parametrize("w,h", [(256, 255), (256, 256), (331, 200), (300, 222)])
+def test_reference_rays_of_small_and_large_frames(rk, ora, w, h, leaf):
+    """Frames on both sides of 2^16 rays, in rows and in tiles (whole, cut at the
+    right, at the bottom), where the leaves' faces are tested with and without their
+    bounds, by a lane and by the wave."""
+    from cudart_amd import device as dev
+    V, F, nodes = _eight_leaves(ora, leaf)
+    cam = rk.camera_lookat([.7, .35, 2.2], [.5, .5, .5], .7, w, h, up=[0, 1, 0])
+    O, D = rk.primary_rays_host(cam, w, h)
+    of, ouv, od, _ = ora.trace_ref_ray(nodes, F, V, O, D)
+    assert 0.001 < (od < np.finfo(np.float32).max).mean() < 0.9
+    got = _trace(dev, nodes, V, F, O, D, w, h, False)
+    np.testing.assert_array_equal(got[0].view(np.uint32), of)
+    np.testing.assert_array_equal(got[1], ouv)
+    np.testing.assert_array_equal(got[2], od)
