@@ -1136,8 +1136,38 @@ __global__ __launch_bounds__(64) void k_units_merge(uint32_t node_count, uint32_
 // faces without the bounds. A 93x52 frame of a small heightfield takes 1.50 ms with
 // them, 1.09 so (loads of 2 faces in flight; 4: 1.15), the 1920x1080 frame the same
 // with both. The first pass, which has many packets, does so for leaves of at most a
-// group (a 1528x859 frame of the 1,280-face sphere: 218 -> 201 us; 24 and 48 faces: no gain).
+// group (a 1528x859 frame of the 1,280-face sphere: 218 -> 201 us; 24 and 48 faces: no
+// gain), through the scalar cache, since every ray of the block tests the same faces:
+// large frames of small meshes 3-5% faster than with a load per lane, 1714x964 of that
+// sphere 244 -> 234 us (230 with every face tested); 4 faces in flight no better than 2
+// (8: 8% slower). Close views of few large faces, where bounds skip little in larger
+// leaves, stay slower than with every face tested from LDS: 1.82 against 1.56 ms at
+// 1497x1497 of 1,126 scattered faces. Six waves per SIMD for five (2 faces at a time
+// in larger leaves) make up for that, but cost large frames of terrains 5-8%.
 constexpr uint32_t kPlainLeaf = 96, kPlainBatch = 2;
+__device__ __forceinline__ void uniform_leaf(const RefMesh& mesh, uint32_t f, uint32_t end, float4 o, float4 d,
+                                             float& depth, uint32_t& fid, float2& coord) {
+  f = __builtin_amdgcn_readfirstlane(f);
+  end = __builtin_amdgcn_readfirstlane(end);
+  for (; f < end; f += kPlainBatch) {
+    float4 v0[kPlainBatch], e1[kPlainBatch], e2[kPlainBatch];
+#pragma unroll
+    for (uint32_t b = 0; b < kPlainBatch; ++b) {
+      typedef const __attribute__((address_space(4))) float uniform_float;
+      uniform_float* r = (uniform_float*)(uintptr_t)(mesh.tris + kRecFloats * (size_t)min(f + b, end - 1u));
+      v0[b] = make_float4(r[0], r[1], r[2], 0.0f);
+      e1[b] = make_float4(r[3], r[4], r[5], 0.0f);
+      e2[b] = make_float4(r[6], r[7], r[8], 0.0f);
+    }
+#pragma unroll
+    for (uint32_t b = 0; b < kPlainBatch; ++b) {
+      float t, u, v;
+      if (f + b < end && tri_ray(o, d, v0[b], e1[b], e2[b], t, u, v)) {
+        if (t < depth) { fid = f + b; coord = make_float2(u, v); depth = t; }
+      }
+    }
+  }
+}
 template <int kS>
 __device__ __forceinline__ bool trace_packet_job(
     const rk::Node* __restrict__ nodes, RefMesh mesh,
@@ -1254,7 +1284,7 @@ __device__ __forceinline__ bool trace_packet_job(
       }
       if (kS == 1) {
         if (in_image) {
-          if (cnt <= kGroup) plain_leaf<kPlainBatch>(mesh, tri_id, tri_id + cnt, orig, dir, depth, fid, coord);
+          if (cnt <= kGroup && mesh.tris) uniform_leaf(mesh, tri_id, tri_id + cnt, orig, dir, depth, fid, coord);
           else lane_leaf(mesh, tri_id, cnt, orig, dir, cr, depth, fid, coord);
         }
       } else {

@@ -131,3 +131,25 @@ def test_reference_rays_of_small_and_large_frames(rk, ora, w, h, leaf):
     np.testing.assert_array_equal(got[0].view(np.uint32), of)
     np.testing.assert_array_equal(got[1], ouv)
     np.testing.assert_array_equal(got[2], od)
+
+
+@pytest.mark.parametrize("leaf", [1, 2, 3, 15, 16, 17, 96, 97])
+@pytest.mark.parametrize("first_pass", [True, False])
+def test_packet_leaf_sizes(rk, ora, leaf, first_pass):
+    """Leaves whose faces come through the scalar cache, without and with their
+    bounds, in the first pass and in the second."""
+    from cudart_amd import device as dev
+    V, F, nodes = _eight_leaves(ora, leaf)
+    w, h = 131, 89
+    cam = rk.camera_lookat([.7, .35, 2.2], [.5, .5, .5], .7, w, h, up=[0, 1, 0])
+    O, D = rk.primary_rays_host(cam, w, h)
+    of, ouv, od, _ = ora.trace_ref_packet(nodes, F, V, O, D, w, h)
+    assert 0.001 < (od < np.finfo(np.float32).max).mean() < 0.9
+    try:
+        dev.set_ref_handoff(packet_faces=0xFFFFFFFF if first_pass else 0)
+        got = _trace(dev, nodes, V, F, O, D, w, h, True)
+    finally:
+        dev.set_ref_handoff()
+    np.testing.assert_array_equal(got[0].view(np.uint32), of)
+    np.testing.assert_array_equal(got[1], ouv)
+    np.testing.assert_array_equal(got[2], od)
