@@ -67,6 +67,7 @@ constexpr uint32_t kOneMax = 4096;  // up to this many keys one workgroup sorts 
 constexpr int kLook = RK_SORT_LOOK;  // look-back status loads in flight per digit
 
 constexpr uint32_t kGroup = 16;  // tiles per look-back group
+constexpr uint32_t kMaxCopies = 8;  // of the digit counts
 
 // Exclusive scan over a block of kT threads of kPer consecutive values each.
 template <int kT, int kPer>
@@ -246,7 +247,13 @@ __global__ __launch_bounds__(kThreads) void k_rs_scatter(const K* __restrict__ k
       total[0] += c;
     }
     rk::atomic_store_relaxed(status + (size_t)tile * D + d, (!kGroups && tile == 0 ? kInc : kAgg) | tag | total[0]);
-    for (uint32_t c = 0; c < copies; ++c) counted[0] += hist[(size_t)c * copy_words + d];
+    // all loads in flight: one after the other, copies cost a pass on 100,000 keys 1 us
+    // of its 8 (a sort of them 47.6 against 42.8 us; 1M 67 against 62)
+    uint32_t part[kMaxCopies];
+#pragma unroll
+    for (uint32_t c = 0; c < kMaxCopies; ++c) part[c] = hist[(size_t)min(c, copies - 1u) * copy_words + d];
+#pragma unroll
+    for (uint32_t c = 0; c < kMaxCopies; ++c) counted[0] += c < copies ? part[c] : 0u;
   }
   block_excl_scan<kThreads, 1>(total, local, s_tmp);
   if (mine) {
@@ -606,7 +613,7 @@ rk_status rk_sort_plan(uint32_t n, int bits, bool anywhere, K* keys, uint32_t* v
     const bool groups = items != kItems;
     p.items = items;
     p.tiles = tiles_of(n, items);
-    p.copies = copies ? std::min<uint32_t>(8u, 1u + p.tiles / 8u) : 1u;
+    p.copies = copies ? std::min(kMaxCopies, 1u + p.tiles / 8u) : 1u;
     p.head_words = p.one ? 1 : 1 + (size_t)p.copies * p.passes * 256;
     p.status_words = p.one ? 0 : ((size_t)p.tiles + (groups ? (p.tiles + kGroup - 1) / kGroup : 0)) * 256;
     RkArena ar(ws, ws_bytes);
