@@ -1361,7 +1361,11 @@ extern "C" rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_fl
       RK_CHECK_LAUNCH();
       big = std::min(2 * big, big_bound);
     }
-    hipLaunchKernelGGL(k_sah_subtrees, dim3(std::min(2048u, n / 256 + 1)), dim3(kTreeThreads), 0, st, s, done);
+    // 8 starting items a workgroup: starts of a face or two make more groups than
+    // n / 256 (hybrid build from 1,280 leaves of one face 111 us with 6 workgroups,
+    // 102 with 161; from 300,000 faces at depth 24 208 and 192)
+    const uint32_t groups = std::max(n / 256, starts_found / 8) + 1;
+    hipLaunchKernelGGL(k_sah_subtrees, dim3(std::min(2048u, groups)), dim3(kTreeThreads), 0, st, s, done);
     RK_CHECK_LAUNCH();
     if ((e = read_ctl(kCtlHist + kHistRead)) != RK_SUCCESS) return e;
     big = level ? got[kCtlBig(level & 1u)] : 0u;
