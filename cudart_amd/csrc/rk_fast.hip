@@ -25,6 +25,7 @@
 // l when it is the right child, so the children of the split between p and
 // p + 1 are records p and p + 1. n records for n faces.
 #include <mutex>
+#include <type_traits>
 
 #include "rk_device.h"
 #include "rk_sort.h"
@@ -753,8 +754,13 @@ constexpr int kXchg = 32, kXchgWords = 4 * kXchg;
 // step only (1: every step); in between they cull against the value they last
 // read, which can only be larger, so they may visit more nodes but find the
 // same closest hit.
+//
+// kApart: leaves' triangles are loaded by instructions of their own, after the
+// nodes' and before the one wait, for rays that share no nodes. With both in one
+// instruction such rays fetch lines into the L1 more than once: 2M incoherent rays on
+// 250,000 faces made 279M requests to the L2 and took 2.35 ms, apart 217M and 1.79.
 template <bool kCount, int kStackN, int kLds, int kWG, bool kOldest = false, int kLeafBatch = 0,
-          int kDonateMin = 1, int kBoundEvery = 1>
+          int kDonateMin = 1, int kBoundEvery = 1, bool kApart = false>
 __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
                                                    uint32_t n_tris, uint32_t root, bool has_ray, float4 orig,
                                                    float4 dir, float depth0, float eps, uint32_t& n_box,
@@ -888,13 +894,19 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
     const bool in_tree = idx < n_tris;
     float4 q0, q1, q2;
     float2 q3;
-    if (owner >= 0 && in_tree && (kLeafBatch == 0 || !at_leaf)) {
+    if (owner >= 0 && in_tree && !(at_leaf && (kLeafBatch != 0 || kApart))) {
       const uint64_t base = at_leaf ? reinterpret_cast<uint64_t>(tris) : reinterpret_cast<uint64_t>(nodes);
       const float4* rec = reinterpret_cast<const float4*>(base + (uint64_t)idx * (at_leaf ? 48u : 64u));
       q0 = rec[0];
       q1 = rec[1];
       q2 = rec[2];
       if (!at_leaf) q3 = *reinterpret_cast<const float2*>(rec + 3);
+    }
+    if (kApart && kLeafBatch == 0 && owner >= 0 && in_tree && at_leaf) {
+      const float4* rec = tris + 3 * (size_t)idx;
+      q0 = rec[0];
+      q1 = rec[1];
+      q2 = rec[2];
     }
     // the owner's best so far bounds a helper's subtree
     float dmax = o_t;
@@ -1108,12 +1120,61 @@ constexpr uint32_t kFetchBoundFaces = 1u << 20;
 // fetched together.
 constexpr uint32_t kMemoryFaces = 1u << 22;
 
+// Between these many faces and from this many rays on, rays in array order that start
+// at different points are traced apart (kApart). With fewer rays, 14 waves per CU, what
+// bounds the trace is the wait per step, and one fetch is faster; with fewer faces the
+// L2 has them, and with more the two are level. 262,144 rays on 70,000, 300,000 and 1M
+// faces: together 177, 371 and 605 us, apart 165, 300 and 565; 196,608 on 300,000: 231
+// and 261; 4M on 1M faces 7.8 and 7.4 ms.
+// A wave of one origin, as a picture's, fetches together: 28 pictures of such trees take
+// 1% longer than with the plain kernel. (Both ways need 89 registers if they may, and 20
+// waves per CU then cost pictures 5%: __launch_bounds__ holds them to 80.)
+constexpr uint32_t kApartFaces = 3u << 14, kApartFacesEnd = 3u << 19, kApartRays = 7u << 15;
+
+// Whether the wave's rays start at one point.
+__device__ __forceinline__ bool one_origin(const float4* __restrict__ origins, uint32_t l, bool has_ray) {
+  const float4 o = has_ray ? origins[l] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const auto first = [](float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); };
+  return __ballot(o.x != first(o.x) || o.y != first(o.y) || o.z != first(o.z)) == 0ull;
+}
+
+// Ray l of this lane (when has_ray), traced and stored.
+template <bool kCount, int kWG, int kLds, bool kOldest, int kLeafBatch, int kDonateMin, int kBoundEvery, bool kApart>
+__device__ __forceinline__ void trace_lane(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
+                                           uint32_t n_tris, const float4* __restrict__ origins,
+                                           const float4* __restrict__ dirs, uint32_t l, bool has_ray,
+                                           uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
+                                           float* __restrict__ depths, float eps,
+                                           unsigned long long* __restrict__ counters, bool reset, uint2* stack,
+                                           uint32_t* xchg) {
+  uint32_t n_box = 0, n_tri = 0;
+  const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const RayHit h = trace_ray_shared<kCount, kStack, kLds, kWG, kOldest, kLeafBatch, kDonateMin, kBoundEvery, kApart>(
+      nodes, tris, n_tris, 0u, has_ray, has_ray ? origins[l] : zero4, has_ray ? dirs[l] : zero4,
+      has_ray ? (reset ? RK_HUGE : depths[l]) : 0.0f, eps, n_box, n_tri, stack, xchg);
+  if (kCount) {
+    atomicAdd(counters, (unsigned long long)n_box);
+    atomicAdd(counters + 1, (unsigned long long)n_tri);
+  }
+  if (has_ray) {
+    if (h.pos != 0xFFFFFFFFu) {
+      faces_id[l] = h.pos;
+      coords[l] = make_float2(h.u, h.v);
+      depths[l] = h.t;
+    } else if (reset) {
+      depths[l] = RK_HUGE;  // the reset a fill kernel would have done; the miss's id and coords stay
+    }
+  }
+}
+
 // kWG threads per workgroup, runs of kRun rays per band (spread_ray; 0: 64
 // consecutive rays per wave), kLds stack entries per lane in LDS. The
-// defaults above are one variant; rk_fast_autotune chooses among several.
+// defaults above are one variant; rk_fast_autotune chooses among several. kFetch:
+// whether nodes and leaves are fetched together or apart, or by the wave's origins.
+enum Fetch { kTogether, kAlwaysApart, kByOrigin };
 template <bool kCount, int kWG, uint32_t kRun, int kLds, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
-          int kBoundEvery = 1, bool kXcdRuns = false>
-__global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
+          int kBoundEvery = 1, bool kXcdRuns = false, Fetch kFetch = kTogether>
+__global__ __launch_bounds__(kWG, kFetch == kByOrigin ? 6 : 1) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
                                                       uint32_t n_tris, const float4* __restrict__ origins,
                                                       const float4* __restrict__ dirs, uint32_t n_rays,
                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
@@ -1131,24 +1192,15 @@ __global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ 
   const bool has_ray = l < n_rays;
   __shared__ uint2 s_stack[kLds * kWG];
   __shared__ uint32_t s_xchg[kWG / 64][kXchgWords];
-  uint32_t n_box = 0, n_tri = 0;
-  const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  const RayHit h = trace_ray_shared<kCount, kStack, kLds, kWG, kOldest, kLeafBatch, kDonateMin, kBoundEvery>(
-      nodes, tris, n_tris, 0u, has_ray, has_ray ? origins[l] : zero4, has_ray ? dirs[l] : zero4,
-      has_ray ? (reset ? RK_HUGE : depths[l]) : 0.0f, eps, n_box, n_tri, s_stack, s_xchg[threadIdx.x >> 6]);
-  if (kCount) {
-    atomicAdd(counters, (unsigned long long)n_box);
-    atomicAdd(counters + 1, (unsigned long long)n_tri);
-  }
-  if (has_ray) {
-    if (h.pos != 0xFFFFFFFFu) {
-      faces_id[l] = h.pos;
-      coords[l] = make_float2(h.u, h.v);
-      depths[l] = h.t;
-    } else if (reset) {
-      depths[l] = RK_HUGE;  // the reset a fill kernel would have done; the miss's id and coords stay
-    }
-  }
+  const auto go = [&](auto apart) {
+    trace_lane<kCount, kWG, kLds, kOldest, kLeafBatch, kDonateMin, kBoundEvery, decltype(apart)::value>(
+        nodes, tris, n_tris, origins, dirs, l, has_ray, faces_id, coords, depths, eps, counters, reset, s_stack,
+        s_xchg[threadIdx.x >> 6]);
+  };
+  if (kFetch == kAlwaysApart || (kFetch == kByOrigin && !one_origin(origins, l, has_ray)))
+    go(std::integral_constant<bool, kFetch != kTogether>());
+  else
+    go(std::integral_constant<bool, false>());
 }
 
 inline unsigned blocks_for(uint32_t n, uint32_t per) { return (n + per - 1) / per; }
@@ -2210,8 +2262,13 @@ extern "C" rk_status rk_fast_trace(rk_stream stream, const rk_fast_bvh* bvh, con
   const TraceVariant* tv = trace_variant(options ? options->config : 0u);
   if (!tv) return RK_ERROR_INVALID_VALUE;
   TraceVariant v = *tv;
-  if ((!options || options->config == 0) && bvh->face_count >= kMemoryFaces)
-    v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32>;
+  if (!options || options->config == 0) {
+    const uint32_t faces = bvh->face_count;
+    if (faces >= kMemoryFaces)
+      v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32>;
+    else if (faces >= kApartFaces && faces < kApartFacesEnd && n_rays >= kApartRays)
+      v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kLdsStack, false, 0, kTraceDonateMin, 1, false, kByOrigin>;
+  }
   return launch_trace_variant(rk_hip_stream(stream), v, bvh, origins, directions, n_rays, faces_id, coords, depths,
                               det_eps_of(options), trace_flags_of(options));
 }
@@ -2338,10 +2395,10 @@ extern "C" rk_status rk_fast_trace_sorted(rk_stream stream, const rk_fast_bvh* b
   const TraceKernel kernel =
       !by_rule ? tv->kernel
       : bvh->face_count >= kFetchBoundFaces
-          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32, 1, true>
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32, 1, true, kAlwaysApart>
       : bvh->face_count >= kXcdFaces
-          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, true>
-          : k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin>;
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, true, kAlwaysApart>
+          : k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, false, kAlwaysApart>;
   hipLaunchKernelGGL(kernel, dim3(blocks_for(n_rays, tv->wg)), dim3(tv->wg), 0, st, nodes,
                      static_cast<const float4*>(bvh->tris), bvh->face_count, o,
                      reinterpret_cast<const float4*>(directions), n_rays, faces_id, reinterpret_cast<float2*>(coords),
