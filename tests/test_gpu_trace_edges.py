@@ -178,3 +178,70 @@ def test_packet_leaf_sizes(rk, ora, leaf, first_pass):
     np.testing.assert_array_equal(got[0].view(np.uint32), of)
     np.testing.assert_array_equal(got[1], ouv)
     np.testing.assert_array_equal(got[2], od)
+
+
+@pytest.mark.parametrize("every", [True, False])
+def test_more_forced_packets_than_the_split_takes(rk, ora, every):
+    """A frame of 1,225 packets, each with a ray (or all its rays) whose direction has
+    a component of 0: the split takes 1,024 of them."""
+    from cudart_amd import device as dev
+    V, F, nodes = _eight_leaves(ora, 16)
+    w, h = 560, 420
+    cam = rk.camera_lookat([2.2, .35, .6], [.5, .5, .5], .6, w, h, up=[0, 1, 0])
+    O, D = rk.primary_rays_host(cam, w, h)
+    O = O.reshape(h, w, 4).copy()
+    D = D.reshape(h, w, 4).copy()
+    pick = np.s_[:, :] if every else np.s_[2::12, 3::16]
+    D[pick][..., 2] = 0
+    O[pick][..., 2] = np.linspace(.1, .9, O[pick].shape[1], dtype=np.float32)
+    O, D = O.reshape(-1, 4), D.reshape(-1, 4)
+    of, ouv, od, _ = ora.trace_ref_packet(nodes, F, V, O, D, w, h)
+    assert 0.01 < (od < np.finfo(np.float32).max).mean() < 0.9
+    got = _trace(dev, nodes, V, F, O, D, w, h, True)
+    np.testing.assert_array_equal(got[0].view(np.uint32), of)
+    np.testing.assert_array_equal(got[1], ouv)
+    np.testing.assert_array_equal(got[2], od)
+
+
+@pytest.mark.parametrize("packet", [True, False])
+def test_split_walks_past_their_hit_lists(rk, ora, packet):
+    """256 subtrees of two faces, layers one behind the other: rays that walk every
+    subtree hit most of them, more than the lists hold (32 entries per ray, 2 per
+    packet's ray, on average)."""
+    from cudart_amd import device as dev
+    rng = np.random.default_rng(8)
+    n, w, h = 256, 64, 48
+    P = np.zeros((n, 2, 3, 3))
+    P[..., 0] = np.linspace(0, 1, n)[:, None, None] + rng.uniform(0, 1e-3, (n, 2, 3))
+    P[:, 0, :, 1:] = [(-.2, -.2), (1.2, -.2), (-.2, 1.2)]
+    P[:, 1, :, 1:] = [(1.2, 1.2), (-.2, 1.2), (1.2, -.2)]
+    P[..., 1:] += rng.normal(0, .02, (n, 2, 3, 2))
+    order = rng.permutation(n)  # the nearest layer in no particular subtree
+    V, F = np.zeros((6 * n, 4), np.float32), np.zeros((2 * n, 4), np.uint32)
+    V[:, :3] = P[order].reshape(-1, 3)
+    F[:, :3] = np.arange(6 * n, dtype=np.uint32).reshape(-1, 3)
+    nodes = np.zeros(2 * n - 1, ora.NODE_DTYPE)
+    for k in range(2 * n - 2, -1, -1):
+        if k >= n - 1:
+            T = V[6 * (k - n + 1):6 * (k - n + 2), :3]
+            nodes[k] = (1 | 2 << 1, 2 * (k - n + 1), T.min(0), T.max(0))
+        else:
+            a, b = nodes[2 * k + 1], nodes[2 * k + 2]
+            nodes[k] = ((k % 3) << 1, 2 * k + 1, np.minimum(a["bmin"], b["bmin"]), np.maximum(a["bmax"], b["bmax"]))
+    O, D = np.zeros((w * h, 4), np.float32), np.zeros((w * h, 4), np.float32)
+    O[:, 0] = -1
+    O[:, 1:3] = rng.uniform(0, 1, (w * h, 2))
+    D[:, 0] = 1
+    D[:, 1] = rng.normal(0, .05, w * h)
+    hits = 0
+    for k in range(n - 1, 2 * n - 1):
+        hits += int((ora.trace_ref_ray(nodes[k:k + 1], F, V, O, D)[2] < np.finfo(np.float32).max).sum())
+    assert hits > 2 * 32 * w * h
+    if packet:
+        of, ouv, od, _ = ora.trace_ref_packet(nodes, F, V, O, D, w, h)
+    else:
+        of, ouv, od, _ = ora.trace_ref_ray(nodes, F, V, O, D)
+    got = _trace(dev, nodes, V, F, O, D, w, h, packet)
+    np.testing.assert_array_equal(got[0].view(np.uint32), of)
+    np.testing.assert_array_equal(got[1], ouv)
+    np.testing.assert_array_equal(got[2], od)
