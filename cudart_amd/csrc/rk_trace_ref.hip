@@ -724,33 +724,24 @@ __global__ __launch_bounds__(256) void k_units_cut(const rk::Node* __restrict__ 
 
 // The walk of ray l by the whole wave with the reference's rules (the same
 // pops, box tests, stack overflow and visit limits), each leaf tested by the
-// whole wave (wave_leaf), from node root with the reference's stack holding
-// sp_base entries below it (0 and 0: the ray's walk), from depth, fid and
-// coord. The stack's entry e is lane e % 64 of st0 (e < 64) or st1.
-struct WalkResult { float depth; uint32_t fid; float2 coord; uint32_t pops; bool stopped; };
-
-__device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint32_t sp_base, float depth,
-                                                uint32_t fid, float2 coord, const rk::Node* __restrict__ nodes,
-                                                RefMesh mesh,
-                                                const float4* __restrict__ origins,
-                                                const float4* __restrict__ dirs, uint32_t node_count,
-                                                uint32_t face_count) {
+// whole wave (wave_leaf), from the depth, face and coordinates given, into them.
+// The stack's entry e is lane e % 64 of st0 (e < 64) or st1.
+__device__ __forceinline__ void wave_walk(uint32_t l, float& depth, uint32_t& fid, float2& coord,
+                                          const rk::Node* __restrict__ nodes, RefMesh mesh,
+                                          const float4* __restrict__ origins, const float4* __restrict__ dirs,
+                                          uint32_t node_count, uint32_t face_count) {
   const int lane = (int)(threadIdx.x & 63u);
   const uint32_t max_visits = 2 * node_count + 2;
   const float4 orig = origins[l], dir = dirs[l];
   const float4 invdir = invdir_of(dir);
   const rk::CullRay cr = cull_ray4(orig, dir);
-  uint32_t st0 = lane == 0 ? root : 0u, st1 = 0u;
+  uint32_t st0 = 0u, st1 = 0u;  // the root
   int sp = 1;
   uint32_t visits = 0;
-  bool stopped = false;
   while (sp > 0 && ++visits <= max_visits) {
     --sp;
     const uint32_t nid = readlane_u32(sp < 64 ? st0 : st1, sp & 63);
-    if (nid >= node_count) {  // never taken for a tree built by this library
-      stopped = true;
-      break;
-    }
+    if (nid >= node_count) break;  // never taken for a tree built by this library
     const NodeRegs nd = load_node(nodes, nid);
     if (rk::node_is_leaf(nd.w0)) {
       const uint32_t first = nd.w1;
@@ -766,10 +757,7 @@ __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint3
       if (box_ray(nd.bmin, nd.bmax, orig, invdir, t) && t < depth) {
         uint32_t nearc, farc;
         children_order(nd.w0, nd.w1, dir, nearc, farc);
-        if ((uint32_t)sp + sp_base + 2u > (uint32_t)kStack) {  // cannot occur for trees of depth <= 94
-          stopped = true;
-          break;
-        }
+        if (sp + 2 > kStack) break;  // cannot occur for trees of depth <= 94
         if (lane == (sp & 63)) {
           if (sp < 64) st0 = farc;
           else st1 = farc;
@@ -783,13 +771,6 @@ __device__ __forceinline__ WalkResult wave_walk(uint32_t l, uint32_t root, uint3
       }
     }
   }
-  WalkResult r;
-  r.depth = depth;
-  r.fid = fid;
-  r.coord = coord;
-  r.pops = visits;
-  r.stopped = stopped;
-  return r;
 }
 
 // The second pass of the per-ray traversal: one wave per ray handed off (and
@@ -805,12 +786,14 @@ __global__ __launch_bounds__(64) void k_trace_ray_wave(const rk::Node* __restric
   const uint32_t count = min(handoff[0], handoff_cap), again = min(handoff[4], redo_cap);
   for (uint32_t i = blockIdx.x; i < count + again; i += gridDim.x) {
     const uint32_t l = i < count ? handoff[kHandoffHead + i] : redo[i - count];
-    const WalkResult r = wave_walk(l, 0u, 0u, depths[l], faces_id[l], coords[l], nodes, mesh, origins, dirs,
-                                   node_count, face_count);
+    float depth = depths[l];
+    uint32_t fid = faces_id[l];
+    float2 coord = coords[l];
+    wave_walk(l, depth, fid, coord, nodes, mesh, origins, dirs, node_count, face_count);
     if (threadIdx.x == 0) {
-      faces_id[l] = r.fid;
-      coords[l] = r.coord;
-      depths[l] = r.depth;
+      faces_id[l] = fid;
+      coords[l] = coord;
+      depths[l] = depth;
     }
   }
 }
