@@ -288,10 +288,10 @@ __device__ __forceinline__ uint32_t block_excl_scan1024(uint32_t v, uint32_t* s_
 //  - a node with a level-L split > a (prefix of the level) stops at the first
 //    one; it splits there if that split is < b;
 //  - for the remaining nodes (suffix) the pointer has left level L: the first
-//    such node walks into the deeper lists (chain_walk); if it stops exactly at
+//    such node walks into the deeper lists (chain_list); if it stops exactly at
 //    the start of level L+1's list, every later suffix node meets the entry test
 //    ptr == idx[L+1] (:375) and is a leaf; otherwise each later node stops at
-//    chain_walk(a).
+//    chain_list(a).
 // What bounds it is the chain from level to level on one CU, so the chain runs
 // in LDS: the first kTopoLists splits (the lists of the top levels, which hold
 // at most 2^L), and the current and the next level's records; memory is read for

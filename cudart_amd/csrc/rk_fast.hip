@@ -614,12 +614,14 @@ constexpr int kStack = RK_TRACE_STACK;
 #ifndef RK_LDS_STACK
 #define RK_LDS_STACK 8
 #endif
-// Stack entries per lane kept in LDS: 8 x 8 B x 64 lanes is 4 KB per wave,
-// far within the 20 waves per CU that the traces' registers allow. Incoherent
-// rays go deeper: 12 entries in batches and sorted traces (1024-mesh batch with 9,
-// 12, 15, 19: 4.01, 3.96, 4.07, 4.09 ms; 1M rays on the 100k soup: 0.824, 0.788,
-// 0.823, 0.848), 15, all that 20 waves leave room for, on trees past the L2 (16M rays on
-// the 10M soup: 24.3, 24.8, 23.2, 23.7 ms).
+// Stack entries per lane kept in LDS: 8 x 8 B x 64 lanes is 4 KB per wave, with the
+// exchange words 4.5: frames have 24 waves per CU by their 80 registers, which leave
+// room for 12 entries. Incoherent rays go deeper: 12 entries in batches (24 waves, or
+// 20 by the queue kernel's 93 registers; 1024-mesh batch with 9, 12, 15, 19: 4.01,
+// 3.96, 4.07, 4.09 ms) and sorted traces (86 registers, 20 waves; 9, 12 and 15 within
+// 1%: 1M rays on the 100k soup 0.61 ms, 2M on 300k faces 1.78), 15, all that 20 waves
+// leave room for, on trees past the L2 (16M sorted rays on the 10M soup with 12, 15
+// and 19: 23.9, 23.9 and 24.6 ms).
 constexpr int kLdsStack = RK_LDS_STACK, kDeepLdsStack = 12, kDeepestLdsStack = 15;
 
 // intersectTriRay, CUDA_raytraceMeshTree.cu:57-89, with vert0.w = edge1.w =
@@ -883,10 +885,10 @@ __device__ __forceinline__ RayHit trace_ray_shared(const FNode* __restrict__ nod
     // This step's record, a node or a leaf's first triangle, is fetched here for
     // both kinds of lanes, with one wait where there would be one in each branch,
     // and meanwhile the owner's bound is read; its address is computed without a
-    // branch. It takes 86 registers, not 64, and 20 waves per CU that wait once are
+    // branch. It takes 80 registers, not 64, and 24 waves per CU that wait once are
     // faster than 32 that wait twice: the 1024-mesh batch 4.35 -> 3.95 ms, the 1920x1080
     // heightfield frame 192 -> 167 us (179 with branches for the address, and then the
-    // 1380x1035 frame of a small heightfield 82 -> 90; 24 waves: no better), the
+    // 1380x1035 frame of a small heightfield 82 -> 90), the
     // 256x256 icosphere frame 63 -> 55, 32 served requests 3.50 -> 3.03 ms.
     const bool at_leaf = (cur & kLeafBit) != 0u;
     const uint32_t first = (cur & ~kLeafBit) >> 4;
@@ -1104,14 +1106,16 @@ static_assert(kTraceWG % 64 == 0 && kTraceWG <= 1024, "whole waves");
 // Sorted rays of a tree that the eight L2s cannot hold between them: workgroups are
 // dealt to the XCDs in turn, so consecutive ones would fetch the same nodes into all
 // eight L2s. With kXcdRuns an XCD takes runs of kXcdRun consecutive workgroups of the
-// order. 16M rays on the 10M soup, with runs of 1, 32, 128, 512 and an eighth of
-// all: 29.3, 27.6, 27.0, 26.6 and 28.1 ms; 2M on 300k faces (34 MB): 1.668 and 1.627
-// with 1 and 512; 1M on 100k: 0.870 and 0.883.
+// order, on trees of kXcdFaces on. Sort and trace of 300k, 1M and 4M rays: on 600k faces
+// 570 -> 512, 1,280 -> 1,225 and 4,300 -> 4,300 us, on 10M faces 957 -> 871, 2,330 -> 2,075
+// and 7,250 -> 6,230; 16M on 10M 24.6 -> 23.9 ms. 2M on 300k faces, 1.71 -> 1.78, are the
+// one slower. Runs of 32, 128 and 512 are within 4%.
 constexpr uint32_t kXcdRun = 512, kXcdFaces = 1u << 18;
 // And from this many faces on, where what bounds the trace is fetching nodes past
 // the L2, idle lanes take subtrees (which the owner might have culled) only on steps
-// where half the wave is idle: 16M rays on the 10M soup 26.6 -> 24.0 ms, 8M on 3M
-// faces 9.52 -> 9.01, 4M on 1M 3.83 -> 3.80; 2M on 300k 1.63 -> 1.65.
+// where half the wave is idle: 16M rays on the 10M soup 26.8 -> 23.9 ms, 8M on 3M
+// faces 13.5 -> 12.4, 4M on 1M 5.17 -> 4.97. On fewer faces it depends on the rays: 300k and
+// 4M on 400k faces 438 -> 476 us and 3.69 -> 3.62 ms.
 constexpr uint32_t kFetchBoundFaces = 1u << 20;
 // Rays in array order may be a picture's, whose rays share nodes and gain from early
 // help, so the same holds only from where the tree is beyond the 256 MB memory-side cache
@@ -2044,7 +2048,9 @@ struct CameraVariant {
   CameraKernel kernel;
 };
 
-// rk_trace_options.config k selects entry k - 1 (0: the first, the default).
+// rk_trace_options.config k selects entry k - 1 (0: the first, or one that is not listed
+// by the sizes, in rk_fast_trace and rk_fast_trace_sorted). All fetch together; for rays
+// that share no nodes those that postpone leaves come out best (2M on 300,000 faces 1.90 ms).
 #define RK_TRACE_VARIANT(wg, run, lds, old, lb, dm) \
   {wg, run, lds, old, lb, dm, 1, k_fast_trace_v<false, wg, run, lds, old != 0, lb, dm>}
 #define RK_TRACE_VARIANT_B(dm, be) {64, 8, 8, 0, 0, dm, be, k_fast_trace_v<false, 64, 8, 8, false, 0, dm, be>}

@@ -1439,8 +1439,9 @@ static std::atomic<uint32_t> g_packet_faces{RK_HANDOFF_AUTO};
 // and 3.78 against 3.27. Which is better below 2^19 rays depends on the view, which
 // a rule by sizes does not see (per-ray, 256 against 4096): the 20k-face icosphere at
 // 512x512 1.02 and 0.50 ms, from twice as far 0.57 and 0.71; 30,000 scattered faces at
-// 704x545 5.31 and 2.72, from twice as far 1.63 and 3.16. Early is never slower than
-// testing every face was; late at 12 rays per face or more was (the last: 2.06).
+// 704x545 5.31 and 2.72, from twice as far 1.63 and 3.16. Of 570 random per-ray
+// frames early left one slower than testing every face, late from 12 rays per face on
+// many (the last: 2.06).
 constexpr uint32_t kAutoRaysBelow = 1u << 19;
 constexpr uint32_t kAutoSmallRayFaces = 256, kAutoSmallPacketFaces = 512;
 static uint32_t limit_of(uint32_t set, uint32_t n_rays, uint32_t small_limit, uint32_t large_limit) {
@@ -1546,10 +1547,11 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
   hipStream_t st = rk_hip_stream(stream);
   const uint32_t n = (uint32_t)width * (uint32_t)height;
   if (coherency) {
-    // A packet whose leaves pass g_packet_faces faces, or one holding a ray
-    // that passes every box test (the packet then visits every leaf, and all
-    // its rays test every face; at its first leaf), is traced on by the second
-    // pass, kPacketSplit threads per ray, from where it was left.
+    // A packet whose leaves pass g_packet_faces faces is traced on by the second
+    // pass, kPacketSplit threads per ray, from where it was left. One holding a ray
+    // that passes every box test (the packet then visits every leaf, and all its
+    // rays test every face) goes at once to walks split by subtree (k_unit_walk,
+    // k_packet_commit), and to the second pass when these do not take it or diverge.
     const uint32_t gx = (uint32_t)(width + kPW - 1) / kPW, gy = (uint32_t)(height + kPH - 1) / kPH;
     const uint32_t faces_limit = limit_of(g_packet_faces.load(std::memory_order_relaxed), n, kAutoSmallPacketFaces,
                                           RK_REF_PACKET_HANDOFF_FACES);
@@ -1595,9 +1597,10 @@ extern "C" rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* no
     }
     if (mesh.tris && hipFreeAsync(const_cast<float*>(mesh.tris), st) != hipSuccess) return RK_ERROR_DEVICE;
   } else {
-    // A ray whose leaves pass g_ray_faces faces, or a ray that passes every
-    // box test (at its first leaf), is traced again by the second pass, one
-    // wave per ray.
+    // A ray whose leaves pass g_ray_faces faces is traced again by the second
+    // pass, one wave per ray. A ray that passes every box test goes at once to walks
+    // split by subtree (k_unit_walk, k_units_merge), and to the second pass when these
+    // do not take it (then at its first leaf) or diverge.
     const uint32_t faces_limit = limit_of(g_ray_faces.load(std::memory_order_relaxed), n, kAutoSmallRayFaces,
                                           RK_REF_HANDOFF_FACES);
     const uint32_t cap = std::min<uint32_t>(n, g_list_cap.load(std::memory_order_relaxed));

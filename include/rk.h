@@ -202,9 +202,9 @@ rk_status rk_build_lbvh(rk_stream stream, rk_uint4* faces, const rk_float4* vert
  * existing_nodes entries of 'nodes' are an LBVH built with tree_complete = 0 (boxes and
  * indices from that build) and each of its leaves is refined. Node ids are breadth-first
  * (the reference's are in atomicAdd order). nodes_capacity >= existing_nodes + 2n - 1.
- * Faces are reordered in place. Synchronises 'stream' once per tree level, except on the first
- * levels (while a level can hold at most min(4096, n/256) nodes); the info words and the face
- * reorder are still queued on 'stream' when it returns. */
+ * Faces are reordered in place. Synchronises 'stream' a few times (with existing nodes once for
+ * their leaves; for each run of queued levels; for the numbering of a deep tree); the info words
+ * and the face reorder are still queued on 'stream' when it returns. */
 size_t rk_build_sah_workspace_size(uint32_t face_count, uint32_t existing_nodes);
 rk_status rk_build_sah(rk_stream stream, rk_uint4* faces, const rk_float4* vertices, uint32_t face_count,
                        const rk_aabox* hitbox, rk_aabox* boxes, uint32_t* indices, rk_bvnode* nodes,
@@ -225,8 +225,8 @@ rk_status rk_raytrace_mesh_tree(rk_stream stream, const rk_bvnode* nodes, uint32
  * traversal whose leaves pass ray_faces faces is traced again from the start by a wave of
  * its own; a packet whose leaves pass packet_faces faces is resumed where it stands with
  * five threads per ray. A ray with a direction component of 0 (every box test passes for
- * it, so it walks the whole tree), or a packet holding one, goes at its first leaf, to
- * walks split by subtree or by parts of the packet on several CUs. The
+ * it, so it walks the whole tree), or a packet holding one, goes at once to walks split by
+ * subtree on several CUs, and to the second pass when there are too many or they fail. The
  * results are the same. What is handed off goes to a per-call list of list_cap entries
  * (1 .. 65536, device memory from the stream's pool); past its end, rays and packets finish
  * in the first pass. UINT32_MAX turns a second pass off. RK_HANDOFF_AUTO (the default for
@@ -373,7 +373,9 @@ rk_status rk_fast_render_camera(rk_stream stream, const rk_fast_bvh* bvh, const 
  * kind, lanes that are done may take the oldest pending subtree of a lane that
  * is not, rather than its newest (steal_oldest). The variant
  * is rk_trace_options.config; rk_fast_trace_variant describes one (camera != 0:
- * a camera variant). */
+ * a camera variant). Config 0 of rk_fast_trace and rk_fast_trace_sorted is the first
+ * variant up to the sizes from which these take kernels of their own: how nodes and leaves
+ * are fetched, deeper LDS stacks, later help. */
 typedef struct rk_trace_tuning {
   uint32_t config;
   uint32_t workgroup, ray_run, bands, lds_stack, xcd_strips;
