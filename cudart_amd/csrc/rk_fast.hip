@@ -1127,13 +1127,15 @@ constexpr uint32_t kMemoryFaces = 1u << 22;
 // Between these many faces and from this many rays on, rays in array order that start
 // at different points are traced apart (kApart). With fewer rays, 14 waves per CU, what
 // bounds the trace is the wait per step, and one fetch is faster; with fewer faces the
-// L2 has them, and with more the two are level. 262,144 rays on 70,000, 300,000 and 1M
-// faces: together 177, 371 and 605 us, apart 165, 300 and 565; 196,608 on 300,000: 231
-// and 261; 4M on 1M faces 7.8 and 7.4 ms.
-// A wave of one origin, as a picture's, fetches together: 28 pictures of such trees take
-// 1% longer than with the plain kernel. (Both ways need 89 registers if they may, and 20
-// waves per CU then cost pictures 5%: __launch_bounds__ holds them to 80.)
-constexpr uint32_t kApartFaces = 3u << 14, kApartFacesEnd = 3u << 19, kApartRays = 7u << 15;
+// L2 has them; with more, where each node is fetched past the L2 anyway, 4-5% is all
+// there is. 262,144 rays on 70,000 and 300,000 faces: together 182 and 372 us, apart 165
+// and 305; 196,608 on 300,000: 231 and 261. 2M on 300,000, 600,000 and 1M: together 2.48,
+// 3.24 and 3.94 ms, apart 1.92, 2.80 and 3.79.
+// A wave of one origin, as a picture's, fetches together, and 28 pictures of such trees
+// take 0.5-2% longer than with the plain kernel (the test's round trip). Both ways need
+// 89 registers if they may, and 20 waves per CU then cost pictures 5%: __launch_bounds__
+// holds them to 80.
+constexpr uint32_t kApartFaces = 3u << 14, kApartFacesEnd = 3u << 18, kApartRays = 7u << 15;
 
 // Whether the wave's rays start at one point.
 __device__ __forceinline__ bool one_origin(const float4* __restrict__ origins, uint32_t l, bool has_ray) {

@@ -28,7 +28,7 @@ def test_sorted_equals_ray_order(rk, faces):
 
 
 @pytest.mark.parametrize("leaf_max", [1, 5])
-@pytest.mark.parametrize("faces", [(3 << 14) - 1, 3 << 14, (3 << 19) - 1, 3 << 19])
+@pytest.mark.parametrize("faces", [(3 << 14) - 1, 3 << 14, (3 << 18) - 1, 3 << 18])
 def test_rays_of_many_origins(rk, faces, leaf_max):
     """Rays in array order where the waves that start at different points fetch leaves
     apart, on both sides of each limit: rays of many origins, of one, and of both in the
