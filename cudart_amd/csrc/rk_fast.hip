@@ -25,7 +25,6 @@
 // l when it is the right child, so the children of the split between p and
 // p + 1 are records p and p + 1. n records for n faces.
 #include <mutex>
-#include <type_traits>
 
 #include "rk_device.h"
 #include "rk_sort.h"
@@ -1124,63 +1123,23 @@ constexpr uint32_t kFetchBoundFaces = 1u << 20;
 // fetched together.
 constexpr uint32_t kMemoryFaces = 1u << 22;
 
-// Between these many faces and from this many rays on, rays in array order that start
-// at different points are traced apart (kApart). With fewer rays, 14 waves per CU, what
-// bounds the trace is the wait per step, and one fetch is faster; with fewer faces the
-// L2 has them; with more, where each node is fetched past the L2 anyway, 4-5% is all
-// there is. 262,144 rays on 70,000 and 300,000 faces: together 182 and 372 us, apart 165
-// and 305; 196,608 on 300,000: 231 and 261. 2M on 300,000, 600,000 and 1M: together 2.48,
-// 3.24 and 3.94 ms, apart 1.92, 2.80 and 3.79.
-// A wave of one origin, as a picture's, fetches together, and 28 pictures of such trees
-// take 0.5-2% longer than with the plain kernel (the test's round trip). Both ways need
-// 89 registers if they may, and 20 waves per CU then cost pictures 5%: __launch_bounds__
-// holds them to 80.
-constexpr uint32_t kApartFaces = 3u << 14, kApartFacesEnd = 3u << 18, kApartRays = 7u << 15;
-
-// Whether the wave's rays start at one point.
-__device__ __forceinline__ bool one_origin(const float4* __restrict__ origins, uint32_t l, bool has_ray) {
-  const float4 o = has_ray ? origins[l] : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  const auto first = [](float x) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x))); };
-  return __ballot(o.x != first(o.x) || o.y != first(o.y) || o.z != first(o.z)) == 0ull;
-}
-
-// Ray l of this lane (when has_ray), traced and stored.
-template <bool kCount, int kWG, int kLds, bool kOldest, int kLeafBatch, int kDonateMin, int kBoundEvery, bool kApart>
-__device__ __forceinline__ void trace_lane(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
-                                           uint32_t n_tris, const float4* __restrict__ origins,
-                                           const float4* __restrict__ dirs, uint32_t l, bool has_ray,
-                                           uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
-                                           float* __restrict__ depths, float eps,
-                                           unsigned long long* __restrict__ counters, bool reset, uint2* stack,
-                                           uint32_t* xchg) {
-  uint32_t n_box = 0, n_tri = 0;
-  const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  const RayHit h = trace_ray_shared<kCount, kStack, kLds, kWG, kOldest, kLeafBatch, kDonateMin, kBoundEvery, kApart>(
-      nodes, tris, n_tris, 0u, has_ray, has_ray ? origins[l] : zero4, has_ray ? dirs[l] : zero4,
-      has_ray ? (reset ? RK_HUGE : depths[l]) : 0.0f, eps, n_box, n_tri, stack, xchg);
-  if (kCount) {
-    atomicAdd(counters, (unsigned long long)n_box);
-    atomicAdd(counters + 1, (unsigned long long)n_tri);
-  }
-  if (has_ray) {
-    if (h.pos != 0xFFFFFFFFu) {
-      faces_id[l] = h.pos;
-      coords[l] = make_float2(h.u, h.v);
-      depths[l] = h.t;
-    } else if (reset) {
-      depths[l] = RK_HUGE;  // the reset a fill kernel would have done; the miss's id and coords stay
-    }
-  }
-}
+// Sorted rays fetch leaves apart (kApart) from this many faces on. Which is better
+// depends on how much the rays hit. Sort and trace of 4M rays on soups of the same area
+// (about one hit in two), 20,000, 80,000, 150,000, 500,000 and 1M faces: together 2.12, 2.29,
+// 2.44, 2.98 and 3.64 ms, apart 2.25, 2.42, 2.53, 2.93 and 3.36. 2M rays on 70,000, 150,000 and
+// 300,000 small faces, of which few are hit: 1.10, 1.61 and 2.28 ms, apart 0.95, 1.29 and
+// 1.78. In array order all fetch together: pictures, which gain 2-30% from it, cannot
+// be told from rays that share no nodes (those lose up to 25% on 50,000 to 1M small
+// faces) but by a test of the waves' origins, which costs pictures 0.5-2%, and with both
+// loops in a kernel 3 registers spill, which costs rays that hit much 15%.
+constexpr uint32_t kApartFaces = 1u << 17;
 
 // kWG threads per workgroup, runs of kRun rays per band (spread_ray; 0: 64
 // consecutive rays per wave), kLds stack entries per lane in LDS. The
-// defaults above are one variant; rk_fast_autotune chooses among several. kFetch:
-// whether nodes and leaves are fetched together or apart, or by the wave's origins.
-enum Fetch { kTogether, kAlwaysApart, kByOrigin };
+// defaults above are one variant; rk_fast_autotune chooses among several.
 template <bool kCount, int kWG, uint32_t kRun, int kLds, bool kOldest = false, int kLeafBatch = 0, int kDonateMin = 1,
-          int kBoundEvery = 1, bool kXcdRuns = false, Fetch kFetch = kTogether>
-__global__ __launch_bounds__(kWG, kFetch == kByOrigin ? 6 : 1) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
+          int kBoundEvery = 1, bool kXcdRuns = false, bool kApart = false>
+__global__ __launch_bounds__(kWG) void k_fast_trace_v(const FNode* __restrict__ nodes, const float4* __restrict__ tris,
                                                       uint32_t n_tris, const float4* __restrict__ origins,
                                                       const float4* __restrict__ dirs, uint32_t n_rays,
                                                       uint32_t* __restrict__ faces_id, float2* __restrict__ coords,
@@ -1198,15 +1157,24 @@ __global__ __launch_bounds__(kWG, kFetch == kByOrigin ? 6 : 1) void k_fast_trace
   const bool has_ray = l < n_rays;
   __shared__ uint2 s_stack[kLds * kWG];
   __shared__ uint32_t s_xchg[kWG / 64][kXchgWords];
-  const auto go = [&](auto apart) {
-    trace_lane<kCount, kWG, kLds, kOldest, kLeafBatch, kDonateMin, kBoundEvery, decltype(apart)::value>(
-        nodes, tris, n_tris, origins, dirs, l, has_ray, faces_id, coords, depths, eps, counters, reset, s_stack,
-        s_xchg[threadIdx.x >> 6]);
-  };
-  if (kFetch == kAlwaysApart || (kFetch == kByOrigin && !one_origin(origins, l, has_ray)))
-    go(std::integral_constant<bool, kFetch != kTogether>());
-  else
-    go(std::integral_constant<bool, false>());
+  uint32_t n_box = 0, n_tri = 0;
+  const float4 zero4 = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  const RayHit h = trace_ray_shared<kCount, kStack, kLds, kWG, kOldest, kLeafBatch, kDonateMin, kBoundEvery, kApart>(
+      nodes, tris, n_tris, 0u, has_ray, has_ray ? origins[l] : zero4, has_ray ? dirs[l] : zero4,
+      has_ray ? (reset ? RK_HUGE : depths[l]) : 0.0f, eps, n_box, n_tri, s_stack, s_xchg[threadIdx.x >> 6]);
+  if (kCount) {
+    atomicAdd(counters, (unsigned long long)n_box);
+    atomicAdd(counters + 1, (unsigned long long)n_tri);
+  }
+  if (has_ray) {
+    if (h.pos != 0xFFFFFFFFu) {
+      faces_id[l] = h.pos;
+      coords[l] = make_float2(h.u, h.v);
+      depths[l] = h.t;
+    } else if (reset) {
+      depths[l] = RK_HUGE;  // the reset a fill kernel would have done; the miss's id and coords stay
+    }
+  }
 }
 
 inline unsigned blocks_for(uint32_t n, uint32_t per) { return (n + per - 1) / per; }
@@ -2270,13 +2238,8 @@ extern "C" rk_status rk_fast_trace(rk_stream stream, const rk_fast_bvh* bvh, con
   const TraceVariant* tv = trace_variant(options ? options->config : 0u);
   if (!tv) return RK_ERROR_INVALID_VALUE;
   TraceVariant v = *tv;
-  if (!options || options->config == 0) {
-    const uint32_t faces = bvh->face_count;
-    if (faces >= kMemoryFaces)
-      v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32>;
-    else if (faces >= kApartFaces && faces < kApartFacesEnd && n_rays >= kApartRays)
-      v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kLdsStack, false, 0, kTraceDonateMin, 1, false, kByOrigin>;
-  }
+  if ((!options || options->config == 0) && bvh->face_count >= kMemoryFaces)
+    v.kernel = k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32>;
   return launch_trace_variant(rk_hip_stream(stream), v, bvh, origins, directions, n_rays, faces_id, coords, depths,
                               det_eps_of(options), trace_flags_of(options));
 }
@@ -2403,10 +2366,12 @@ extern "C" rk_status rk_fast_trace_sorted(rk_stream stream, const rk_fast_bvh* b
   const TraceKernel kernel =
       !by_rule ? tv->kernel
       : bvh->face_count >= kFetchBoundFaces
-          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32, 1, true, kAlwaysApart>
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepestLdsStack, false, 0, 32, 1, true, true>
       : bvh->face_count >= kXcdFaces
-          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, true, kAlwaysApart>
-          : k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, false, kAlwaysApart>;
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, true, true>
+      : bvh->face_count >= kApartFaces
+          ? k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin, 1, false, true>
+          : k_fast_trace_v<false, kTraceWG, kSpreadRun, kDeepLdsStack, false, 0, kTraceDonateMin>;
   hipLaunchKernelGGL(kernel, dim3(blocks_for(n_rays, tv->wg)), dim3(tv->wg), 0, st, nodes,
                      static_cast<const float4*>(bvh->tris), bvh->face_count, o,
                      reinterpret_cast<const float4*>(directions), n_rays, faces_id, reinterpret_cast<float2*>(coords),
