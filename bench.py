@@ -76,17 +76,17 @@ TRACE_TRAFFIC_BYTES = (102_101 * 2 + 10_575) * 1024
 # (profiles/case_kernels.md).
 BUILD_KERNELS = {  # kernel: (us, HBM read KiB, HBM write KiB, launches per build)
     "heightfield": {
-        "k_fast_prep": (14.53, 26_740, 39_561, 1),
-        "k_rs_scatter": (16.44, 9_768, 10_169, 4),
-        "k_fast_hierarchy": (46.36, 47_530, 114_420, 1),
-        "k_hier_reduce": (16.61, 618, 777, 2),
+        "k_fast_prep": (14.82, 26_740, 39_561, 1),
+        "k_rs_scatter": (15.16, 9_768, 10_169, 4),
+        "k_fast_hierarchy": (46.48, 47_530, 114_420, 1),
+        "k_hier_reduce": (16.62, 618, 777, 2),
     },
     "soup": {
-        "k_fast_prep": (204.4, 625_130, 429_701, 1),
-        "k_rs_hist": (43.45, 78_300, 9_899, 1),
-        "k_rs_scatter": (63.01, 131_978, 135_924, 8),
-        "k_fast_hierarchy": (781.1, 2_926_534, 1_177_784, 1),
-        "k_hier_reduce": (20.42, 3_416, 4_688, 3),
+        "k_fast_prep": (204.2, 625_130, 429_701, 1),
+        "k_rs_hist": (42.99, 78_300, 9_899, 1),
+        "k_rs_scatter": (61.08, 131_978, 135_924, 8),
+        "k_fast_hierarchy": (783.6, 2_926_534, 1_177_784, 1),
+        "k_hier_reduce": (19.91, 3_416, 4_688, 3),
     },
 }
 HBM_PEAK_GBS = 8000.0

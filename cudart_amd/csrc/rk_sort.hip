@@ -12,7 +12,7 @@
 // Below 2^21 keys a pass is bound by latency, at most a few tiles per CU, and
 // the look-back has two levels: a tile adds the counts of the tiles before it
 // in its group of 16, all in flight at once, and looks back over groups (1M
-// pairs: 15.1 against 16.8 us per pass; with one level the prefixes advance 8
+// pairs: 15.2 against 16.8 us per pass; with one level the prefixes advance 8
 // tiles per round trip). Above, tiles queue on every CU and overlap each other.
 // Slower: ranks from eight ballots per key (158 against 155 us per 1M-face
 // build, 1613 against 1577 for 10M); wider digits, 10 bits (three passes for
