@@ -472,7 +472,8 @@ __device__ __forceinline__ uint32_t octant_of(float4 dir) {
 // The stack keeps the reference's 96 entries and its overflow rule; the first
 // kLdsStack entries of each lane live in LDS (entry e of lane x at
 // e * 64 + x), deeper ones in scratch (trees of depth <= 31 need at most 33),
-// so a CU holds 20 waves of this kernel instead of 6.
+// so a CU holds 16 waves of this kernel instead of 6, as its 101 registers allow (20,
+// with 7 spilled: no faster over 140 frames).
 //
 // A wave's rays are a tile of 16 x 4 pixels where that fills nearly all lanes
 // (tiled_rays), else 64 in a row: neighbours in the picture walk the same nodes
